@@ -12,15 +12,25 @@ import math
 import numpy as np
 import torch
 
-import bench
-
 pkg = importlib.import_module("cpp-tensorlib_amd")
 qwen = importlib.import_module("cpp-tensorlib_amd.qwen")
 model = importlib.import_module("cpp-tensorlib_amd.model")
 
 QWEN = {"0.5B": qwen.QWEN_05B, "7B": qwen.QWEN_7B}
 CONTEXT = {"0.5B": 2304, "7B": 4352}           # what a model is created for
-FOLDER = {"Lusadra": (bench.LUSADRA_SIZES, bench.lusadra_config), "Girirax": (bench.GIRIRAX_SIZES, bench.girirax_config)}
+# The folder designs at the sizes of bench.py. Lusadra: heads, key heads, head size and window of the attention; heads,
+# key and value size of the linear attention. Girirax (state-space and latent-attention layers in turn): heads, value
+# size, state and groups; heads, key, rotated, value size, latent and query rank.
+SIZES = {
+    "Lusadra": {
+        "small": dict(layers=12, vocab=32000, width=896, left=(14, 2, 64, 512), right=(7, 64, 128), ff=4864),
+        "medium": dict(layers=8, vocab=32000, width=2048, left=(16, 4, 128, 1024), right=(16, 64, 128), ff=8192),
+        "large": dict(layers=4, vocab=32000, width=3584, left=(28, 4, 128, 1024), right=(28, 64, 128), ff=18944)},
+    "Girirax": {
+        "small": dict(layers=12, vocab=32000, width=896, ssm=(28, 64, 128, 1), latent=(14, 64, 32, 64, 256, 384), ff=4864),
+        "medium": dict(layers=8, vocab=32000, width=2048, ssm=(64, 64, 128, 8), latent=(16, 128, 64, 128, 512, 768), ff=8192),
+        "large": dict(layers=4, vocab=32000, width=3584, ssm=(112, 64, 128, 8), latent=(28, 128, 64, 128, 512, 1536), ff=18944)},
+}
 RANK = 16                                        # of Lusadra's decay inputs
 
 
@@ -80,6 +90,27 @@ def draw(rng):
                     tb=rng.random() < 0.3)
     rows, cols = rng.choice([(4864, 896), (896, 4864), (3584, 3584), (18944, 3584), (3584, 18944)])
     return dict(kind=kind, rows=rows + rng.randint(-40, 40), cols=cols, to=rng.choice(["q4", "bf16"]))
+
+
+def _config(c):
+    """The config.json of a folder design."""
+    z = SIZES[c["design"]][c["size"]]
+    mlp = {"kind": "dense", "ff": z["ff"]}
+    base = {"architecture": c["design"], "vocab": z["vocab"], "width": z["width"], "norm": {"eps": 1e-6}}
+    if c["design"] == "Lusadra":
+        H, G, D, window = z["left"]
+        h, d, v = z["right"]
+        left = {"heads": H, "kv_heads": G, "dim": D, "vdim": D, "mask": {"size": window}, "scale": D ** -0.5,
+                "q_temp": {"coef": 0.1, "every": 1024}}
+        mixer = {"left": left, "right": {"heads": h, "dim": d, "vdim": v, "tau": 16.0}, "left_scale": 0.7, "right_scale": 0.7}
+        return dict(base, layers=[{"type": "parallel", "mixer": mixer, "mlp": mlp}] * z["layers"], loop=None)
+    h, p, n, g = z["ssm"]
+    H, D, R, V, L, Q = z["latent"]
+    ssm = {"heads": h, "vdim": p, "state": n, "groups": g, "conv": 4, "norm_groups": g}
+    att = {"heads": H, "dim": D, "rot_dim": R, "vdim": V, "kv_rank": L, "q_rank": Q, "scale": (D + R) ** -0.5,
+           "rot": {"base": 1e6, "dims": R}}
+    pair = [{"type": "mamba2", "mixer": ssm, "mlp": mlp}, {"type": "latent_attention", "mixer": att, "mlp": mlp}]
+    return dict(base, embedding={"scale": 4.0}, residual_mult=0.5, layers=pair * (z["layers"] // 2))
 
 
 # ---- what a program holds before the call -----------------------------------------------------------
@@ -151,9 +182,8 @@ def prepare(case, seed):
         s["tokens"] = _tokens(seed, c.get("tokens", 1), d["vocab"])
         return s
     if c["kind"] == "turn":
-        sizes, config = FOLDER[c["design"]]
-        z = sizes[c["size"]]
-        m = model.Model.random(config(z), seed=seed, rank=RANK, max_ctx=4096, chunk=512)
+        z = SIZES[c["design"]][c["size"]]
+        m = model.Model.random(_config(c), seed=seed, rank=RANK, max_ctx=4096, chunk=512)
         return dict(case=c, m=_Closing(m), tokens=_tokens(seed, c["prompt"] + c["tokens"], z["vocab"]))
     if c["kind"] == "attention":
         q, k, v = _attention_inputs(c, seed)
@@ -212,15 +242,17 @@ def _qwen_weights(d):
 def _turn_weights(c):
     """(weights of all layers, of the head, bytes of state a token reads and writes, numbers per cached position and
     the multiply-adds of a query with one of them, positions a query sees at most), over all layers."""
-    z = FOLDER[c["design"]][0][c["size"]]
+    z = SIZES[c["design"]][c["size"]]
     n, head = z["layers"], z["width"] * z["vocab"]
     if c["design"] == "Lusadra":
         H, G, D, window = z["left"]
         h, d, v = z["right"]
-        return n * bench.lusadra_weights(z), head, n * 8 * h * d * v, n * 4 * G * D, n * 2 * H * D, window
-    h, p, s, _ = z["ssm"]
-    H, D, R, V, L, _ = z["latent"]
-    return n // 2 * sum(bench.girirax_weights(z)), head, n // 2 * 8 * h * p * s, n // 2 * 2 * (L + R), n // 2 * H * (2 * L + R), 1 << 30
+        layer = z["width"] * (3 * H * D + G * D + 2 * h * d + 3 * h * v + RANK + 2 * z["ff"])
+        return n * layer, head, n * 8 * h * d * v, n * 4 * G * D, n * 2 * H * D, window
+    h, p, s, g = z["ssm"]
+    H, D, R, V, L, Q = z["latent"]
+    pair = z["width"] * (3 * h * p + 2 * g * s + h + Q + L + R + 2 * H * V + 6 * z["ff"]) + Q * H * (D + R) + L * H * (D + V)
+    return n // 2 * pair, head, n // 2 * 8 * h * p * s, n // 2 * 2 * (L + R), n // 2 * H * (2 * L + R), 1 << 30
 
 
 def work(case):
@@ -234,7 +266,7 @@ def work(case):
                 "flops": 2 * (d["n_layers"] * layer * T + head) + 4 * d["n_layers"] * d["n_q_heads"] * d["head_dim"] * seen}
     if c["kind"] == "turn":
         layers, head, state, row, query, most = _turn_weights(c)
-        P, N, vocab = c["prompt"], c["tokens"], FOLDER[c["design"]][0][c["size"]]["vocab"]
+        P, N, vocab = c["prompt"], c["tokens"], SIZES[c["design"]][c["size"]]["vocab"]
         bytes_ = (2 * (layers + head) + state) * (1 + N) + 4 * vocab * (1 + N)
         bytes_ += row * sum(min(p + 1, most) for p in range(P, P + N)) + row * P
         seen = sum(min(p + 1, most) for p in range(P + N))
@@ -411,8 +443,8 @@ def _lin(x, w):
     return torch.cat([x @ w[i:i + 16384].to(D64).T for i in range(0, len(w), 16384)], -1)
 
 
-def _lusadra_exact(z, tokens, seed):
-    cfg, S = bench.lusadra_config(z), _Stream(seed)
+def _lusadra_exact(c, z, tokens, seed):
+    cfg, S = _config(c), _Stream(seed)
     E, eps, T = z["width"], cfg["norm"]["eps"], len(tokens)
     layers = []
     for lc in cfg["layers"]:
@@ -459,8 +491,8 @@ def _lusadra_exact(z, tokens, seed):
     return _rms(x, eps) * onorm, head
 
 
-def _girirax_exact(z, tokens, seed):
-    cfg, S = bench.girirax_config(z), _Stream(seed)
+def _girirax_exact(c, z, tokens, seed):
+    cfg, S = _config(c), _Stream(seed)
     E, eps, T, mult = z["width"], cfg["norm"]["eps"], len(tokens), cfg["residual_mult"]
     layers = []
     for lc in cfg["layers"]:
@@ -531,9 +563,9 @@ def exact(case, seed):
     if c["kind"] in ("step", "prompt"):
         return _qwen_exact(c, seed)
     if c["kind"] == "turn":
-        z = FOLDER[c["design"]][0][c["size"]]
+        z = SIZES[c["design"]][c["size"]]
         tokens = _tokens(seed, c["prompt"] + c["tokens"], z["vocab"])
-        rows, head = (_lusadra_exact if c["design"] == "Lusadra" else _girirax_exact)(z, tokens, seed)
+        rows, head = (_lusadra_exact if c["design"] == "Lusadra" else _girirax_exact)(c, z, tokens, seed)
         return [v[None] for v in _lin(rows[c["prompt"] - 1:], head)]
     if c["kind"] == "attention":
         q, k, v = _attention_inputs(c, seed)
