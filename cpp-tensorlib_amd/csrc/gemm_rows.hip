@@ -1,0 +1,439 @@
+// Products of a few rows: C[M,N] = A[M,K] f32 . W[N,K]^T for a short prompt, W bf16 rows or int4 groups.
+//
+// What bounds it: with M of a few dozen the weight is read once and hardly reused, and what is left is the
+// chain of latencies of one block. gemm_bf16_nt_kernel (prefill.hip) walks K in slabs of 32 through LDS, two
+// barriers and one load round trip per slab: ten slabs were 20 us for weights that take 2 us to read. Here a
+// block has no barrier until its sums are complete: its eight wavefronts split the block's K range between
+// them (wavefront w takes the 32-k steps w, w + 8, ...), each with the WHOLE tile's accumulators, and loads
+// both operands straight into the registers of the MFMA that uses them, several steps ahead. The sums meet in
+// LDS once at the end, in a fixed order.
+//
+// Both operands of v_mfma_f32_16x16x32_bf16 are K-contiguous per lane: lane l supplies row l % 16 and k
+// 8 (l / 16) .. + 8 - one 16-byte load of a bf16 weight (64 contiguous bytes of every row), two of an f32
+// activation (128). Every activation is cut exactly into three bf16 terms in registers (gemm_bf16_nt_kernel's
+// arithmetic: exact products, fp32 sums). Tiles of 16 rows waste less of a ragged M than tiles of 32 or 64.
+//
+// int4: a lane's 16-byte load is the 32 weights of ONE scale group; four groups lie in the four lane quarters
+// and are traded (two swaps of lane halves, two of 16-lane rows, for four steps) so that a step multiplies one
+// group: its sums start at zero and join the accumulators times the group's scale, as in gemm_bf16_nt_kernel.
+#include <type_traits>
+
+#include "gemm_shared.hpp"
+
+namespace tlhip {
+namespace rows {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kWaves = 8, kStep = 32;
+constexpr int kMaxTM = 5;
+
+// Steps of activations in flight per wavefront (int4: a divisor of four): 2 KB of LDS per row tile each.
+__host__ __device__ constexpr int stages(int TM, bool q4) { return TM <= 2 ? 4 : TM == 3 && !q4 ? 3 : 2; }
+__host__ __device__ constexpr int lds_bytes(int TM, int TN, bool q4) {
+  const int ring = kWaves * stages(TM, q4) * TM * 2048, sums = 4 * 16 * TM * (16 * TN + 4) * 4;
+  return ring > sums ? ring : sums;
+}
+
+// 8 floats -> their three bf16 terms (by truncation: x = hi + mid + lo exactly for normal x)
+__device__ __forceinline__ void split3(const f32x4& x0, const f32x4& x1, frag16 p[3]) {
+  const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    const uint32_t u0 = __float_as_uint(x[2 * b]), u1 = __float_as_uint(x[2 * b + 1]);
+    const float r0 = x[2 * b] - __uint_as_float(u0 & 0xffff0000u), r1 = x[2 * b + 1] - __uint_as_float(u1 & 0xffff0000u);
+    const uint32_t m0 = __float_as_uint(r0), m1 = __float_as_uint(r1);
+    const float s0 = r0 - __uint_as_float(m0 & 0xffff0000u), s1 = r1 - __uint_as_float(m1 & 0xffff0000u);
+    p[0][b] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+    p[1][b] = __builtin_amdgcn_perm(m1, m0, 0x07060302u);
+    p[2][b] = __builtin_amdgcn_perm(__float_as_uint(s1), __float_as_uint(s0), 0x07060302u);
+  }
+}
+
+// 8 nibbles (k ascending, value = nibble - 8) -> 8 bf16, exact
+__device__ __forceinline__ frag16 nib8(uint32_t w) {
+  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;   // even k, odd k
+  frag16 o;
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    const float e = (float)((lo >> (8 * b)) & 0xffu) - 8.0f, d = (float)((hi >> (8 * b)) & 0xffu) - 8.0f;
+    o[b] = __builtin_amdgcn_perm(__float_as_uint(d), __float_as_uint(e), 0x07060302u);
+  }
+  return o;
+}
+
+__device__ __forceinline__ f32x4 mma(const frag16& a, const frag16& b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Grid: x = row blocks (fastest) x column tiles, y = K-split parts of `part_units` units (bf16: steps of 32 k,
+// int4: 128 k); part y goes to C + y * M * ldc. N, ff, GU and the order of a gated tile's columns as in
+// gemm_bf16_nt_kernel: a tile's first 8 TN columns are gate features, the rest the same features' up rows.
+template <int TM, int TN, bool GU, bool Q4>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* __restrict__ A, const void* __restrict__ W,
+                                                                  const float* __restrict__ scales, float* __restrict__ C,
+                                                                  int M, int N, int K, int part_units, int ldc, int ff,
+                                                                  int row_blocks) {
+  constexpr int BM = 16 * TM, BN = 16 * TN, LD = BN + 4;
+  constexpr int ST = stages(TM, Q4), kSlot = TM * 2048;
+  extern __shared__ __attribute__((aligned(1024))) float red[];   // activations in flight, then [4][BM][LD] sums
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, quarter = lane >> 4;
+  // one contiguous run of tiles per XCD, row blocks fastest: those share a weight tile in one L2
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
+  const int lid = xcd * q8 + min(xcd, r8) + within;
+  const int m0 = lid % row_blocks * BM, n0 = lid / row_blocks * BN;
+  C += (size_t)blockIdx.y * M * ldc;
+  const int units = Q4 ? K / 128 : K / kStep, ubeg = blockIdx.y * part_units, uend = min(units, ubeg + part_units);
+  const int first = ubeg + wave, mine = first < uend ? (uend - first + kWaves - 1) / kWaves : 0;
+
+  // byte offsets of this lane's rows (clamped into the operands: what lies past an edge is not stored). A 1 KB copy
+  // of activations is eight rows of 128 bytes, the 16-byte chunks of row r in the order c ^ (r & 7), which spreads
+  // the fragment reads (16 rows, one chunk) over the LDS banks.
+  uint32_t aoff[TM][2], woff[TN], soff[Q4 ? TN : 1];
+#pragma unroll
+  for (int t = 0; t < TM; t++)
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      aoff[t][h] = (uint32_t)min(m0 + 16 * t + 8 * h + (lane >> 3), M - 1) * (uint32_t)(K * 4) + ((lane & 7) ^ (lane >> 3)) * 16;
+  const int frag[2] = {r16 * 128 + ((2 * quarter) ^ (r16 & 7)) * 16, r16 * 128 + ((2 * quarter + 1) ^ (r16 & 7)) * 16};
+  char* ring = reinterpret_cast<char*>(red) + wave * (ST * kSlot);
+#pragma unroll
+  for (int j = 0; j < TN; j++) {
+    const int col = 16 * j + r16;
+    int r;
+    if (GU) {
+      const int f = min((n0 >> 1) + col % (BN / 2), N - 1);
+      r = f + (col >= BN / 2 ? ff : 0);
+    } else {
+      r = min(n0 + col, N - 1);
+    }
+    woff[j] = (uint32_t)r * (uint32_t)(Q4 ? K / 2 : K * 2) + quarter * 16;
+    if (Q4) soff[j] = (uint32_t)r * (uint32_t)(K / 8);
+  }
+  const char* Ab = reinterpret_cast<const char*>(A);
+  const char* Wb = static_cast<const char*>(W);
+  const char* Sb = reinterpret_cast<const char*>(scales);
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int t = 0; t < TM; t++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  if (mine > 0) {
+    auto load_a = [&](int u, uint32_t step) {      // u: slot, step: of 32 k
+#pragma unroll
+      for (int t = 0; t < TM; t++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(Ab + (aoff[t][h] + step * 128u)),
+                                           (__attribute__((address_space(3))) void*)(ring + u * kSlot + t * 2048 + h * 1024), 16, 0, 0);
+    };
+    // all but my youngest `n` loads have landed (copies into LDS are waited for by count: the compiler does not see them)
+    auto landed = [](auto n) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory"); };
+    auto cut = [&](int u, int t, frag16 p[3]) {
+      const char* at = ring + u * kSlot + t * 2048;
+      split3(*reinterpret_cast<const f32x4*>(at + frag[0]), *reinterpret_cast<const f32x4*>(at + frag[1]), p);
+    };
+    if constexpr (!Q4) {
+      frag16 w[ST][TN];
+      auto load = [&](int u, int i) {              // slot u takes my i-th step
+        const uint32_t step = (uint32_t)(first + kWaves * i);
+        load_a(u, step);
+#pragma unroll
+        for (int j = 0; j < TN; j++) w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + step * 64u));
+        __builtin_amdgcn_sched_barrier(0);         // (else the compiler gathers the loads of all slots behind the last one's products)
+      };
+      auto compute = [&](int u) {
+#pragma unroll
+        for (int t = 0; t < TM; t++) {
+          frag16 p[3];
+          cut(u, t, p);
+#pragma unroll
+          for (int e = 0; e < 3; e++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[t][j] = mma(p[e], w[u][j], acc[t][j]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      // every load is of a step that exists: one past the end would cost what a real one costs
+      int it = 0;
+#pragma unroll
+      for (int u = 0; u < ST; u++)
+        if (u < mine) load(u, u);
+      for (; it + 2 * ST <= mine; it += ST) {
+#pragma unroll
+        for (int u = 0; u < ST; u++) {
+          landed(std::integral_constant<int, (ST - 1) * (2 * TM + TN)>{});
+          compute(u);
+          load(u, it + u + ST);
+        }
+      }
+      landed(std::integral_constant<int, 0>{});
+#pragma unroll
+      for (int u = 0; u < ST; u++) {
+        if (it + u < mine) compute(u);
+        if (it + u + ST < mine) load(u, it + u + ST);
+      }
+      landed(std::integral_constant<int, 0>{});
+#pragma unroll
+      for (int u = 0; u < ST; u++)
+        if (it + u + ST < mine) compute(u);
+    } else {
+      // a unit is four steps; W and the scales of the next unit and the activations of the next steps are on
+      // their way while one is multiplied
+      frag16 w[2][TN];
+      f32x4 s[2][TN];
+      auto load_w = [&](int u, int i) {
+        const uint32_t unit = (uint32_t)(first + kWaves * i);
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + unit * 64u));
+          s[u][j] = *reinterpret_cast<const f32x4*>(Sb + (soff[j] + unit * 16u));
+        }
+      };
+      auto step_of = [&](int i) { return (uint32_t)(4 * (first + kWaves * (i >> 2)) + (i & 3)); };   // my i-th step: 4 per unit
+      // words of four groups -> one word of each of the four quarters' groups: afterwards w[u][j][g] is the eight
+      // weights of group g that this lane's quarter multiplies
+      auto trade = [&](int u) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          uint32_t x[4] = {w[u][j][0], w[u][j][1], w[u][j][2], w[u][j][3]};
+          auto y = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
+          x[0] = y[0]; x[2] = y[1];
+          y = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
+          x[1] = y[0]; x[3] = y[1];
+          y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+          x[0] = y[0]; x[1] = y[1];
+          y = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
+          x[2] = y[0]; x[3] = y[1];
+          w[u][j] = frag16{x[0], x[1], x[2], x[3]};
+        }
+      };
+      auto compute = [&](int u, int g) {           // group g of the unit in slot u
+        frag16 b[TN];
+#pragma unroll
+        for (int j = 0; j < TN; j++) b[j] = nib8(w[u][j][g]);
+#pragma unroll
+        for (int t = 0; t < TM; t++) {
+          frag16 p[3];
+          cut(g % ST, t, p);
+          f32x4 grp[TN];
+#pragma unroll
+          for (int e = 0; e < 3; e++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) grp[j] = mma(p[e], b[j], e == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : grp[j]);
+#pragma unroll
+          for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[t][j][v] = fmaf(grp[j][v], s[u][j][g], acc[t][j][v]);
+          if (TM >= 3) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      // unit `it` in slot u; `more`: the next unit exists (its activations follow in), `far`: the one after it too
+      auto unit = [&](int u, int it, auto steady) {
+        const bool more = decltype(steady)::value || it + 1 < mine, far = decltype(steady)::value || it + 2 < mine;
+        trade(u);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          // younger than this step's activations: those of ST - 1 steps, and the unit of weights issued between
+          if (!decltype(steady)::value) landed(std::integral_constant<int, 0>{});
+          else if (g == 0) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
+          else if (g == 1) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
+          else if (ST == 4) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
+          else landed(std::integral_constant<int, (ST - 1) * 2 * TM>{});
+          compute(u, g);
+          if (g + ST < 4 || more) load_a(g % ST, step_of(4 * it + g + ST));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (far) load_w(u, it + 2);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      load_w(0, 0);
+      if (mine > 1) load_w(1, 1);
+#pragma unroll
+      for (int u = 0; u < ST; u++) load_a(u, step_of(u));
+      __builtin_amdgcn_sched_barrier(0);
+      int it = 0;
+      if (mine > 3) {                              // (the first unit's weights were not issued between its activations: no count)
+        unit(0, 0, std::false_type{});
+        it = 1;
+        for (; it + 3 < mine; it += 2) {
+          unit(1, it, std::true_type{});
+          unit(0, it + 1, std::true_type{});
+        }
+        unit(1, it, std::false_type{});
+        it++;
+      }
+      for (; it < mine; it++) {
+        if ((it & 1) == 0) unit(0, it, std::false_type{});
+        else unit(1, it, std::false_type{});
+      }
+    }
+  }
+
+  // acc[t][j][v] of lane l: row 16 t + 4 (l / 16) + v, column 16 j + l % 16. Wavefronts 4..7 hand theirs to 0..3,
+  // whose four sums everyone then adds up.
+  auto put = [&](float* dst) {
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) dst[(16 * t + 4 * quarter + v) * LD + 16 * j + r16] = acc[t][j][v];
+  };
+  __syncthreads();                                 // (the sums take the place of activations that other wavefronts read)
+  float* slot = red + (size_t)(wave & 3) * BM * LD;
+  if (wave >= 4) put(slot);
+  __syncthreads();
+  if (wave < 4) {
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[t][j][v] += slot[(16 * t + 4 * quarter + v) * LD + 16 * j + r16];
+    put(slot);                                     // (the lane's own entries: nobody else reads them before the barrier)
+  }
+  __syncthreads();
+  const bool wide = (ldc & 3) == 0;
+  auto total = [&](int row, int col) {
+    f32x4 x[4];
+#pragma unroll
+    for (int w4 = 0; w4 < 4; w4++) x[w4] = *reinterpret_cast<const f32x4*>(red + ((size_t)w4 * BM + row) * LD + col);
+    return (x[0] + x[1]) + (x[2] + x[3]);
+  };
+  auto store = [&](float* dst, const f32x4& o, int left) {
+    if (wide && left >= 4) {
+      *reinterpret_cast<f32x4*>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (e < left) dst[e] = o[e];
+    }
+  };
+  if (GU && gridDim.y == 1) {
+    for (int i = tid; i < BM * (BN / 8); i += 64 * kWaves) {
+      const int row = i / (BN / 8), c = i % (BN / 8) * 4, gm = m0 + row, f = (n0 >> 1) + c;
+      if (gm >= M || f >= N) continue;
+      const f32x4 g = total(row, c), u = total(row, c + BN / 2);
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] = (g[e] * (1.0f / (1.0f + expf(-g[e])))) * u[e];   // swiglu_kernel's arithmetic
+      store(C + (size_t)gm * ldc + f, o, N - f);
+    }
+    return;
+  }
+  for (int i = tid; i < BM * (BN / 4); i += 64 * kWaves) {
+    const int row = i / (BN / 4), c = i % (BN / 4) * 4, gm = m0 + row, gn = n0 + c;
+    if (gm >= M || (!GU && gn >= N)) continue;     // gated parts are whole tiles wide
+    store(C + (size_t)gm * ldc + gn, total(row, c), GU ? 4 : N - gn);
+  }
+}
+
+template <int TM, int TN, bool GU, bool Q4>
+int run(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int M, int N, int K, int ldc, int ff) {
+  constexpr int lds = lds_bytes(TM, TN, Q4);
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows_kernel<TM, TN, GU, Q4>),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
+  gemm_rows_kernel<TM, TN, GU, Q4><<<dim3((unsigned)(P.tiles * P.row_blocks), (unsigned)P.S), dim3(64 * kWaves), lds, ctx().stream>>>(
+      A, W, scales, C, M, N, K, P.part_units, ldc, ff, P.row_blocks);
+  return TLHIP_OK;
+}
+
+template <int TM>
+int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int M, int N, int K, int ldc, int ff, bool gu) {
+  const bool q4 = scales != nullptr;
+  switch (P.TN + (gu ? 16 : 0) + (q4 ? 32 : 0)) {   // (int4 over four column tiles: the registers hold one row tile)
+    case 1: return run<TM, 1, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 2: return run<TM, 2, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 4: return run<TM, 4, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 18: return run<TM, 2, true, false>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 20: return run<TM, 4, true, false>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 33: return run<TM, 1, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 34: return run<TM, 2, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 36:
+      if constexpr (TM == 1) return run<TM, 4, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      break;
+    case 50: return run<TM, 2, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 52:
+      if constexpr (TM == 1) return run<TM, 4, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      break;
+  }
+  return fail(TLHIP_EUNSUPPORTED, "gemm_rows: no kernel for this plan");
+}
+
+}  // namespace rows
+
+// Row tiles per block, columns per tile and K splits that an estimate of the time likes best; S == 0 where
+// gemm_bf16_nt_kernel is the better one or the shape is not taken.
+//
+// The estimate, fitted to 280 runs (K 384 .. 18944, N 384 .. 37888, M 8 .. 120; rms error 24 %): a step of a block's
+// eight wavefronts takes the CU's vector memory path 35 clocks per KB of activations and 60 per KB of weights (whose
+// lanes cover 16 rows each), or its SIMDs, with two wavefronts each, the clocks of their matrix or vector
+// instructions (5.5 per element cut, 23 per eight nibbles; int4 measured 1.8 times that); a block starts and ends in
+// 3500 clocks and 60 per accumulator tile; a launch costs 2 us.
+// The other kernel, measured over the same shapes: 6 us and 0.4 us per 32-k slab (1.0 with two blocks on a CU) up to 64
+// rows, above that 17 us and 0.35 (0.8). It is kept where its 128 x 256 tiles pay: products of more than a few rows
+// whose weight keeps every CU busy for several rounds (M = 64, 4608 x 3584: 14.9 us against 16.8 here).
+// Measured, us, other kernel -> this one: 896 x 896 at 5 / 37 / 77 rows 10.5 / 10.0 / 20.5 -> 3.6 / 3.7 / 4.4; 4864 x 896
+// gated 14.4 / 16.0 / 25.4 -> 7.8 / 11.1 / 13.4; 896 x 4864 11.0 / 11.4 / 21.7 -> 4.9 / 7.0 / 9.6; 18944 x 3584 gated
+// 111 / 111 -> 63 / 92; int4 119 / 127 -> 53 / 93.
+RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S) {
+  using rows::kMaxTM;
+  RowsPlan best;
+  const int64_t rows_w = (gu ? 2 : 1) * N;
+  if (M > 128 || K % (q4 ? 128 : 32) != 0 || M * K * 4 >= (int64_t(1) << 32) || rows_w * K * (q4 ? 1 : 4) / 2 >= (int64_t(1) << 32))
+    return best;                                   // (32-bit byte offsets)
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t t16 = cdiv(M, 16), cus = ctx().cus, units = K / (q4 ? 128 : 32), steps = q4 ? 4 : 1;
+  best.row_blocks = (int)cdiv(t16, kMaxTM);
+  const int TM = best.TM = (int)cdiv(t16, best.row_blocks);
+  double least = 0;
+  for (int TN = q4 && TM > 1 ? 2 : 4; TN >= (gu ? 2 : 1); TN /= 2) {   // (what the registers hold)
+    const int64_t tiles = cdiv(rows_w, 16 * TN);
+    for (int64_t S = 1; S <= std::min<int64_t>(max_S, units); S++) {
+      const int64_t per = cdiv(units, S), blocks = tiles * best.row_blocks * S;
+      if (cdiv(units, per) != S) continue;
+      const double n = (double)(cdiv(per, rows::kWaves) * steps);    // steps of a wavefront
+      const double mem = 8 * (70.0 * TM + (q4 ? 30.0 : 60.0) * TN);
+      const double math = 2 * (q4 ? 1.8 * std::max(48.0 * TM * TN, 176.0 * TM + TN * (92.0 + 16 * TM)) : std::max(48.0 * TM * TN, 176.0 * TM));
+      const double rounds = blocks <= 2 * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus;
+      double us = 2 + rounds * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100;
+      // parts written and read, and, gated, their launch (a plain product is planned like one left as parts, whose sum
+      // its consumer forms: the two are the same bits)
+      if (S > 1) us += (double)S * M * rows_w * 4 / 4e6 + (gu ? 5 : 0);
+      if (best.S == 0 || us < least) {
+        least = us;
+        best.TN = TN;
+        best.S = (int)S;
+        best.tiles = (int)tiles;
+        best.part_units = (int)per;
+      }
+    }
+  }
+  if (M > 16) {
+    const int64_t bm = M > 64 ? 128 : 64, bn = M > 64 && !q4 ? 256 : 128, tiles = cdiv(M, bm) * cdiv(rows_w, bn), slabs = K / 32;
+    const int64_t S = std::max<int64_t>(1, std::min(std::min<int64_t>(max_S, 2 * cus / tiles), slabs / 8));
+    const double other = M > 64 ? 17 + (double)slabs / S * (tiles * S <= 96 ? 0.35 : 0.8) : 6 + (double)slabs / S * (tiles * S <= cus ? 0.4 : 1.0);
+    if (other + (gu && S > 1 ? 5 : 0) < least) best.S = 0;
+  }
+  return best;
+}
+
+int launch_gemm_rows(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K,
+                     int64_t ldc, bool gu) {
+  switch (P.TM) {
+    case 1: return rows::run_tm<1>(P, A, W, scales, C, (int)M, (int)N, (int)K, (int)ldc, (int)N, gu);
+    case 2: return rows::run_tm<2>(P, A, W, scales, C, (int)M, (int)N, (int)K, (int)ldc, (int)N, gu);
+    case 3: return rows::run_tm<3>(P, A, W, scales, C, (int)M, (int)N, (int)K, (int)ldc, (int)N, gu);
+    case 4: return rows::run_tm<4>(P, A, W, scales, C, (int)M, (int)N, (int)K, (int)ldc, (int)N, gu);
+    case 5: return rows::run_tm<5>(P, A, W, scales, C, (int)M, (int)N, (int)K, (int)ldc, (int)N, gu);
+  }
+  return fail(TLHIP_EUNSUPPORTED, "gemm_rows: no kernel for this plan");
+}
+
+}  // namespace tlhip

@@ -10,6 +10,15 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t frag16 __attribute__((ext_vector_type(4)));   // eight 16-bit operands of one lane
 
+// gemm_rows.hip: products of a few rows. S == 0: not a shape it takes.
+struct RowsPlan {
+  int TM = 0, TN = 0, S = 0, tiles = 0, row_blocks = 0, part_units = 0;
+};
+// max_S: the most K splits allowed
+RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S);
+int launch_gemm_rows(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K,
+                     int64_t ldc, bool gu);
+
 // defined in prefill.hip
 __global__ void splitk_sum_kernel(const float4* __restrict__ part, float4* __restrict__ C, int M, int n4,
                                   int ldc4, int S);

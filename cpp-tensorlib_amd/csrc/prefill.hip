@@ -481,6 +481,18 @@ using namespace tlhip;
 
 extern "C" {
 
+// C[M][n] (rows ldc apart) = the sum of the S parts [M][part_w]; half > 0: gated parts, strips of `half`
+// gate features followed by their up values.
+static void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t part_w, int64_t ldc, int S, int half) {
+  const dim3 grid((unsigned)(((size_t)M * n / 4 + 255) / 256));
+  if (half > 0)
+    splitk_sum_swiglu_kernel<<<grid, dim3(256), 0, ctx().stream>>>(reinterpret_cast<const float4*>(parts), reinterpret_cast<float4*>(C), (int)M,
+                                                                   (int)(n / 4), (int)(part_w / 4), (int)(ldc / 4), S, half / 4);
+  else
+    splitk_sum_kernel<<<grid, dim3(256), 0, ctx().stream>>>(reinterpret_cast<const float4*>(parts), reinterpret_cast<float4*>(C), (int)M,
+                                                            (int)(n / 4), (int)(ldc / 4), S);
+}
+
 // Three forms of one launcher.
 //   plain: C[M][N] is the product.
 //   parts (S_out != nullptr): the K-split parts are the result - C is then the caller's buffer,
@@ -523,6 +535,21 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   const int64_t slots = (int64_t)c.cus * 2;
   const int per = gu ? 2 : 1;                             // tile columns per unit of N
   const bool can_split = (N % 4) == 0 && aligned16(C);   // the part sum works on float4s
+  if (aligned16(C)) {   // a few rows: a kernel of their own
+    int64_t max_S = can_split ? 16 : 1;
+    if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
+    const RowsPlan P = plan_gemm_rows(M, N, K, gu, q4, max_S);
+    if (P.S > 0) {
+      const bool sum = P.S > 1 && !want_parts;
+      const int64_t part_w = gu ? (int64_t)P.tiles * 16 * P.TN : N;
+      float* dst = sum ? static_cast<float*>(scratch((size_t)P.S * M * part_w * sizeof(float))) : pc;
+      if (!dst) return fail(TLHIP_ENOMEM, "tlhip_gemm_bf16_nt: no scratch for K-split parts");
+      if (want_parts) *S_out = P.S;
+      if (int rc = launch_gemm_rows(P, pa, W, static_cast<const float*>(scales), dst, M, N, K, sum ? part_w : N, gu)) return rc;
+      if (sum) launch_part_sum(dst, pc, M, N, part_w, N, P.S, gu ? 8 * P.TN : 0);
+      TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+    }
+  }
   const bool half = q4 && M > 64 && c.tune_gemm_planes != 3;
   const size_t ea_bytes = half ? (((size_t)M * sizeof(int) + 255) & ~(size_t)255) : 0;
   struct Piece { int64_t n0, n; int S; int variant; };    // columns (features) [n0, n0 + n)
@@ -623,18 +650,7 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
       default: return fail(TLHIP_EUNSUPPORTED, "tlhip_gemm_bf16_nt: no kernel for this plan");
     }
 #undef TLHIP_GEMM
-    if (S > 1 && !want_parts) {
-      const size_t total4 = (size_t)M * P.n / 4;
-      const dim3 sgrid((unsigned)((total4 + 255) / 256));
-      if (gu)
-        splitk_sum_swiglu_kernel<<<sgrid, dim3(256), 0, c.stream>>>(
-            reinterpret_cast<const float4*>(dst), reinterpret_cast<float4*>(pc + P.n0), (int)M,
-            (int)(P.n / 4), (int)(part_w / 4), (int)(N / 4), S, bn / 4 / 4);
-      else
-        splitk_sum_kernel<<<sgrid, dim3(256), 0, c.stream>>>(
-            reinterpret_cast<const float4*>(dst), reinterpret_cast<float4*>(pc + P.n0), (int)M,
-            (int)(P.n / 4), (int)(N / 4), S);
-    }
+    if (S > 1 && !want_parts) launch_part_sum(dst, pc + P.n0, M, P.n, part_w, N, S, gu ? bn / 4 : 0);
   }
   TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
 }

@@ -1,0 +1,84 @@
+"""GPU parity: the products of a few rows (csrc/gemm_rows.hip) at the edges of their tiles: rows around the 16-row
+tiles and the blocks of up to five of them, columns that fill no tile, K of one step, of fewer steps than wavefronts and
+of several rounds, both weight formats, plain, gated and left as K-split parts.
+
+Every product is compared with float64. A sum of n fp32 additions is off by at most n 2^-24 of the sum of its terms'
+magnitudes; here n is three terms per 32-k step of a wavefront's chain, the 32 products inside an instruction and the
+eight wavefronts' sums."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 16, 128), (2, 33, 128), (5, 200, 256), (16, 896, 896), (17, 130, 128), (37, 1152, 896), (64, 64, 3584),
+          (65, 100, 128), (77, 896, 4864), (80, 36, 2048), (81, 260, 384), (97, 128, 896), (128, 72, 640)]
+
+
+def _weights(orc, fmt, N, K, seed):
+    """(device bytes, float64 values) of an [N, K] weight."""
+    if fmt == "bf16":
+        w = orc.to_bf16(orc.normal(N * K, seed, std=0.02)).reshape(N, K)
+        return w, orc.bf16_widen(w).reshape(N, K).astype(np.float64)
+    rng = np.random.default_rng(seed)
+    packed = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    scales = rng.uniform(0.002, 0.006, (N, K // 32)).astype(np.float32)
+    nib = np.stack([packed & 15, packed >> 4], -1).reshape(N, K // 32, 32).astype(np.float64) - 8
+    return np.concatenate([packed.ravel(), scales.ravel().view(np.uint8)]), (nib * scales[:, :, None]).reshape(N, K)
+
+
+def _slack(A, W, K):
+    return (3 * K / 32 + 40) * 2.0 ** -24 * (np.abs(A) @ np.abs(W).T)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "q4"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_plain_and_parts(lib, orc, fmt, M, N, K):
+    print("case gemm_rows", fmt, M, N, K, flush=True)
+    A = orc.normal(M * K, 21).reshape(M, K)
+    w, W = _weights(orc, fmt, N, K, 22)
+    want, slack = A.astype(np.float64) @ W.T, _slack(A.astype(np.float64), W, K)
+    da, dw = lib.to_device(A), lib.to_device(w)
+    out, parts = lib.to_device(np.full((M, N), np.nan, np.float32)), lib.to_device(np.full((16, M, N), np.nan, np.float32))
+    if fmt == "bf16":
+        lib.gemm_bf16_nt(da, dw, out, M, N, K)
+        n = lib.gemm_bf16_nt_parts(da, dw, parts, M, N, K)
+    else:
+        lib.gemm_q4_nt(da, dw, out, M, N, K)
+        n = lib.gemm_q4_nt_parts(da, dw, parts, M, N, K)
+    assert 1 <= n <= 16
+    assert np.all(np.abs(out.numpy() - want) <= slack)
+    got = parts.numpy()
+    assert np.all(np.abs(got[:n].astype(np.float64).sum(0) - want) <= slack)
+    assert np.isnan(got[n:]).all()                 # nothing written past the parts
+    for b in (da, dw, out, parts):
+        b.free()
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "q4"])
+@pytest.mark.parametrize("M,ff,K", [(1, 8, 128), (5, 4864, 896), (16, 100, 128), (33, 31, 256), (77, 4864, 896), (81, 200, 384), (128, 17, 128)])
+def test_gated(lib, orc, fmt, M, ff, K):
+    print("case gemm_rows gated", fmt, M, ff, K, flush=True)
+    A = orc.normal(M * K, 23).reshape(M, K)
+    w, W = _weights(orc, fmt, 2 * ff, K, 24)
+    p, s = A.astype(np.float64) @ W.T, _slack(A.astype(np.float64), W, K)
+    g, u, sg, su = p[:, :ff], p[:, ff:], s[:, :ff], s[:, ff:]
+    act = g / (1 + np.exp(-g))
+    da, dw, out = lib.to_device(A), lib.to_device(w), lib.to_device(np.full((M, ff), np.nan, np.float32))
+    (lib.gemm_bf16_nt_swiglu if fmt == "bf16" else lib.gemm_q4_nt_swiglu)(da, dw, out, M, ff, K)
+    # the slope of x sigmoid(x) is below 1.1; the gate itself costs a few roundings
+    assert np.all(np.abs(out.numpy() - act * u) <= 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u))
+    for b in (da, dw, out):
+        b.free()
+
+
+def test_whole_numbers_are_exact_and_columns_land_where_they_belong(lib, orc):
+    """Integer operands give exact integers whatever the order of the sums; every entry of the result differs."""
+    rng = np.random.default_rng(31)
+    for M, N, K in ((5, 70, 96), (40, 300, 160), (77, 896, 512), (96, 1000, 1024)):
+        A = rng.integers(-300, 300, (M, K)).astype(np.float32) + 0.5
+        Wf = rng.integers(-60, 60, (N, K)).astype(np.float32)
+        da, dw, out = lib.to_device(A), lib.to_device(orc.to_bf16(Wf).reshape(N, K)), lib.empty((M, N))
+        lib.gemm_bf16_nt(da, dw, out, M, N, K)
+        assert np.array_equal(out.numpy().astype(np.float64), A.astype(np.float64) @ Wf.astype(np.float64).T), (M, N, K)
+        for b in (da, dw, out):
+            b.free()
