@@ -14,6 +14,8 @@
 // 4 wavefronts (2 x 2) per block, 128 x 128 block tile, 64 x 64 per wavefront (2 x 2 MFMA
 // tiles, 64 accumulator registers), K slabs of 16; the next slab's global loads are in
 // flight while the current one is multiplied.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace tlhip {
@@ -202,6 +204,235 @@ int launch_sgemm_mfma(const float* pa, int64_t lda, int ta, const float* pb, int
   if (S > 1) {
     const size_t n = (size_t)M * N;
     sgemm_sum_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(dst, pc, n, S, scale, offset, epi);
+  }
+  return 0;
+}
+
+// ---- up to a few hundred rows -----------------------------------------------------------------------------
+// C[M,N] = A[M,K] . op(B) without LDS in the loop: the eight wavefronts of a block split its K range between them
+// (wavefront w takes the 16-k steps w, w + 8, ...), each with the whole 16 TM x 64 tile's accumulators, and both operands
+// go from memory into the registers of v_mfma_f32_16x16x4_f32 that uses them, ST steps ahead; the sums meet in LDS
+// once, in a fixed order. Lane l supplies row l % 16 of A and, of its quarter q = l / 16, the k 4 q .. 4 q + 3 of a step
+// as one 16-byte load, one number per product; B is read four columns wide ([K][N]: columns 4 (l % 16) + j, rows
+// 4 q + s, whole 256-byte runs) or like A ([N][K]).
+// What bounds it: below about 64 rows reading B, above that the matrix pipe (32 clocks per 2048 operations; 60 to 80 of its
+// 157 TFLOP/s, which is also what the LDS-tiled kernel above reaches). That one has two barriers per 16 k and reads
+// ragged tiles element by element, the vector-ALU kernel of fewer than 128 rows had no K split at all. us, before ->
+// now: 5 x 4864 x 896 164 -> 8.6, 5 x 896 x 4864 865 -> 10.7, 64 x 3584 x 3584 767 -> 32, 158 x 1153 x 901 41 -> 13,
+// 333 x 4864 x 896 66 -> 47, 450 x 4608 x 3589 260 -> 218.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // rows need not be 16-byte aligned
+
+constexpr int kSrWaves = 8, kSrStep = 16, kSrBN = 64, kSrLD = kSrBN + 4;
+
+template <int TM, int TB>
+__global__ __launch_bounds__(64 * kSrWaves, 2) void sgemm_rows_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ B,
+                                                                      int64_t ldb, float* __restrict__ C, int M, int N, int K, float scale,
+                                                                      float offset, int epi, int kchunk, int row_blocks) {
+  constexpr int BM = 16 * TM, ST = TM <= 2 ? 4 : 3;
+  extern __shared__ __attribute__((aligned(16))) float sums[];
+  float (*red)[BM][kSrLD] = reinterpret_cast<float (*)[BM][kSrLD]>(sums);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, quarter = lane >> 4;
+  // one contiguous run of tiles per XCD, row blocks fastest: they read the same columns of B
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
+  const int lid = xcd * q8 + min(xcd, r8) + within;
+  const int m0 = lid % row_blocks * BM, n0 = lid / row_blocks * kSrBN;
+  const int kbeg = blockIdx.y * kchunk, kend = min(K, kbeg + kchunk);
+  C += (size_t)blockIdx.y * M * N;                 // K-split parts are dense
+  // whole steps, the first `whole` of this block's range; what is left of K is one ragged step
+  const int steps = (kend - kbeg) / kSrStep, mine = wave < steps ? (steps - wave + kSrWaves - 1) / kSrWaves : 0;
+  const bool edge = n0 + kSrBN > N;                // (the block's last columns are read one by one, clamped)
+
+  const float *arow[TM], *bcol[TB ? 4 : 1];
+#pragma unroll
+  for (int t = 0; t < TM; t++) arow[t] = A + (size_t)min(m0 + 16 * t + r16, M - 1) * lda;   // (rows past the edge: not stored)
+  if (TB) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) bcol[TB ? j : 0] = B + (size_t)min(n0 + 16 * j + r16, N - 1) * ldb;
+  } else {
+    bcol[0] = B + (edge ? 0 : n0 + 4 * r16);
+  }
+  f32x4 acc[TM][4];
+#pragma unroll
+  for (int t = 0; t < TM; t++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  f32x4 a[ST][TM], b[ST][4];                       // b: TB column tile j, k 4 q ..; else row 4 q + s, column tiles 0 .. 3
+  auto load = [&](int u, int i) {
+    const int k = kbeg + kSrStep * (wave + kSrWaves * i) + 4 * quarter;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (TB) {
+        b[u][j] = *reinterpret_cast<const f32x4u*>(bcol[TB ? j : 0] + k);
+      } else if (!edge) {
+        b[u][j] = *reinterpret_cast<const f32x4u*>(bcol[0] + (size_t)(k + j) * ldb);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) b[u][j][e] = bcol[0][(size_t)(k + j) * ldb + min(n0 + 4 * r16 + e, N - 1)];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TM; t++) a[u][t] = *reinterpret_cast<const f32x4u*>(arow[t] + k);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto compute = [&](int u) {
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int t = 0; t < TM; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][t][s], TB ? b[u][j][s] : b[u][s][j], acc[t][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // every load is of a step that exists: one past the end would cost what a real one costs
+  int it = 0;
+#pragma unroll
+  for (int u = 0; u < ST; u++)
+    if (u < mine) load(u, u);
+  for (; it + 2 * ST <= mine; it += ST) {
+#pragma unroll
+    for (int u = 0; u < ST; u++) {
+      compute(u);
+      load(u, it + u + ST);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < ST; u++) {
+    if (it + u < mine) compute(u);
+    if (it + u + ST < mine) load(u, it + u + ST);
+  }
+#pragma unroll
+  for (int u = 0; u < ST; u++)
+    if (it + u + ST < mine) compute(u);
+  // the ragged step: k past the end is zero on both sides (a zero against an infinity would not do)
+  if (kbeg + steps * kSrStep < kend && wave == steps % kSrWaves) {
+    const int k = kbeg + steps * kSrStep + 4 * quarter;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const bool in = k + s < kend;
+      const int kk = min(k + s, kend - 1);
+      float bv[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const float v = TB ? bcol[TB ? j : 0][kk] : B[(size_t)kk * ldb + min(n0 + 4 * r16 + j, N - 1)];
+        bv[j] = in ? v : 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < TM; t++) {
+        const float v = arow[t][kk], av = in ? v : 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[j], acc[t][j], 0, 0, 0);
+      }
+    }
+  }
+
+  // acc[t][j][v] of lane l: row 16 t + 4 (l / 16) + v, column l % 16 of column tile j. Wavefronts 4..7 hand theirs to
+  // 0..3, whose four sums everyone then adds up.
+  auto entry = [&](float* dst, int t, int v) { return dst + (16 * t + 4 * quarter + v) * kSrLD + (TB ? r16 : 4 * r16); };
+  auto put = [&](float* dst) {
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        float* p = entry(dst, t, v);
+        if (TB) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) p[16 * j] = acc[t][j][v];
+        } else {
+          *reinterpret_cast<f32x4*>(p) = f32x4{acc[t][0][v], acc[t][1][v], acc[t][2][v], acc[t][3][v]};
+        }
+      }
+  };
+  float* slot = &red[wave & 3][0][0];
+  if (wave >= 4) put(slot);
+  __syncthreads();
+  if (wave < 4) {
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const float* p = entry(slot, t, v);
+        if (TB) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[t][j][v] += p[16 * j];
+        } else {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[t][j][v] += x[j];
+        }
+      }
+    put(slot);
+  }
+  __syncthreads();
+  const bool wide = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+  for (int i = tid; i < BM * (kSrBN / 4); i += 64 * kSrWaves) {
+    const int row = i / (kSrBN / 4), c = i % (kSrBN / 4) * 4, gm = m0 + row, gn = n0 + c;
+    if (gm >= M || gn >= N) continue;
+    f32x4 o = (*reinterpret_cast<const f32x4*>(&red[0][row][c]) + *reinterpret_cast<const f32x4*>(&red[1][row][c])) +
+              (*reinterpret_cast<const f32x4*>(&red[2][row][c]) + *reinterpret_cast<const f32x4*>(&red[3][row][c]));
+    if (epi)
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] = add_rn(mul_rn(o[e], scale), offset);
+    float* dst = C + (size_t)gm * N + gn;
+    if (wide) {
+      *reinterpret_cast<f32x4*>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (gn + e < N) dst[e] = o[e];
+    }
+  }
+}
+
+// The same for A as it is stored ([M][K]); the caller has checked the arguments.
+int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb, int tb, float* pc, int M, int N, int K, float scale,
+                      float offset, int epi) {
+  // Row blocks and K splits (parts in scratch, summed in a fixed order) that an estimate in clocks likes best: a block
+  // takes 1600 clocks per row tile and 128 k, and 6000 to start and end; blocks run one to a CU, so tiles that make a
+  // round and a bit are cut smaller until they make whole rounds; parts are written and read at 2.5 KB a clock, and their
+  // launch is 11000. (333 x 3584 x 3584: 175 us with 336 tiles of full K, 128 with three splits.)
+  const int t16 = (M + 15) / 16, cus = ctx().cus;
+  const int64_t columns = (N + kSrBN - 1) / kSrBN;
+  int rb = 1, TM = 1, S = 1;
+  double least = -1;
+  for (int r = (t16 + 3) / 4; r <= (t16 + 3) / 4 + 2 && r <= t16; r++) {
+    const int tm = (t16 + r - 1) / r;
+    for (int s = 1; s <= 16 && (s == 1 || K / s >= 64); s++) {
+      const double rounds = (double)((r * columns * s + cus - 1) / cus), steps = (double)(((K + s - 1) / s + 127) / 128);
+      const double t = rounds * (steps * 1600 * tm + 6000) + (s > 1 ? 11000 + 8.0 * s * M * N / 2500 : 0);
+      if (least < 0 || t < least) { least = t; rb = r; TM = tm; S = s; }
+    }
+  }
+  const int64_t tiles = rb * columns;
+  int kchunk = K;
+  float* dst = pc;
+  if (S > 1) {
+    kchunk = ((K + S - 1) / S + kSrStep - 1) / kSrStep * kSrStep;
+    S = (K + kchunk - 1) / kchunk;
+    dst = S > 1 ? static_cast<float*>(scratch((size_t)S * M * N * sizeof(float))) : pc;
+    if (!dst) return fail(TLHIP_ENOMEM, "tlhip_gemm: no scratch for %d K-splits", S);
+  }
+  const dim3 grid((unsigned)tiles, (unsigned)S);
+  const int kepi = S > 1 ? 0 : epi;
+  const auto run = [&](auto tm, auto t_b) {
+    constexpr int TM_ = decltype(tm)::value, TB_ = decltype(t_b)::value, lds = 4 * 16 * TM_ * kSrLD * (int)sizeof(float);
+    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(sgemm_rows_kernel<TM_, TB_>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
+    sgemm_rows_kernel<TM_, TB_><<<grid, dim3(64 * kSrWaves), lds, ctx().stream>>>(pa, lda, pb, ldb, dst, M, N, K, scale, offset, kepi, kchunk, rb);
+    return 0;
+  };
+  using std::integral_constant;
+  const auto by_tm = [&](auto t_b) {
+    return TM == 1 ? run(integral_constant<int, 1>{}, t_b) : TM == 2 ? run(integral_constant<int, 2>{}, t_b)
+         : TM == 3 ? run(integral_constant<int, 3>{}, t_b) : run(integral_constant<int, 4>{}, t_b);
+  };
+  if (int rc = tb ? by_tm(integral_constant<int, 1>{}) : by_tm(integral_constant<int, 0>{})) return rc;
+  if (S > 1) {
+    const size_t n = (size_t)M * N;
+    sgemm_sum_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx().stream>>>(dst, pc, n, S, scale, offset, epi);
   }
   return 0;
 }
