@@ -259,3 +259,39 @@ def test_load_gguf_refuses_what_it_cannot_take(tmp_path, what):
         W.qwen2_file(path, d, w)
     with pytest.raises(RuntimeError, match="load_gguf failed"):
         qwen.QwenGPU.from_gguf(path, fmt="q4", max_ctx=64)
+
+
+@pytest.mark.parametrize("st", [F32, F16])
+def test_quantize_q4_beside_its_rounding_boundaries(lib, orc, st):
+    """Weights a few units in the last place around (n + 1/2) scale and n scale, where a quotient that is not correctly
+    rounded would land on the other side, and groups that hold infinities and NaN: nibbles and scales bit for bit those
+    of the division."""
+    rng = np.random.default_rng(71)
+    rows, K = 600, 320
+    top = np.abs(rng.standard_normal((rows, K // 32, 1)) * 10.0 ** rng.integers(-4, 4, (rows, K // 32, 1))).astype(np.float32) + np.float32(1e-7)
+    if st == F16:
+        top = np.minimum(top, 6e4).astype(np.float16).astype(np.float32)
+    scale = np.maximum(top, np.float32(1e-8)) / np.float32(7)
+    n = rng.integers(0, 7, (rows, K // 32, 32)) + np.where(rng.random((rows, K // 32, 32)) < 0.7, 0.5, 0.0)
+    near = (n * scale.astype(np.float64)).astype(np.float32)
+    w = np.minimum(np.abs((near.view(np.int32) + rng.integers(-3, 4, near.shape).astype(np.int32)).view(np.float32)), top)
+    w = np.where(np.isfinite(w), w, 0).astype(np.float32)
+    w[..., 0:1] = top                                     # the group's largest: its scale is known
+    w *= np.where(rng.random(w.shape) < 0.5, -1, 1).astype(np.float32)
+    w = w.reshape(rows, K)
+    w[5, 3], w[6, 40], w[7, 100], w[7, 101] = np.inf, np.nan, -np.inf, np.nan
+    host = w.astype(np.float16).view(np.uint16) if st == F16 else w
+    wide = orc.f16_widen(host).reshape(rows, K) if st == F16 else w
+    src, q4 = lib.to_device(host), lib.to_device(np.zeros(orc.q4_bytes(rows, K), np.uint8))
+    lib.quantize_q4(src, st, q4, rows, K)
+    got = q4.numpy()
+    with np.errstate(all="ignore"):
+        g = wide.reshape(-1, 32)
+        big = np.fmax(np.fmax.reduce(np.abs(g), 1), np.float32(1e-8))
+        sc = (big / np.float32(7)).astype(np.float32)
+        d = (g / sc[:, None]).astype(np.float32)
+        q = np.copysign(np.floor(np.abs(d)) + (np.abs(d) - np.floor(np.abs(d)) >= 0.5), d)
+        nib = np.where(np.isnan(q), 0, np.clip(q, -8, 7) + 8).astype(np.uint8).reshape(rows, K)
+    assert np.array_equal(got[rows * K // 2:].view(np.float32), sc)
+    assert np.array_equal(got[:rows * K // 2].reshape(rows, K // 2), nib[:, 0::2] | nib[:, 1::2] << 4)
+    src.free(); q4.free()
