@@ -1,0 +1,340 @@
+// Prompt-chunk GEMM over an int4 weight: C[M,N] = A[M,K] f32 . dequant(W)^T, formed as the sum over groups of
+// scale * (A . q) - the decode GEMV's arithmetic on the matrix pipe, in the terms of gemm_bf16_nt_kernel's int4 form for
+// more than 64 rows: row m of A times 2^ea[m] as two f16 terms (one fp32 rounding per product), nibbles exact in f16, a
+// group's sums started at zero and added to the accumulators times its scale.
+//
+// What bounded that form (244 TFLOP/s): vector instructions. Every block cut its rows of A again, slab by slab
+// (128 instructions per lane and slab of 32 k beside 16 MFMAs), and a nibble took two instructions. Here:
+//   * A is cut once per product (q4_image_kernel; the pass that found the exponents did half of it) into images of
+//     64 rows x 32 k, both terms, 8 KB, rows in the bank-conflict-free order the fragment reads expect, so that a unit
+//     of four slabs is 32 contiguous KB that go to LDS by global_load_lds, without registers;
+//   * the nibbles a lane multiplies come to it directly: its wavefront owns 64 columns (64 x 64 outputs, four
+//     wavefronts side by side), a 16-byte load is one group of one column, and two half-wave swaps per two groups give
+//     each half its k. Masked in place, a nibble is an f16 with its value (or 16 times that) in the last bits of 1024, so
+//     eight of them take nine instructions; the k order that gives (0 4 1 5 2 6 3 7) is the one the images are
+//     written in.
+// 102 vector instructions beside 16 MFMAs per slab and wavefront are left, 64 of them the scales'; they and the MFMAs of a
+// SIMD's two wavefronts add up (512 x 32768 x 3584: 235 us = 510 TFLOP/s; without the scales 192, without all of it and the
+// loads 148; wave priorities and a staggered start change nothing). Two blocks per CU, two barriers per 128 k.
+// Rows come in blocks of 64: 301 rows waste 6 % of the products, 128-row tiles waste 28 %. us, before -> now: 301 rows
+// gated 37888 x 3584 303 -> 209, 3584 x 18944 150 -> 113, 4608 x 3584 48 -> 42; 512 rows 393 -> 320, 207 -> 176, 61 -> 58.
+#include "gemm_shared.hpp"
+
+namespace tlhip {
+namespace q4 {
+
+constexpr int kBM = 64, kBN = 256, kSlab = 32, kPlane = kBM * kSlab * 2, kImage = 2 * kPlane, kUnit = 4 * kImage;
+
+__device__ __forceinline__ int image_off(int row, int chunk) {   // 16-byte chunk (8 k) of a row inside a plane
+  return row * (kSlab * 2) + ((chunk ^ ((row >> 1) & 3)) << 4);
+}
+
+// One block per row of the images (rows past M are zero rows): the row's exponent and its two f16 terms. The row stays
+// in registers between the two steps: up to RR runs of eight k per thread, K <= 2048 RR.
+template <int RR>
+__global__ __launch_bounds__(256) void q4_image_kernel(const float* __restrict__ A, int* __restrict__ ea, char* __restrict__ img,
+                                                       int M, int K) {
+  __shared__ uint32_t part[4];
+  const int gm = blockIdx.x, t = threadIdx.x, k8 = K / 8, row = gm % kBM;
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  f32x4 v[RR][2];
+  uint32_t mx = 0;
+  const f32x4* src = reinterpret_cast<const f32x4*>(A + (size_t)min(gm, M - 1) * K);
+#pragma unroll
+  for (int i = 0; i < RR; i++) {
+    const int q = t + 256 * i;
+    const bool in = q < k8 && gm < M;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      v[i][h] = in ? src[2 * q + h] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; e++) mx = max(mx, __float_as_uint(v[i][h][e]) & 0x7fffffffu);
+    }
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
+  if ((t & 63) == 0) part[t >> 6] = mx;
+  __syncthreads();
+  mx = max(max(part[0], part[1]), max(part[2], part[3]));
+  const int e = row_exponent((int)(mx >> 23), mx == 0);
+  const float s = pow2f(e);
+  if (t == 0 && gm < M) ea[gm] = e;
+  char* dst = img + (size_t)(gm / kBM) * (K / kSlab) * kImage;
+#pragma unroll
+  for (int i = 0; i < RR; i++) {
+    const int q = t + 256 * i;                     // run q of the row: slab q / 4, chunk q % 4
+    if (q >= k8) break;
+    const f32x4 a = v[i][0] * s, b = v[i][1] * s;
+    frag16 hi, lo;
+#pragma unroll
+    for (int p = 0; p < 4; p++) {                  // pairs (0 4) (1 5) (2 6) (3 7)
+      uint32_t h2, l2;
+      split2_f16<false>(a[p], b[p], h2, l2);
+      hi[p] = h2;
+      lo[p] = l2;
+    }
+    char* o = dst + (size_t)(q >> 2) * kImage + image_off(row, q & 3);
+    *reinterpret_cast<frag16*>(o) = hi;
+    *reinterpret_cast<frag16*>(o + kPlane) = lo;
+  }
+}
+
+// eight nibbles of a word as f16 weights n - 8, k in the images' order
+__device__ __forceinline__ frag16 nib8(uint32_t w) {
+  const f16x2 off = {(_Float16)-1032.0f, (_Float16)-1032.0f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, off16 = {(_Float16)-72.0f, (_Float16)-72.0f};
+  const uint32_t u = w >> 8;
+  auto low = [&](uint32_t x) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, (x & 0x000f000fu) | 0x64006400u) + off); };
+  auto high = [&](uint32_t x) {                    // 1024 + 16 n: (that) / 16 - 72, exact
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (x & 0x00f000f0u) | 0x64006400u), sixteenth, off16));
+  };
+  return frag16{low(w), high(w), low(u), high(u)};
+}
+
+__device__ __forceinline__ f32x16 mma(const frag16& a, const frag16& b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// Grid: x = row blocks (fastest) x column tiles, y = K-split parts of `part_units` units of 128 k; part y goes to
+// C + y * M * ldc. n0 in tile columns; N = columns of this launch (gated: features), W and scales at its first row.
+// GU: a wavefront's 64 columns are 32 gate features and their up rows (ff rows further down); under a split the raw
+// parts are stored in that order and splitk_sum_swiglu_kernel gates after the sum.
+template <bool GU>
+__global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict__ Aimg, const int* __restrict__ ea, const uint8_t* __restrict__ W,
+                                                         const float* __restrict__ scales, float* __restrict__ C, int M, int N, int K,
+                                                         int part_units, int ldc, int ff, int row_blocks) {
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  extern __shared__ __attribute__((aligned(1024))) char ring[];   // two units of A
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
+  const int lid = xcd * q8 + min(xcd, r8) + within;   // one contiguous run of tiles per XCD
+  const int rb = lid % row_blocks, n0 = lid / row_blocks * kBN;
+  const int groups = K / kSlab, ubeg = blockIdx.y * part_units, nu = min((groups + 3) / 4, ubeg + part_units) - ubeg;
+  C += (size_t)blockIdx.y * M * ldc;
+
+  // this lane's columns (clamped: what lies past the edge is not stored)
+  const uint8_t* wrow[2];
+  const float* srow[2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    int64_t r;
+    if (GU) r = min((n0 >> 1) + wave * 32 + l32, N - 1) + (j ? (int64_t)ff : 0);
+    else r = min(n0 + wave * 64 + j * 32 + l32, N - 1);
+    wrow[j] = W + r * (K / 2);
+    srow[j] = scales + r * groups;
+  }
+  const char* asrc = Aimg + ((size_t)rb * groups + 4 * ubeg) * kImage;
+  // my eighth of a unit's copy (past the last group: the images end, so the copy stops there)
+  auto copy = [&](int u, int stage) {
+    const int have = min(4, groups - 4 * (ubeg + u)) * (kImage / 1024);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int piece = min(wave * 8 + i, have - 1);   // (a repeated piece lands in a slab that is not multiplied)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(asrc + (size_t)u * kUnit + piece * 1024 + lane * 16),
+                                       (__attribute__((address_space(3))) void*)(ring + stage * kUnit + (wave * 8 + i) * 1024), 16, 0, 0);
+    }
+  };
+  frag16 w[2][2][2];                               // [set][column tile][groups 0 1 | 2 3]
+  f32x4u s[2][2];
+  auto load_w = [&](int set, int u) {
+    const int g0 = 4 * (ubeg + u);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+#pragma unroll
+      for (int p = 0; p < 2; p++) w[set][j][p] = *reinterpret_cast<const frag16*>(wrow[j] + 16 * min(g0 + 2 * p + half, groups - 1));
+      if (g0 + 4 <= groups) {
+        s[set][j] = *reinterpret_cast<const f32x4u*>(srow[j] + g0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[set][j][e] = srow[j][min(g0 + e, groups - 1)];
+      }
+    }
+  };
+  auto barrier = [] {                              // without the fence that would wait for every copy in flight
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+  int aoff[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++) aoff[ks] = image_off(l32, ks * 2 + half);   // (32 rows further down: 32 row lengths, the same swizzle)
+
+  auto slab = [&](const char* at, int set, int g) {
+    frag16 b[2][2];                                // [16-k step][column tile]
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) b[ks][j] = nib8(w[set][j][g >> 1][2 * ks + (g & 1)]);
+    f32x16 grp[2][2];                              // four chains of products side by side
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int p = 0; p < 2; p++) {                // (the second terms first would cost precision at long K: 1.9e-7 for 1.3e-7)
+        frag16 a[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) a[i] = *reinterpret_cast<const frag16*>(at + aoff[ks] + p * kPlane + i * 32 * kSlab * 2);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) grp[i][j] = mma(a[i], b[ks][j], ks + p == 0 ? f32x16{} : grp[i][j]);
+      }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[i][j][v] = fmaf(grp[i][j][v], s[set][j][g], acc[i][j][v]);
+  };
+  auto unit = [&](int set, int u) {
+    // my copies and loads of unit u have landed (those of u + 1 - eight copies, six loads - may be in flight); past the
+    // barrier that holds for every wavefront
+    if (4 * (ubeg + u) + 8 <= groups && u + 1 < nu) asm volatile("s_waitcnt vmcnt(14)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    barrier();
+    // words of groups (half) and 2 + (half): a half's k of both groups of a pair
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        frag16& x = w[set][j][p];
+        const auto y = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
+        const auto z = __builtin_amdgcn_permlane32_swap(x[2], x[3], false, false);
+        x = frag16{y[0], y[1], z[0], z[1]};        // [16-k step][group of the pair]
+      }
+    const char* at = ring + set * kUnit;
+    const int have = min(4, groups - 4 * (ubeg + u));
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      if (g < have) slab(at + g * kImage, set, g);
+    barrier();                                     // everyone is done with this stage
+    if (u + 2 < nu) {
+      copy(u + 2, set);
+      load_w(set, u + 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  copy(0, 0);
+  load_w(0, 0);
+  if (nu > 1) {
+    copy(1, 1);
+    load_w(1, 1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  for (int u = 0; u < nu; u += 2) {
+    unit(0, u);
+    if (u + 1 < nu) unit(1, u + 1);
+  }
+
+  // acc[v] of lane l: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32. The row's exponent comes back out, exactly.
+  const int m0 = rb * kBM;
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int gm = m0 + i * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+      if (gm >= M) continue;
+      const int e = ea[gm];
+      if (GU && gridDim.y == 1) {
+        const int f = (n0 >> 1) + wave * 32 + l32;
+        if (f >= N) continue;
+        const float g = ldexpf(acc[i][0][v], -e), sg = 1.0f / (1.0f + expf(-g));   // swiglu_kernel's arithmetic
+        C[(size_t)gm * ldc + f] = (g * sg) * ldexpf(acc[i][1][v], -e);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          const int gn = n0 + wave * 64 + j * 32 + l32;
+          if (!GU && gn >= N) continue;            // gated parts are whole tiles wide
+          C[(size_t)gm * ldc + gn] = ldexpf(acc[i][j][v], -e);
+        }
+      }
+    }
+}
+
+}  // namespace q4
+
+static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The three forms of gemm_bf16_nt_impl (prefill.hip), which has checked the arguments. can_split: the part sums work on
+// float4s. Work is shaped to whole rounds of the 2 * CUs block slots: fewer tiles than slots -> K split; more -> the
+// columns that make whole rounds with full K, the rest split over K in a second launch.
+int gemm_q4_prompt(const float* A, const uint8_t* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K, size_t parts_bytes,
+                   int* S_out, bool gu, bool can_split) {
+  using namespace q4;
+  Context& c = ctx();
+  const int per = gu ? 2 : 1;
+  const int64_t w = kBN / per, rb = cdiv(M, kBM), tn = cdiv(N, w), slots = 2 * (int64_t)c.cus, groups = K / kSlab, units = cdiv(groups, 4);
+  const bool want_parts = S_out != nullptr;
+  struct Piece { int64_t tn0, tcols; int S; } pieces[2];
+  int npieces = 0;
+  auto pick_S = [&](int64_t tiles) {
+    if (!can_split || tiles >= slots) return 1;
+    int64_t S = std::min<int64_t>(slots / tiles, 16);
+    while (S > 1 && units / S < 2) S--;            // at least 256 k per part
+    if (want_parts)
+      while (S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) S--;
+    return (int)S;
+  };
+  const int64_t per_round = slots / rb;
+  if (rb * tn <= slots || per_round == 0 || !can_split || want_parts) {
+    pieces[npieces++] = Piece{0, tn, pick_S(rb * tn)};
+  } else {
+    const int64_t main_tn = tn / per_round * per_round;
+    pieces[npieces++] = Piece{0, main_tn, 1};
+    if (main_tn < tn) pieces[npieces++] = Piece{main_tn, tn - main_tn, pick_S(rb * (tn - main_tn))};
+  }
+  const size_t ea_bytes = ((size_t)M * sizeof(int) + 1023) & ~(size_t)1023, img_bytes = (size_t)rb * groups * kImage;
+  size_t parts_need = 0;
+  if (!want_parts)
+    for (int i = 0; i < npieces; i++)
+      if (pieces[i].S > 1) {
+        const int64_t part_w = gu ? pieces[i].tcols * kBN : std::min<int64_t>(pieces[i].tcols * w, N - pieces[i].tn0 * w);
+        parts_need = std::max(parts_need, (size_t)pieces[i].S * M * part_w * sizeof(float));
+      }
+  char* sbase = static_cast<char*>(scratch(ea_bytes + img_bytes + parts_need));
+  if (!sbase) return kNoScratch;
+  int* ea = reinterpret_cast<int*>(sbase);
+  char* img = sbase + ea_bytes;
+  const auto image = [&](auto kernel) { kernel<<<dim3((unsigned)(rb * kBM)), dim3(256), 0, c.stream>>>(A, ea, img, (int)M, (int)K); };
+  if (K <= 2048) image(q4_image_kernel<1>);
+  else if (K <= 4096) image(q4_image_kernel<2>);
+  else if (K <= 8192) image(q4_image_kernel<4>);
+  else if (K <= 20480) image(q4_image_kernel<10>);
+  else image(q4_image_kernel<16>);
+  for (int i = 0; i < npieces; i++) {
+    const Piece& P = pieces[i];
+    const int64_t n0 = P.tn0 * w, pn = std::min<int64_t>(P.tcols * w, N - n0), part_w = gu ? P.tcols * kBN : pn;
+    const int64_t part_units = cdiv(units, P.S);
+    const int S = (int)cdiv(units, part_units);
+    float* dst = C + n0;
+    int64_t ldc = N;
+    if (want_parts) {
+      *S_out = S;
+    } else if (S > 1) {
+      dst = reinterpret_cast<float*>(sbase + ea_bytes + img_bytes);
+      ldc = part_w;
+    }
+    if (rb * P.tcols > 0x7fffffff || part_w > 0x7fffffff) return fail(TLHIP_EUNSUPPORTED, "tlhip_gemm_q4_nt: too many tiles for one grid");
+    const dim3 grid((unsigned)(rb * P.tcols), (unsigned)S);
+    const uint8_t* wp = W + (size_t)n0 * K / 2;
+    const float* sp = scales + (size_t)n0 * groups;
+    const auto run = [&](auto kernel, hipError_t set) {
+      if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
+      kernel<<<grid, dim3(256), 2 * kUnit, c.stream>>>(img, ea, wp, sp, dst, (int)M, (int)pn, (int)K, (int)part_units, (int)ldc, (int)N, (int)rb);
+      return 0;
+    };
+    static const hipError_t set_plain = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_q4_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kUnit);
+    static const hipError_t set_gated = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_q4_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kUnit);
+    if (int rc = gu ? run(gemm_q4_kernel<true>, set_gated) : run(gemm_q4_kernel<false>, set_plain)) return rc;
+    if (S > 1 && !want_parts) launch_part_sum(dst, C + n0, M, pn, part_w, N, S, gu ? 32 : 0);
+  }
+  return TLHIP_OK;
+}
+
+}  // namespace tlhip

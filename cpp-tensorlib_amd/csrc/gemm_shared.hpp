@@ -19,7 +19,16 @@ RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64
 int launch_gemm_rows(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K,
                      int64_t ldc, bool gu);
 
+// gemm_q4.hip: products of more than 64 rows over an int4 weight, in the three forms of tlhip_gemm_q4_nt*. kNoScratch:
+// nothing was launched, for want of scratch (a recording may not grow it); the caller has a form that needs less.
+constexpr int kNoScratch = 1;
+int gemm_q4_prompt(const float* A, const uint8_t* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K, size_t parts_bytes,
+                   int* S_out, bool gu, bool can_split);
+
 // defined in prefill.hip
+// C[M][n] (rows ldc apart) = the sum of the S parts [M][part_w]; half > 0: gated parts, strips of `half`
+// gate features followed by their up values.
+void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t part_w, int64_t ldc, int S, int half);
 __global__ void splitk_sum_kernel(const float4* __restrict__ part, float4* __restrict__ C, int M, int n4,
                                   int ldc4, int S);
 __global__ void splitk_sum_swiglu_kernel(const float4* __restrict__ part, float4* __restrict__ out, int M,

@@ -475,15 +475,7 @@ __global__ __launch_bounds__(256) void splitk_sum_swiglu_kernel(const float4* __
   out[m * ldc4 + f4] = o;
 }
 
-}  // namespace tlhip
-
-using namespace tlhip;
-
-extern "C" {
-
-// C[M][n] (rows ldc apart) = the sum of the S parts [M][part_w]; half > 0: gated parts, strips of `half`
-// gate features followed by their up values.
-static void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t part_w, int64_t ldc, int S, int half) {
+void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t part_w, int64_t ldc, int S, int half) {
   const dim3 grid((unsigned)(((size_t)M * n / 4 + 255) / 256));
   if (half > 0)
     splitk_sum_swiglu_kernel<<<grid, dim3(256), 0, ctx().stream>>>(reinterpret_cast<const float4*>(parts), reinterpret_cast<float4*>(C), (int)M,
@@ -492,6 +484,12 @@ static void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, 
     splitk_sum_kernel<<<grid, dim3(256), 0, ctx().stream>>>(reinterpret_cast<const float4*>(parts), reinterpret_cast<float4*>(C), (int)M,
                                                             (int)(n / 4), (int)(ldc / 4), S);
 }
+
+}  // namespace tlhip
+
+using namespace tlhip;
+
+extern "C" {
 
 // Three forms of one launcher.
 //   plain: C[M][N] is the product.
@@ -538,12 +536,17 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   if (aligned16(C)) {   // a few rows: a kernel of their own
     int64_t max_S = can_split ? 16 : 1;
     if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
-    const RowsPlan P = plan_gemm_rows(M, N, K, gu, q4, max_S);
+    RowsPlan P = plan_gemm_rows(M, N, K, gu, q4, max_S);
+    const auto part_width = [&] { return gu ? (int64_t)P.tiles * 16 * P.TN : N; };
+    char* parts = nullptr;
+    if (P.S > 1 && !want_parts) {
+      parts = static_cast<char*>(scratch((size_t)P.S * M * part_width() * sizeof(float)));
+      if (!parts) P = plan_gemm_rows(M, N, K, gu, q4, 1);   // no scratch to be had (a recording may not grow it): no parts
+    }
     if (P.S > 0) {
       const bool sum = P.S > 1 && !want_parts;
-      const int64_t part_w = gu ? (int64_t)P.tiles * 16 * P.TN : N;
-      float* dst = sum ? static_cast<float*>(scratch((size_t)P.S * M * part_w * sizeof(float))) : pc;
-      if (!dst) return fail(TLHIP_ENOMEM, "tlhip_gemm_bf16_nt: no scratch for K-split parts");
+      const int64_t part_w = part_width();
+      float* dst = sum ? reinterpret_cast<float*>(parts) : pc;
       if (want_parts) *S_out = P.S;
       if (int rc = launch_gemm_rows(P, pa, W, static_cast<const float*>(scales), dst, M, N, K, sum ? part_w : N, gu)) return rc;
       if (sum) launch_part_sum(dst, pc, M, N, part_w, N, P.S, gu ? 8 * P.TN : 0);
@@ -552,6 +555,13 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   }
   const bool half = q4 && M > 64 && c.tune_gemm_planes != 3;
   const size_t ea_bytes = half ? (((size_t)M * sizeof(int) + 255) & ~(size_t)255) : 0;
+  // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
+  // against 50, 301 x 37888 x 3584 209 against 303)
+  if (half && K <= 32768 && (per * N >= 2048 || K <= 1024)) {
+    const int rc = gemm_q4_prompt(pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, parts_bytes, S_out, gu, can_split);
+    if (rc < 0) return rc;
+    if (rc != kNoScratch) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+  }
   struct Piece { int64_t n0, n; int S; int variant; };    // columns (features) [n0, n0 + n)
   Piece pieces[2];
   int npieces = 0;

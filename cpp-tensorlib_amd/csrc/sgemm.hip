@@ -412,7 +412,11 @@ int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb
     kchunk = ((K + S - 1) / S + kSrStep - 1) / kSrStep * kSrStep;
     S = (K + kchunk - 1) / kchunk;
     dst = S > 1 ? static_cast<float*>(scratch((size_t)S * M * N * sizeof(float))) : pc;
-    if (!dst) return fail(TLHIP_ENOMEM, "tlhip_gemm: no scratch for %d K-splits", S);
+    if (!dst) {                                    // no scratch to be had (a recording may not grow it): no parts
+      dst = pc;
+      S = 1;
+      kchunk = K;
+    }
   }
   const dim3 grid((unsigned)tiles, (unsigned)S);
   const int kepi = S > 1 ? 0 : epi;

@@ -1,0 +1,53 @@
+"""GPU parity: int4 products of more than 64 rows (csrc/gemm_q4.hip) at the edges of their 64-row and 256-column tiles, of
+their units of four groups (K not a multiple of 128 too) and of their K splits, against float64.
+
+Activations enter as two f16 terms of a row scaled by a power of two: 2^-24 of each product's magnitude (the cases' rows
+hold no element 2^24 below their largest); the sums are fp32, 32 products inside two instructions per term, then one
+addition per group and one per part."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(lib, orc, M, rows, K, seed):
+    A = orc.normal(M * K, seed).reshape(M, K)
+    A = np.where(np.abs(A) < 1e-4, np.float32(1e-4), A).astype(np.float32)
+    rng = np.random.default_rng(seed)
+    packed = rng.integers(0, 256, (rows, K // 2), dtype=np.uint8)
+    scales = rng.uniform(0.002, 0.006, (rows, K // 32)).astype(np.float32)
+    nib = np.stack([packed & 15, packed >> 4], -1).reshape(rows, K // 32, 32).astype(np.float64) - 8
+    W, A64 = (nib * scales[:, :, None]).reshape(rows, K), A.astype(np.float64)
+    slack = (K / 32 + 100) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W).T)
+    return lib.to_device(A), lib.to_device(np.concatenate([packed.ravel(), scales.ravel().view(np.uint8)])), A64 @ W.T, slack
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 2048, 32), (129, 2049, 160), (200, 257, 896), (192, 2304, 128), (301, 2500, 1056), (320, 4608, 3584),
+                                   (512, 3584, 1024), (193, 70000, 256), (1000, 2300, 384)])
+def test_plain_and_parts(lib, orc, M, N, K):
+    print("case gemm_q4", M, N, K, flush=True)
+    da, dw, want, slack = _case(lib, orc, M, N, K, 81)
+    out = lib.to_device(np.full((M, N), np.nan, np.float32))
+    parts = lib.to_device(np.full((4, M, N), np.nan, np.float32))
+    lib.gemm_q4_nt(da, dw, out, M, N, K)
+    n = lib.gemm_q4_nt_parts(da, dw, parts, M, N, K)
+    assert 1 <= n <= 4
+    assert np.all(np.abs(out.numpy() - want) <= slack)
+    got = parts.numpy()
+    assert np.all(np.abs(got[:n].astype(np.float64).sum(0) - want) <= slack)
+    assert np.isnan(got[n:]).all()
+    for b in (da, dw, out, parts):
+        b.free()
+
+
+@pytest.mark.parametrize("M,ff,K", [(66, 1024, 32), (129, 1100, 160), (301, 4864, 896), (512, 1030, 384), (200, 18944, 128)])
+def test_gated(lib, orc, M, ff, K):
+    print("case gemm_q4 gated", M, ff, K, flush=True)
+    da, dw, p, s = _case(lib, orc, M, 2 * ff, K, 83)
+    g, u, sg, su = p[:, :ff], p[:, ff:], s[:, :ff], s[:, ff:]
+    act, out = g / (1 + np.exp(-g)), lib.to_device(np.full((M, ff), np.nan, np.float32))
+    lib.gemm_q4_nt_swiglu(da, dw, out, M, ff, K)
+    # the slope of x sigmoid(x) is below 1.1; the gate itself costs a few roundings
+    assert np.all(np.abs(out.numpy() - act * u) <= 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u))
+    for b in (da, dw, out):
+        b.free()
