@@ -595,10 +595,12 @@ struct RowTune { int R, KW, bpc, nw, lpr; };
 //  * many rows per CU: whole rows per wavefront (KW = 1), 2 to 4 rows in flight per lane group;
 //  * few rows per CU: K is split over KW wavefronts of a block so that every CU still has a
 //    tile, one chunk per wavefront where the chunks allow it.
-static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int cus, int lds_per_cu, const RowTune& tn) {
+// pro: what stages x.
+static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int pro, int cus, int lds_per_cu, const RowTune& tn) {
   RowCfg c{};
   const double waste64 = (double)((upr + 63) / 64 * 64) / upr, waste16 = (double)((upr + 15) / 16 * 16) / upr;
-  int lpr = (waste64 >= 1.3 && waste16 < waste64) ? 16 : 64;
+  // (a bf16 row has four times the units: 64 lanes up to twice the row's; 3072 x 768 3.4 us against 4.1 with 16)
+  int lpr = (waste64 >= (E == 8 && N / cus < 17 ? 2.0 : 1.3) && waste16 < waste64) ? 16 : 64;
   if (tn.lpr == 16 || tn.lpr == 64) lpr = tn.lpr;
   const int qn = 64 / lpr;
   const int chunks = (upr + lpr - 1) / lpr;
@@ -631,6 +633,29 @@ static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int cus, int lds_per_cu, 
   while (KW > chunks) {  // not enough K to split that far: more row groups instead
     KW /= 2;
     if (R > 1) R /= 2; else if (nw > 4) nw /= 2;
+  }
+  if (E == 8 && lpr == 64 && xbytes + 8192 <= (size_t)lds_per_cu) {
+    // bf16, whose rows are long for their number (us before -> now; cold weights):
+    //  * up to 16 rows per CU: one tile per CU of its share of the rows, four to a wavefront, and K over as many
+    //    wavefronts as the block takes, where they get as many chunks each (16 rows and two splits left half the CUs of
+    //    2048 x 12288 without a tile: 12.3 -> 9.8; 2048 x 4096 8.4 -> 7.2, 2048 x 2048 4.7 -> 3.9, 896 x 4864 4.9 -> 4.3,
+    //    3392 x 2048 7.4 -> 6.7; 3584 x 3584, seven chunks over four, would be 6.9 for 6.6);
+    //  * up to 31 rows and three chunks: the same without the split, whose halves are uneven (5376 x 1536 6.2 -> 5.4);
+    //  * 32 to 127 rows: small blocks, whose ends fall apart in time, as long as they hold x in what a thread requests up
+    //    front (18960 x 2048 15.9 -> 14.0, 32000 x 2048 23.4 -> 21.8, 9728 x 896 6.5 -> 6.0), else of eight wavefronts
+    //    (33000 x 3584: 37.4 so, 38.9 with four, 39.8 with one such block per CU). The post-norm's sums are every block's
+    //    own, so few large ones there (16496 x 3584 24.2 -> 21.9, 24.8 with small ones; 10304 x 2048 12.4 -> 10.7, 9728 x 896 gated 8.8 -> 7.9).
+    const int rows = (int)std::min<int64_t>((N + cus - 1) / cus, 1 << 20), groups = (rows + 3) / 4;
+    if (rows <= 16) {
+      const int kw = std::min(16 / groups, chunks);
+      if ((chunks + kw - 1) / kw * kw * 10 <= chunks * 11) { R = 4; KW = kw; nw = groups * kw; want_bpc = 1; }
+    } else if (rows < 32) {
+      if (chunks <= 3) { R = 4; KW = 1; nw = groups; want_bpc = 2; }
+    } else if (rows_per_cu >= 32 && rows_per_cu < 128) {
+      R = 2; KW = 1;
+      nw = pro == kPostnorm ? 12 : upr <= 256 ? 4 : 8;
+      want_bpc = pro == kPostnorm ? 2 : 16 / nw;
+    }
   }
   if (tn.nw > 0) nw = tn.nw;
   if (tn.R > 0) R = tn.R;
@@ -688,12 +713,12 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
   if (EPI != kStore && N > max_rows) return fail(TLHIP_EUNSUPPORTED, "gemv: gate|up matrix too large for one launch");
   for (int64_t n0 = 0; n0 < N; n0 += max_rows) {
     const int64_t n = N - n0 < max_rows ? N - n0 : max_rows;
-    RowCfg cfg = pick_rows_cfg(n, upr, Fmt::E, c.cus, c.lds_per_cu, tn);
+    RowCfg cfg = pick_rows_cfg(n, upr, Fmt::E, PRO, c.cus, c.lds_per_cu, tn);
     if (EPI != kStore && cfg.R == 1) {   // a lane group needs a gate row and its up row
       RowTune two = tn;
       two.R = 2;
       if (cfg.nw / cfg.KW >= 2 && cfg.nw > 4) two.nw = cfg.nw / 2;   // keeps the rows of a block tile
-      cfg = pick_rows_cfg(n, upr, Fmt::E, c.cus, c.lds_per_cu, two);
+      cfg = pick_rows_cfg(n, upr, Fmt::E, PRO, c.cus, c.lds_per_cu, two);
     }
     if (PRO == kAttnMerge) cfg.lds += (size_t)pro.heads * (kMergeMax + 1) * sizeof(float);
     if (PRO == kPostnorm) cfg.lds += (size_t)(std::max(pro.parts, cfg.nw) + pro.parts) * sizeof(float);
