@@ -247,8 +247,12 @@ class sequence {
     for (int64_t w0 = 0; w0 < n; w0 += step) {
       const int64_t k = std::min(step, n - w0);
       if (!room(std::min(step, n))) return false;
-      for (int64_t i = 0; i < k; i++) reinterpret_cast<int32_t*>(idx_host_)[i] = (int32_t)want[w0 + i];
-      hip::upload(idx_, idx_host_, k);
+      if (k == 1) {
+        hip::upload_u32(idx_, (unsigned)want[w0]);   // (in order with the chunk's launches, which a copy would wait for)
+      } else {
+        for (int64_t i = 0; i < k; i++) reinterpret_cast<int32_t*>(idx_host_)[i] = (int32_t)want[w0 + i];
+        hip::upload(idx_, idx_host_, k);
+      }
       bool ok = hip::gather_rows(chunk_rows(m_), idx_, rows_, chunk_row_width(m_), k, T);
       ok = ok && (k == 1 ? gemv(head(m_), rows_, out_) : gemm(head(m_), rows_, out_, k));
       if (!ok) return false;

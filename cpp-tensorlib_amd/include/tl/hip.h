@@ -570,9 +570,10 @@ struct context {
     return &e->derived.back();
   }
   // device -> staging
-  void pull(extent& e) {
-    f.memcpy_d2h(e.staging, e.base, e.size);
+  bool pull(extent& e) {
+    const bool ok = f.memcpy_d2h(e.staging, e.base, e.size) == 0;
     e.live = extent::side::either;
+    return ok;
   }
 };
 
@@ -704,9 +705,10 @@ inline void sync_to_host(void* native, bool for_write) {
   auto& c = context::get();
   extent* e = c.ready ? c.buffers.containing(native) : nullptr;
   if (!e) return;
+  // (the copy back waits for what is queued: a wait of its own before it is 5 to 10 us per decode step)
+  if (e->staging && e->live == extent::side::device && c.pull(*e)) c.pending = false;
   if (c.pending) flush();
   if (!e->staging) return;
-  if (e->live == extent::side::device) c.pull(*e);
   if (for_write) e->live = extent::side::staging;
 }
 
@@ -744,13 +746,17 @@ inline bool download_raw(void* dst_host, const void* src_dev, int64_t bytes) {
   return bytes == 0 || c.f.memcpy_d2h(dst_host, src_dev, (size_t)bytes) == 0;
 }
 
-// A 4-byte device scalar (a position, a token id) set from the host.
+// A 4-byte device scalar (a position, a token id) set from the host: the value travels with a launch, in order with the
+// others and not waited for.
 inline void upload_u32(void* native, unsigned val) {
   auto& c = context::get();
   extent* e = c.ready ? c.buffers.containing(native) : nullptr;
   if (!e || !e->staging || e->size < sizeof val) return;
   std::memcpy(e->staging, &val, sizeof val);
-  c.push(*e, sizeof val);
+  if (c.capturing || c.f.fill_u32(e->base, val, 1) != 0) return c.push(*e, sizeof val);
+  c.forget_derived(*e);
+  e->live = extent::side::either;
+  c.pending = true;
 }
 
 // ---- the seam ------------------------------------------------------------------
