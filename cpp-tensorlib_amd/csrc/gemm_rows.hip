@@ -375,13 +375,14 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 // eight wavefronts takes the CU's vector memory path 35 clocks per KB of activations and 60 per KB of weights (whose
 // lanes cover 16 rows each), or its SIMDs, with two wavefronts each, the clocks of their matrix or vector
 // instructions (5.5 per element cut, 23 per eight nibbles; int4 measured 1.8 times that); a block starts and ends in
-// 3500 clocks and 60 per accumulator tile; a launch costs 2 us.
+// 3500 clocks and 60 per accumulator tile; bf16 blocks past the first round cost a fifth more; a launch costs 2 us.
 // The other kernel, measured over the same shapes: 6 us and 0.4 us per 32-k slab (1.0 with two blocks on a CU) up to 64
 // rows, above that 17 us and 0.35 (0.8). It is kept where its 128 x 256 tiles pay: products of more than a few rows
 // whose weight keeps every CU busy for several rounds (M = 64, 4608 x 3584: 14.9 us against 16.8 here).
 // Measured, us, other kernel -> this one: 896 x 896 at 5 / 37 / 77 rows 10.5 / 10.0 / 20.5 -> 3.6 / 3.7 / 4.4; 4864 x 896
-// gated 14.4 / 16.0 / 25.4 -> 7.8 / 11.1 / 13.4; 896 x 4864 11.0 / 11.4 / 21.7 -> 4.9 / 7.0 / 9.6; 18944 x 3584 gated
-// 111 / 111 -> 63 / 92; int4 119 / 127 -> 53 / 93.
+// gated 14.4 / 16.0 / 25.4 -> 7.8 / 11.1 / 13.4; 896 x 4864 11.0 / 11.4 / 21.7 -> 4.9 / 7.0 / 9.6; 9728 x 896 at 48 and 64
+// rows 16.8 / 17.8 -> 10.8 / 11.9; 18944 x 3584 gated 111 / 111 -> 63 / 92; int4 119 / 127 -> 53 / 93. 18960 x 2048 at 24 to
+// 64 rows stays with the other one (30 us; 32 to 40 here in parts).
 RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S) {
   using rows::kMaxTM;
   RowsPlan best;
@@ -393,6 +394,7 @@ RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64
   best.row_blocks = (int)cdiv(t16, kMaxTM);
   const int TM = best.TM = (int)cdiv(t16, best.row_blocks);
   double least = 0;
+  const double own_sum = gu || (!q4 && N > 8192) ? 5 : 0;   // (18960 x 2048 at 32 rows: 33.6 us in two parts)
   for (int TN = q4 && TM > 1 ? 2 : 4; TN >= (gu ? 2 : 1); TN /= 2) {   // (what the registers hold)
     const int64_t tiles = cdiv(rows_w, 16 * TN);
     for (int64_t S = 1; S <= std::min<int64_t>(max_S, units); S++) {
@@ -401,11 +403,13 @@ RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64
       const double n = (double)(cdiv(per, rows::kWaves) * steps);    // steps of a wavefront
       const double mem = 8 * (70.0 * TM + (q4 ? 30.0 : 60.0) * TN);
       const double math = 2 * (q4 ? 1.8 * std::max(48.0 * TM * TN, 176.0 * TM + TN * (92.0 + 16 * TM)) : std::max(48.0 * TM * TN, 176.0 * TM));
-      const double rounds = blocks <= 2 * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus;
-      double us = 2 + rounds * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100;
-      // parts written and read, and, gated, their launch (a plain product is planned like one left as parts, whose sum
-      // its consumer forms: the two are the same bits)
-      if (S > 1) us += (double)S * M * rows_w * 4 / 4e6 + (gu ? 5 : 0);
+      // (every CU is busy without a split, and the parts of more than a row tile cost more than the last round's gaps)
+      if (!q4 && S > 1 && M > 16 && tiles * best.row_blocks > cus) break;
+      const double rounds = blocks <= (q4 ? 2 : 4) * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus;
+      double us = 2 + rounds * (!q4 && rounds > 1 ? 1.2 : 1.0) * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100;
+      // parts written and read, and their launch, which a gated product has and a wide one (a narrow one is planned as if
+      // left as parts, whose sum its consumer forms: the two are the same bits)
+      if (S > 1) us += (double)S * M * rows_w * 4 / 4e6 + own_sum;
       if (best.S == 0 || us < least) {
         least = us;
         best.TN = TN;
@@ -419,7 +423,7 @@ RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64
     const int64_t bm = M > 64 ? 128 : 64, bn = M > 64 && !q4 ? 256 : 128, tiles = cdiv(M, bm) * cdiv(rows_w, bn), slabs = K / 32;
     const int64_t S = std::max<int64_t>(1, std::min(std::min<int64_t>(max_S, 2 * cus / tiles), slabs / 8));
     const double other = M > 64 ? 17 + (double)slabs / S * (tiles * S <= 96 ? 0.35 : 0.8) : 6 + (double)slabs / S * (tiles * S <= cus ? 0.4 : 1.0);
-    if (other + (gu && S > 1 ? 5 : 0) < least) best.S = 0;
+    if (other + (S > 1 ? own_sum : 0) < least) best.S = 0;
   }
   return best;
 }
