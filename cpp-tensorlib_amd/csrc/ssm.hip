@@ -4,7 +4,7 @@
 //   y = (S^T C + skip_h x) silu(z)
 // decay_h is the base-2 log of the decay per unit of dt (negative). Everything is f32.
 //
-// Decode: one block per head (ssm_step_kernel). Prompt chunks in pieces of C tokens, with l_t the sum of
+// Decode: one launch (ssm_step_kernel). Prompt chunks in pieces of C tokens, with l_t the sum of
 // the log decays since the piece began:
 //   y_t = 2^l_t C_t^T S_0 + sum_(s <= t) (C_t . B_s) 2^(l_t - l_s) dt_s x_s
 //   S_C = 2^l_C S_0 + sum_s 2^(l_C - l_s) dt_s B_s x_s^T
@@ -37,53 +37,69 @@ __host__ __device__ inline SsmDims ssm_dims(const tlhip_ssm& a) {
 }
 __host__ __device__ inline int ssm_ld(int V) { return (V + 3) & ~3; }
 
-// sum over the taps of channel c for the token at position p; `now` is the token's own input
+// sum over the taps of channel c for the token at position p; `now` is the token's own input. The rows of four taps are
+// requested together: one by one they were three round trips of the step.
 __device__ __forceinline__ float conv_step(const tlhip_ssm& a, const SsmDims& d, const float* __restrict__ ring, int p, int c, float now) {
   const float* w = static_cast<const float*>(a.conv_w);
+  const int first = (p + 1) % d.taps;  // slot of position p - (taps - 1)
   float s = 0.f;
-  for (int j = 0; j < d.taps - 1; j++) {
-    const int q = p - (d.taps - 1) + j;
-    const float x = ring[(size_t)(max(q, 0) % d.taps) * d.ch + c];
-    s = fmaf(w[(size_t)j * d.ch + c], q >= 0 ? x : 0.f, s);
+  for (int j0 = 0; j0 < d.taps - 1; j0 += 4) {
+    float x[4], f[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int j = min(j0 + k, d.taps - 2), slot = first + j < d.taps ? first + j : first + j - d.taps;
+      x[k] = ring[(size_t)slot * d.ch + c];
+      f[k] = w[(size_t)j * d.ch + c];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (j0 + k < d.taps - 1) s = fmaf(f[k], p - (d.taps - 1) + j0 + k >= 0 ? x[k] : 0.f, s);
   }
   return fmaf(w[(size_t)(d.taps - 1) * d.ch + c], now, s) + static_cast<const float*>(a.conv_b)[c];
 }
 
-// Decode step of one head, 512 threads: a thread owns one float4 column of every ng-th state row.
+// Decode step, 512 threads: a thread owns one float4 column of every ng-th state row. SLICED: a block takes 16 of a head's
+// columns, else all of them. The step is a chain of round trips (position, state and convolution inputs, sums), so the
+// slices are there to shorten it: four times the blocks, one state row to a thread, the sum over the rows by shuffles
+// instead of 32 LDS reads in turn (28 heads of 128 x 64: 6.6 us whole, 5.1 in slices). Each slice convolves its
+// group's B and C again.
+template <bool SLICED>
 __global__ __launch_bounds__(512) void ssm_step_kernel(const float* __restrict__ u, float* __restrict__ y, const tlhip_ssm a,
                                                        int pos, const uint32_t* __restrict__ d_pos) {
   extern __shared__ __attribute__((aligned(16))) float ssm_lds[];
   const SsmDims d = ssm_dims(a);
-  const int tid = threadIdx.x, h = blockIdx.x, per = d.H / d.G, g = h / per;
+  const int slices = SLICED ? d.V >> 4 : 1, tid = threadIdx.x, h = blockIdx.x / slices, slice = blockIdx.x - h * slices, col0 = 16 * slice;
+  const int per = d.H / d.G, g = h / per;
   const int p = d_pos ? (int)*d_pos : pos;
-  const int ld = ssm_ld(d.V), nv4 = ld >> 2, ng = 512 / nv4, v4 = tid % nv4, ng0 = tid / nv4;
+  const int ld = ssm_ld(d.V), cols = SLICED ? 16 : ld, nv4 = cols >> 2, ng = 512 / nv4, v4 = tid % nv4, ng0 = tid / nv4;
   const bool live = ng0 < ng;
-  float* xs = ssm_lds;                 // [ld] convolved x of the head
-  float* Bs = xs + ld;                 // [N]
+  float* xs = ssm_lds;                 // [cols] convolved x of the block's columns
+  float* Bs = xs + cols;               // [N]
   float* Cs = Bs + d.N;                // [N]
-  float* red = Cs + d.N + ((4 - (ld + 2 * d.N) % 4) & 3);   // [ng][ld]
-  const size_t slot = (size_t)d.H * d.N * ld;
-  const float* src = static_cast<const float*>(a.ssm_state) + (size_t)(p & 1) * slot + (size_t)h * d.N * ld;
-  float* dst = static_cast<float*>(a.ssm_state) + (size_t)((p + 1) & 1) * slot + (size_t)h * d.N * ld;
-  constexpr int PRE = 8;               // rows of this thread requested up front
+  float* red = Cs + d.N + ((4 - (cols + 2 * d.N) % 4) & 3);   // [ng][ld], sliced: [wavefronts][16]
+  const size_t slot = (size_t)d.H * d.N * ld, at = (size_t)h * d.N * ld + col0 + 4 * v4;
+  const float* src = static_cast<const float*>(a.ssm_state) + (size_t)(p & 1) * slot + at;
+  float* dst = static_cast<float*>(a.ssm_state) + (size_t)((p + 1) & 1) * slot + at;
+  constexpr int PRE = SLICED ? 2 : 8;  // rows of this thread requested up front
   float4 st[PRE];
 #pragma unroll
   for (int i = 0; i < PRE; i++) {
     const int n = ng0 + i * ng;
-    st[i] = live && p > 0 && n < d.N ? *reinterpret_cast<const float4*>(src + (size_t)n * ld + 4 * v4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    st[i] = live && p > 0 && n < d.N ? *reinterpret_cast<const float4*>(src + (size_t)n * ld) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  const float z = SLICED && tid < 16 ? u[a.z_off + h * d.V + col0 + tid] : 0.f;
   float* ring = static_cast<float*>(a.conv_state);
   const float dt = softplus_f(u[a.dt_off + h] + static_cast<const float*>(a.dt_bias)[h]);
   const float w = exp2f(static_cast<const float*>(a.decay)[h] * dt);
-  // this head's x and its group's B and C; the input row is kept for the coming tokens (B, C: by the group's first head)
-  for (int i = tid; i < ld + 2 * d.N; i += 512) {
+  // the block's x and its group's B and C; the input row is kept for the coming tokens (B, C: by the group's first block)
+  for (int i = tid; i < cols + 2 * d.N; i += 512) {
     int c;
     bool keep = true;
-    if (i < ld) c = i < d.V ? h * d.V + i : -1;
+    if (i < cols) c = col0 + i < d.V ? h * d.V + col0 + i : -1;
     else {
-      const int n = i - ld;
+      const int n = i - cols;
       c = d.inner + (n < d.N ? g * d.N + n : (d.G + g) * d.N + n - d.N);
-      keep = h == g * per;
+      keep = h == g * per && slice == 0;
     }
     float v = 0.f;
     if (c >= 0) {
@@ -94,33 +110,55 @@ __global__ __launch_bounds__(512) void ssm_step_kernel(const float* __restrict__
     ssm_lds[i] = v;
   }
   __syncthreads();
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   if (live) {
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     const float x0 = dt * xs[4 * v4], x1 = dt * xs[4 * v4 + 1], x2 = dt * xs[4 * v4 + 2], x3 = dt * xs[4 * v4 + 3];
     const auto row = [&](int n, float4 s) {
       const float b = Bs[n], c = Cs[n];
       s.x = fmaf(w, s.x, b * x0); s.y = fmaf(w, s.y, b * x1); s.z = fmaf(w, s.z, b * x2); s.w = fmaf(w, s.w, b * x3);
-      *reinterpret_cast<float4*>(dst + (size_t)n * ld + 4 * v4) = s;
+      *reinterpret_cast<float4*>(dst + (size_t)n * ld) = s;
       o.x = fmaf(c, s.x, o.x); o.y = fmaf(c, s.y, o.y); o.z = fmaf(c, s.z, o.z); o.w = fmaf(c, s.w, o.w);
     };
 #pragma unroll
     for (int i = 0; i < PRE; i++)
       if (ng0 + i * ng < d.N) row(ng0 + i * ng, st[i]);
     for (int n = ng0 + PRE * ng; n < d.N; n += ng)
-      row(n, p > 0 ? *reinterpret_cast<const float4*>(src + (size_t)n * ld + 4 * v4) : make_float4(0.f, 0.f, 0.f, 0.f));
-    *reinterpret_cast<float4*>(red + ng0 * ld + 4 * v4) = o;
+      row(n, p > 0 ? *reinterpret_cast<const float4*>(src + (size_t)n * ld) : make_float4(0.f, 0.f, 0.f, 0.f));
   }
-  __syncthreads();
-  for (int v = tid; v < d.V; v += 512) {
-    float t = 0.f;
-    for (int k = 0; k < ng; k++) t += red[k * ld + v];
+  const auto finish = [&](int v, float t, float zv) {
     t = fmaf(static_cast<const float*>(a.skip)[h], xs[v], t);
-    y[a.y_off + h * d.V + v] = t * silu_f(u[a.z_off + h * d.V + v]);
+    y[a.y_off + h * d.V + col0 + v] = t * silu_f(zv);
+  };
+  if constexpr (SLICED) {
+#pragma unroll
+    for (int m = 4; m < 64; m *= 2) {
+      o.x += __shfl_xor(o.x, m, kWave); o.y += __shfl_xor(o.y, m, kWave);
+      o.z += __shfl_xor(o.z, m, kWave); o.w += __shfl_xor(o.w, m, kWave);
+    }
+    if ((tid & 63) < 4) *reinterpret_cast<float4*>(red + (tid >> 6) * 16 + 4 * (tid & 63)) = o;
+    __syncthreads();
+    if (tid < 16) {
+      float t = red[tid];
+#pragma unroll
+      for (int k = 1; k < 8; k++) t += red[16 * k + tid];
+      finish(tid, t, z);
+    }
+  } else {
+    if (live) *reinterpret_cast<float4*>(red + ng0 * ld + 4 * v4) = o;
+    __syncthreads();
+    for (int v = tid; v < d.V; v += 512) {
+      float t = 0.f;
+      for (int k = 0; k < ng; k++) t += red[k * ld + v];
+      finish(v, t, u[a.z_off + h * d.V + v]);
+    }
   }
 }
+// up to four blocks per CU, and whole slices
+static bool ssm_sliced(const tlhip_ssm& a) { return a.vdim % 16 == 0 && a.heads * (a.vdim / 16) <= 4 * (int64_t)ctx().cus; }
 static size_t ssm_step_lds(const tlhip_ssm& a) {
+  const bool sliced = ssm_sliced(a);
   const int ld = ssm_ld((int)a.vdim), ng = 512 / (ld >> 2);
-  return (size_t)(ld + 2 * (int)a.state + 4 + ng * ld) * sizeof(float);
+  return (size_t)((sliced ? 16 : ld) + 2 * (int)a.state + 4 + (sliced ? 8 * 16 : ng * ld)) * sizeof(float);
 }
 
 // ---- prompt chunks -------------------------------------------------------------------------------
@@ -477,8 +515,10 @@ int tlhip_ssm_step(const void* u, void* y, const tlhip_ssm* a, int64_t pos, cons
   Context& c = ctx();
   const size_t lds = ssm_step_lds(*a);
   if (lds > (size_t)c.lds_per_cu) return fail(TLHIP_EUNSUPPORTED, "tlhip_ssm_step: not enough LDS");
-  hipLaunchKernelGGL(ssm_step_kernel, dim3((unsigned)a->heads), dim3(512), lds, c.stream, static_cast<const float*>(u),
-                     static_cast<float*>(y), *a, (int)pos, static_cast<const uint32_t*>(d_pos));
+  const bool sliced = ssm_sliced(*a);
+  hipLaunchKernelGGL(sliced ? ssm_step_kernel<true> : ssm_step_kernel<false>, dim3((unsigned)(a->heads * (sliced ? a->vdim / 16 : 1))),
+                     dim3(512), lds, c.stream, static_cast<const float*>(u), static_cast<float*>(y), *a, (int)pos,
+                     static_cast<const uint32_t*>(d_pos));
   TLHIP_CHECK_LAUNCH(TLHIP_C_SSM);
 }
 
