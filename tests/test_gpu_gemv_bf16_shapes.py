@@ -67,3 +67,28 @@ def test_gated(lib, ff, K):
     assert np.all(np.abs(act.numpy() - gate * z[ff:]) <= 1.1 * err[:ff] * (np.abs(z[ff:]) + err[ff:]) + np.abs(gate) * err[ff:] + 1e-6 * np.abs(gate * z[ff:]))
     for b in (dx, dd, dw, dW, dg, act, out):
         b.free()
+
+
+@pytest.mark.parametrize("n,parts,K", [(4096, 8, 4096), (7168, 8, 7168), (256, 2, 264), (384, 3, 520), (1000, 1, 1008), (7, 1, 8), (1200, 8, 1200), (512, 1, 520)])
+def test_normed_runs(lib, n, parts, K):
+    """Runs of half wavefronts and others, one and several, in rows shorter than the product's K; the row itself is exact to
+    the norm's few roundings."""
+    print("case bf16 normed runs", n, parts, K, flush=True)
+    N = 700
+    bits, W = _weight(N, K, n)
+    g = np.random.default_rng(9)
+    x, d, w, b = (g.standard_normal(K).astype(np.float32) for _ in range(4))
+    w[n:] = 0
+    for with_x, with_b in ((1, 1), (0, 0)):
+        v = (d + with_b * b).astype(np.float64)[:n].reshape(parts, -1)
+        s = np.zeros(K)
+        s[:n] = (v / np.sqrt(np.mean(v * v, axis=1, keepdims=True) + 1e-6)).ravel() * w[:n]
+        s += with_x * x
+        dx, dd, db, dw, dW = (lib.to_device(a) for a in (x, d, b, w, bits))
+        y, out = lib.to_device(np.full(N, np.nan, np.float32)), lib.to_device(np.full(K, np.nan, np.float32))
+        lib.gemv_bf16_row_postnorm(dx if with_x else None, dd, db if with_b else None, dw, n, parts, out, dW, y, N, K, 1e-6)
+        # v carries one rounding, its mean square and root (K / 1024 + 20) / 2 together, the product and sum three
+        assert np.all(np.abs(out.numpy() - s) <= (K / 2048 + 16) * 2.0 ** -24 * (np.abs(s) + np.abs(with_x * x) + 1))
+        _near(y.numpy(), W, s, (K / 2048 + 16) * 2.0 ** -24 * np.abs(W).sum(1).max() * np.abs(s).max())
+        for a in (dx, dd, db, dw, dW, y, out):
+            a.free()
