@@ -176,6 +176,31 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return t;
 }
 
+// part(0) + part(1) + ... + part(S - 1), added in that order. The parts of a product lie in another die's cache or beyond:
+// requested one by one each was a round trip, so four are at once (77 rows of 896 in up to seven parts normed: 5.6 us, 3.4
+// so and in blocks of 256 threads).
+__device__ __forceinline__ float plus(float a, float b) { return a + b; }
+__device__ __forceinline__ float4 plus(const float4& a, const float4& b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+template <typename F>
+__device__ __forceinline__ auto sum_parts(int S, F part) {
+  auto a = part(0);
+  int s = 1;
+  for (; s + 4 <= S; s += 4) {
+    const auto b = part(s), c = part(s + 1), d = part(s + 2), e = part(s + 3);
+    a = plus(plus(plus(plus(a, b), c), d), e);
+  }
+  if (s + 3 == S) {
+    const auto b = part(s), c = part(s + 1), d = part(s + 2);
+    a = plus(plus(plus(a, b), c), d);
+  } else if (s + 2 == S) {
+    const auto b = part(s), c = part(s + 1);
+    a = plus(plus(a, b), c);
+  } else if (s < S) {
+    a = plus(a, part(s));
+  }
+  return a;
+}
+
 __device__ __forceinline__ float bf16_lo(uint32_t packed) {  // element 0 of a pair
   return __uint_as_float(packed << 16);
 }

@@ -228,11 +228,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_aimage_kernel(const float* x, co
       if (i < n4) {
         v[k] = x4[i];
         wv[k] = w4[i];
-        float4 d = d4[i];
-        for (int sidx = 1; sidx < S; sidx++) {     // K-split parts, ascending
-          const float4 e = d4[sidx * (part_stride >> 2) + i];
-          d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w;
-        }
+        float4 d = sum_parts(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
         if constexpr (POST) {
           if (bias) {
             const float4 e = reinterpret_cast<const float4*>(bias)[i];

@@ -97,13 +97,13 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
   for (int i = threadIdx.x; i < n; i += 256) hout[base + i] = (src[base + i] * inv) * w[i];
 }
 
-// Wide variant for rows that fit the registers of one 1024-thread block
-// (n % 4 == 0, n <= 4*1024*RV): every thread keeps its float4s of the row and of
+// Wide variant for rows that fit the registers of one block of NT threads
+// (n % 4 == 0, n <= 4*NT*RV): every thread keeps its float4s of the row and of
 // the weight in VGPRs, so the row is read once and nothing waits on a second
 // pass. This is the model shape (n = 896 ... 8192), for one row of a decode step and for
 // the 512 rows of a prompt chunk alike (6.6 us against 11.1 us for 512 x 3584).
-template <bool RES, int RV>
-__global__ __launch_bounds__(1024) void rmsnorm_wide_kernel(const float* __restrict__ x,
+template <bool RES, int RV, int NT>
+__global__ __launch_bounds__(NT) void rmsnorm_wide_kernel(const float* __restrict__ x,
                                                             const float* __restrict__ delta,
                                                             const float* __restrict__ w,
                                                             float* __restrict__ xout,
@@ -120,33 +120,29 @@ __global__ __launch_bounds__(1024) void rmsnorm_wide_kernel(const float* __restr
   float acc = 0.f;
 #pragma unroll
   for (int k = 0; k < RV; k++) {
-    const int i = threadIdx.x + k * 1024;
+    const int i = threadIdx.x + k * NT;
     if (i < n4) {
       v[k] = x4[i];
       wv[k] = w4[i];
       if (RES) {
-        float4 d = d4[i];
-        for (int sidx = 1; sidx < S; sidx++) {   // K-split parts, ascending
-          const float4 e = d4[sidx * (part_stride >> 2) + i];
-          d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w;
-        }
+        const float4 d = sum_parts(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
         v[k].x += d.x; v[k].y += d.y; v[k].z += d.z; v[k].w += d.w;
       }
     }
   }
 #pragma unroll
   for (int k = 0; k < RV; k++) {
-    const int i = threadIdx.x + k * 1024;
+    const int i = threadIdx.x + k * NT;
     if (i < n4) {
       if (RES) reinterpret_cast<float4*>(xout + base)[i] = v[k];
       acc += (v[k].x * v[k].x + v[k].y * v[k].y) + (v[k].z * v[k].z + v[k].w * v[k].w);
     }
   }
-  const float sum = block_sum<16>(acc, red);
+  const float sum = block_sum<NT / 64>(acc, red);
   const float inv = 1.0f / sqrtf(sum * (1.0f / (float)n) + eps);
 #pragma unroll
   for (int k = 0; k < RV; k++) {
-    const int i = threadIdx.x + k * 1024;
+    const int i = threadIdx.x + k * NT;
     if (i < n4) {
       float4 o;
       o.x = (v[k].x * inv) * wv[k].x; o.y = (v[k].y * inv) * wv[k].y;
@@ -162,10 +158,12 @@ static void launch_rmsnorm(const float* x, const float* delta, const float* w, f
   hipStream_t st = ctx().stream;
   const size_t ps = (size_t)(rows * n);   // delta parts, when S > 1
   const bool wide_ok = (n % 4) == 0 && aligned16(w) && aligned16(hout);
-  if (wide_ok && n <= 4096)
-    rmsnorm_wide_kernel<RES, 1><<<dim3((unsigned)rows), dim3(1024), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps);
-  else if (wide_ok && n <= 8192)
-    rmsnorm_wide_kernel<RES, 2><<<dim3((unsigned)rows), dim3(1024), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps);
+  // (blocks of no more wavefronts than the row has work for: the others only meet the barriers)
+  const auto wide = [&](auto kernel, int nt) { kernel<<<dim3((unsigned)rows), dim3(nt), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps); };
+  if (wide_ok && n <= 1024) wide(rmsnorm_wide_kernel<RES, 1, 256>, 256);
+  else if (wide_ok && n <= 2048) wide(rmsnorm_wide_kernel<RES, 1, 512>, 512);
+  else if (wide_ok && n <= 4096) wide(rmsnorm_wide_kernel<RES, 1, 1024>, 1024);
+  else if (wide_ok && n <= 8192) wide(rmsnorm_wide_kernel<RES, 2, 1024>, 1024);
   else
     rmsnorm_kernel<RES><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps);
 }
@@ -394,12 +392,7 @@ __global__ __launch_bounds__(256) void qkv_rope_fill_kernel(
   // S > 1: qkv is the S K-split parts of the projection, part_stride floats apart, added up in
   // ascending order as the part-sum launch would have
   auto ld4 = [&](const float* p) {
-    float4 a = *reinterpret_cast<const float4*>(p);
-    for (int sidx = 1; sidx < S; sidx++) {
-      const float4 b = *reinterpret_cast<const float4*>(p + sidx * part_stride);
-      a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-    }
-    return a;
+    return sum_parts(S, [&](int s) { return *reinterpret_cast<const float4*>(p + s * part_stride); });
   };
   const int half = D >> 1, q4 = half >> 2;            // float4 groups per half row
   const int rot_per_t = (Hq + Hkv) * q4, v_per_t = Hkv * (D >> 2);

@@ -441,11 +441,7 @@ __global__ __launch_bounds__(256) void splitk_sum_kernel(const float4* __restric
                                                          int ldc4, int S) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, total = (size_t)M * n4;
   if (i >= total) return;
-  float4 a = part[i];
-  for (int sidx = 1; sidx < S; sidx++) {
-    const float4 b = part[sidx * total + i];
-    a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-  }
+  const float4 a = sum_parts(S, [&](int s) { return part[s * total + i]; });
   const size_t m = i / n4;
   C[m * ldc4 + (i - m * n4)] = a;
 }
@@ -453,6 +449,8 @@ __global__ __launch_bounds__(256) void splitk_sum_kernel(const float4* __restric
 // The same for the parts of a GU launch: out[m][f] = swiglu(sum_s gate part, sum_s up part). Parts are
 // [M][nv] in tile column order: per wavefront strip of 2 * HW columns, HW gate features then their
 // up values. pf4 = features / 4 of this piece, ldc4 = row stride of out in float4s.
+struct GateUp4 { float4 g, u; };
+__device__ __forceinline__ GateUp4 plus(const GateUp4& a, const GateUp4& b) { return GateUp4{plus(a.g, b.g), plus(a.u, b.u)}; }
 __global__ __launch_bounds__(256) void splitk_sum_swiglu_kernel(const float4* __restrict__ part,
                                                                 float4* __restrict__ out, int M, int pf4,
                                                                 int nv4, int ldc4, int S, int hw4) {
@@ -461,12 +459,8 @@ __global__ __launch_bounds__(256) void splitk_sum_swiglu_kernel(const float4* __
   const size_t m = i / pf4;
   const int f4 = (int)(i - m * pf4);
   const size_t gi = m * nv4 + (size_t)(f4 / hw4) * 2 * hw4 + f4 % hw4, total = (size_t)M * nv4;
-  float4 g = part[gi], u = part[gi + hw4];
-  for (int sidx = 1; sidx < S; sidx++) {
-    const float4 a = part[sidx * total + gi], b = part[sidx * total + gi + hw4];
-    g.x += a.x; g.y += a.y; g.z += a.z; g.w += a.w;
-    u.x += b.x; u.y += b.y; u.z += b.z; u.w += b.w;
-  }
+  const GateUp4 gu = sum_parts(S, [&](int s) { return GateUp4{part[s * total + gi], part[s * total + gi + hw4]}; });
+  const float4 g = gu.g, u = gu.u;
   float4 o;
   o.x = (g.x * (1.0f / (1.0f + expf(-g.x)))) * u.x;
   o.y = (g.y * (1.0f / (1.0f + expf(-g.y)))) * u.y;

@@ -61,11 +61,11 @@ __global__ __launch_bounds__(256) void embed_scaled_kernel(const uint16_t* __res
   out[(size_t)t * ld + c] = c < width ? __uint_as_float((uint32_t)table[(size_t)tok * ldt + c] << 16) * scale : 0.f;
 }
 
-// xout = x + rms(parts + bias) * w, one block of 1024 threads per row, RV float4s a thread.
-template <int RV>
-__global__ __launch_bounds__(1024) void postnorm_rows_kernel(const float* x, const float* __restrict__ delta, int S,
-                                                             size_t part_stride, const float* __restrict__ bias,
-                                                             const float* __restrict__ w, float* xout, int n, float eps) {
+// xout = x + rms(parts + bias) * w, a block of NT threads per row, RV float4s a thread.
+template <int RV, int NT>
+__global__ __launch_bounds__(NT) void postnorm_rows_kernel(const float* x, const float* __restrict__ delta, int S,
+                                                           size_t part_stride, const float* __restrict__ bias,
+                                                           const float* __restrict__ w, float* xout, int n, float eps) {
   __shared__ float red[16];
   const size_t base = (size_t)blockIdx.x * n;
   const int n4 = n >> 2;
@@ -73,16 +73,12 @@ __global__ __launch_bounds__(1024) void postnorm_rows_kernel(const float* x, con
   float acc = 0.f;
 #pragma unroll
   for (int k = 0; k < RV; k++) {
-    const int i = threadIdx.x + k * 1024;
+    const int i = threadIdx.x + k * NT;
     if (i < n4) {
       const float4* d4 = reinterpret_cast<const float4*>(delta + base);
       xv[k] = reinterpret_cast<const float4*>(x + base)[i];
       wv[k] = reinterpret_cast<const float4*>(w)[i];
-      v[k] = d4[i];
-      for (int s = 1; s < S; s++) {    // K-split parts, ascending
-        const float4 e = d4[s * (part_stride >> 2) + i];
-        v[k].x += e.x; v[k].y += e.y; v[k].z += e.z; v[k].w += e.w;
-      }
+      v[k] = sum_parts(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
       if (bias) {
         const float4 e = reinterpret_cast<const float4*>(bias)[i];
         v[k].x += e.x; v[k].y += e.y; v[k].z += e.z; v[k].w += e.w;
@@ -90,10 +86,10 @@ __global__ __launch_bounds__(1024) void postnorm_rows_kernel(const float* x, con
       acc += (v[k].x * v[k].x + v[k].y * v[k].y) + (v[k].z * v[k].z + v[k].w * v[k].w);
     }
   }
-  const float inv = 1.0f / sqrtf(block_sum<16>(acc, red) / (float)n + eps);
+  const float inv = 1.0f / sqrtf(block_sum<NT / 64>(acc, red) / (float)n + eps);
 #pragma unroll
   for (int k = 0; k < RV; k++) {
-    const int i = threadIdx.x + k * 1024;
+    const int i = threadIdx.x + k * NT;
     if (i < n4)
       reinterpret_cast<float4*>(xout + base)[i] =
           make_float4(fmaf(v[k].x * inv, wv[k].x, xv[k].x), fmaf(v[k].y * inv, wv[k].y, xv[k].y),
@@ -225,8 +221,10 @@ int tlhip_postnorm_res_parts(const void* x, const void* parts, int64_t S, const 
   if (aimage)
     return postnorm_aimage(static_cast<const float*>(x), static_cast<const float*>(parts), (int)S, static_cast<const float*>(bias),
                            static_cast<const float*>(norm_w), static_cast<float*>(xout), (int)n, eps, (int)rows, aimage);
-  auto fn = n <= 4096 ? postnorm_rows_kernel<1> : n <= 8192 ? postnorm_rows_kernel<2> : postnorm_rows_kernel<8>;
-  hipLaunchKernelGGL(fn, dim3((unsigned)rows), dim3(1024), 0, ctx().stream, static_cast<const float*>(x), static_cast<const float*>(parts),
+  const int nt = n <= 1024 ? 256 : n <= 2048 ? 512 : 1024;   // no more wavefronts than the row has work for
+  auto fn = n <= 1024 ? postnorm_rows_kernel<1, 256> : n <= 2048 ? postnorm_rows_kernel<1, 512> : n <= 4096 ? postnorm_rows_kernel<1, 1024>
+          : n <= 8192 ? postnorm_rows_kernel<2, 1024> : postnorm_rows_kernel<8, 1024>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)rows), dim3((unsigned)nt), 0, ctx().stream, static_cast<const float*>(x), static_cast<const float*>(parts),
                      (int)S, (size_t)(rows * n), static_cast<const float*>(bias), static_cast<const float*>(norm_w),
                      static_cast<float*>(xout), (int)n, eps);
   TLHIP_CHECK_LAUNCH(TLHIP_C_RMSNORM_RES);

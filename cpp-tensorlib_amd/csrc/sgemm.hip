@@ -163,8 +163,7 @@ __global__ __launch_bounds__(256) void sgemm_sum_kernel(const float* __restrict_
                                                         size_t n, int S, float scale, float offset, int epi) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  float a = part[i];
-  for (int s = 1; s < S; s++) a += part[(size_t)s * n + i];
+  const float a = sum_parts(S, [&](int s) { return part[(size_t)s * n + i]; });
   C[i] = epi ? add_rn(mul_rn(a, scale), offset) : a;
 }
 
