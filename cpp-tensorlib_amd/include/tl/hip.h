@@ -570,10 +570,9 @@ struct context {
     return &e->derived.back();
   }
   // device -> staging
-  bool pull(extent& e) {
-    const bool ok = f.memcpy_d2h(e.staging, e.base, e.size) == 0;
+  void pull(extent& e) {
+    f.memcpy_d2h(e.staging, e.base, e.size);
     e.live = extent::side::either;
-    return ok;
   }
 };
 
@@ -705,10 +704,9 @@ inline void sync_to_host(void* native, bool for_write) {
   auto& c = context::get();
   extent* e = c.ready ? c.buffers.containing(native) : nullptr;
   if (!e) return;
-  // (the copy back waits for what is queued: a wait of its own before it is 5 to 10 us per decode step)
-  if (e->staging && e->live == extent::side::device && c.pull(*e)) c.pending = false;
   if (c.pending) flush();
   if (!e->staging) return;
+  if (e->live == extent::side::device) c.pull(*e);
   if (for_write) e->live = extent::side::staging;
 }
 
