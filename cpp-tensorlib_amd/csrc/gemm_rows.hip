@@ -16,6 +16,12 @@
 // int4: a lane's 16-byte load is the 32 weights of ONE scale group; four groups lie in the four lane quarters
 // and are traded (two swaps of lane halves, two of 16-lane rows, for four steps) so that a step multiplies one
 // group: its sums start at zero and join the accumulators times the group's scale, as in gemm_bf16_nt_kernel.
+//
+// int4 above 64 rows (RANGED): the other kernels for these products scale every row of A by its exponent, so a row of
+// any finite magnitude comes out right there, while three bf16 terms as they are lose their last bits below 2^-110 and
+// a group's sum of 256 times the magnitude overflows above 2^119. Both show in the results, as values that are not
+// finite or as four in a row that are tiny. Only then does a block look for its rows' largest magnitudes, and only where
+// one is outside 2^-100 .. 2^100 does it multiply once more with scaled rows and store what comes out of that.
 #include <type_traits>
 
 #include "gemm_shared.hpp"
@@ -70,7 +76,7 @@ __device__ __forceinline__ f32x4 mma(const frag16& a, const frag16& b, f32x4 c) 
 // Grid: x = row blocks (fastest) x column tiles, y = K-split parts of `part_units` units (bf16: steps of 32 k,
 // int4: 128 k); part y goes to C + y * M * ldc. N, ff, GU and the order of a gated tile's columns as in
 // gemm_bf16_nt_kernel: a tile's first 8 TN columns are gate features, the rest the same features' up rows.
-template <int TM, int TN, bool GU, bool Q4>
+template <int TM, int TN, bool GU, bool Q4, bool RANGED>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* __restrict__ A, const void* __restrict__ W,
                                                                   const float* __restrict__ scales, float* __restrict__ C,
                                                                   int M, int N, int K, int part_units, int ldc, int ff,
@@ -116,12 +122,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
   const char* Sb = reinterpret_cast<const char*>(scales);
 
   f32x4 acc[TM][TN];
-#pragma unroll
-  for (int t = 0; t < TM; t++)
-#pragma unroll
-    for (int j = 0; j < TN; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float row_scale[TM];                             // RANGED: of this lane's row in each row tile
 
-  if (mine > 0) {
+  // the wavefront's share of the product into acc; scaled: A's rows times row_scale
+  auto multiply = [&](auto scaled) {
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (mine == 0) return;
     auto load_a = [&](int u, uint32_t step) {      // u: slot, step: of 32 k
 #pragma unroll
       for (int t = 0; t < TM; t++)
@@ -134,7 +143,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
     auto landed = [](auto n) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory"); };
     auto cut = [&](int u, int t, frag16 p[3]) {
       const char* at = ring + u * kSlot + t * 2048;
-      split3(*reinterpret_cast<const f32x4*>(at + frag[0]), *reinterpret_cast<const f32x4*>(at + frag[1]), p);
+      f32x4 x0 = *reinterpret_cast<const f32x4*>(at + frag[0]), x1 = *reinterpret_cast<const f32x4*>(at + frag[1]);
+      if constexpr (decltype(scaled)::value) {
+        x0 *= row_scale[t];
+        x1 *= row_scale[t];
+      }
+      split3(x0, x1, p);
     };
     if constexpr (!Q4) {
       frag16 w[ST][TN];
@@ -272,7 +286,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
         else unit(1, it, std::false_type{});
       }
     }
-  }
+  };
 
   // acc[t][j][v] of lane l: row 16 t + 4 (l / 16) + v, column 16 j + l % 16. Wavefronts 4..7 hand theirs to 0..3,
   // whose four sums everyone then adds up.
@@ -284,20 +298,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
 #pragma unroll
         for (int v = 0; v < 4; v++) dst[(16 * t + 4 * quarter + v) * LD + 16 * j + r16] = acc[t][j][v];
   };
-  __syncthreads();                                 // (the sums take the place of activations that other wavefronts read)
   float* slot = red + (size_t)(wave & 3) * BM * LD;
-  if (wave >= 4) put(slot);
-  __syncthreads();
-  if (wave < 4) {
-#pragma unroll
-    for (int t = 0; t < TM; t++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[t][j][v] += slot[(16 * t + 4 * quarter + v) * LD + 16 * j + r16];
-    put(slot);                                     // (the lane's own entries: nobody else reads them before the barrier)
-  }
-  __syncthreads();
   const bool wide = (ldc & 3) == 0;
   auto total = [&](int row, int col) {
     f32x4 x[4];
@@ -314,32 +315,102 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
         if (e < left) dst[e] = o[e];
     }
   };
-  if (GU && gridDim.y == 1) {
-    for (int i = tid; i < BM * (BN / 8); i += 64 * kWaves) {
-      const int row = i / (BN / 8), c = i % (BN / 8) * 4, gm = m0 + row, f = (n0 >> 1) + c;
-      if (gm >= M || f >= N) continue;
-      const f32x4 g = total(row, c), u = total(row, c + BN / 2);
-      f32x4 o;
+  auto odd = [](const f32x4& o) {                  // RANGED: not finite, or nothing but tiny values
+    const float m = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3])));
+    const float z = (o[0] + o[1]) * 0.f + (o[2] + o[3]) * 0.f;
+    return m < 0x1p-40f || z != 0.f;
+  };
+  int* found = reinterpret_cast<int*>(red + 4 * BM * LD);   // RANGED: two words behind the sums
+  static_assert(!RANGED || (4 * BM * LD + 2) * 4 <= lds_bytes(TM, TN, Q4), "room for the words");
+  auto any_of_block = [&](bool mine_too, int word) {
+    if (mine_too) found[word] = 1;
+    __syncthreads();
+    return found[word] != 0;
+  };
+  // the wavefronts' sums joined and stored; true where a sum of this thread's is odd
+  auto finish = [&] {
+    bool o_dd = false;
+    __syncthreads();                               // (the sums take the place of activations that other wavefronts read)
+    if (RANGED && tid < 2) found[tid] = 0;
+    if (wave >= 4) put(slot);
+    __syncthreads();
+    if (wave < 4) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) o[e] = (g[e] * (1.0f / (1.0f + expf(-g[e])))) * u[e];   // swiglu_kernel's arithmetic
-      store(C + (size_t)gm * ldc + f, o, N - f);
+      for (int t = 0; t < TM; t++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) acc[t][j][v] += slot[(16 * t + 4 * quarter + v) * LD + 16 * j + r16];
+      put(slot);                                   // (the lane's own entries: nobody else reads them before the barrier)
     }
-    return;
-  }
-  for (int i = tid; i < BM * (BN / 4); i += 64 * kWaves) {
-    const int row = i / (BN / 4), c = i % (BN / 4) * 4, gm = m0 + row, gn = n0 + c;
-    if (gm >= M || (!GU && gn >= N)) continue;     // gated parts are whole tiles wide
-    store(C + (size_t)gm * ldc + gn, total(row, c), GU ? 4 : N - gn);
+    __syncthreads();
+    if (GU && gridDim.y == 1) {
+      for (int i = tid; i < BM * (BN / 8); i += 64 * kWaves) {
+        const int row = i / (BN / 8), c = i % (BN / 8) * 4, gm = m0 + row, f = (n0 >> 1) + c;
+        if (gm >= M || f >= N) continue;
+        const f32x4 g = total(row, c), u = total(row, c + BN / 2);
+        if (RANGED) o_dd |= odd(g) || odd(u);
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = (g[e] * (1.0f / (1.0f + expf(-g[e])))) * u[e];   // swiglu_kernel's arithmetic
+        store(C + (size_t)gm * ldc + f, o, N - f);
+      }
+    } else {
+      for (int i = tid; i < BM * (BN / 4); i += 64 * kWaves) {
+        const int row = i / (BN / 4), c = i % (BN / 4) * 4, gm = m0 + row, gn = n0 + c;
+        if (gm >= M || (!GU && gn >= N)) continue;   // gated parts are whole tiles wide
+        const f32x4 o = total(row, c);
+        if (RANGED) o_dd |= odd(o);
+        store(C + (size_t)gm * ldc + gn, o, GU ? 4 : N - gn);
+      }
+    }
+    return o_dd;
+  };
+  multiply(std::false_type{});
+  if constexpr (!RANGED) {
+    finish();
+  } else if (any_of_block(finish(), 0)) {
+    int ex[TM];
+    bool far = false;
+#pragma unroll
+    for (int t = 0; t < TM; t++) {                 // the largest magnitude of what this wavefront cuts of a row
+      const char* row = Ab + (size_t)min(m0 + 16 * t + r16, M - 1) * K * 4 + quarter * 32;
+      uint32_t m = 0;
+#pragma unroll 1
+      for (int i = 0; i < 4 * mine; i++) {
+        const uint4* x = reinterpret_cast<const uint4*>(row + (size_t)(4 * (first + kWaves * (i >> 2)) + (i & 3)) * 128);
+        const uint4 x0 = x[0], x1 = x[1];
+        m = max(m, max(max(x0.x & 0x7fffffffu, x0.y & 0x7fffffffu), max(x0.z & 0x7fffffffu, x0.w & 0x7fffffffu)));
+        m = max(m, max(max(x1.x & 0x7fffffffu, x1.y & 0x7fffffffu), max(x1.z & 0x7fffffffu, x1.w & 0x7fffffffu)));
+      }
+      m = max(m, (uint32_t)__shfl_xor((int)m, 16));
+      m = max(m, (uint32_t)__shfl_xor((int)m, 32));
+      far |= m != 0u && (m < __float_as_uint(0x1p-100f) || m > __float_as_uint(0x1p100f));
+      ex[t] = row_exponent((int)(m >> 23), m == 0u);
+      row_scale[t] = pow2f(ex[t]);
+    }
+    if (!any_of_block(far, 1)) return;             // zeros, or weights that are
+    __syncthreads();                               // (the words lie where copies are about to land)
+    multiply(std::true_type{});
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int e = __shfl(ex[t], 4 * quarter + v);   // the exponent of row 16 t + 4 quarter + v comes back out
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[t][j][v] = ldexpf(acc[t][j][v], -e);
+      }
+    finish();
   }
 }
 
-template <int TM, int TN, bool GU, bool Q4>
+template <int TM, int TN, bool GU, bool Q4, bool RANGED = false>
 int run(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int M, int N, int K, int ldc, int ff) {
   constexpr int lds = lds_bytes(TM, TN, Q4);
-  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows_kernel<TM, TN, GU, Q4>),
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows_kernel<TM, TN, GU, Q4, RANGED>),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
-  gemm_rows_kernel<TM, TN, GU, Q4><<<dim3((unsigned)(P.tiles * P.row_blocks), (unsigned)P.S), dim3(64 * kWaves), lds, ctx().stream>>>(
+  gemm_rows_kernel<TM, TN, GU, Q4, RANGED><<<dim3((unsigned)(P.tiles * P.row_blocks), (unsigned)P.S), dim3(64 * kWaves), lds, ctx().stream>>>(
       A, W, scales, C, M, N, K, P.part_units, ldc, ff, P.row_blocks);
   return TLHIP_OK;
 }
@@ -347,18 +418,34 @@ int run(const RowsPlan& P, const float* A, const void* W, const float* scales, f
 template <int TM>
 int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int M, int N, int K, int ldc, int ff, bool gu) {
   const bool q4 = scales != nullptr;
+  if constexpr (TM >= 3) {                         // more than 64 rows are blocks of three to five row tiles
+    if (q4 && M > 64) {
+      switch (P.TN + (gu ? 16 : 0)) {
+        case 1: return run<TM, 1, false, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+        case 2: return run<TM, 2, false, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+        case 18: return run<TM, 2, true, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      }
+      return fail(TLHIP_EUNSUPPORTED, "gemm_rows: no kernel for this plan");
+    }
+  }
   switch (P.TN + (gu ? 16 : 0) + (q4 ? 32 : 0)) {   // (int4 over four column tiles: the registers hold one row tile)
     case 1: return run<TM, 1, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
     case 2: return run<TM, 2, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
     case 4: return run<TM, 4, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
     case 18: return run<TM, 2, true, false>(P, A, W, scales, C, M, N, K, ldc, ff);
     case 20: return run<TM, 4, true, false>(P, A, W, scales, C, M, N, K, ldc, ff);
-    case 33: return run<TM, 1, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
-    case 34: return run<TM, 2, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 33:
+      if constexpr (TM <= 4) return run<TM, 1, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      break;
+    case 34:
+      if constexpr (TM <= 4) return run<TM, 2, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      break;
     case 36:
       if constexpr (TM == 1) return run<TM, 4, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;
-    case 50: return run<TM, 2, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 50:
+      if constexpr (TM <= 4) return run<TM, 2, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      break;
     case 52:
       if constexpr (TM == 1) return run<TM, 4, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;

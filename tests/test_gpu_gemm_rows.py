@@ -82,3 +82,32 @@ def test_whole_numbers_are_exact_and_columns_land_where_they_belong(lib, orc):
         assert np.array_equal(out.numpy().astype(np.float64), A.astype(np.float64) @ Wf.astype(np.float64).T), (M, N, K)
         for b in (da, dw, out):
             b.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 896, 896), (77, 301, 896), (96, 260, 2048), (128, 900, 384)])
+def test_int4_rows_of_any_magnitude(lib, orc, M, N, K):
+    """Above 64 rows an int4 product holds rows of any finite magnitude, denormal ones too, beside ordinary ones and rows
+    of zeros, whichever kernel forms it. Results below 2^-126 keep what a denormal holds, once per part of the sum."""
+    print("case gemm_rows magnitudes", M, N, K, flush=True)
+    w, W = _weights(orc, "q4", N, K, 25)
+    da, dw, out, parts = lib.empty((M, K)), lib.to_device(w), lib.empty((M, N)), lib.empty((16, M, N))
+    for exps in (np.linspace(-140, 126, M), np.where(np.arange(M) % 9 == 4, 124, 0), np.where(np.arange(M) == M - 1, -130, 0)):
+        A = np.clip(orc.normal(M * K, 26).reshape(M, K), -1.9, 1.9).astype(np.float64) * 2.0 ** np.round(exps)[:, None]
+        A[3], A[7, : K // 2] = 0.0, 0.0
+        A = A.astype(np.float32)
+        want, slack = A.astype(np.float64) @ W.T, _slack(A.astype(np.float64), W, K) + 20 * 2.0 ** -149
+        lib.gemm_q4_nt(da.upload(A), dw, out, M, N, K)
+        assert np.all(np.abs(out.numpy() - want) <= slack)
+        n = lib.gemm_q4_nt_parts(da, dw, parts, M, N, K)
+        assert np.all(np.abs(parts.numpy()[:n].astype(np.float64).sum(0) - want) <= slack)
+    ff = N // 2
+    A = np.where(np.abs(exps)[:, None] > 0, A * np.float32(2.0 ** 60), A * np.float32(2.0 ** -120))
+    p, s = A.astype(np.float64) @ W[:2 * ff].T, _slack(A.astype(np.float64), W[:2 * ff], K)
+    g, u, sg, su = p[:, :ff], p[:, ff:], s[:, :ff], s[:, ff:]
+    act, packed = g / (1 + np.exp(-g)), w[:2 * ff * K // 2]
+    dw.upload(np.concatenate([packed, w[N * K // 2:][:2 * ff * K // 8]]))
+    gated = lib.empty((M, ff))
+    lib.gemm_q4_nt_swiglu(da.upload(A), dw, gated, M, ff, K)
+    assert np.all(np.abs(gated.numpy() - act * u) <= 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u) + 2.0 ** -149)
+    for b in (da, dw, out, parts, gated):
+        b.free()
