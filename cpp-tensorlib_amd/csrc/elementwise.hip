@@ -290,7 +290,8 @@ int tlhip_gemm(const void* a, int64_t a_off, int64_t lda, int ta, const void* b,
   // product is whole 128 x 128 tiles of aligned rows and at least two of them tall, where the LDS-tiled kernel reads
   // each operand once per tile (512 x 4608 x 3584: 215 us against 258; but 333 x 4864 x 896: 66 against 46).
   const bool whole = m >= 256 && (m % 128) == 0 && (n % 128) == 0 && (k % 16) == 0 && (lda % 4) == 0 && (ldb % 4) == 0 && aligned16(pa) && aligned16(pb);
-  if (!ta && k >= 16 && m <= 1024 && !whole && (m + 15) / 16 * ((n + 63) / 64) < 0x7fffffff) {
+  // (2^23 blocks of 512 threads are what a grid's x can count)
+  if (!ta && k >= 16 && m <= 1024 && !whole && (m + 15) / 16 * ((n + 63) / 64) < (1 << 23)) {
     const int rc = launch_sgemm_rows(pa, lda, pb, ldb, tb, po, (int)m, (int)n, (int)k, scale, offset, epi);
     if (rc != 0) return rc;
     TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM);

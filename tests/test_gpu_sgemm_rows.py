@@ -55,3 +55,17 @@ def test_strided_views_and_byte_offsets(lib, orc):
     assert np.array_equal(out.numpy()[3:].reshape(M, N).astype(np.float64), want)
     for b in (da, db, out):
         b.free()
+
+
+def test_more_columns_than_a_grid_of_its_blocks_counts(lib, orc):
+    """2^29 columns and a few: one row of B is read for all of them (a row stride of zero), so only the result is large."""
+    N, K = (1 << 29) + 70, 16
+    a, b = np.arange(1, K + 1, dtype=np.float32), np.arange(K, dtype=np.float32) - 5
+    da, db, out = lib.to_device(a), lib.to_device(b), lib.empty_bytes(N * 4)
+    lib.gemm(da, K, 0, db, 0, 1, out, 1, N, K)
+    for first in (0, (1 << 28) - 7, N - 1000):
+        got = np.empty(1000, np.float32)
+        lib._chk(lib.c.tlhip_memcpy_d2h(got.ctypes.data, out.ptr + first * 4, got.nbytes))
+        assert np.all(got == a @ b), first
+    for x in (da, db, out):
+        x.free()
