@@ -14,6 +14,7 @@
 // 4 wavefronts (2 x 2) per block, 128 x 128 block tile, 64 x 64 per wavefront (2 x 2 MFMA
 // tiles, 64 accumulator registers), K slabs of 16; the next slab's global loads are in
 // flight while the current one is multiplied.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -385,9 +386,10 @@ __global__ __launch_bounds__(64 * kSrWaves, 2) void sgemm_rows_kernel(const floa
   }
 }
 
-// The same for A as it is stored ([M][K]); the caller has checked the arguments.
+// The same for A as it is stored ([M][K]); the caller has checked the arguments. tiled: the LDS-tiled kernel takes the
+// product too; 1 is returned, and nothing launched, where it is the better one.
 int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb, int tb, float* pc, int M, int N, int K, float scale,
-                      float offset, int epi) {
+                      float offset, int epi, bool tiled) {
   // Row blocks and K splits (parts in scratch, summed in a fixed order) that an estimate in clocks likes best: a block
   // takes 1600 clocks per row tile and 128 k, and 6000 to start and end; blocks run one to a CU, so tiles that make a
   // round and a bit are cut smaller until they make whole rounds; parts are written and read at 2.5 KB a clock, and their
@@ -403,6 +405,13 @@ int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb
       const double t = rounds * (steps * 1600 * tm + 6000) + (s > 1 ? 11000 + 8.0 * s * M * N / 2500 : 0);
       if (least < 0 || t < least) { least = t; rb = r; TM = tm; S = s; }
     }
+  }
+  // With fewer than 256 k there is nothing to split, and blocks in several rounds each start and end for two steps or
+  // less. The LDS-tiled kernel's time there, measured from 128 x 128 to 1024 x 9000: 6 us and 1.5 for every 16 k, over
+  // 256 tiles in proportion (986 x 7459 x 22: 15 us, 42 here; 614 x 4098 x 29 9.8 and 17; 300 x 2000 x 60 11 and 7.6).
+  if (tiled && K < 256) {
+    const double tiles128 = (double)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
+    if (least > 2100 * (6 + 1.5 * ((K + 15) / 16) * std::max(1.0, tiles128 / 256))) return 1;
   }
   const int64_t tiles = rb * columns;
   int kchunk = K;
