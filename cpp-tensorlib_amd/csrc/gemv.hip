@@ -102,7 +102,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   const int groups = nw / KW;        // wavefront row groups per block tile
   const int rows_per_tile = groups * QN * R;
   const int wrow = (wn * QN + q) * R;  // this lane's first row inside a tile
-  float* psum = fw;                                         // sums of squares (then 1 / rms, where a block reads the row again): post-norm producer
+  float* psum = fw;                                         // sums of squares (kPostnormLong: then 1 / rms): post-norm producers
   constexpr bool kPair = EPI != kStore;
   const auto act = [&](float g, float u, int i) {
     return EPI == kGeglu ? gelu_tanh(g + pro.gu_bias[i]) * (u + pro.gu_bias[N / 2 + i]) : gated(g, u);
@@ -120,7 +120,8 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   const float4* d4 = reinterpret_cast<const float4*>(pro.delta);
   // float4s a thread requests up front: all of x up to 20 floats per thread (K = 18944 on 1024
   // threads), 8 per thread in the norm form, whose vector is the hidden size (registers)
-  constexpr int PL = PRO == kRmsnorm || PRO == kPostnorm ? 2 : 5;
+  constexpr bool kPost = PRO == kPostnorm || PRO == kPostnormLong;
+  constexpr int PL = PRO == kRmsnorm || kPost ? 2 : 5;
   float4 px[PL], pa[PL], pn[PL], pb[PL];
   // attention-merge producer: this thread's first float4 of the first kPre splits' accumulators, and
   // the (head, split) pair whose maximum and sum it weighs
@@ -144,8 +145,8 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       const int i = min(tid + k * (int)blockDim.x, n4 - 1);
       if (PRO != kAttnMerge) px[k] = x4[i];
       if (PRO != kPlain && PRO != kAttnMerge) pa[k] = aux4[i];
-      if (PRO == kRmsnorm || PRO == kPostnorm) pn[k] = reinterpret_cast<const float4*>(pro.norm_w)[i];
-      if (PRO == kPostnorm && pro.bias) pb[k] = reinterpret_cast<const float4*>(pro.bias)[i];
+      if (PRO == kRmsnorm || kPost) pn[k] = reinterpret_cast<const float4*>(pro.norm_w)[i];
+      if (kPost && pro.bias) pb[k] = reinterpret_cast<const float4*>(pro.bias)[i];
     }
   }
   asm volatile("" ::: "memory");
@@ -196,38 +197,35 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     __syncthreads();
   }
 
-  // Post-norm producer: 1 / rms of every run. Where the threads hold the row (and runs end at half a wavefront's 128
-  // values) the squares are summed from the registers requested above: read again, behind the first weights, they kept
-  // the block waiting for those (in a step's trace 9728 x 896 gated 8.4 -> 7.8 us, 3868 x 896 5.4 -> 4.2).
-  bool held = false;
-  float inv_all = 0.f;                 // held, one run
+  // Post-norm producer: 1 / rms of every run, summed from the registers requested above (runs end at half a wavefront's
+  // 128 values): read again, behind the first weights, they kept the block waiting for those (in a step's trace 9728 x 896
+  // gated 8.4 -> 7.8 us, 3868 x 896 5.4 -> 4.2).
+  float inv_all = 0.f;                 // of one run
   if constexpr (PRO == kPostnorm) {
-    held = n4 <= PL * (int)blockDim.x && (pro.parts == 1 || pro.part_len % 128 == 0);
-    if (held) {
-      const int n = pro.parts * pro.part_len;
+    const int n = pro.parts * pro.part_len;
 #pragma unroll
-      for (int k = 0; k < PL; k++) {
-        const int e = 4 * (tid + k * (int)blockDim.x);
-        float4 v = pa[k];
-        if (pro.bias) { v.x += pb[k].x; v.y += pb[k].y; v.z += pb[k].z; v.w += pb[k].w; }
-        float ss = e < n ? v.x * v.x : 0.f;
-        ss = e + 1 < n ? fmaf(v.y, v.y, ss) : ss;
-        ss = e + 2 < n ? fmaf(v.z, v.z, ss) : ss;
-        ss = e + 3 < n ? fmaf(v.w, v.w, ss) : ss;
-        const LanePair p = swap16(ss, ss);
-        ss = p.first + p.second;
-        ss = dpp_add_f32<0x140>(dpp_add_f32<0x141>(dpp_add_f32<0x4E>(dpp_add_f32<0xB1>(ss))));
-        if ((lane & 31) == 0) psum[2 * (wave + k * nw) + (lane >> 5)] = ss;   // of values 128 (this index) ..
-      }
-      __syncthreads();
-      if (pro.parts == 1) {
-        const float t = wave_sum(lane < 2 * PL * nw ? psum[lane] : 0.f);
-        inv_all = 1.0f / sqrtf(t / (float)pro.part_len + pro.eps);
-      }
+    for (int k = 0; k < PL; k++) {
+      const int e = 4 * (tid + k * (int)blockDim.x);
+      float4 v = pa[k];
+      if (pro.bias) { v.x += pb[k].x; v.y += pb[k].y; v.z += pb[k].z; v.w += pb[k].w; }
+      float ss = e < n ? v.x * v.x : 0.f;
+      ss = e + 1 < n ? fmaf(v.y, v.y, ss) : ss;
+      ss = e + 2 < n ? fmaf(v.z, v.z, ss) : ss;
+      ss = e + 3 < n ? fmaf(v.w, v.w, ss) : ss;
+      const LanePair p = swap16(ss, ss);
+      ss = p.first + p.second;
+      ss = dpp_add_f32<0x140>(dpp_add_f32<0x141>(dpp_add_f32<0x4E>(dpp_add_f32<0xB1>(ss))));
+      if ((lane & 31) == 0) psum[2 * (wave + k * nw) + (lane >> 5)] = ss;   // of values 128 (this index) ..
+    }
+    __syncthreads();
+    if (pro.parts == 1) {
+      const float t = wave_sum(lane < 2 * PL * nw ? psum[lane] : 0.f);
+      inv_all = 1.0f / sqrtf(t / (float)pro.part_len + pro.eps);
     }
   }
-  // Else a run is summed by `seg` wavefronts where there are fewer runs than wavefronts, in a fixed order.
-  if (PRO == kPostnorm && !held) {
+  // In a pass of their own a run's squares are summed by `seg` wavefronts where there are fewer runs than wavefronts, in a
+  // fixed order.
+  if constexpr (PRO == kPostnormLong) {
     const int seg = pro.parts < nw ? nw / pro.parts : 1, sums = pro.parts * seg, len = pro.part_len;
     for (int s = wave; s < sums; s += nw) {
       const int p = s / seg, b = p * len;
@@ -282,14 +280,14 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       if (!have) {
         v = x4[i];
         if (PRO == kSwiglu) aux = x4[n4 + i];
-        if (PRO == kRmsnorm || PRO == kPostnorm) { nv = reinterpret_cast<const float4*>(pro.norm_w)[i]; if (d4) aux = d4[i]; }
-        if (PRO == kPostnorm && pro.bias) ab = reinterpret_cast<const float4*>(pro.bias)[i];
+        if (PRO == kRmsnorm || kPost) { nv = reinterpret_cast<const float4*>(pro.norm_w)[i]; if (d4) aux = d4[i]; }
+        if (kPost && pro.bias) ab = reinterpret_cast<const float4*>(pro.bias)[i];
       }
-      if constexpr (PRO == kPostnorm) {
+      if constexpr (kPost) {
         if (pro.bias) { aux.x += ab.x; aux.y += ab.y; aux.z += ab.z; aux.w += ab.w; }
         const int last = pro.parts - 1;
         float i0 = inv_all, i1 = inv_all, i2 = inv_all, i3 = inv_all;
-        if (!held) {
+        if constexpr (PRO == kPostnormLong) {
           const auto inv_of = [&](int e) { return psum[last == 0 ? 0 : min(e / pro.part_len, last)]; };
           i0 = inv_of(4 * i), i1 = inv_of(4 * i + 1), i2 = inv_of(4 * i + 2), i3 = inv_of(4 * i + 3);
         } else if (last > 0) {           // four values lie in one run
@@ -333,7 +331,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
           if (pro.xout && blockIdx.x == 0) reinterpret_cast<float4*>(pro.xout)[i] = v;
           v.x *= nv.x; v.y *= nv.y; v.z *= nv.z; v.w *= nv.w;
         }
-        if (PRO == kPostnorm && pro.xout && blockIdx.x == 0) reinterpret_cast<float4*>(pro.xout)[i] = v;
+        if (kPost && pro.xout && blockIdx.x == 0) reinterpret_cast<float4*>(pro.xout)[i] = v;
       }
       const int u = i / J, j = i - u * J;
       if (live) xs[((u / LPR) * J + j) * XS + (u & (LPR - 1))] = Fmt::stage(v);
@@ -637,7 +635,7 @@ static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int pro, int cus, int lds
   RowCfg c{};
   const double waste64 = (double)((upr + 63) / 64 * 64) / upr, waste16 = (double)((upr + 15) / 16 * 16) / upr;
   // (a bf16 row has four times the units: 64 lanes up to twice the row's; 3072 x 768 3.4 us against 4.1 with 16)
-  int lpr = (waste64 >= (E == 8 && N / cus < 17 ? 2.0 : 1.3) && waste16 < waste64) ? 16 : 64;
+  int lpr = (waste64 >= (E == 8 && pro != kPostnormLong && N / cus < 17 ? 2.0 : 1.3) && waste16 < waste64) ? 16 : 64;
   if (tn.lpr == 16 || tn.lpr == 64) lpr = tn.lpr;
   const int qn = 64 / lpr;
   const int chunks = (upr + lpr - 1) / lpr;
@@ -671,24 +669,29 @@ static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int pro, int cus, int lds
     KW /= 2;
     if (R > 1) R /= 2; else if (nw > 4) nw /= 2;
   }
-  if (E == 8 && lpr == 64 && xbytes + 8192 <= (size_t)lds_per_cu) {
+  if (E == 8 && lpr == 64 && pro != kPostnormLong && xbytes + 8192 <= (size_t)lds_per_cu) {
     // bf16, whose rows are long for their number (us before -> now; cold weights):
     //  * up to 16 rows per CU: one tile per CU of its share of the rows, four to a wavefront, and K over as many
     //    wavefronts as the block takes, where they get as many chunks each (16 rows and two splits left half the CUs of
     //    2048 x 12288 without a tile: 12.3 -> 9.8; 2048 x 4096 8.4 -> 7.2, 2048 x 2048 4.7 -> 3.9, 896 x 4864 4.9 -> 4.3,
     //    3392 x 2048 7.4 -> 6.7; 3584 x 3584, seven chunks over four, would be 6.9 for 6.6);
-    //  * up to 31 rows and three chunks: the same without the split, whose halves are uneven (5376 x 1536 6.2 -> 5.4);
+    //    Not for one row per CU behind a gate, whose two wavefronts would be slow to form x (256 x 1024 3.4 -> 3.5);
+    //  * up to 31 rows and three chunks: the same without the split, whose halves are uneven (5376 x 1536 6.2 -> 5.4). The
+    //    halves of two chunks are even, which a plain x gains from (5120 x 896 4.5 with the split, 4.7 without);
     //  * 32 to 127 rows: small blocks, whose ends fall apart in time, as long as they hold x in what a thread requests up
     //    front (18960 x 2048 15.9 -> 14.0, 32000 x 2048 23.4 -> 21.8, 9728 x 896 6.5 -> 6.0), else of eight wavefronts
     //    (33000 x 3584: 37.4 so, 38.9 with four, 39.8 with one such block per CU). The post-norm's sums are every block's
     //    own, so few large ones there (16496 x 3584 24.2 -> 21.9, 24.8 with small ones; 10304 x 2048 12.4 -> 10.7, 9728 x 896 gated 8.8 -> 7.9).
+    //    Blocks that form x anew from memory (normed, over 8192 long) or at length (gated, short rows) stay few: 8192 x 14336
+    //    normed 40.4 and 43.1 so, 8192 x 896 gated 5.6 and 6.1.
+    // A post-norm whose row no block holds keeps the shapes above: 1024 x 12288 15.5 us, 16.7 in these.
     const int rows = (int)std::min<int64_t>((N + cus - 1) / cus, 1 << 20), groups = (rows + 3) / 4;
-    if (rows <= 16) {
+    if (rows <= 16 && !(pro == kSwiglu && rows <= 1)) {
       const int kw = std::min(16 / groups, chunks);
       if ((chunks + kw - 1) / kw * kw * 10 <= chunks * 11) { R = 4; KW = kw; nw = groups * kw; want_bpc = 1; }
-    } else if (rows < 32) {
-      if (chunks <= 3) { R = 4; KW = 1; nw = groups; want_bpc = 2; }
-    } else if (rows_per_cu >= 32 && rows_per_cu < 128) {
+    } else if (rows > 16 && rows < 32) {
+      if (chunks <= 3 && (chunks != 2 || pro != kPlain)) { R = 4; KW = 1; nw = groups; want_bpc = 2; }
+    } else if (rows_per_cu >= 32 && rows_per_cu < 128 && !(pro == kRmsnorm && upr > 1024) && !(pro == kSwiglu && chunks <= 2)) {
       R = 2; KW = 1;
       nw = pro == kPostnorm ? 12 : upr <= 256 ? 4 : 8;
       want_bpc = pro == kPostnorm ? 2 : 16 / nw;
@@ -750,12 +753,22 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
   if (EPI != kStore && N > max_rows) return fail(TLHIP_EUNSUPPORTED, "gemv: gate|up matrix too large for one launch");
   for (int64_t n0 = 0; n0 < N; n0 += max_rows) {
     const int64_t n = N - n0 < max_rows ? N - n0 : max_rows;
-    RowCfg cfg = pick_rows_cfg(n, upr, Fmt::E, PRO, c.cus, c.lds_per_cu, tn);
-    if (EPI != kStore && cfg.R == 1) {   // a lane group needs a gate row and its up row
-      RowTune two = tn;
-      two.R = 2;
-      if (cfg.nw / cfg.KW >= 2 && cfg.nw > 4) two.nw = cfg.nw / 2;   // keeps the rows of a block tile
-      cfg = pick_rows_cfg(n, upr, Fmt::E, PRO, c.cus, c.lds_per_cu, two);
+    const auto pick = [&](int producer) {
+      RowCfg g = pick_rows_cfg(n, upr, Fmt::E, producer, c.cus, c.lds_per_cu, tn);
+      if (EPI != kStore && g.R == 1) {   // a lane group needs a gate row and its up row
+        RowTune two = tn;
+        two.R = 2;
+        if (g.nw / g.KW >= 2 && g.nw > 4) two.nw = g.nw / 2;   // keeps the rows of a block tile
+        g = pick_rows_cfg(n, upr, Fmt::E, producer, c.cus, c.lds_per_cu, two);
+      }
+      return g;
+    };
+    RowCfg cfg = pick(PRO);
+    bool held = false;                   // the post-norm's row, by the threads of a block of this shape
+    if constexpr (PRO == kPostnorm) {
+      const auto holds = [&] { return upr * (Fmt::E / 4) <= 2 * 64 * cfg.nw && (pro.parts == 1 || pro.part_len % 128 == 0); };
+      if (!holds()) cfg = pick(kPostnormLong);
+      held = holds();
     }
     if (PRO == kAttnMerge) cfg.lds += (size_t)pro.heads * (kMergeMax + 1) * sizeof(float);
     if (PRO == kPostnorm) cfg.lds += (size_t)std::max(std::max(pro.parts, cfg.nw) + pro.parts, 4 * cfg.nw) * sizeof(float);
@@ -763,6 +776,8 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
     const int rows_per_tile = (cfg.nw / cfg.KW) * (64 / cfg.lpr) * cfg.R;
     const int ntiles = (int)((n + rows_per_tile - 1) / rows_per_tile);
     auto fn = cfg.lpr == 16 ? pick_rows_fn<Fmt, PRO, 16, EPI>(cfg.R) : pick_rows_fn<Fmt, PRO, 64, EPI>(cfg.R);
+    if constexpr (PRO == kPostnorm)
+      if (!held) fn = cfg.lpr == 16 ? pick_rows_fn<Fmt, kPostnormLong, 16, EPI>(cfg.R) : pick_rows_fn<Fmt, kPostnormLong, 64, EPI>(cfg.R);
     if (!fn) return fail(TLHIP_EINVAL, "rows per wavefront must be 1, 2, 4 or 8");
     if (cfg.lds > 48 * 1024) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),

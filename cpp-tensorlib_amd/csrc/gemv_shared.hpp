@@ -166,6 +166,9 @@ __device__ __forceinline__ float wave_sum_rows(float (&a)[R], int lane) {
 //   kPostnorm: x = in (when there is one) + (delta + bias) / rms * norm_w, the norm over `parts` runs of part_len
 //             entries, each by its own root mean square; block 0 writes x to xout. The factor is needed before
 //             anything can be staged, so the block meets a barrier for it; the weights are on their way meanwhile.
+//             The block's threads hold the whole row, which is where the squares come from.
+//   kPostnormLong: the same for rows that the threads do not hold, or runs that end inside half a wavefront's 128 values:
+//             the squares come from a pass of their own.
 // How a block leaves its results (EPI):
 //   kStore:  y[row] = dot.
 //   kGateUp: W is [gate rows | up rows] (N/2 each); a lane group owns R/2 gate rows and the
@@ -173,7 +176,7 @@ __device__ __forceinline__ float wave_sum_rows(float (&a)[R], int lane) {
 //            activation in the GEMV that produces it, once per element, instead of in every
 //            block of the GEMV that consumes it.
 //   kGeglu:  as kGateUp with y[i] = gelu_tanh(g + gu_bias[i]) * (u + gu_bias[N/2 + i]).
-enum { kPlain = 0, kSwiglu = 1, kRmsnorm = 2, kAttnMerge = 3, kPostnorm = 4 };
+enum { kPlain = 0, kSwiglu = 1, kRmsnorm = 2, kAttnMerge = 3, kPostnorm = 4, kPostnormLong = 5 };
 constexpr int kMergeMax = 16;  // splits the kAttnMerge producer takes (its lanes per head)
 enum { kStore = 0, kGateUp = 1, kGeglu = 2 };
 __device__ __forceinline__ float gated(float g, float u) { return (g * (1.0f / (1.0f + expf(-g)))) * u; }
@@ -188,7 +191,7 @@ struct Producer {
   float eps;
   // kAttnMerge: x points at the partials [heads*S] m | [heads*S] l | [heads*S][D] acc
   int S = 0, heads = 0, D = 0;
-  // kPostnorm
+  // kPostnorm, kPostnormLong
   const float* bias = nullptr;
   int parts = 0, part_len = 0, add_x = 0;
   // kGeglu

@@ -37,11 +37,15 @@ def test_plain_and_normed(lib, N, K):
     lib.gemv_bf16_row_postnorm(dx, dd, None, dw, K, 1, out, dW, y, N, K, 1e-6)
     n = d.astype(np.float64)
     _near(y.numpy(), W, x + n / np.sqrt(np.mean(n * n) + 1e-6) * w)
+    if K % 56 == 0:                                # runs that do not end at 128 values
+        r = n.reshape(7, -1)
+        lib.gemv_bf16_row_postnorm(dx, dd, None, dw, K, 7, out, dW, y, N, K, 1e-6)
+        _near(y.numpy(), W, x + (r / np.sqrt(np.mean(r * r, axis=1, keepdims=True) + 1e-6)).ravel() * w)
     for b in (dx, dd, dw, dW, y, out):
         b.free()
 
 
-@pytest.mark.parametrize("ff,K", [(1, 64), (1537, 904), (4096, 776), (4097, 2048), (9480, 520), (16200, 136)])
+@pytest.mark.parametrize("ff,K", [(1, 64), (1537, 904), (4096, 776), (4097, 2048), (9480, 520), (16200, 136), (130, 8712), (700, 8200)])
 def test_gated(lib, ff, K):
     print("case bf16 gated rows", ff, K, flush=True)
     bits, W = _weight(2 * ff, K, ff + K)
