@@ -153,8 +153,9 @@ __global__ __launch_bounds__(512) void ssm_step_kernel(const float* __restrict__
     }
   }
 }
-// up to four blocks per CU, and whole slices
-static bool ssm_sliced(const tlhip_ssm& a) { return a.vdim % 16 == 0 && a.heads * (a.vdim / 16) <= 4 * (int64_t)ctx().cus; }
+// up to two blocks per CU, and whole slices (heads of 64 and 128 state rows, us, whole -> slices: 28 6.6 -> 5.1, 112 (448
+// slices) 6.1 -> 6.1, 160 6.4 -> 7.2; 256 heads of 16 state rows 4.9 -> 7.3)
+static bool ssm_sliced(const tlhip_ssm& a) { return a.vdim % 16 == 0 && a.heads * (a.vdim / 16) <= 2 * (int64_t)ctx().cus; }
 static size_t ssm_step_lds(const tlhip_ssm& a) {
   const bool sliced = ssm_sliced(a);
   const int ld = ssm_ld((int)a.vdim), ng = 512 / (ld >> 2);
