@@ -593,18 +593,15 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const tlhip_la
 }
 
 // ---- splits joined, values' up-projection, gate ---------------------------------------------------
-// Block (slice of out_rows value rows, head, TQ <= 4 tokens) of NT threads; G groups of threads share the splits.
+// Block (slice of ROWS value rows, head, TQ <= 4 tokens) of NT threads; G groups of threads share the splits.
 constexpr int kMaxSplits = 64;
-// A single token's blocks take 16 rows on 512 threads: every block joins the splits again (64 KB of a latent of 256), but
-// no thread more than eight of them at once (14 heads of 64 over 256: 7.5 us with 32 rows on 1024 threads, 6.6 so).
-constexpr int out_rows(int TQ) { return TQ == 1 ? 16 : 32; }
 __host__ __device__ inline int out_groups(int NT, int TQ, int LV) { const int n = TQ * (LV / 4); return n >= NT ? 1 : NT / n; }
-template <int TQ, int NT>
+template <int TQ, int NT, int ROWS>
 __global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict__ u, int64_t ldu, float* __restrict__ y, int64_t ldy,
                                                         const tlhip_latent_attn a, const float* __restrict__ part, int T, int S,
                                                         int rows, int slices) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  constexpr int NW = NT / 64, kOutRows = out_rows(TQ);
+  constexpr int NW = NT / 64;
   const Dims d = dims_of(a);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int slice = blockIdx.x % slices, h = blockIdx.x / slices % d.H, t0 = blockIdx.x / slices / d.H * TQ;
@@ -613,9 +610,9 @@ __global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict_
   float* w = oc + G * TQ * LV;         // [TQ][S] the splits' weights
   const size_t R = (size_t)rows;
   const float *pm = part, *pl = part + (size_t)S * R, *pa = pl + (size_t)S * R;
-  const int v1 = min(d.V, (slice + 1) * kOutRows), vw = slice * kOutRows + wave;
+  const int v1 = min(d.V, (slice + 1) * ROWS), vw = slice * ROWS + wave;
   const u32x4* uv = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.uv)) + (size_t)h * d.V * n8;
-  constexpr int PRE = kOutRows / NW < 2 ? 1 : 2;     // rows whose weights are requested up front
+  constexpr int PRE = ROWS / NW < 2 ? 1 : 2;     // rows whose weights are requested up front
   u32x4 pre[PRE];
   float gate[PRE];                     // (of a single token)
 #pragma unroll
@@ -879,9 +876,15 @@ static int launch(const float* u, int64_t ldu, const float* q, int64_t ldq, floa
   if (!fa) return fail(TLHIP_EUNSUPPORTED, "tlhip_latent_attn: latent and rotated dims beyond what the kernel holds");
   const size_t la = kExact ? (size_t)NQ * d.DS * 1024 + 2 * 16 * 1024 : 0;
   if (int rc = allow(reinterpret_cast<const void*>(fa), la)) return rc;
-  const int oslices = (d.V + out_rows(TQ) - 1) / out_rows(TQ), ont = TQ == 1 ? 512 : 256;
+  // A single token's blocks take 16 rows on 512 threads while that is no more than a block per CU and 10 MB of partials that
+  // they read: every block joins all splits again, but no thread more than eight of them at once. (Against 32 rows on 1024
+  // threads: 14 heads of 64 over 256 in 64 splits 6.6 us for 7.5; 20 of 64 over 512 the whole step 1.02 times as fast, 28 of
+  // 128 over 512 0.87 times, 40 of 128 over 256 0.89 times.)
+  const int64_t blocks16 = (int64_t)d.H * ((d.V + 15) / 16);
+  const bool narrow = TQ == 1 && blocks16 <= c.cus && blocks16 * S * LV <= 5 << 19;
+  const int out_rows = narrow ? 16 : 32, oslices = (d.V + out_rows - 1) / out_rows, ont = narrow ? 512 : TQ == 1 ? 1024 : 256;
   const size_t lo = o_mfma ? lom : (size_t)TQ * (out_groups(ont, TQ, LV) * LV + S) * sizeof(float);
-  auto fo = TQ == 1 ? latent_out_kernel<1, 512> : latent_out_kernel<4, 256>;
+  auto fo = narrow ? latent_out_kernel<1, 512, 16> : TQ == 1 ? latent_out_kernel<1, 1024, 32> : latent_out_kernel<4, 256, 32>;
   auto fom = o_vec ? latent_out_mfma_kernel<true> : latent_out_mfma_kernel<false>;
   if (int rc = allow(o_mfma ? reinterpret_cast<const void*>(fom) : reinterpret_cast<const void*>(fo), lo)) return rc;
 
