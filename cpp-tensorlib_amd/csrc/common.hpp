@@ -178,13 +178,18 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 
 // part(0) + part(1) + ... + part(S - 1), added in that order. The parts of a product lie in another die's cache or beyond:
 // requested one by one each was a round trip, so four are at once (77 rows of 896 in up to seven parts normed: 5.6 us, 3.4
-// so and in blocks of 256 threads).
+// so and in blocks of 256 threads). That is more code, which the short kernels that call this feel: PLAIN is the loop, for
+// launches of one or two parts (512 rows of 3584 in two parts normed: 5.6 us, 6.2 in the other form).
 __device__ __forceinline__ float plus(float a, float b) { return a + b; }
 __device__ __forceinline__ float4 plus(const float4& a, const float4& b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-template <typename F>
+template <bool PLAIN = false, typename F>
 __device__ __forceinline__ auto sum_parts(int S, F part) {
   auto a = part(0);
   int s = 1;
+  if constexpr (PLAIN) {
+    for (; s < S; s++) a = plus(a, part(s));
+    return a;
+  }
   for (; s + 4 <= S; s += 4) {
     const auto b = part(s), c = part(s + 1), d = part(s + 2), e = part(s + 3);
     a = plus(plus(plus(plus(a, b), c), d), e);

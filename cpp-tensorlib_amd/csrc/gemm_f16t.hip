@@ -201,12 +201,12 @@ __global__ __launch_bounds__(256) void a_image_kernel(const float* __restrict__ 
 // x and xout may be the same buffer (a thread writes only what it has read).
 // POST: the norm is of what is added instead, xout = x + ((parts + bias) / rms) w (the arithmetic of
 // postnorm_rows_kernel, seqops.hip), and the image is that of xout; hout is not written.
-template <int RV, bool POST = false>
+template <int RV, bool POST, bool PLAIN>
 __global__ __launch_bounds__(1024) void rmsnorm_aimage_kernel(const float* x, const float* __restrict__ delta,
                                                               const float* __restrict__ w, float* xout,
                                                               float* __restrict__ hout, int n, float eps, int S,
                                                               size_t part_stride, int* __restrict__ ea,
-                                                              char* __restrict__ img, int M, const float* __restrict__ bias = nullptr) {
+                                                              char* __restrict__ img, int M, const float* __restrict__ bias) {
   __shared__ float red[16];
   __shared__ uint32_t part[16], cnt[16];
   const int gm = blockIdx.x, t = threadIdx.x, n4 = n >> 2, nslab = n / kBK;
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_aimage_kernel(const float* x, co
       if (i < n4) {
         v[k] = x4[i];
         wv[k] = w4[i];
-        float4 d = sum_parts(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
+        float4 d = sum_parts<PLAIN>(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
         if constexpr (POST) {
           if (bias) {
             const float4 e = reinterpret_cast<const float4*>(bias)[i];
@@ -867,14 +867,12 @@ int tlhip_rmsnorm_res_parts_aimage(const void* x, const void* parts, int64_t S, 
   const dim3 grid((unsigned)(timg * f16t::kTile)), block(1024);
   const size_t ps = (size_t)(rows * n);
   hipStream_t st = ctx().stream;
-  if (n <= 4096)
-    f16t::rmsnorm_aimage_kernel<1><<<grid, block, 0, st>>>(static_cast<const float*>(x), static_cast<const float*>(parts),
-                                                         static_cast<const float*>(w), static_cast<float*>(xout),
-                                                         static_cast<float*>(hout), (int)n, eps, (int)S, ps, ea, img, (int)rows);
-  else
-    f16t::rmsnorm_aimage_kernel<2><<<grid, block, 0, st>>>(static_cast<const float*>(x), static_cast<const float*>(parts),
-                                                         static_cast<const float*>(w), static_cast<float*>(xout),
-                                                         static_cast<float*>(hout), (int)n, eps, (int)S, ps, ea, img, (int)rows);
+  const auto run = [&](auto kernel) {
+    kernel<<<grid, block, 0, st>>>(static_cast<const float*>(x), static_cast<const float*>(parts), static_cast<const float*>(w),
+                                   static_cast<float*>(xout), static_cast<float*>(hout), (int)n, eps, (int)S, ps, ea, img, (int)rows, nullptr);
+  };
+  if (n <= 4096) S > 2 ? run(f16t::rmsnorm_aimage_kernel<1, false, false>) : run(f16t::rmsnorm_aimage_kernel<1, false, true>);
+  else S > 2 ? run(f16t::rmsnorm_aimage_kernel<2, false, false>) : run(f16t::rmsnorm_aimage_kernel<2, false, true>);
   TLHIP_CHECK_LAUNCH(TLHIP_C_RMSNORM_RES);
 }
 
@@ -920,7 +918,8 @@ int postnorm_aimage(const float* x, const float* parts, int S, const float* bias
   if (timg * f16t::kTile > 0x7fffffff) return fail(TLHIP_EUNSUPPORTED, "tlhip_postnorm_res_parts: too many rows");
   int* ea = static_cast<int*>(aimage);
   char* img = static_cast<char*>(aimage) + (((size_t)rows * sizeof(int) + 1023) & ~(size_t)1023);
-  auto fn = n <= 4096 ? f16t::rmsnorm_aimage_kernel<1, true> : f16t::rmsnorm_aimage_kernel<2, true>;
+  auto fn = S > 2 ? (n <= 4096 ? f16t::rmsnorm_aimage_kernel<1, true, false> : f16t::rmsnorm_aimage_kernel<2, true, false>)
+                  : (n <= 4096 ? f16t::rmsnorm_aimage_kernel<1, true, true> : f16t::rmsnorm_aimage_kernel<2, true, true>);
   hipLaunchKernelGGL(fn, dim3((unsigned)(timg * f16t::kTile)), dim3(1024), 0, ctx().stream, x, parts, w, xout, (float*)nullptr, n, eps, S,
                      (size_t)rows * n, ea, img, rows, bias);
   TLHIP_CHECK_LAUNCH(TLHIP_C_RMSNORM_RES);

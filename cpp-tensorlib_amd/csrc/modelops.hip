@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
 // the weight in VGPRs, so the row is read once and nothing waits on a second
 // pass. This is the model shape (n = 896 ... 8192), for one row of a decode step and for
 // the 512 rows of a prompt chunk alike (6.6 us against 11.1 us for 512 x 3584).
-template <bool RES, int RV, int NT>
+template <bool RES, int RV, int NT, bool PLAIN>
 __global__ __launch_bounds__(NT) void rmsnorm_wide_kernel(const float* __restrict__ x,
                                                             const float* __restrict__ delta,
                                                             const float* __restrict__ w,
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_wide_kernel(const float* __restric
       v[k] = x4[i];
       wv[k] = w4[i];
       if (RES) {
-        const float4 d = sum_parts(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
+        const float4 d = sum_parts<PLAIN>(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
         v[k].x += d.x; v[k].y += d.y; v[k].z += d.z; v[k].w += d.w;
       }
     }
@@ -160,10 +160,12 @@ static void launch_rmsnorm(const float* x, const float* delta, const float* w, f
   const bool wide_ok = (n % 4) == 0 && aligned16(w) && aligned16(hout);
   // (blocks of no more wavefronts than the row has work for: the others only meet the barriers)
   const auto wide = [&](auto kernel, int nt) { kernel<<<dim3((unsigned)rows), dim3(nt), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps); };
-  if (wide_ok && n <= 1024) wide(rmsnorm_wide_kernel<RES, 1, 256>, 256);
-  else if (wide_ok && n <= 2048) wide(rmsnorm_wide_kernel<RES, 1, 512>, 512);
-  else if (wide_ok && n <= 4096) wide(rmsnorm_wide_kernel<RES, 1, 1024>, 1024);
-  else if (wide_ok && n <= 8192) wide(rmsnorm_wide_kernel<RES, 2, 1024>, 1024);
+  // (1024 threads keep enough requests in flight by themselves: rows of 3584 are 3 % slower in fours with eight parts, 6 % with
+  // two; of 5120 in eight parts 7 % faster)
+  if (wide_ok && n <= 1024) S > 2 ? wide(rmsnorm_wide_kernel<RES, 1, 256, false>, 256) : wide(rmsnorm_wide_kernel<RES, 1, 256, true>, 256);
+  else if (wide_ok && n <= 2048) S > 2 ? wide(rmsnorm_wide_kernel<RES, 1, 512, false>, 512) : wide(rmsnorm_wide_kernel<RES, 1, 512, true>, 512);
+  else if (wide_ok && n <= 4096) wide(rmsnorm_wide_kernel<RES, 1, 1024, true>, 1024);
+  else if (wide_ok && n <= 8192) S > 4 ? wide(rmsnorm_wide_kernel<RES, 2, 1024, false>, 1024) : wide(rmsnorm_wide_kernel<RES, 2, 1024, true>, 1024);
   else
     rmsnorm_kernel<RES><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps);
 }
@@ -383,7 +385,7 @@ template <> __device__ __forceinline__ void kv_store4<uint16_t>(uint16_t* p, con
   *reinterpret_cast<uint2*>(p) = make_uint2(lo, hi);
 }
 
-template <typename KT>
+template <typename KT, bool PLAIN>
 __global__ __launch_bounds__(256) void qkv_rope_fill_kernel(
     const float* __restrict__ qkv, const float* __restrict__ bq, const float* __restrict__ bk,
     const float* __restrict__ bv, const float2* __restrict__ table, float* __restrict__ qh,
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(256) void qkv_rope_fill_kernel(
   // S > 1: qkv is the S K-split parts of the projection, part_stride floats apart, added up in
   // ascending order as the part-sum launch would have
   auto ld4 = [&](const float* p) {
-    return sum_parts(S, [&](int s) { return *reinterpret_cast<const float4*>(p + s * part_stride); });
+    return sum_parts<PLAIN>(S, [&](int s) { return *reinterpret_cast<const float4*>(p + s * part_stride); });
   };
   const int half = D >> 1, q4 = half >> 2;            // float4 groups per half row
   const int rot_per_t = (Hq + Hkv) * q4, v_per_t = Hkv * (D >> 2);
@@ -729,14 +731,19 @@ int tlhip_qkv_rope_fill_parts(const void* qkv, int64_t n_parts, const void* bq, 
     return fail(TLHIP_EINVAL, "tlhip_qkv_rope_fill: operands must be 16-byte aligned");
   const int Hq = (int)n_q_heads, Hkv = (int)n_kv_heads;
   const int64_t total = T * ((int64_t)(Hq + Hkv) * (D / 8) + (int64_t)Hkv * (D / 4));
-#define TLHIP_FILL(KT_)                                                                              \
-  qkv_rope_fill_kernel<KT_><<<dim3(blocks_for(total)), dim3(256), 0, ctx().stream>>>(                \
+#define TLHIP_FILL(KT_, PLAIN_)                                                                      \
+  qkv_rope_fill_kernel<KT_, PLAIN_><<<dim3(blocks_for(total)), dim3(256), 0, ctx().stream>>>(       \
       static_cast<const float*>(qkv), static_cast<const float*>(bq), static_cast<const float*>(bk), \
       static_cast<const float*>(bv), static_cast<const float2*>(table), static_cast<float*>(qh),    \
       static_cast<KT_*>(Kc), static_cast<KT_*>(Vc), (int)T, Hq, Hkv, (int)D, pos0, kv_max,        \
       (int)n_parts, (size_t)(T * (Hq + 2 * Hkv) * D))
-  if (kv_bf16) TLHIP_FILL(uint16_t);
-  else TLHIP_FILL(float);
+  if (n_parts > 2) {
+    if (kv_bf16) TLHIP_FILL(uint16_t, false);
+    else TLHIP_FILL(float, false);
+  } else {
+    if (kv_bf16) TLHIP_FILL(uint16_t, true);
+    else TLHIP_FILL(float, true);
+  }
 #undef TLHIP_FILL
   TLHIP_CHECK_LAUNCH(TLHIP_C_KV_FILL);
 }

@@ -1,5 +1,7 @@
 // Row ops around the layers: token rows with sinusoidal positions, sums into the residual stream, row
 // gathers, norms of what a sublayer wrote, the PolyNorm and gated GELU activations of a chunk.
+#include <type_traits>
+
 #include "common.hpp"
 #include "gemv_shared.hpp"
 #include "polynorm.hpp"
@@ -62,7 +64,7 @@ __global__ __launch_bounds__(256) void embed_scaled_kernel(const uint16_t* __res
 }
 
 // xout = x + rms(parts + bias) * w, a block of NT threads per row, RV float4s a thread.
-template <int RV, int NT>
+template <int RV, int NT, bool PLAIN>
 __global__ __launch_bounds__(NT) void postnorm_rows_kernel(const float* x, const float* __restrict__ delta, int S,
                                                            size_t part_stride, const float* __restrict__ bias,
                                                            const float* __restrict__ w, float* xout, int n, float eps) {
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(NT) void postnorm_rows_kernel(const float* x, const
       const float4* d4 = reinterpret_cast<const float4*>(delta + base);
       xv[k] = reinterpret_cast<const float4*>(x + base)[i];
       wv[k] = reinterpret_cast<const float4*>(w)[i];
-      v[k] = sum_parts(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
+      v[k] = sum_parts<PLAIN>(S, [&](int s) { return d4[s * (part_stride >> 2) + i]; });
       if (bias) {
         const float4 e = reinterpret_cast<const float4*>(bias)[i];
         v[k].x += e.x; v[k].y += e.y; v[k].z += e.z; v[k].w += e.w;
@@ -222,8 +224,12 @@ int tlhip_postnorm_res_parts(const void* x, const void* parts, int64_t S, const 
     return postnorm_aimage(static_cast<const float*>(x), static_cast<const float*>(parts), (int)S, static_cast<const float*>(bias),
                            static_cast<const float*>(norm_w), static_cast<float*>(xout), (int)n, eps, (int)rows, aimage);
   const int nt = n <= 1024 ? 256 : n <= 2048 ? 512 : 1024;   // no more wavefronts than the row has work for
-  auto fn = n <= 1024 ? postnorm_rows_kernel<1, 256> : n <= 2048 ? postnorm_rows_kernel<1, 512> : n <= 4096 ? postnorm_rows_kernel<1, 1024>
-          : n <= 8192 ? postnorm_rows_kernel<2, 1024> : postnorm_rows_kernel<8, 1024>;
+  const auto pick = [&](auto plain) {
+    constexpr bool P = decltype(plain)::value;
+    return n <= 1024 ? postnorm_rows_kernel<1, 256, P> : n <= 2048 ? postnorm_rows_kernel<1, 512, P> : n <= 4096 ? postnorm_rows_kernel<1, 1024, P>
+         : n <= 8192 ? postnorm_rows_kernel<2, 1024, P> : postnorm_rows_kernel<8, 1024, P>;
+  };
+  auto fn = S > 2 ? pick(std::false_type{}) : pick(std::true_type{});
   hipLaunchKernelGGL(fn, dim3((unsigned)rows), dim3((unsigned)nt), 0, ctx().stream, static_cast<const float*>(x), static_cast<const float*>(parts),
                      (int)S, (size_t)(rows * n), static_cast<const float*>(bias), static_cast<const float*>(norm_w),
                      static_cast<float*>(xout), (int)n, eps);
