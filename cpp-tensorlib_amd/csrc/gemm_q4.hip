@@ -261,34 +261,49 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
 
 static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// The three forms of gemm_bf16_nt_impl (prefill.hip), which has checked the arguments. can_split: the part sums work on
-// float4s. Work is shaped to whole rounds of the 2 * CUs block slots: fewer tiles than slots -> K split; more -> the
-// columns that make whole rounds with full K, the rest split over K in a second launch.
-int gemm_q4_prompt(const float* A, const uint8_t* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K, size_t parts_bytes,
-                   int* S_out, bool gu, bool can_split) {
+// can_split: the part sums work on float4s. Work is shaped to whole rounds of the 2 * CUs block slots: fewer tiles than slots
+// -> K split; more -> the columns that make whole rounds with full K, the rest split over K in a second launch. The time, fitted to
+// 400 runs (65 to 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 %): 11.2 us for two launches, 4 per million numbers
+// cut, a unit of 128 k 2.7 or, with two blocks on a CU, 4.1.
+Q4Plan plan_gemm_q4(int64_t M, int64_t N, int64_t K, size_t parts_bytes, bool want_parts, bool gu, bool can_split) {
   using namespace q4;
-  Context& c = ctx();
+  Q4Plan plan;
   const int per = gu ? 2 : 1;
-  const int64_t w = kBN / per, rb = cdiv(M, kBM), tn = cdiv(N, w), slots = 2 * (int64_t)c.cus, groups = K / kSlab, units = cdiv(groups, 4);
-  const bool want_parts = S_out != nullptr;
-  struct Piece { int64_t tn0, tcols; int S; } pieces[2];
-  int npieces = 0;
+  const int64_t cus = ctx().cus, w = kBN / per, rb = cdiv(M, kBM), tn = cdiv(N, w), slots = 2 * cus, units = cdiv(K / kSlab, 4);
   auto pick_S = [&](int64_t tiles) {
     if (!can_split || tiles >= slots) return 1;
     int64_t S = std::min<int64_t>(slots / tiles, 16);
     while (S > 1 && units / S < 2) S--;            // at least 256 k per part
     if (want_parts)
       while (S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) S--;
-    return (int)S;
+    return (int)cdiv(units, cdiv(units, S));
   };
   const int64_t per_round = slots / rb;
   if (rb * tn <= slots || per_round == 0 || !can_split || want_parts) {
-    pieces[npieces++] = Piece{0, tn, pick_S(rb * tn)};
+    plan.pieces[plan.npieces++] = {0, tn, pick_S(rb * tn)};
   } else {
     const int64_t main_tn = tn / per_round * per_round;
-    pieces[npieces++] = Piece{0, main_tn, 1};
-    if (main_tn < tn) pieces[npieces++] = Piece{main_tn, tn - main_tn, pick_S(rb * (tn - main_tn))};
+    plan.pieces[plan.npieces++] = {0, main_tn, 1};
+    if (main_tn < tn) plan.pieces[plan.npieces++] = {main_tn, tn - main_tn, pick_S(rb * (tn - main_tn))};
   }
+  plan.us = 11.2 + 4e-6 * (double)M * K;
+  for (int i = 0; i < plan.npieces; i++) {
+    const Q4Plan::Piece& P = plan.pieces[i];
+    plan.us += (double)cdiv(units, P.S) * slab_us(rb * P.tcols * P.S, cus, 2.67, 4.1);
+    if (P.S > 1) plan.us += 0.35e-6 * P.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
+  }
+  return plan;
+}
+
+// The three forms of gemm_bf16_nt_impl (prefill.hip), which has checked the arguments.
+int gemm_q4_prompt(const Q4Plan& plan, const float* A, const uint8_t* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K,
+                   int* S_out, bool gu) {
+  using namespace q4;
+  Context& c = ctx();
+  const int64_t w = gu ? kBN / 2 : kBN, rb = cdiv(M, kBM), groups = K / kSlab, units = cdiv(groups, 4);
+  const bool want_parts = S_out != nullptr;
+  const Q4Plan::Piece* pieces = plan.pieces;
+  const int npieces = plan.npieces;
   const size_t ea_bytes = ((size_t)M * sizeof(int) + 1023) & ~(size_t)1023, img_bytes = (size_t)rb * groups * kImage;
   size_t parts_need = 0;
   if (!want_parts)
@@ -308,10 +323,10 @@ int gemm_q4_prompt(const float* A, const uint8_t* W, const float* scales, float*
   else if (K <= 20480) image(q4_image_kernel<10>);
   else image(q4_image_kernel<16>);
   for (int i = 0; i < npieces; i++) {
-    const Piece& P = pieces[i];
+    const Q4Plan::Piece& P = pieces[i];
     const int64_t n0 = P.tn0 * w, pn = std::min<int64_t>(P.tcols * w, N - n0), part_w = gu ? P.tcols * kBN : pn;
-    const int64_t part_units = cdiv(units, P.S);
-    const int S = (int)cdiv(units, part_units);
+    const int S = P.S;
+    const int64_t part_units = cdiv(units, S);
     float* dst = C + n0;
     int64_t ldc = N;
     if (want_parts) {

@@ -455,64 +455,70 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 
 }  // namespace rows
 
-// Row tiles per block, columns per tile and K splits that an estimate of the time likes best; S == 0 where
-// gemm_bf16_nt_kernel is the better one or the shape is not taken.
+// Row tiles per block, columns per tile and K splits that an estimate of the time likes best; S == 0 where the shape is not
+// taken.
 //
-// The estimate, fitted to 280 runs (K 384 .. 18944, N 384 .. 37888, M 8 .. 120; rms error 24 %): a step of a block's
-// eight wavefronts takes the CU's vector memory path 35 clocks per KB of activations and 60 per KB of weights (whose
-// lanes cover 16 rows each), or its SIMDs, with two wavefronts each, the clocks of their matrix or vector
-// instructions (5.5 per element cut, 23 per eight nibbles; int4 measured 1.8 times that); a block starts and ends in
-// 3500 clocks and 60 per accumulator tile; bf16 blocks past the first round cost a fifth more; a launch costs 2 us.
-// The other kernel, measured over the same shapes: 6 us and 0.4 us per 32-k slab (1.0 with two blocks on a CU) up to 64
-// rows, above that 17 us and 0.35 (0.8). It is kept where its 128 x 256 tiles pay: products of more than a few rows
-// whose weight keeps every CU busy for several rounds (M = 64, 4608 x 3584: 14.9 us against 16.8 here).
+// The estimate that chooses, fitted to 280 runs (K 384 .. 18944, N 384 .. 37888, M 8 .. 120): a step of a block's eight
+// wavefronts takes the CU's vector memory path 35 clocks per KB of activations and 60 per KB of weights (whose lanes cover
+// 16 rows each), or its SIMDs, with two wavefronts each, the clocks of their matrix or vector instructions (5.5 per element
+// cut, 23 per eight nibbles; int4 measured 1.8 times that); a block starts and ends in 3500 clocks and 60 per accumulator
+// tile; bf16 blocks past the first round cost a fifth more; a launch costs 2 us. `us` is the chosen plan's time fitted again,
+// to 1000 runs (error 10 to 13 %) and 5 to 12 % up: the caller weighs it against the time of the kernel it would take instead.
 // Measured, us, other kernel -> this one: 896 x 896 at 5 / 37 / 77 rows 10.5 / 10.0 / 20.5 -> 3.6 / 3.7 / 4.4; 4864 x 896
 // gated 14.4 / 16.0 / 25.4 -> 7.8 / 11.1 / 13.4; 896 x 4864 11.0 / 11.4 / 21.7 -> 4.9 / 7.0 / 9.6; 9728 x 896 at 48 and 64
-// rows 16.8 / 17.8 -> 10.8 / 11.9; 18944 x 3584 gated 111 / 111 -> 63 / 92; int4 119 / 127 -> 53 / 93. 18960 x 2048 at 24 to
-// 64 rows stays with the other one (30 us; 32 to 40 here in parts).
-RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S) {
-  using rows::kMaxTM;
+// rows 16.8 / 17.8 -> 10.8 / 11.9; 18944 x 3584 gated 111 / 111 -> 63 / 92; int4 119 / 127 -> 53 / 93.
+static RowsPlan plan_row_blocks(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S, int64_t row_blocks) {
   RowsPlan best;
-  const int64_t rows_w = (gu ? 2 : 1) * N;
-  if (M > 128 || K % (q4 ? 128 : 32) != 0 || M * K * 4 >= (int64_t(1) << 32) || rows_w * K * (q4 ? 1 : 4) / 2 >= (int64_t(1) << 32))
-    return best;                                   // (32-bit byte offsets)
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  const int64_t t16 = cdiv(M, 16), cus = ctx().cus, units = K / (q4 ? 128 : 32), steps = q4 ? 4 : 1;
-  best.row_blocks = (int)cdiv(t16, kMaxTM);
-  const int TM = best.TM = (int)cdiv(t16, best.row_blocks);
+  const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / (q4 ? 128 : 32), steps = q4 ? 4 : 1;
+  best.row_blocks = (int)row_blocks;
+  const int TM = best.TM = (int)cdiv(cdiv(M, 16), row_blocks);
   double least = 0;
   const double own_sum = gu || (!q4 && N > 8192) ? 5 : 0;   // (18960 x 2048 at 32 rows: 33.6 us in two parts)
   for (int TN = q4 && TM > 1 ? 2 : 4; TN >= (gu ? 2 : 1); TN /= 2) {   // (what the registers hold)
     const int64_t tiles = cdiv(rows_w, 16 * TN);
     for (int64_t S = 1; S <= std::min<int64_t>(max_S, units); S++) {
-      const int64_t per = cdiv(units, S), blocks = tiles * best.row_blocks * S;
+      const int64_t per = cdiv(units, S), blocks = tiles * row_blocks * S;
       if (cdiv(units, per) != S) continue;
       const double n = (double)(cdiv(per, rows::kWaves) * steps);    // steps of a wavefront
       const double mem = 8 * (70.0 * TM + (q4 ? 30.0 : 60.0) * TN);
       const double math = 2 * (q4 ? 1.8 * std::max(48.0 * TM * TN, 176.0 * TM + TN * (92.0 + 16 * TM)) : std::max(48.0 * TM * TN, 176.0 * TM));
       // (every CU is busy without a split, and the parts of more than a row tile cost more than the last round's gaps)
-      if (!q4 && S > 1 && M > 16 && tiles * best.row_blocks > cus) break;
+      if (!q4 && S > 1 && M > 16 && tiles * row_blocks > cus) break;
       const double rounds = blocks <= (q4 ? 2 : 4) * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus;
-      double us = 2 + rounds * (!q4 && rounds > 1 ? 1.2 : 1.0) * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100;
+      const double parts = S > 1 ? (double)S * M * rows_w * 4 / 1e6 : 0;
       // parts written and read, and their launch, which a gated product has and a wide one (a narrow one is planned as if
       // left as parts, whose sum its consumer forms: the two are the same bits)
-      if (S > 1) us += (double)S * M * rows_w * 4 / 4e6 + own_sum;
+      const double us = 2 + rounds * (!q4 && rounds > 1 ? 1.2 : 1.0) * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100 +
+                        (S > 1 ? parts / 4 + own_sum : 0);
       if (best.S == 0 || us < least) {
         least = us;
         best.TN = TN;
         best.S = (int)S;
         best.tiles = (int)tiles;
         best.part_units = (int)per;
+        // fewer steps than wavefronts leave some idle; five row tiles of int4 spill, and int4 blocks in turn wait for what
+        // they would have loaded ahead
+        const double work = rounds * n * std::max(mem * (double)std::min<int64_t>(rows::kWaves, per) / rows::kWaves, per > 4 ? math : math / 2) / 2100;
+        best.us = q4 ? 2 + work * (TM == 5 ? 1.3 : 1.0) * (rounds > 2 ? 1.2 : rounds > 1 ? 0.81 : 0.74) + rounds * (0.3 + 0.18 * TM * TN) + parts
+                     : 0.85 + 1.15 * work + rounds * (1.2 + 0.18 * TM * TN) + 0.75 * parts;
       }
     }
   }
-  if (M > 16) {
-    const int64_t bm = M > 64 ? 128 : 64, bn = M > 64 && !q4 ? 256 : 128, tiles = cdiv(M, bm) * cdiv(rows_w, bn), slabs = K / 32;
-    const int64_t S = std::max<int64_t>(1, std::min(std::min<int64_t>(max_S, 2 * cus / tiles), slabs / 8));
-    const double other = M > 64 ? 17 + (double)slabs / S * (tiles * S <= 96 ? 0.35 : 0.8) : 6 + (double)slabs / S * (tiles * S <= cus ? 0.4 : 1.0);
-    if (other + (S > 1 ? own_sum : 0) < least) best.S = 0;
-  }
   return best;
+}
+
+RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S) {
+  const int64_t rows_w = (gu ? 2 : 1) * N, t16 = (M + 15) / 16;
+  if (M > 128 || K % (q4 ? 128 : 32) != 0 || M * K * 4 >= (int64_t(1) << 32) || rows_w * K * (q4 ? 1 : 4) / 2 >= (int64_t(1) << 32))
+    return RowsPlan{};                             // (32-bit byte offsets)
+  const auto plan = [&](int64_t row_blocks) { return plan_row_blocks(M, N, K, gu, q4, max_S, row_blocks); };
+  if (!q4 || t16 != 5) return plan((t16 + rows::kMaxTM - 1) / rows::kMaxTM);
+  // int4 with 65 to 80 rows: one block of five row tiles, or two of three (77 x 640 x 768 7.8 us and 6.1; 74 x 4609 x 11008, whose
+  // K cannot be split, 76 and 107)
+  const RowsPlan one = plan(1), two = plan(2);
+  const auto all = [](const RowsPlan& P) { return P.us + (P.S > 1 ? kPartSumUs : 0); };
+  return two.S > 0 && (one.S == 0 || all(two) < all(one)) ? two : one;
 }
 
 int launch_gemm_rows(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K,

@@ -13,6 +13,7 @@ typedef uint32_t frag16 __attribute__((ext_vector_type(4)));   // eight 16-bit o
 // gemm_rows.hip: products of a few rows. S == 0: not a shape it takes.
 struct RowsPlan {
   int TM = 0, TN = 0, S = 0, tiles = 0, row_blocks = 0, part_units = 0;
+  double us = 0;                       // what the product takes so, its parts' traffic included, the launch that adds them up not
 };
 // max_S: the most K splits allowed
 RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S);
@@ -22,8 +23,20 @@ int launch_gemm_rows(const RowsPlan& P, const float* A, const void* W, const flo
 // gemm_q4.hip: products of more than 64 rows over an int4 weight, in the three forms of tlhip_gemm_q4_nt*. kNoScratch:
 // nothing was launched, for want of scratch (a recording may not grow it); the caller has a form that needs less.
 constexpr int kNoScratch = 1;
-int gemm_q4_prompt(const float* A, const uint8_t* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K, size_t parts_bytes,
-                   int* S_out, bool gu, bool can_split);
+struct Q4Plan {
+  struct Piece { int64_t tn0, tcols; int S; } pieces[2];   // tile columns, K splits
+  int npieces = 0;
+  double us = 0;                       // as in RowsPlan
+};
+Q4Plan plan_gemm_q4(int64_t M, int64_t N, int64_t K, size_t parts_bytes, bool want_parts, bool gu, bool can_split);
+int gemm_q4_prompt(const Q4Plan& plan, const float* A, const uint8_t* W, const float* scales, float* C, int64_t M, int64_t N, int64_t K,
+                   int* S_out, bool gu);
+// The launch that adds a product's parts up costs this beside their traffic; blocks of kernels that run two to a CU: us for a
+// K slab or unit with one block per CU, with two, and beyond that in proportion.
+constexpr double kPartSumUs = 2.2;
+inline double slab_us(int64_t blocks, int64_t cus, double one, double two) {
+  return blocks <= cus ? one : blocks <= 2 * cus ? two : two * (double)blocks / (double)(2 * cus);
+}
 
 // defined in prefill.hip
 // C[M][n] (rows ldc apart) = the sum of the S parts [M][part_w]; half > 0: gated parts, strips of `half`

@@ -527,35 +527,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   const int64_t slots = (int64_t)c.cus * 2;
   const int per = gu ? 2 : 1;                             // tile columns per unit of N
   const bool can_split = (N % 4) == 0 && aligned16(C);   // the part sum works on float4s
-  if (aligned16(C)) {   // a few rows: a kernel of their own
-    int64_t max_S = can_split ? 16 : 1;
-    if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
-    RowsPlan P = plan_gemm_rows(M, N, K, gu, q4, max_S);
-    const auto part_width = [&] { return gu ? (int64_t)P.tiles * 16 * P.TN : N; };
-    char* parts = nullptr;
-    if (P.S > 1 && !want_parts) {
-      parts = static_cast<char*>(scratch((size_t)P.S * M * part_width() * sizeof(float)));
-      if (!parts) P = plan_gemm_rows(M, N, K, gu, q4, 1);   // no scratch to be had (a recording may not grow it): no parts
-    }
-    if (P.S > 0) {
-      const bool sum = P.S > 1 && !want_parts;
-      const int64_t part_w = part_width();
-      float* dst = sum ? reinterpret_cast<float*>(parts) : pc;
-      if (want_parts) *S_out = P.S;
-      if (int rc = launch_gemm_rows(P, pa, W, static_cast<const float*>(scales), dst, M, N, K, sum ? part_w : N, gu)) return rc;
-      if (sum) launch_part_sum(dst, pc, M, N, part_w, N, P.S, gu ? 8 * P.TN : 0);
-      TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
-    }
-  }
   const bool half = q4 && M > 64 && c.tune_gemm_planes != 3;
   const size_t ea_bytes = half ? (((size_t)M * sizeof(int) + 255) & ~(size_t)255) : 0;
-  // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
-  // against 50, 301 x 37888 x 3584 209 against 303)
-  if (half && K <= 32768 && (per * N >= 2048 || K <= 1024)) {
-    const int rc = gemm_q4_prompt(pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, parts_bytes, S_out, gu, can_split);
-    if (rc < 0) return rc;
-    if (rc != kNoScratch) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
-  }
   struct Piece { int64_t n0, n; int S; int variant; };    // columns (features) [n0, n0 + n)
   Piece pieces[2];
   int npieces = 0;
@@ -590,6 +563,52 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
     else pieces[npieces++] = Piece{0, N, pick_S(t64), 2};
   }
   static const int kBm[4] = {128, 64, 64, 128}, kBn[4] = {256, 128, 64, 128};
+  // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
+  // against 50, 301 x 37888 x 3584 209 against 303)
+  const bool images = half && K <= 32768 && (per * N >= 2048 || K <= 1024);
+  Q4Plan q4_plan;
+  if (images) q4_plan = plan_gemm_q4(M, N, K, parts_bytes, want_parts, gu, can_split);
+  // A few rows: a kernel of their own, above 16 where it is the faster one. What the others take, fitted to 1000 runs (17 to
+  // 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 to 9 %): a start, and a time per 32-k slab with one and two blocks on a CU.
+  if (aligned16(C)) {
+    int64_t max_S = can_split ? 16 : 1;
+    if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
+    RowsPlan P = plan_gemm_rows(M, N, K, gu, q4, max_S);
+    if (M > 16 && P.S > 0) {
+      double other = images ? q4_plan.us : 0;
+      for (int pi = 0; !images && pi < npieces; pi++) {
+        const Piece& O = pieces[pi];
+        const int bm = kBm[O.variant], bn = kBn[O.variant];
+        const int64_t slabs = cdiv(cdiv(K, O.S), kBK), blocks = cdiv(M, bm) * cdiv(O.n, bn / per) * cdiv(cdiv(K, kBK), slabs);
+        if (M <= 64 && q4) other += 2.4 + (double)slabs * slab_us(blocks, c.cus, 0.965, 1.13);
+        else if (M <= 64) other += 2.2 + (double)slabs * (bn > 64 ? slab_us(blocks, c.cus, 0.9, 1.12) : slab_us(blocks, c.cus, 0.65, 0.95));
+        else if (q4) other += 12.1 + (double)slabs * slab_us(blocks, c.cus, 1.03, 1.03);
+        else other += 7 + (double)slabs * slab_us(blocks, c.cus, 1.5, 2.18);
+        if (O.S > 1) other += (M <= 64 ? 0.65e-6 : 0.36e-6) * O.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
+      }
+      if (P.us + (P.S > 1 && !want_parts ? kPartSumUs : 0) > other) P.S = 0;
+    }
+    const auto part_width = [&] { return gu ? (int64_t)P.tiles * 16 * P.TN : N; };
+    char* parts = nullptr;
+    if (P.S > 1 && !want_parts) {
+      parts = static_cast<char*>(scratch((size_t)P.S * M * part_width() * sizeof(float)));
+      if (!parts) P = plan_gemm_rows(M, N, K, gu, q4, 1);   // no scratch to be had (a recording may not grow it): no parts
+    }
+    if (P.S > 0) {
+      const bool sum = P.S > 1 && !want_parts;
+      const int64_t part_w = part_width();
+      float* dst = sum ? reinterpret_cast<float*>(parts) : pc;
+      if (want_parts) *S_out = P.S;
+      if (int rc = launch_gemm_rows(P, pa, W, static_cast<const float*>(scales), dst, M, N, K, sum ? part_w : N, gu)) return rc;
+      if (sum) launch_part_sum(dst, pc, M, N, part_w, N, P.S, gu ? 8 * P.TN : 0);
+      TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+    }
+  }
+  if (images) {
+    const int rc = gemm_q4_prompt(q4_plan, pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, S_out, gu);
+    if (rc < 0) return rc;
+    if (rc != kNoScratch) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+  }
   // One scratch request for the whole call (a second, larger one could move the buffer): the
   // exponents of A's rows first, then room for the largest piece's K-split parts.
   size_t parts_need = 0;
