@@ -7,6 +7,8 @@
 // uploaded as they are and these kernels write the decode formats straight into the
 // weight buffers. All of it is byte/integer work at HBM speed, bit-identical to the
 // host arithmetic.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace tlhip {
@@ -277,17 +279,20 @@ int tlhip_quantize_q4(const void* src, int src_type, void* packed, void* scales,
   if (!aligned16(src) || !aligned16(packed) || (reinterpret_cast<uintptr_t>(scales) & 3u))
     return fail(TLHIP_EINVAL, "tlhip_quantize_q4: src and packed must be 16-byte aligned, scales 4-byte");
   const int64_t groups = rows * (K / 32);
-  const int64_t blocks = (2 * groups + 255) / 256;
-  if (blocks > 0x7fffffff) return fail(TLHIP_EUNSUPPORTED, "tlhip_quantize_q4: too many groups");
-  uint2* pk = static_cast<uint2*>(packed);
-  float* sc = static_cast<float*>(scales);
-  const dim3 grid((unsigned)blocks), block(256);
-  if (src_type == TLHIP_T_F32)
-    quantize_q4_kernel<TLHIP_T_F32><<<grid, block, 0, ctx().stream>>>(static_cast<const float*>(src), pk, sc, groups);
-  else if (src_type == TLHIP_T_F16)
-    quantize_q4_kernel<TLHIP_T_F16><<<grid, block, 0, ctx().stream>>>(static_cast<const uint16_t*>(src), pk, sc, groups);
-  else
-    quantize_q4_kernel<TLHIP_T_BF16><<<grid, block, 0, ctx().stream>>>(static_cast<const uint16_t*>(src), pk, sc, groups);
+  if ((groups + 255) / 256 > 0x7fffffff) return fail(TLHIP_EUNSUPPORTED, "tlhip_quantize_q4: too many groups");
+  // (a grid's x counts threads in 32 bits, and a group takes two: at most 2^30 groups a launch)
+  for (int64_t g0 = 0; g0 < groups; g0 += (int64_t)1 << 30) {
+    const int64_t n = std::min<int64_t>(groups - g0, (int64_t)1 << 30);
+    uint2* pk = static_cast<uint2*>(packed) + 2 * g0;
+    float* sc = static_cast<float*>(scales) + g0;
+    const dim3 grid((unsigned)((2 * n + 255) / 256)), block(256);
+    if (src_type == TLHIP_T_F32)
+      quantize_q4_kernel<TLHIP_T_F32><<<grid, block, 0, ctx().stream>>>(static_cast<const float*>(src) + 32 * g0, pk, sc, n);
+    else if (src_type == TLHIP_T_F16)
+      quantize_q4_kernel<TLHIP_T_F16><<<grid, block, 0, ctx().stream>>>(static_cast<const uint16_t*>(src) + 32 * g0, pk, sc, n);
+    else
+      quantize_q4_kernel<TLHIP_T_BF16><<<grid, block, 0, ctx().stream>>>(static_cast<const uint16_t*>(src) + 32 * g0, pk, sc, n);
+  }
   TLHIP_CHECK_LAUNCH(TLHIP_C_QUANTIZE_Q4);
 }
 

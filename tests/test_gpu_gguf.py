@@ -295,3 +295,32 @@ def test_quantize_q4_beside_its_rounding_boundaries(lib, orc, st):
     assert np.array_equal(got[rows * K // 2:].view(np.float32), sc)
     assert np.array_equal(got[:rows * K // 2].reshape(rows, K // 2), nib[:, 0::2] | nib[:, 1::2] << 4)
     src.free(); q4.free()
+
+
+def test_quantize_q4_of_more_groups_than_a_grid_counts(lib, orc):
+    """2^31 groups and a few thousand: two threads a group are more than one launch holds. The first and last groups and those
+    around each 2^30 are checked; the rows between hold whatever the memory does."""
+    groups, part = (1 << 31) + 4096, 2048
+    K, need = 32 * 2048, ((1 << 31) + 4096) * (64 + 16 + 4)
+    if lib.device_info()["hbm_bytes"] < 1.3 * need:
+        pytest.skip("the matrix and its int4 form take 180 GB")
+    try:
+        whole = lib.empty_bytes(need)
+    except RuntimeError:
+        pytest.skip("no room for the matrix and its int4 form")
+    src, packed, scales = whole.ptr, whole.ptr + groups * 64, whole.ptr + groups * 80
+    w = orc.normal(part * 32, 91).astype(np.float16).view(np.uint16)
+    q, s = lib.to_device(np.zeros(part * 16, np.uint8)), lib.to_device(np.zeros(part, np.float32))
+    first = lib.to_device(w)
+    lib._chk(lib.c.tlhip_quantize_q4(first.ptr, F16, q.ptr, s.ptr, 1, part * 32, 32))
+    at = [0, (1 << 30) - part // 2, (1 << 31) - part // 2, groups - part]
+    for g in at:
+        lib._chk(lib.c.tlhip_memcpy_h2d(src + g * 64, w.ctypes.data, w.nbytes))
+    lib._chk(lib.c.tlhip_quantize_q4(src, F16, packed, scales, groups // 2048, K, 32))
+    for g in at:
+        nib, sc = np.empty(part * 16, np.uint8), np.empty(part, np.float32)
+        lib._chk(lib.c.tlhip_memcpy_d2h(nib.ctypes.data, packed + g * 16, nib.nbytes))
+        lib._chk(lib.c.tlhip_memcpy_d2h(sc.ctypes.data, scales + g * 4, sc.nbytes))
+        assert np.array_equal(nib, q.numpy()) and np.array_equal(sc, s.numpy()), g
+    for b in (whole, first, q, s):
+        b.free()
