@@ -161,11 +161,12 @@ static void launch_rmsnorm(const float* x, const float* delta, const float* w, f
   // (blocks of no more wavefronts than the row has work for: the others only meet the barriers)
   const auto wide = [&](auto kernel, int nt) { kernel<<<dim3((unsigned)rows), dim3(nt), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps); };
   // (1024 threads keep enough requests in flight by themselves: rows of 3584 are 3 % slower in fours with eight parts, 6 % with
-  // two; of 5120 in eight parts 7 % faster)
+  // two; two rounds of them do not: rows of 5120 are 7 % faster in fours with eight parts, of 4392 11 % with four, though 5 %
+  // slower with two)
   if (wide_ok && n <= 1024) S > 2 ? wide(rmsnorm_wide_kernel<RES, 1, 256, false>, 256) : wide(rmsnorm_wide_kernel<RES, 1, 256, true>, 256);
   else if (wide_ok && n <= 2048) S > 2 ? wide(rmsnorm_wide_kernel<RES, 1, 512, false>, 512) : wide(rmsnorm_wide_kernel<RES, 1, 512, true>, 512);
   else if (wide_ok && n <= 4096) wide(rmsnorm_wide_kernel<RES, 1, 1024, true>, 1024);
-  else if (wide_ok && n <= 8192) S > 4 ? wide(rmsnorm_wide_kernel<RES, 2, 1024, false>, 1024) : wide(rmsnorm_wide_kernel<RES, 2, 1024, true>, 1024);
+  else if (wide_ok && n <= 8192) S > 2 ? wide(rmsnorm_wide_kernel<RES, 2, 1024, false>, 1024) : wide(rmsnorm_wide_kernel<RES, 2, 1024, true>, 1024);
   else
     rmsnorm_kernel<RES><<<dim3((unsigned)rows), dim3(256), 0, st>>>(x, delta, w, xout, hout, (int)n, eps, S, ps);
 }
