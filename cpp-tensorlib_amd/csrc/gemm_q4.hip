@@ -264,7 +264,8 @@ static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // can_split: the part sums work on float4s. Work is shaped to whole rounds of the 2 * CUs block slots: fewer tiles than slots
 // -> K split; more -> the columns that make whole rounds with full K, the rest split over K in a second launch. The time, fitted to
 // 400 runs (65 to 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 %): 11.2 us for two launches, 4 per million numbers
-// cut, a unit of 128 k 2.7 or, with two blocks on a CU, 4.1.
+// cut, a unit of 128 k 2.7 or, with two blocks on a CU, 4.1. Above 128 rows, to 11000 runs (129 to 1024 rows, N 128 .. 40000, K 128 ..
+// 20480; error 7 %): the same and the outputs, with whole rounds of blocks: 14 x 37 tiles are two.
 Q4Plan plan_gemm_q4(int64_t M, int64_t N, int64_t K, size_t parts_bytes, bool want_parts, bool gu, bool can_split) {
   using namespace q4;
   Q4Plan plan;
@@ -285,6 +286,17 @@ Q4Plan plan_gemm_q4(int64_t M, int64_t N, int64_t K, size_t parts_bytes, bool wa
     const int64_t main_tn = tn / per_round * per_round;
     plan.pieces[plan.npieces++] = {0, main_tn, 1};
     if (main_tn < tn) plan.pieces[plan.npieces++] = {main_tn, tn - main_tn, pick_S(rb * (tn - main_tn))};
+  }
+  const double outputs = 1e-6 * (double)M * (double)(per * N);
+  if (M > 128) {
+    plan.us = 9.8 + 2.7e-6 * (double)M * K + 0.88 * outputs + 9 * (plan.npieces - 1);
+    for (int i = 0; i < plan.npieces; i++) {
+      const Q4Plan::Piece& P = plan.pieces[i];
+      const int64_t part_groups = std::min(4 * cdiv(units, P.S), K / kSlab);
+      plan.us += (double)part_groups / 4 * rounds_us(rb * P.tcols * P.S, cus, 2.69, 3.7);
+      if (P.S > 1) plan.us += 1.04e-6 * P.S * M * per * std::min<int64_t>(N, P.tcols * w) + (want_parts ? 0 : 3.3);
+    }
+    return plan;
   }
   plan.us = 11.2 + 4e-6 * (double)M * K;
   for (int i = 0; i < plan.npieces; i++) {

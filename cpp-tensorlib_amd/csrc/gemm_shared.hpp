@@ -37,6 +37,10 @@ constexpr double kPartSumUs = 2.2;
 inline double slab_us(int64_t blocks, int64_t cus, double one, double two) {
   return blocks <= cus ? one : blocks <= 2 * cus ? two : two * (double)blocks / (double)(2 * cus);
 }
+// the same with whole rounds of blocks, whose columns do not differ enough in time to fill the last one's gaps
+inline double rounds_us(int64_t blocks, int64_t cus, double one, double two) {
+  return blocks <= cus ? one : two * (double)((blocks + 2 * cus - 1) / (2 * cus));
+}
 
 // defined in prefill.hip
 // C[M][n] (rows ldc apart) = the sum of the S parts [M][part_w]; half > 0: gated parts, strips of `half`

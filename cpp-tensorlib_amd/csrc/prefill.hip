@@ -565,9 +565,25 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   static const int kBm[4] = {128, 64, 64, 128}, kBn[4] = {256, 128, 64, 128};
   // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
   // against 50, 301 x 37888 x 3584 209 against 303)
-  const bool images = half && K <= 32768 && (per * N >= 2048 || K <= 1024);
+  bool images = half && K <= 32768 && (per * N >= 2048 || K <= 1024);
   Q4Plan q4_plan;
   if (images) q4_plan = plan_gemm_q4(M, N, K, parts_bytes, want_parts, gu, can_split);
+  const auto part_slabs = [&](const Piece& O) { return cdiv(cdiv(K, O.S), kBK); };
+  const auto part_blocks = [&](const Piece& O) {
+    return cdiv(M, kBm[O.variant]) * cdiv(O.n, kBn[O.variant] / per) * cdiv(cdiv(K, kBK), part_slabs(O));
+  };
+  // Above 128 rows also by what the two take, where the images' tiles are a round and a bit and these are one (us, images and here:
+  // 613 x 6528 x 5248 169 and 134, 705 x 10880 x 3584 in parts 195 and 161, 847 x 9344 x 256 33 and 26). This kernel's time is fitted
+  // to the 11000 runs of plan_gemm_q4 (error 5 %); 5 % are the images', for the errors of both.
+  if (images && M > 128) {
+    double here = 10.1 + 0.9e-6 * (double)M * (double)(per * N) + 7.3 * (npieces - 1);
+    for (int pi = 0; pi < npieces; pi++) {
+      const Piece& O = pieces[pi];
+      here += (double)part_slabs(O) * rounds_us(part_blocks(O), c.cus, 0.98, 1.22);
+      if (O.S > 1) here += 1.2e-6 * O.S * M * per * O.n + (want_parts ? 0 : 2.7);
+    }
+    images = 0.95 * q4_plan.us < here;
+  }
   // A few rows: a kernel of their own, above 16 where it is the faster one. What the others take, fitted to 1000 runs (17 to
   // 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 to 9 %): a start, and a time per 32-k slab with one and two blocks on a CU.
   if (aligned16(C)) {
@@ -578,8 +594,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
       double other = images ? q4_plan.us : 0;
       for (int pi = 0; !images && pi < npieces; pi++) {
         const Piece& O = pieces[pi];
-        const int bm = kBm[O.variant], bn = kBn[O.variant];
-        const int64_t slabs = cdiv(cdiv(K, O.S), kBK), blocks = cdiv(M, bm) * cdiv(O.n, bn / per) * cdiv(cdiv(K, kBK), slabs);
+        const int bn = kBn[O.variant];
+        const int64_t slabs = part_slabs(O), blocks = part_blocks(O);
         if (M <= 64 && q4) other += 2.4 + (double)slabs * slab_us(blocks, c.cus, 0.965, 1.13);
         else if (M <= 64) other += 2.2 + (double)slabs * (bn > 64 ? slab_us(blocks, c.cus, 0.9, 1.12) : slab_us(blocks, c.cus, 0.65, 0.95));
         else if (q4) other += 12.1 + (double)slabs * slab_us(blocks, c.cus, 1.03, 1.03);

@@ -23,7 +23,8 @@ def _case(lib, orc, M, rows, K, seed):
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 2048, 32), (129, 2049, 160), (200, 257, 896), (192, 2304, 128), (301, 2500, 1056), (320, 4608, 3584),
-                                   (512, 3584, 1024), (193, 70000, 256), (1000, 2300, 384)])
+                                   (512, 3584, 1024), (193, 70000, 256), (1000, 2300, 384),
+                                   (847, 9344, 256)])
 def test_plain_and_parts(lib, orc, M, N, K):
     print("case gemm_q4", M, N, K, flush=True)
     da, dw, want, slack = _case(lib, orc, M, N, K, 81)
@@ -40,7 +41,8 @@ def test_plain_and_parts(lib, orc, M, N, K):
         b.free()
 
 
-@pytest.mark.parametrize("M,ff,K", [(66, 1024, 32), (129, 1100, 160), (301, 4864, 896), (512, 1030, 384), (200, 18944, 128)])
+@pytest.mark.parametrize("M,ff,K", [(66, 1024, 32), (129, 1100, 160), (301, 4864, 896), (512, 1030, 384), (200, 18944, 128),
+                                    (731, 2304, 416), (727, 1501, 416)])
 def test_gated(lib, orc, M, ff, K):
     print("case gemm_q4 gated", M, ff, K, flush=True)
     da, dw, p, s = _case(lib, orc, M, 2 * ff, K, 83)
