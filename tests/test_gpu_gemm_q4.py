@@ -53,3 +53,49 @@ def test_gated(lib, orc, M, ff, K):
     assert np.all(np.abs(out.numpy() - act * u) <= 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u))
     for b in (da, dw, out):
         b.free()
+
+
+@pytest.mark.parametrize("M,K", [(65, 2016), (65, 2080), (65, 4064), (65, 4128), (65, 8160), (65, 8224), (65, 20448), (65, 20512), (65, 32736),
+                                 (65, 32800), (129, 2048), (129, 4096), (129, 20480), (129, 32768)])
+def test_rows_at_the_limits_of_the_images_kernels(lib, orc, M, K):
+    """A row's image is cut by threads that hold the whole row: one to sixteen runs of eight k each, to 2048, 4096, 8192, 20480 and
+    32768 k. Longer rows are multiplied without images."""
+    N = 2048
+    print("case gemm_q4 limits", M, N, K, flush=True)
+    da, dw, want, slack = _case(lib, orc, M, N, K, 85)
+    out = lib.to_device(np.full((M, N), np.nan, np.float32))
+    lib.gemm_q4_nt(da, dw, out, M, N, K)
+    assert np.all(np.abs(out.numpy() - want) <= slack)
+    for b in (da, dw, out):
+        b.free()
+
+
+def test_infinities_and_nan_stay_in_their_rows(lib, orc):
+    M, N, K = 301, 2049, 896
+    print("case gemm_q4 not finite", M, N, K, flush=True)
+    da, dw, _, _ = _case(lib, orc, M, N, K, 87)
+    out, A = lib.empty((M, N)), da.numpy()
+    lib.gemm_q4_nt(da, dw, out, M, N, K)
+    clean = out.numpy()
+    A[3, 5], A[200, K - 1] = np.inf, np.nan
+    lib.gemm_q4_nt(da.upload(A), dw, out, M, N, K)
+    got, rest = out.numpy(), [r for r in range(M) if r not in (3, 200)]
+    assert np.isnan(got[[3, 200]]).all() and np.array_equal(got[rest], clean[rest])
+    for b in (da, dw, out):
+        b.free()
+
+
+def test_recorded_without_room_for_the_images(fresh_lib, recorded, orc):
+    """The images of 200 rows of 16384 take 16 MB; a recording that finds 8 MB multiplies without them."""
+    M, N, K = 200, 2049, 16384
+    print("case gemm_q4 recorded", M, N, K, flush=True)
+    da, dw, want, slack = _case(fresh_lib, orc, M, N, K, 89)
+    out = fresh_lib.empty((M, N))
+    fresh_lib.gemm_q4_nt(da, dw, out, 65, 2048, 32)   # (scratch comes in 8 MB at least)
+    for got in recorded(lambda: fresh_lib.gemm_q4_nt(da, dw, out, M, N, K), out):
+        assert np.all(np.abs(got - want) <= slack)
+    before = fresh_lib.alloc_calls()
+    fresh_lib.gemm_q4_nt(da, dw, out, M, N, K)
+    assert fresh_lib.alloc_calls() > before and np.all(np.abs(out.numpy() - want) <= slack)
+    for b in (da, dw, out):
+        b.free()

@@ -1,6 +1,6 @@
 """GPU parity: the products of a few rows (csrc/gemm_rows.hip) at the edges of their tiles: rows around the 16-row
 tiles and the blocks of up to five of them, columns that fill no tile, K of one step, of fewer steps than wavefronts and
-of several rounds, both weight formats, plain, gated and left as K-split parts.
+of many steps to a wavefront, both weight formats, plain, gated and left as K-split parts.
 
 Every product is compared with float64. A sum of n fp32 additions is off by at most n 2^-24 of the sum of its terms'
 magnitudes; here n is three terms per 32-k step of a wavefront's chain, the 32 products inside an instruction and the
@@ -67,6 +67,89 @@ def test_gated(lib, orc, fmt, M, ff, K):
     (lib.gemm_bf16_nt_swiglu if fmt == "bf16" else lib.gemm_q4_nt_swiglu)(da, dw, out, M, ff, K)
     # the slope of x sigmoid(x) is below 1.1; the gate itself costs a few roundings
     assert np.all(np.abs(out.numpy() - act * u) <= 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u))
+    for b in (da, dw, out):
+        b.free()
+
+
+@pytest.mark.parametrize("fmt,K", [("bf16", 2048), ("bf16", 9216), ("q4", 4096), ("q4", 4736), ("q4", 9216)])
+def test_many_steps_to_a_wavefront(lib, orc, fmt, K):
+    """Columns that are no multiple of four keep K in one part: a wavefront's steps go through its slots several times (bf16: 8 and
+    36 steps in two to four slots; int4: four, five and nine units in two), for every number of row tiles. The sums' order
+    does not depend on the tiles, so the first five rows of every product are the bits of the five-row product, which only
+    this kernel forms: the others are formed by it too."""
+    N = 33
+    A = orc.normal(128 * K, 27).reshape(128, K)
+    w, W = _weights(orc, fmt, N, K, 28)
+    dw, five = lib.to_device(w), None
+    for M in (5, 17, 33, 49, 77, 96, 128):
+        print("case gemm_rows long", fmt, M, N, K, flush=True)
+        da, out = lib.to_device(A[:M]), lib.to_device(np.full((M, N), np.nan, np.float32))
+        (lib.gemm_bf16_nt if fmt == "bf16" else lib.gemm_q4_nt)(da, dw, out, M, N, K)
+        got, A64 = out.numpy(), A[:M].astype(np.float64)
+        assert np.all(np.abs(got - A64 @ W.T) <= _slack(A64, W, K)), M
+        five = got if five is None else five
+        assert np.array_equal(got[:5], five), M
+        da.free(); out.free()
+    dw.free()
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "q4"])
+def test_many_steps_of_wide_gated_tiles(lib, orc, fmt):
+    """The same of a gated product wide enough for the widest tiles: 20 steps or five units to a wavefront."""
+    ff, K = 4865, 5120
+    A = orc.normal(40 * K, 29).reshape(40, K)
+    w, W = _weights(orc, fmt, 2 * ff, K, 30)
+    p, s = A.astype(np.float64) @ W.T, _slack(A.astype(np.float64), W, K)
+    g, u, sg, su = p[:, :ff], p[:, ff:], s[:, :ff], s[:, ff:]
+    act = g / (1 + np.exp(-g))
+    bound = 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u)
+    dw, five = lib.to_device(w), None
+    for M in (5, 20, 40):
+        print("case gemm_rows long gated", fmt, M, ff, K, flush=True)
+        da, out = lib.to_device(A[:M]), lib.to_device(np.full((M, ff), np.nan, np.float32))
+        (lib.gemm_bf16_nt_swiglu if fmt == "bf16" else lib.gemm_q4_nt_swiglu)(da, dw, out, M, ff, K)
+        got = out.numpy()
+        assert np.all(np.abs(got - (act * u)[:M]) <= bound[:M]), M
+        five = got if five is None else five
+        assert np.array_equal(got[:5], five), M
+        da.free(); out.free()
+    dw.free()
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [("bf16", 40, 130, 896), ("q4", 40, 130, 896), ("q4", 77, 896, 896), ("q4", 128, 900, 384)])
+def test_infinities_and_nan_stay_in_their_rows(lib, orc, fmt, M, N, K):
+    """An infinity and a NaN make their rows NaN (an infinity's lower terms are); the other rows keep their bits, also where
+    a block multiplies once more for them."""
+    print("case gemm_rows not finite", fmt, M, N, K, flush=True)
+    A = orc.normal(M * K, 33).reshape(M, K)
+    w, _ = _weights(orc, fmt, N, K, 34)
+    da, dw, out = lib.to_device(A), lib.to_device(w), lib.empty((M, N))
+    call = lib.gemm_bf16_nt if fmt == "bf16" else lib.gemm_q4_nt
+    call(da, dw, out, M, N, K)
+    clean = out.numpy()
+    A[3, 5], A[M - 1, K - 1] = np.inf, np.nan
+    call(da.upload(A), dw, out, M, N, K)
+    got, rest = out.numpy(), [r for r in range(M) if r not in (3, M - 1)]
+    assert np.isnan(got[[3, M - 1]]).all() and np.array_equal(got[rest], clean[rest])
+    for b in (da, dw, out):
+        b.free()
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [("bf16", 37, 896, 4864), ("bf16", 77, 896, 4864), ("q4", 20, 896, 4864), ("q4", 77, 896, 4864)])
+def test_recorded_without_scratch(fresh_lib, recorded, orc, fmt, M, N, K):
+    """Where the parts of a split K have no room the product is formed in one part."""
+    print("case gemm_rows recorded", fmt, M, N, K, flush=True)
+    A = orc.normal(M * K, 35).reshape(M, K)
+    w, W = _weights(orc, fmt, N, K, 36)
+    want, slack = A.astype(np.float64) @ W.T, _slack(A.astype(np.float64), W, K)
+    da, dw, out = fresh_lib.to_device(A), fresh_lib.to_device(w), fresh_lib.empty((M, N))
+    call = fresh_lib.gemm_bf16_nt if fmt == "bf16" else fresh_lib.gemm_q4_nt
+    call(da, dw, out, 1, 16, 128)                  # (the first launch of a library loads its kernels)
+    for got in recorded(lambda: call(da, dw, out, M, N, K), out):
+        assert np.all(np.abs(got - want) <= slack)
+    before = fresh_lib.alloc_calls()
+    call(da, dw, out, M, N, K)                     # with scratch to be had: in parts
+    assert fresh_lib.alloc_calls() > before and np.all(np.abs(out.numpy() - want) <= slack)
     for b in (da, dw, out):
         b.free()
 

@@ -25,6 +25,27 @@ def test_edges(lib, orc, M, N, K, tb):
         b.free()
 
 
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(16, 70, 2100), (30, 131, 1300), (45, 67, 1607), (64, 129, 2049), (100, 65, 1500)])
+def test_recorded_without_scratch(fresh_lib, recorded, orc, M, N, K, tb):
+    """Where the parts of a split K have no room a block takes all of it: 10 to 17 steps to a wavefront, whose three or four
+    slots of registers are filled several times, for one to four row tiles."""
+    print("case sgemm rows recorded", M, N, K, tb, flush=True)
+    A, B = orc.normal(M * K, 66).reshape(M, K), orc.normal(N * K, 67).reshape((N, K) if tb else (K, N))
+    Bd = (B.T if tb else B).astype(np.float64)
+    want, slack = A.astype(np.float64) @ Bd, (K + 8) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(Bd))
+    da, db, out = fresh_lib.to_device(A), fresh_lib.to_device(B), fresh_lib.empty((M, N))
+    call = lambda m, n, k: fresh_lib.gemm(da, K, 0, db, K if tb else N, tb, out, m, n, k)
+    call(1, 1, 16)                                 # (the first launch of a library loads its kernels)
+    for got in recorded(lambda: call(M, N, K), out):
+        assert np.all(np.abs(got - want) <= slack)
+    before = fresh_lib.alloc_calls()
+    call(M, N, K)                                  # with scratch to be had: in parts
+    assert fresh_lib.alloc_calls() > before and np.all(np.abs(out.numpy() - want) <= slack)
+    for b in (da, db, out):
+        b.free()
+
+
 @pytest.mark.parametrize("M,N,K", [(20, 130, 37), (70, 90, 700)])
 def test_infinities_and_nan_stay_where_they_are(lib, orc, M, N, K):
     """A row with an infinity gives infinities of the sign of the column's weight, one with a NaN gives NaN, a zero
