@@ -116,8 +116,9 @@ __global__ __launch_bounds__(256) void softmax_kernel(const float* __restrict__ 
 }
 
 // General f32 GEMM with transposed-view operands and an affine epilogue, VALU form:
-// 64x64 tile, 16-wide K slab through LDS, 4x4 outputs per thread. Serves fewer than 16 k and
-// small transposed A; everything else runs on the matrix-pipe kernels of sgemm.hip.
+// 64x64 tile, 16-wide K slab through LDS, 4x4 outputs per thread. Serves what the matrix-pipe kernels of
+// sgemm.hip do not: fewer than 16 k; fewer than 128 rows or columns of a transposed A or of one with more than 1024
+// rows; under 128 rows, many columns of less than 48 k (launch_sgemm_rows); row or column counts past those kernels' grids.
 __global__ __launch_bounds__(256) void sgemm_kernel(const float* __restrict__ A, int64_t lda,
                                                     int ta, const float* __restrict__ B,
                                                     int64_t ldb, int tb, float* __restrict__ C,

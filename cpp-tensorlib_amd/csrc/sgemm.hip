@@ -387,7 +387,7 @@ __global__ __launch_bounds__(64 * kSrWaves, 2) void sgemm_rows_kernel(const floa
 }
 
 // The same for A as it is stored ([M][K]); the caller has checked the arguments. tiled: the LDS-tiled kernel takes the
-// product too; 1 is returned, and nothing launched, where it is the better one.
+// product too, else the vector-ALU kernel; 1 is returned, and nothing launched, where that is the better one.
 int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb, int tb, float* pc, int M, int N, int K, float scale,
                       float offset, int epi, bool tiled) {
   // Row blocks and K splits (parts in scratch, summed in a fixed order) that an estimate in clocks likes best: a block
@@ -414,6 +414,11 @@ int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb
     if (least > 2100 * (6 + 1.5 * ((K + 15) / 16) * std::max(1.0, tiles128 / 256))) return 1;
   }
   const int64_t tiles = rb * columns;
+  // Fewer than 128 rows or columns, which is what the vector-ALU kernel is left with: more than one, two and four rounds of
+  // these blocks for K up to 16, 32 and 47 cost more than its 64 x 64 tiles, which meet no one at their end (us, here and there: 100 x
+  // 25000 x 16 15 and 10, 127 x 60000 x 20 32 and 24, 100 x 60000 x 33 31 and 28; 64 x 12000 x 16 4.6 and 5.6). With up to 32 rows
+  // half of such a tile or more is empty (16 x 30000 x 16: 4.0 and 5.0).
+  if (!tiled && K < 48 && M > 32 && tiles >> ((K + 15) / 16 - 1) > cus) return 1;
   int kchunk = K;
   float* dst = pc;
   if (S > 1) {
