@@ -15,6 +15,7 @@
 // tiles, 64 accumulator registers), K slabs of 16; the next slab's global loads are in
 // flight while the current one is multiplied.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -168,29 +169,40 @@ __global__ __launch_bounds__(256) void sgemm_sum_kernel(const float* __restrict_
   C[i] = epi ? add_rn(mul_rn(a, scale), offset) : a;
 }
 
-// Launches the matrix-pipe GEMM; the caller has checked the arguments.
-int launch_sgemm_mfma(const float* pa, int64_t lda, int ta, const float* pb, int64_t ldb, int tb, float* pc,
-                      int M, int N, int K, float scale, float offset, int epi) {
-  const int64_t tiles = (int64_t)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
-  // Too few tiles to fill the chip: split K over gridDim.z (at least 256 of K per slice) into
-  // scratch parts that are summed in a fixed order - deterministic, no atomics.
+// 16-byte loads need aligned bases and row strides that keep every row aligned
+static bool sgemm_aligned(const float* pa, int64_t lda, const float* pb, int64_t ldb) {
+  return aligned16(pa) && aligned16(pb) && (lda % 4) == 0 && (ldb % 4) == 0;
+}
+// Too few tiles to fill the chip: split K over gridDim.z (at least 256 of K per slice) into
+// scratch parts that are summed in a fixed order - deterministic, no atomics.
+static int sgemm_mfma_splits(int64_t tiles, int K) {
   int S = 1;
   if (tiles < ctx().cus) {
     S = (int)((2 * (int64_t)ctx().cus + tiles - 1) / tiles);
     if (S > 8) S = 8;
     while (S > 1 && K / S < 256) S--;
   }
+  if (S > 1) {
+    const int kchunk = ((K + S - 1) / S + kSgBK - 1) / kSgBK * kSgBK;
+    S = (K + kchunk - 1) / kchunk;
+  }
+  return S;
+}
+
+// Launches the matrix-pipe GEMM; the caller has checked the arguments.
+int launch_sgemm_mfma(const float* pa, int64_t lda, int ta, const float* pb, int64_t ldb, int tb, float* pc,
+                      int M, int N, int K, float scale, float offset, int epi) {
+  const int64_t tiles = (int64_t)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
+  const int S = sgemm_mfma_splits(tiles, K);
   int kchunk = K;
   float* dst = pc;
   if (S > 1) {
     kchunk = ((K + S - 1) / S + kSgBK - 1) / kSgBK * kSgBK;
-    S = (K + kchunk - 1) / kchunk;
-    dst = S > 1 ? static_cast<float*>(scratch((size_t)S * M * N * sizeof(float))) : pc;
+    dst = static_cast<float*>(scratch((size_t)S * M * N * sizeof(float)));
     if (!dst) return fail(TLHIP_ENOMEM, "tlhip_gemm: no scratch for %d K-splits", S);
   }
   const dim3 grid((unsigned)((N + kSgBN - 1) / kSgBN), (unsigned)((M + kSgBM - 1) / kSgBM), (unsigned)S);
-  // 16-byte loads need aligned bases and row strides that keep every row aligned
-  const int aligned = aligned16(pa) && aligned16(pb) && (lda % 4) == 0 && (ldb % 4) == 0;
+  const int aligned = sgemm_aligned(pa, lda, pb, ldb);
   hipStream_t st = ctx().stream;
   const int kepi = S > 1 ? 0 : epi;   // the part sum applies the epilogue when K is split
 #define TLHIP_SGEMM(TA_, TB_)                                                                         \
@@ -406,19 +418,30 @@ int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb
       if (least < 0 || t < least) { least = t; rb = r; TM = tm; S = s; }
     }
   }
-  // With fewer than 256 k there is nothing to split, and blocks in several rounds each start and end for two steps or
-  // less. The LDS-tiled kernel's time there, measured from 128 x 128 to 1024 x 9000: 6 us and 1.5 for every 16 k, over
-  // 256 tiles in proportion (986 x 7459 x 22: 15 us, 42 here; 614 x 4098 x 29 9.8 and 17; 300 x 2000 x 60 11 and 7.6).
-  if (tiled && K < 256) {
-    const double tiles128 = (double)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
-    if (least > 2100 * (6 + 1.5 * ((K + 15) / 16) * std::max(1.0, tiles128 / 256))) return 1;
+  // The LDS-tiled kernel is the better one where blocks in several rounds each start and end for a few steps, and for many
+  // columns of a middling K (986 x 7459 x 22: 15 us, 42 here; 864 x 18126 x 308 117 and 181; but 300 x 2000 x 60 11 and 7.6). Both
+  // times in us, fitted to 2210 runs (128 to 1024 rows, 128 to 150000 columns, K 16 .. 5000; errors 8 and 6 %): a start; for every
+  // round of blocks its own start and end and its steps of 16 k (per row tile here); the outputs' megabytes, twice for parts; and
+  // the launch that adds those up.
+  if (tiled) {
+    const int64_t tiles128 = (int64_t)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
+    const int St = sgemm_mfma_splits(tiles128, K);
+    const auto steps = [&](int parts) { return (double)(((K + parts - 1) / parts + kSgBK - 1) / kSgBK); };
+    const auto mb = [&](int parts) { return 4e-6 * M * N * (parts > 1 ? 2 * parts : 1); };
+    const double here = 2.2 + std::ceil((double)rb * columns * S / cus) * (1.15 + TM * (0.25 + (tb ? 0.81 : 0.72) * steps(S) / kSrWaves)) +
+                        0.28 * mb(S) + (S > 1 ? 2.2 : 0);
+    const double fill = (double)tiles128 * St / cus;   // blocks run two to a CU, and the last round's gaps are partly filled
+    const double there = 5.5 + std::max(1.0, 0.14 * fill + 0.86 * std::ceil(fill)) *
+                                   (steps(St) * (sgemm_aligned(pa, lda, pb, ldb) ? 1.41 : 1.57) - 1) + 0.16 * mb(St) + (St > 1 ? 7.9 : 0);
+    // (its parts need scratch, which a recording may not grow: the product stays here then)
+    if (here > 1.02 * there && (St == 1 || scratch((size_t)St * M * N * sizeof(float)))) return 1;
   }
   const int64_t tiles = rb * columns;
   // Fewer than 128 rows or columns, which is what the vector-ALU kernel is left with: more than one, two and four rounds of
   // these blocks for K up to 16, 32 and 47 cost more than its 64 x 64 tiles, which meet no one at their end (us, here and there: 100 x
-  // 25000 x 16 15 and 10, 127 x 60000 x 20 32 and 24, 100 x 60000 x 33 31 and 28; 64 x 12000 x 16 4.6 and 5.6). With up to 32 rows
-  // half of such a tile or more is empty (16 x 30000 x 16: 4.0 and 5.0).
-  if (!tiled && K < 48 && M > 32 && tiles >> ((K + 15) / 16 - 1) > cus) return 1;
+  // 25000 x 16 15 and 10, 127 x 60000 x 20 32 and 24, 100 x 60000 x 33 31 and 28; 64 x 12000 x 16 4.6 and 5.6). Up to 32 rows leave
+  // half of such a tile empty: twice the rounds (26 x 102934 x 24 22 and 15, 16 x 30000 x 16 4.0 and 5.0).
+  if (!tiled && K < 48 && M > 16 && tiles >> ((K + 15) / 16 - (M > 32 ? 1 : 0)) > cus) return 1;
   int kchunk = K;
   float* dst = pc;
   if (S > 1) {

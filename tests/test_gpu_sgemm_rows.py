@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("tb", [0, 1])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 16), (2, 3, 17), (5, 70, 31), (16, 64, 128), (17, 65, 129), (33, 4, 200), (48, 257, 64), (64, 896, 4864),
                                    (65, 100, 1000), (127, 63, 16), (129, 130, 97), (200, 1153, 901), (333, 640, 896), (1000, 61, 65),
-                                   (33, 16500, 16), (33, 16320, 16), (100, 25003, 20), (127, 40001, 33), (64, 70000, 47)])
+                                   (33, 16500, 16), (33, 16320, 16), (100, 25003, 20), (127, 40001, 33), (64, 70000, 47), (17, 33100, 16),
+                                   (208, 5518, 296), (864, 4021, 308), (153, 17729, 245)])
 def test_edges(lib, orc, M, N, K, tb):
     print("case sgemm rows", M, N, K, tb, flush=True)
     A, B = orc.normal(M * K, 61).reshape(M, K), orc.normal(N * K, 62).reshape((N, K) if tb else (K, N))
