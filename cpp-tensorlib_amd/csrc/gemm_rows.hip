@@ -498,10 +498,15 @@ static RowsPlan plan_row_blocks(int64_t M, int64_t N, int64_t K, bool gu, bool q
         best.tiles = (int)tiles;
         best.part_units = (int)per;
         // fewer steps than wavefronts leave some idle; five row tiles of int4 spill, and int4 blocks in turn wait for what
-        // they would have loaded ahead
-        const double work = rounds * n * std::max(mem * (double)std::min<int64_t>(rows::kWaves, per) / rows::kWaves, per > 4 ? math : math / 2) / 2100;
+        // they would have loaded ahead; over many blocks, wavefronts with a unit more than others even out (38 x 18088 gated x
+        // 2560, 20 units over eight wavefronts: 64 us here, 89 in the 64-row tiles)
+        const double own = q4 && blocks > 2 * cus && per > rows::kWaves ? 1.05 * (double)per / rows::kWaves * steps : n;
+        const double work = rounds * own * std::max(mem * (double)std::min<int64_t>(rows::kWaves, per) / rows::kWaves, per > 4 ? math : math / 2) / 2100;
         best.us = q4 ? 2 + work * (TM == 5 ? 1.3 : 1.0) * (rounds > 2 ? 1.2 : rounds > 1 ? 0.81 : 0.74) + rounds * (0.3 + 0.18 * TM * TN) + parts
                      : 0.85 + 1.15 * work + rounds * (1.2 + 0.18 * TM * TN) + 0.75 * parts;
+        // many columns of a short K (14000 runs, N 20000 .. 160000): 24 x 21497 gated x 512 int4 24.8 us for an estimate of 20.3, 111 x
+        // 10540 gated x 256 bf16 15.3 for 19.9
+        if (blocks > 2 * cus) best.us *= q4 ? (per <= 4 ? 1.2 : 1.0) : M > 64 && K <= 384 ? 0.78 : 1.0;
       }
     }
   }
@@ -512,6 +517,10 @@ RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64
   const int64_t rows_w = (gu ? 2 : 1) * N, t16 = (M + 15) / 16;
   if (M > 128 || K % (q4 ? 128 : 32) != 0 || M * K * 4 >= (int64_t(1) << 32) || rows_w * K * (q4 ? 1 : 4) / 2 >= (int64_t(1) << 32))
     return RowsPlan{};                             // (32-bit byte offsets)
+  // Up to 16 rows nothing else is as fast, save for int4 with so few units that most wavefronts of a block have none and so many
+  // columns that blocks come in more rounds than that: up to 65000 columns x 128 twice what the 64-row tiles take, x 256 1.4 times;
+  // up to 32768 x 256 0.9 times
+  if (q4 && M <= 16 && K < 512 && (rows_w + 63) / 64 > K / 128 * (int64_t)ctx().cus) return RowsPlan{};
   const auto plan = [&](int64_t row_blocks) { return plan_row_blocks(M, N, K, gu, q4, max_S, row_blocks); };
   if (!q4 || t16 != 5) return plan((t16 + rows::kMaxTM - 1) / rows::kMaxTM);
   // int4 with 65 to 80 rows: one block of five row tiles, or two of three (77 x 640 x 768 7.8 us and 6.1; 74 x 4609 x 11008, whose

@@ -11,7 +11,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 16, 128), (2, 33, 128), (5, 200, 256), (16, 896, 896), (17, 130, 128), (37, 1152, 896), (64, 64, 3584),
-          (65, 100, 128), (77, 896, 4864), (80, 36, 2048), (81, 260, 384), (97, 128, 896), (128, 72, 640)]
+          (65, 100, 128), (77, 896, 4864), (80, 36, 2048), (81, 260, 384), (97, 128, 896), (128, 72, 640),
+          (9, 18500, 128), (16, 18300, 128), (60, 33000, 128)]
 
 
 def _weights(orc, fmt, N, K, seed):
