@@ -79,7 +79,8 @@ __global__ __launch_bounds__(256) void q4_image_kernel(const float* __restrict__
   }
 }
 
-// eight nibbles of a word as f16 weights n - 8, k in the images' order
+// eight nibbles of a word as f16 weights n - 8, k in the images' order. Masked into the last bits of 1024, upper nibbles sixteen
+// times as large: the magic-number conversion of int4 weights (Kim et al., "Who Says Elephants Can't Run", 2022), from the f16 format.
 __device__ __forceinline__ frag16 nib8(uint32_t w) {
   const f16x2 off = {(_Float16)-1032.0f, (_Float16)-1032.0f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, off16 = {(_Float16)-72.0f, (_Float16)-72.0f};
   const uint32_t u = w >> 8;

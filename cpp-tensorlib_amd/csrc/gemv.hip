@@ -674,7 +674,7 @@ static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int pro, int cus, int lds
     //  * up to 16 rows per CU: one tile per CU of its share of the rows, four to a wavefront, and K over as many
     //    wavefronts as the block takes, where they get as many chunks each (16 rows and two splits left half the CUs of
     //    2048 x 12288 without a tile: 12.3 -> 9.8; 2048 x 4096 8.4 -> 7.2, 2048 x 2048 4.7 -> 3.9, 896 x 4864 4.9 -> 4.3,
-    //    3392 x 2048 7.4 -> 6.7; 3584 x 3584, seven chunks over four, would be 6.9 for 6.6);
+    //    3392 x 2048 7.4 -> 6.7; 3584 x 3584, seven chunks over four, would be 6.9 for 6.6).
     //    Not for one row per CU behind a gate, whose two wavefronts would be slow to form x (256 x 1024 3.4 -> 3.5);
     //  * up to 31 rows and three chunks: the same without the split, whose halves are uneven (5376 x 1536 6.2 -> 5.4). The
     //    halves of two chunks are even, which a plain x gains from (5120 x 896 4.5 with the split, 4.7 without);
