@@ -565,7 +565,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   static const int kBm[4] = {128, 64, 64, 128}, kBn[4] = {256, 128, 64, 128};
   // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
   // against 50, 301 x 37888 x 3584 209 against 303)
-  bool images = half && K <= 32768 && (per * N >= 2048 || K <= 1024);
+  const bool images_fit = half && K <= 32768 && (per * N >= 2048 || K <= 1024);
+  bool images = images_fit;
   Q4Plan q4_plan;
   if (images) q4_plan = plan_gemm_q4(M, N, K, parts_bytes, want_parts, gu, can_split);
   const auto part_slabs = [&](const Piece& O) { return cdiv(cdiv(K, O.S), kBK); };
@@ -639,7 +640,20 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   char* sbase = nullptr;
   if (ea_bytes + parts_need > 0) {
     sbase = static_cast<char*>(scratch(ea_bytes + parts_need));
-    if (!sbase) return fail(TLHIP_ENOMEM, "tlhip_gemm_bf16_nt: no scratch for row exponents and K-split parts");
+    if (!sbase) {   // (a recording may not grow it) what would have been slower, if it needs less
+      const RowsPlan P = aligned16(C) ? plan_gemm_rows(M, N, K, gu, q4, 1) : RowsPlan{};
+      if (P.S > 0) {
+        if (want_parts) *S_out = 1;
+        if (int rc = launch_gemm_rows(P, pa, W, static_cast<const float*>(scales), pc, M, N, K, N, gu)) return rc;
+        TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+      }
+      if (images_fit && !images) {
+        const int rc = gemm_q4_prompt(q4_plan, pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, S_out, gu);
+        if (rc < 0) return rc;
+        if (rc != kNoScratch) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+      }
+      return fail(TLHIP_ENOMEM, "tlhip_gemm_bf16_nt: no scratch for row exponents and K-split parts");
+    }
   }
   int* ea = reinterpret_cast<int*>(sbase);
   if (half) row_exponent_f32_kernel<<<dim3((unsigned)M), dim3(256), 0, c.stream>>>(pa, (int)K, ea);

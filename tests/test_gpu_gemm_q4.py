@@ -99,3 +99,17 @@ def test_recorded_without_room_for_the_images(fresh_lib, recorded, orc):
     assert fresh_lib.alloc_calls() > before and np.all(np.abs(out.numpy() - want) <= slack)
     for b in (da, dw, out):
         b.free()
+
+
+def test_recorded_without_room_for_parts(fresh_lib, recorded, orc):
+    """359 rows of this weight are formed without images, in two parts of 31 MB; a recording with room for the images only (3 MB)
+    takes those."""
+    M, N, K = 359, 10880, 1792
+    print("case gemm_q4 recorded parts", M, N, K, flush=True)
+    da, dw, want, slack = _case(fresh_lib, orc, M, N, K, 91)
+    out = fresh_lib.empty((M, N))
+    fresh_lib.gemm_q4_nt(da, dw, out, 65, 2048, 32)   # (scratch comes in 8 MB at least)
+    for got in recorded(lambda: fresh_lib.gemm_q4_nt(da, dw, out, M, N, K), out):
+        assert np.all(np.abs(got - want) <= slack)
+    for b in (da, dw, out):
+        b.free()

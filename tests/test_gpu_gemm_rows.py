@@ -136,9 +136,11 @@ def test_infinities_and_nan_stay_in_their_rows(lib, orc, fmt, M, N, K):
         b.free()
 
 
-@pytest.mark.parametrize("fmt,M,N,K", [("bf16", 37, 896, 4864), ("bf16", 77, 896, 4864), ("q4", 20, 896, 4864), ("q4", 77, 896, 4864)])
+@pytest.mark.parametrize("fmt,M,N,K", [("bf16", 37, 896, 4864), ("bf16", 77, 896, 4864), ("q4", 20, 896, 4864), ("q4", 77, 896, 4864),
+                                         ("bf16", 64, 4608, 3584), ("q4", 128, 4608, 3584)])
 def test_recorded_without_scratch(fresh_lib, recorded, orc, fmt, M, N, K):
-    """Where the parts of a split K have no room the product is formed in one part."""
+    """Where the parts of a split K have no room the product is formed in one part, also one that another kernel would have formed
+    in parts (the last two)."""
     print("case gemm_rows recorded", fmt, M, N, K, flush=True)
     A = orc.normal(M * K, 35).reshape(M, K)
     w, W = _weights(orc, fmt, N, K, 36)
