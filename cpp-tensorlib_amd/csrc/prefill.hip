@@ -601,7 +601,7 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
         else if (M <= 64) other += 2.2 + (double)slabs * (bn > 64 ? slab_us(blocks, c.cus, 0.9, 1.12) : slab_us(blocks, c.cus, 0.65, 0.95)) *
                                              (bn == 64 && O.S == 1 && blocks > 3 * c.cus ? 0.85 : 1);   // (four blocks to a CU: 60 x 64982 x 768 32 us, 43 by rows)
         else if (q4) other += 12.1 + (double)slabs * slab_us(blocks, c.cus, 1.03, 1.03);
-        else other += 7 + (double)slabs * slab_us(blocks, c.cus, 1.5, 2.18);
+        else other += (gu && K <= 256 ? 9 : 7) + (double)slabs * slab_us(blocks, c.cus, 1.5, 2.18);   // (67 x 10732 gated x 128: 16.2 us, 10.8 by rows)
         if (O.S > 1) other += (M <= 64 ? 0.65e-6 : 0.36e-6) * O.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
       }
       if (P.us + (P.S > 1 && !want_parts ? kPartSumUs : 0) > other) P.S = 0;
