@@ -289,7 +289,8 @@ int tlhip_gemm(const void* a, int64_t a_off, int64_t lda, int ta, const void* b,
   const int epi = !(scale == 1.0f && offset == 0.0f);
   // Up to 1024 rows of an A that is stored as it is read: the kernel that splits K inside its blocks, unless the
   // product is whole 128 x 128 tiles of aligned rows and at least two of them tall, where the LDS-tiled kernel reads
-  // each operand once per tile (512 x 4608 x 3584: 215 us against 258; but 333 x 4864 x 896: 66 against 46).
+  // each operand once per tile (512 x 4608 x 3584: 215 us against 258; but 333 x 4864 x 896: 66 against 46), or that
+  // kernel's or the vector-ALU kernel's estimated time is less (launch_sgemm_rows returns 1).
   const bool tiled = m >= 128 && n >= 128 && k >= 16 && (m + 127) / 128 <= 65535;
   const bool whole = m >= 256 && (m % 128) == 0 && (n % 128) == 0 && (k % 16) == 0 && (lda % 4) == 0 && (ldb % 4) == 0 && aligned16(pa) && aligned16(pb);
   // (2^23 blocks of 512 threads are what a grid's x can count)
