@@ -148,6 +148,7 @@ SIGNATURES = {
     "tlhip_ssm_chunk": (cint, [P, i64, P, i64, P, i64, i64]),
     "tlhip_latent_cache_bytes": (i64, [i64, i64, i64, i64, cint]),
     "tlhip_latent_attn_run": (cint, [P, i64, P, i64, P, i64, P, i64, i64, P]),
+    "tlhip_embed_rows": (cint, [P, cint, P, i64, P, i64, i64]),
     "tlhip_tune_gemv_q4": (cint, [cint, cint, cint, cint, cint]),
     "tlhip_tune_gemv_cols": (cint, [cint]),
     "tlhip_tune_attn_prefill": (cint, [cint]),
@@ -663,6 +664,10 @@ class TlHip:
 
     def gather_rows(self, src, idx, out, n, rows, src_rows):
         self._chk(self.c.tlhip_gather_rows(src.ptr, idx.ptr, out.ptr, n, rows, src_rows))
+
+    def embed_rows(self, table, table_type, ids, out, hidden, vocab):
+        ids = np.ascontiguousarray(ids, np.int64)
+        self._chk(self.c.tlhip_embed_rows(table.ptr, table_type, ids.ctypes.data_as(P), len(ids), out.ptr, hidden, vocab))
 
     def tune_attn_prefill(self, kernel):
         """0 / False: built-in choice, 1 / True: VALU kernel, 2: fp32 matrix pipe, 4: f16 terms."""

@@ -212,6 +212,45 @@ __global__ __launch_bounds__(256) void embed_gather_f16_kernel(const uint16_t* _
   out[j] = f16_bits_to_f32(table[static_cast<size_t>(tok) * hidden + j]);
 }
 
+// out[t][j] = widen(table[ids[t]][j]). The ids ride in the launch's arguments: no copy to wait for (a prompt of 512 x 3584
+// widened on the host and copied took 600 us, this 6). Bound by the launch; V numbers a thread.
+template <int M> struct TokenIds { int id[M]; };   // a launch of one id carries few
+constexpr int kFewIds = 8, kManyIds = 768;
+template <bool F16, int V, int M>
+__global__ __launch_bounds__(256) void embed_rows_kernel(const uint16_t* __restrict__ table, const TokenIds<M> ids,
+                                                         float* __restrict__ out, int hidden) {
+  const int t = blockIdx.y, j = (blockIdx.x * 256 + threadIdx.x) * V;
+  if (j >= hidden) return;
+  const uint16_t* row = table + (size_t)ids.id[t] * hidden + j;
+  float* o = out + (size_t)t * hidden + j;
+  if constexpr (V == 8) {
+    const uint4 w = *reinterpret_cast<const uint4*>(row);
+    const uint32_t d[4] = {w.x, w.y, w.z, w.w};
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      f[2 * i] = F16 ? f16_bits_to_f32((uint16_t)(d[i] & 0xffffu)) : bf16_lo(d[i]);
+      f[2 * i + 1] = F16 ? f16_bits_to_f32((uint16_t)(d[i] >> 16)) : bf16_hi(d[i]);
+    }
+    reinterpret_cast<float4*>(o)[0] = make_float4(f[0], f[1], f[2], f[3]);
+    reinterpret_cast<float4*>(o)[1] = make_float4(f[4], f[5], f[6], f[7]);
+  } else {
+    *o = F16 ? f16_bits_to_f32(*row) : __uint_as_float((uint32_t)*row << 16);
+  }
+}
+
+template <bool F16, int V, int M>
+static void launch_embed_rows(const void* table, const int64_t* ids, int64_t T, float* out, int64_t hidden) {
+  const unsigned gx = (unsigned)((hidden + 256 * V - 1) / (256 * V));
+  for (int64_t t0 = 0; t0 < T; t0 += M) {
+    const int n = (int)std::min<int64_t>(T - t0, M);
+    TokenIds<M> a{};
+    for (int t = 0; t < n; t++) a.id[t] = (int)ids[t0 + t];
+    embed_rows_kernel<F16, V, M><<<dim3(gx, (unsigned)n), dim3(256), 0, ctx().stream>>>(
+        static_cast<const uint16_t*>(table), a, out + t0 * hidden, (int)hidden);
+  }
+}
+
 static bool known_type(int t) { return t == TLHIP_T_F32 || t == TLHIP_T_F16 || t == TLHIP_T_BF16; }
 
 }  // namespace tlhip
@@ -308,6 +347,22 @@ int tlhip_embed_gather_f16(const void* table, const void* d_token, void* out, in
   hipError_t e_ = hipGetLastError();
   if (e_ != hipSuccess) return hip_fail(e_, "kernel launch");
   return TLHIP_OK;
+}
+
+int tlhip_embed_rows(const void* table, int table_type, const int64_t* ids, int64_t T, void* out, int64_t hidden, int64_t vocab) {
+  TLHIP_REQUIRE_READY();
+  const char* who = "tlhip_embed_rows";
+  if (!table || !ids || !out) return fail(TLHIP_EINVAL, "%s: null pointer", who);
+  if (table_type != TLHIP_T_F16 && table_type != TLHIP_T_BF16) return fail(TLHIP_EINVAL, "%s: an f16 or bf16 table", who);
+  if (T <= 0 || hidden <= 0 || vocab <= 0 || hidden > (1 << 30) || vocab > 0x7fffffff) return fail(TLHIP_EINVAL, "%s: bad shape", who);
+  for (int64_t t = 0; t < T; t++)
+    if (ids[t] < 0 || ids[t] >= vocab) return fail(TLHIP_EINVAL, "%s: id outside the table", who);
+  const bool f16 = table_type == TLHIP_T_F16, wide = hidden % 8 == 0 && aligned16(table) && aligned16(out), few = T <= kFewIds;
+  const auto go = wide ? (few ? (f16 ? launch_embed_rows<true, 8, kFewIds> : launch_embed_rows<false, 8, kFewIds>)
+                              : (f16 ? launch_embed_rows<true, 8, kManyIds> : launch_embed_rows<false, 8, kManyIds>))
+                       : (f16 ? launch_embed_rows<true, 1, kManyIds> : launch_embed_rows<false, 1, kManyIds>);
+  go(table, ids, T, static_cast<float*>(out), hidden);
+  TLHIP_CHECK_LAUNCH(TLHIP_C_EMBED);
 }
 
 }  // extern "C"

@@ -155,6 +155,7 @@ struct api {
                         int64_t);
   int (*qkv_rope_append_tab)(void*, const void*, const void*, const void*, void*, void*, int64_t, int64_t,
                              int64_t, int64_t, const void*, int64_t, const void*, int) = nullptr;
+  int (*embed_rows)(const void*, int, const int64_t*, int64_t, void*, int64_t, int64_t) = nullptr;
   int (*embed_gather_bf16)(const void*, const void*, void*, int64_t, int64_t) = nullptr;
   int (*token_advance)(void*, const void*, void*, int64_t) = nullptr;
   int (*gemv_q4_swiglu)(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t) = nullptr;
@@ -394,6 +395,7 @@ struct context {
               bind(f.attn_decode_qkv, "tlhip_attn_decode_qkv") &&
               bind(f.tune_gemv_cols, "tlhip_tune_gemv_cols") && bind(f.convert, "tlhip_convert") && bind(f.convert_transpose, "tlhip_convert_transpose") &&
               bind(f.quantize_q4, "tlhip_quantize_q4") && bind(f.embed_gather_f16, "tlhip_embed_gather_f16") &&
+              bind(f.embed_rows, "tlhip_embed_rows") &&
               bind(f.embed_gather_bf16, "tlhip_embed_gather_bf16") &&
               bind(f.token_advance, "tlhip_token_advance") &&
               bind(f.gemv_q4_swiglu, "tlhip_gemv_q4_swiglu") &&
@@ -1306,6 +1308,16 @@ inline bool embed_gather_f16(void* table, void* d_token, void* out, int64_t hidd
   L.reads(table, d_token);
   L.writes(out);
   return L.sent(L.lib.embed_gather_f16(table, d_token, out, hidden, vocab));
+}
+
+// out[T, hidden] = widened rows ids[0..T) of an f16 or bf16 table on the device; the ids travel with the launch. false, with
+// nothing launched, for an id outside [0, vocab).
+inline bool embed_rows(void* table, bool f16, const int64_t* ids, int64_t T, void* out, int64_t hidden, int64_t vocab) {
+  launch L;
+  if (!L.ok) return false;
+  L.reads(table);
+  L.writes(out);
+  return L.sent(L.lib.embed_rows(table, f16 ? 1 : 2, ids, T, out, hidden, vocab));
 }
 
 // ---- device-resident greedy loop -----------------------------------------------------------

@@ -70,7 +70,6 @@ struct scratch {
   void* res[2] = {nullptr, nullptr};
   void *hb = nullptr, *h2b = nullptr, *qkvb = nullptr, *ab = nullptr, *mb = nullptr, *gub = nullptr,
        *mdb = nullptr, *logitsb = nullptr, *embedb = nullptr;
-  float* embed_host = nullptr;
   float* logits_host = nullptr;
 };
 
@@ -83,7 +82,6 @@ struct prefill_scratch {
   void* rope = nullptr;         // (cos, sin)[T][head_dim/2] of the chunk being run
   void* parts = nullptr;        // K-split parts of the o-proj / down products, read by the residual norm
   int64_t parts_bytes = 0;
-  float* emb_host = nullptr;
 };
 
 // GPU time per region of a decode step, from events on the library's stream around the launches
@@ -99,14 +97,13 @@ struct step_prof {
 struct model {
   dims d{};
   prefill_scratch ps;
-  std::vector<uint16_t> embed;  // [vocab, hidden] bf16 or f16 rows, gathered on the host (qm:530-535)
+  void* embed = nullptr;        // [vocab, hidden] bf16 or f16 rows on the device (the reference gathers on the host, qm:530-535)
   bool embed_f16 = false;       // rows are IEEE half, as a model file stores token_embd (qm:297)
   void* onorm = nullptr;
   linear lm_head;
   std::vector<layer> layers;
   scratch s;
   void* rope_tab = nullptr;            // (cos, sin)[head_dim/2] of the step being run
-  void* embed_dev = nullptr;           // the embedding table on the device (greedy_loop only)
   void* attn_partials = nullptr;       // split partials of the device-position attention
   int64_t attn_partials_bytes = 0;
   bool ready = false;
@@ -193,7 +190,7 @@ inline bool init(model& M, const dims& d) {
   M.layers.assign((size_t)d.n_layers, layer{});
   auto A = [](int64_t n) { return hip::alloc(n * 4, nullptr); };
   scratch& S = M.s;
-  S.embedb = hip::alloc(d.hidden * 4, &S.embed_host);
+  S.embedb = A(d.hidden);
   S.res[0] = A(d.hidden);
   S.res[1] = A(d.hidden);
   S.hb = A(d.hidden);
@@ -259,10 +256,32 @@ inline bool set_layer_bf16(model& M, int64_t li, const layer_blobs_bf16& b) {
          L.wd.w;
 }
 
+// The embedding table, [vocab, hidden] rows of 16 bits, onto the device through a pinned block (a copy from pageable memory
+// runs at a fraction of the link's rate); the one before it is let go.
+inline bool set_embed(model& M, const void* rows, bool f16) {
+  const int64_t bytes = M.d.vocab * M.d.hidden * 2, blk = std::min(bytes, int64_t(32) << 20);
+  if (M.embed) hip::release(M.embed, 0, nullptr);
+  M.embed = hip::alloc_device(bytes);
+  M.embed_f16 = f16;
+  float* stage_host = nullptr;
+  void* stage = M.embed ? hip::alloc(blk, &stage_host) : nullptr;
+  if (!stage) return false;
+  bool ok = true;
+  for (int64_t o = 0; o < bytes && ok; o += blk) {
+    const int64_t n = std::min(blk, bytes - o);
+    std::memcpy(stage_host, static_cast<const char*>(rows) + o, (size_t)n);
+    hip::upload(stage, stage_host, (n + 3) / 4);
+    ok = hip::copy_d2d(static_cast<char*>(M.embed) + o, stage, n);
+    hip::flush();   // the staging block is used again
+  }
+  hip::release(stage, blk, stage_host);
+  return ok;
+}
+
 inline bool set_head_bf16(model& M, const uint16_t* embed_bf16, const float* onorm,
                           const uint16_t* outw_kn) {
   const dims& d = M.d;
-  M.embed.assign(embed_bf16, embed_bf16 + d.vocab * d.hidden);
+  if (!set_embed(M, embed_bf16, false)) return false;
   M.onorm = detail::dev_from_host(onorm, d.hidden * 4);
   std::vector<uint16_t> rows((size_t)(d.vocab * d.hidden));
   detail::transpose_kn(outw_kn, rows.data(), d.hidden, d.vocab);
@@ -275,7 +294,7 @@ inline bool set_head_bf16(model& M, const uint16_t* embed_bf16, const float* ono
 inline bool set_head_q4(model& M, const uint16_t* embed_bf16, const float* onorm,
                         const uint8_t* outw_q4) {
   const dims& d = M.d;
-  M.embed.assign(embed_bf16, embed_bf16 + d.vocab * d.hidden);
+  if (!set_embed(M, embed_bf16, false)) return false;
   M.onorm = detail::dev_from_host(onorm, d.hidden * 4);
   M.lm_head = linear{detail::dev_from_host(outw_q4, q4_bytes(d.vocab, d.hidden)), d.vocab, d.hidden,
                      wfmt::q4};
@@ -339,9 +358,9 @@ inline bool set_random(model& M, uint32_t seed, wfmt fmt) {
   }
   M.lm_head = make(d.vocab, d.hidden);
   M.onorm = detail::dev_from_host(hvec(d.hidden, 1.f, 0.02f).data(), d.hidden * 4);
-  M.embed.resize((size_t)(d.vocab * d.hidden));
-  for (size_t i = 0; i < M.embed.size(); i++)
-    M.embed[i] = f32_to_bf16(0.02f * ((float)(int32_t)next() * (1.0f / 2147483648.0f)));
+  std::vector<uint16_t> embed((size_t)(d.vocab * d.hidden));
+  for (auto& v : embed) v = f32_to_bf16(0.02f * ((float)(int32_t)next() * (1.0f / 2147483648.0f)));
+  ok = ok && set_embed(M, embed.data(), false);
   hip::flush();
   M.ready = ok && M.onorm;
   return M.ready;
@@ -555,13 +574,10 @@ inline bool load_gguf(model& M, const gguf::model& g, wfmt fmt, int64_t max_ctx 
   }
   if (ok) {
     const gguf::tensor_info* emb = g.tensor("token_embd.weight");
-    if (emb->type == gguf::ggml_type::f16) M.embed_f16 = true;
-    else if (emb->type == gguf::ggml_type::bf16) M.embed_f16 = false;
-    else ok = detail::why_(why, "token_embd.weight: f16 or bf16 expected");
-    if (ok) {
-      const uint16_t* rows = static_cast<const uint16_t*>(emb->data);
-      M.embed.assign(rows, rows + d.vocab * E);
-    }
+    if (emb->type != gguf::ggml_type::f16 && emb->type != gguf::ggml_type::bf16)
+      ok = detail::why_(why, "token_embd.weight: f16 or bf16 expected");
+    else if (!set_embed(M, emb->data, emb->type == gguf::ggml_type::f16))
+      ok = detail::why_(why, "token_embd.weight: no room on the device");
   }
   hip::flush();
   cv.destroy();
@@ -576,18 +592,10 @@ inline void set_cache_pos(model& M, int64_t p) {
   for (auto& L : M.layers) L.cache.pos = p;
 }
 
-// Widen one embedding row into the staged input (host gather, one small H2D).
-// false for a token id outside [0, vocab): nothing is read or uploaded.
+// The step's input: the token's embedding row, widened on the device. false for a token id outside [0, vocab): nothing is
+// read or launched.
 inline bool stage_embed(model& M, int64_t token) {
-  const dims& d = M.d;
-  if (token < 0 || token >= d.vocab) return false;
-  const uint16_t* r = M.embed.data() + (size_t)token * d.hidden;
-  if (M.embed_f16)
-    for (int64_t j = 0; j < d.hidden; j++) M.s.embed_host[j] = f16_to_f32(r[j]);
-  else
-    for (int64_t j = 0; j < d.hidden; j++) M.s.embed_host[j] = bf16_to_f32(r[j]);
-  hip::upload(M.s.embedb, M.s.embed_host, d.hidden);
-  return true;
+  return hip::embed_rows(M.embed, M.embed_f16, &token, 1, M.s.embedb, M.d.hidden, M.d.vocab);
 }
 
 // All layers + final norm + lm_head on the scratch buffers, no allocation, no
@@ -746,7 +754,7 @@ inline bool prefill_reserve(model& M, int64_t T) {
   auto A = [](int64_t n) { return hip::alloc_device(n * 4); };
   for (void* b : {P.emb, P.h, P.h2, P.qkv, P.qkvh, P.ah, P.at, P.gu, P.mb, P.md, P.res[0], P.res[1], P.rope, P.parts})
     if (b) hip::release(b, 0, nullptr);
-  P.emb = hip::alloc(T * d.hidden * 4, &P.emb_host);
+  P.emb = A(T * d.hidden);
   P.h = A(T * d.hidden);
   P.h2 = A(T * d.hidden);
   P.qkv = A(T * d.qkv_dim());
@@ -833,46 +841,11 @@ inline bool prefill_layers(model& M, int64_t T) {
   return ok;
 }
 
-// Gather T embedding rows on the host and upload them as the chunk input.
-// false for a token id outside [0, vocab), before anything is read.
+// The chunk's input: T embedding rows, widened on the device. false for a token id outside [0, vocab), before anything is read.
 inline bool stage_chunk(model& M, const int64_t* tokens, int64_t T) {
-  const dims& d = M.d;
   for (int64_t t = 0; t < T; t++)
-    if (tokens[t] < 0 || tokens[t] >= d.vocab) return false;
-  if (!prefill_reserve(M, T)) return false;
-  for (int64_t t = 0; t < T; t++) {
-    const uint16_t* r = M.embed.data() + (size_t)tokens[t] * d.hidden;
-    float* o = M.ps.emb_host + t * d.hidden;
-    if (M.embed_f16)
-      for (int64_t j = 0; j < d.hidden; j++) o[j] = f16_to_f32(r[j]);
-    else
-      for (int64_t j = 0; j < d.hidden; j++) o[j] = bf16_to_f32(r[j]);
-  }
-  hip::upload(M.ps.emb, M.ps.emb_host, T * d.hidden);
-  return true;
-}
-
-// Copy the host embedding table to the device once, through a pinned staging block.
-inline bool upload_embed(model& M) {
-  if (M.embed_dev) return true;
-  const int64_t bytes = (int64_t)M.embed.size() * 2;
-  if (bytes <= 0) return false;
-  M.embed_dev = hip::alloc_device(bytes);
-  if (!M.embed_dev) return false;
-  const int64_t blk = int64_t(32) << 20;
-  float* stage_host = nullptr;
-  void* stage = hip::alloc(blk, &stage_host);
-  if (!stage) return false;
-  bool ok = true;
-  for (int64_t o = 0; o < bytes && ok; o += blk) {
-    const int64_t n = std::min(blk, bytes - o);
-    std::memcpy(stage_host, reinterpret_cast<const char*>(M.embed.data()) + o, (size_t)n);
-    hip::upload(stage, stage_host, (n + 3) / 4);
-    ok = hip::copy_d2d(static_cast<char*>(M.embed_dev) + o, stage, n);
-    hip::flush();   // the staging block is reused
-  }
-  hip::release(stage, blk, stage_host);
-  return ok;
+    if (tokens[t] < 0 || tokens[t] >= M.d.vocab) return false;
+  return prefill_reserve(M, T) && hip::embed_rows(M.embed, M.embed_f16, tokens, T, M.ps.emb, M.d.hidden, M.d.vocab);
 }
 
 // ---- what the decode loops (decode_loop.h) ask of a model --------------------------------------
@@ -889,19 +862,19 @@ inline bool step_layers(model& M, int64_t pos, void* d_pos = nullptr, bool advan
 // The same with its input taken from a token id on the device.
 inline bool step_layers_from(model& M, void* d_tok, void* d_pos) {
   const dims& d = M.d;
-  const bool ok = M.embed_f16 ? hip::embed_gather_f16(M.embed_dev, d_tok, M.s.embedb, d.hidden, d.vocab)
-                              : hip::embed_gather_bf16(M.embed_dev, d_tok, M.s.embedb, d.hidden, d.vocab);
+  const bool ok = M.embed_f16 ? hip::embed_gather_f16(M.embed, d_tok, M.s.embedb, d.hidden, d.vocab)
+                              : hip::embed_gather_bf16(M.embed, d_tok, M.s.embedb, d.hidden, d.vocab);
   return ok && step_layers(M, 0, d_pos, /*advance=*/false);
 }
 // What steps with the position on the device need besides the model; false: this model has no such steps.
-inline bool reserve_device_steps(model& M, bool device_tokens) {
+inline bool reserve_device_steps(model& M, bool) {
   const dims& d = M.d;
   if (M.layers.empty() || !M.fused || !hip::graph_available()) return false;
   if (!M.attn_partials) {
     M.attn_partials_bytes = hip::attn_partials_bytes(d.n_q_heads, d.n_kv_heads, context_capacity(M), d.head_dim);
     M.attn_partials = hip::alloc_device(M.attn_partials_bytes);
   }
-  return M.attn_partials && (!device_tokens || upload_embed(M));
+  return M.attn_partials && M.embed;
 }
 // T prompt tokens through all layers at the caches' position; final-norm rows in chunk_rows().
 inline bool prompt_chunk(model& M, const int64_t* tokens, int64_t T) {

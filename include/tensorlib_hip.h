@@ -324,6 +324,9 @@ int tlhip_quantize_q4(const void* src, int src_type, void* packed, void* scales,
  * the reference gathers it (qwen_model.h:297, 531-540). */
 int tlhip_embed_gather_f16(const void* table, const void* d_token, void* out, int64_t hidden,
                            int64_t vocab);
+/* out[T][hidden] f32 = widened rows ids[0 .. T) (host memory, read before the call returns; every one within [0, vocab) or
+ * nothing is launched) of a [vocab, hidden] table of TLHIP_T_F16 or TLHIP_T_BF16. Capturable; the ids are then fixed. */
+int tlhip_embed_rows(const void* table, int table_type, const int64_t* ids, int64_t T, void* out, int64_t hidden, int64_t vocab);
 
 /* ---- GEMVs that produce their own activation vector (no single reference
  * counterpart) -----------------------------------------------------------------
