@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void sgemm_kernel(const float* __restrict__ A,
 }
 
 int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb, int tb, float* pc, int M, int N, int K, float scale,
-                      float offset, int epi, bool tiled);
+                      float offset, int epi, bool tiled, bool whole);
 int launch_sgemm_mfma(const float* pa, int64_t lda, int ta, const float* pb, int64_t ldb, int tb, float* pc,
                       int M, int N, int K, float scale, float offset, int epi);   // sgemm.hip
 
@@ -290,12 +290,13 @@ int tlhip_gemm(const void* a, int64_t a_off, int64_t lda, int ta, const void* b,
   // Up to 1024 rows of an A that is stored as it is read: the kernel that splits K inside its blocks, unless the
   // product is whole 128 x 128 tiles of aligned rows and at least two of them tall, where the LDS-tiled kernel reads
   // each operand once per tile (512 x 4608 x 3584: 215 us against 258; but 333 x 4864 x 896: 66 against 46), or that
-  // kernel's or the vector-ALU kernel's estimated time is less (launch_sgemm_rows returns 1).
+  // kernel's or the vector-ALU kernel's estimated time is less (launch_sgemm_rows returns 1). From 128 columns and k on the kernel
+  // that works in bf16 terms comes first where its estimate is less than theirs.
   const bool tiled = m >= 128 && n >= 128 && k >= 16 && (m + 127) / 128 <= 65535;
   const bool whole = m >= 256 && (m % 128) == 0 && (n % 128) == 0 && (k % 16) == 0 && (lda % 4) == 0 && (ldb % 4) == 0 && aligned16(pa) && aligned16(pb);
   // (2^23 blocks of 512 threads are what a grid's x can count)
-  if (!ta && k >= 16 && m <= 1024 && !whole && (m + 15) / 16 * ((n + 63) / 64) < (1 << 23)) {
-    const int rc = launch_sgemm_rows(pa, lda, pb, ldb, tb, po, (int)m, (int)n, (int)k, scale, offset, epi, tiled);
+  if (!ta && k >= 16 && m <= 1024 && (m + 15) / 16 * ((n + 63) / 64) < (1 << 23)) {
+    const int rc = launch_sgemm_rows(pa, lda, pb, ldb, tb, po, (int)m, (int)n, (int)k, scale, offset, epi, tiled, whole);
     if (rc < 0) return rc;
     if (rc == 0) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM);
   }

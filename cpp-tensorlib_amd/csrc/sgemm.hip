@@ -169,6 +169,10 @@ __global__ __launch_bounds__(256) void sgemm_sum_kernel(const float* __restrict_
   C[i] = epi ? add_rn(mul_rn(a, scale), offset) : a;
 }
 
+void launch_sgemm_sum(const float* part, float* C, size_t n, int S, float scale, float offset, int epi) {
+  sgemm_sum_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx().stream>>>(part, C, n, S, scale, offset, epi);
+}
+
 // 16-byte loads need aligned bases and row strides that keep every row aligned
 static bool sgemm_aligned(const float* pa, int64_t lda, const float* pb, int64_t ldb) {
   return aligned16(pa) && aligned16(pb) && (lda % 4) == 0 && (ldb % 4) == 0;
@@ -214,8 +218,7 @@ int launch_sgemm_mfma(const float* pa, int64_t lda, int ta, const float* pb, int
   else TLHIP_SGEMM(1, 1);
 #undef TLHIP_SGEMM
   if (S > 1) {
-    const size_t n = (size_t)M * N;
-    sgemm_sum_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(dst, pc, n, S, scale, offset, epi);
+    launch_sgemm_sum(dst, pc, (size_t)M * N, S, scale, offset, epi);
   }
   return 0;
 }
@@ -398,10 +401,14 @@ __global__ __launch_bounds__(64 * kSrWaves, 2) void sgemm_rows_kernel(const floa
   }
 }
 
+int launch_sgemm_split(const float* pa, int64_t lda, const float* pb, int64_t ldb, int tb, float* pc, int M, int N, int K, float scale,
+                       float offset, int epi, double other_us, int other_steps);
 // The same for A as it is stored ([M][K]); the caller has checked the arguments. tiled: the LDS-tiled kernel takes the
-// product too, else the vector-ALU kernel; 1 is returned, and nothing launched, where that is the better one.
+// product too, else the vector-ALU kernel; 1 is returned, and nothing launched, where that is the better one. whole: the
+// LDS-tiled kernel is better than this one in any case. Ahead of either goes the product in bf16 terms (sgemm_split.hip) where its
+// estimate is the least.
 int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb, int tb, float* pc, int M, int N, int K, float scale,
-                      float offset, int epi, bool tiled) {
+                      float offset, int epi, bool tiled, bool whole) {
   // Row blocks and K splits (parts in scratch, summed in a fixed order) that an estimate in clocks likes best: a block
   // takes 1600 clocks per row tile and 128 k, and 6000 to start and end; blocks run one to a CU, so tiles that make a
   // round and a bit are cut smaller until they make whole rounds; parts are written and read at 2.5 KB a clock, and their
@@ -423,19 +430,21 @@ int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb
   // times in us, fitted to 2210 runs (128 to 1024 rows, 128 to 150000 columns, K 16 .. 5000; errors 8 and 6 %): a start; for every
   // round of blocks its own start and end and its steps of 16 k (per row tile here); the outputs' megabytes, twice for parts; and
   // the launch that adds those up.
-  if (tiled) {
-    const int64_t tiles128 = (int64_t)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
-    const int St = sgemm_mfma_splits(tiles128, K);
-    const auto steps = [&](int parts) { return (double)(((K + parts - 1) / parts + kSgBK - 1) / kSgBK); };
-    const auto mb = [&](int parts) { return 4e-6 * M * N * (parts > 1 ? 2 * parts : 1); };
-    const double here = 2.2 + std::ceil((double)rb * columns * S / cus) * (1.15 + TM * (0.25 + (tb ? 0.81 : 0.72) * steps(S) / kSrWaves)) +
-                        0.28 * mb(S) + (S > 1 ? 2.2 : 0);
-    const double fill = (double)tiles128 * St / cus;   // blocks run two to a CU, and the last round's gaps are partly filled
-    const double there = 5.5 + std::max(1.0, 0.14 * fill + 0.86 * std::ceil(fill)) *
-                                   (steps(St) * (sgemm_aligned(pa, lda, pb, ldb) ? 1.41 : 1.57) - 1) + 0.16 * mb(St) + (St > 1 ? 7.9 : 0);
-    // (its parts need scratch, which a recording may not grow: the product stays here then)
-    if (here > 1.02 * there && (St == 1 || scratch((size_t)St * M * N * sizeof(float)))) return 1;
-  }
+  const int64_t tiles128 = (int64_t)((N + kSgBN - 1) / kSgBN) * ((M + kSgBM - 1) / kSgBM);
+  const int St = sgemm_mfma_splits(tiles128, K);
+  const auto steps = [&](int parts) { return (double)(((K + parts - 1) / parts + kSgBK - 1) / kSgBK); };
+  const auto mb = [&](int parts) { return 4e-6 * M * N * (parts > 1 ? 2 * parts : 1); };
+  const double here = 2.2 + std::ceil((double)rb * columns * S / cus) * (1.15 + TM * (0.25 + (tb ? 0.81 : 0.72) * steps(S) / kSrWaves)) +
+                      0.28 * mb(S) + (S > 1 ? 2.2 : 0);
+  const double fill = (double)tiles128 * St / cus;   // blocks run two to a CU, and the last round's gaps are partly filled
+  const double there = 5.5 + std::max(1.0, 0.14 * fill + 0.86 * std::ceil(fill)) *
+                                 (steps(St) * (sgemm_aligned(pa, lda, pb, ldb) ? 1.41 : 1.57) - 1) + 0.16 * mb(St) + (St > 1 ? 7.9 : 0);
+  const bool to_tiles = whole || (tiled && here > 1.02 * there);
+  // (a wavefront of the LDS-tiled kernel adds up all of its block's K, here an eighth)
+  if (const int rc = launch_sgemm_split(pa, lda, pb, ldb, tb, pc, M, N, K, scale, offset, epi, to_tiles ? there : here,
+                                        (int)steps(to_tiles ? St : S) / (to_tiles ? 1 : kSrWaves)); rc != 1) return rc;
+  // (its parts need scratch, which a recording may not grow: the product stays here then)
+  if (to_tiles && (whole || St == 1 || scratch((size_t)St * M * N * sizeof(float)))) return 1;
   const int64_t tiles = rb * columns;
   // Fewer than 128 rows or columns, which is what the vector-ALU kernel is left with: more than one, two and four rounds of
   // these blocks for K up to 16, 32 and 47 cost more than its 64 x 64 tiles, which meet no one at their end (us, here and there: 100 x
@@ -471,8 +480,7 @@ int launch_sgemm_rows(const float* pa, int64_t lda, const float* pb, int64_t ldb
   };
   if (int rc = tb ? by_tm(integral_constant<int, 1>{}) : by_tm(integral_constant<int, 0>{})) return rc;
   if (S > 1) {
-    const size_t n = (size_t)M * N;
-    sgemm_sum_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx().stream>>>(dst, pc, n, S, scale, offset, epi);
+    launch_sgemm_sum(dst, pc, (size_t)M * N, S, scale, offset, epi);
   }
   return 0;
 }
