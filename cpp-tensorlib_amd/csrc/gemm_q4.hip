@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
     const int have = min(4, groups - 4 * (ubeg + u)) * (kImage / 1024);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const int piece = min(wave * 8 + i, have - 1);   // (a repeated piece lands in a slab that is not multiplied)
+      const int piece = min(wave * 8 + i, have - 1);   // (a repeated piece lands in a slab whose scales are zero)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(asrc + (size_t)u * kUnit + piece * 1024 + lane * 16),
                                        (__attribute__((address_space(3))) void*)(ring + stage * kUnit + (wave * 8 + i) * 1024), 16, 0, 0);
     }
@@ -167,33 +167,44 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
 #pragma unroll
   for (int ks = 0; ks < 2; ks++) aoff[ks] = image_off(l32, ks * 2 + half);   // (32 rows further down: 32 row lengths, the same swizzle)
 
-  auto slab = [&](const char* at, int set, int g) {
-    frag16 b[2][2];                                // [16-k step][column tile]
+  // A slab in two halves of 32 rows, i = 0 and 1. Between the matrix instructions of one half go the vector instructions of
+  // its neighbours: the scales of the half before it, the nibbles of the next slab. Each half's eight products keep the matrix
+  // pipe for 256 clocks; in a run of their own, as the scales after them, they kept the wavefront from issuing anything else.
+  frag16 a[4], b[2][2];                            // A: [16-k step, term]; weights: [16-k step][column tile]
+  f32x16 grp[2][2];                                // [half][column tile]: the sums of a group, its scales still to come
+  float ps[2] = {0.f, 0.f};                        // those of the half before
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+  for (int j = 0; j < 2; j++)
 #pragma unroll
-      for (int ks = 0; ks < 2; ks++) b[ks][j] = nib8(w[set][j][g >> 1][2 * ks + (g & 1)]);
-    f32x16 grp[2][2];                              // four chains of products side by side
+    for (int v = 0; v < 16; v++) grp[1][j][v] = 0.f;
+  auto fetch = [&](const char* at, int i, int q) __attribute__((always_inline)) { a[q] = *reinterpret_cast<const frag16*>(at + aoff[q >> 1] + (q & 1) * kPlane + i * 32 * kSlab * 2); };
+  auto nibbles = [&](int set, int g, int ks, int j) __attribute__((always_inline)) { b[ks][j] = nib8(w[set][j][g >> 1][2 * ks + (g & 1)]); };
+  auto scaled = [&](int i, int q) __attribute__((always_inline)) {   // a quarter of half i's sums
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++)
+    for (int v = 8 * (q & 1); v < 8 * (q & 1) + 8; v++) acc[i][q >> 1][v] = fmaf(grp[i][q >> 1][v], ps[q >> 1], acc[i][q >> 1][v]);
+    asm volatile("" : "+v"(acc[i][q >> 1]));       // (here: the compiler would gather the slabs' scales, and spill their sums)
+  };
+  // next: where the slab after this one lies (nullptr: the unit ends)
+  auto slab = [&](const char* at, const char* next, int set, int g) __attribute__((always_inline)) {
 #pragma unroll
-      for (int p = 0; p < 2; p++) {                // (the second terms first would cost precision at long K: 1.9e-7 for 1.3e-7)
-        frag16 a[2];
+    for (int i = 0; i < 2; i++) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) a[i] = *reinterpret_cast<const frag16*>(at + aoff[ks] + p * kPlane + i * 32 * kSlab * 2);
+      for (int q = 0; q < 4; q++) {                // (the second terms first would cost precision at long K: 1.9e-7 for 1.3e-7)
+        const int ks = q >> 1;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int j = 0; j < 2; j++) grp[i][j] = mma(a[i], b[ks][j], ks + p == 0 ? f32x16{} : grp[i][j]);
+        for (int j = 0; j < 2; j++) grp[i][j] = mma(a[q], b[ks][j], q == 0 ? f32x16{} : grp[i][j]);
+        if (i == 0) fetch(at, 1, q);
+        else if (next) fetch(next, 0, q);
+        scaled(1 - i, q);
+        if (i == 0 && q < 2) nibbles(set, g, 1, q);
+        if (i == 1 && q >= 2 && next) nibbles(set, g + 1, 0, q - 2);
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[i][j][v] = fmaf(grp[i][j][v], s[set][j][g], acc[i][j][v]);
+      for (int j = 0; j < 2; j++) ps[j] = s[set][j][g];
+    }
   };
-  auto unit = [&](int set, int u) {
+  auto unit = [&](int set, int u) __attribute__((always_inline)) {
     // my copies and loads of unit u have landed (those of u + 1 - eight copies, six loads - may be in flight); past the
     // barrier that holds for every wavefront
     if (4 * (ubeg + u) + 8 <= groups && u + 1 < nu) asm volatile("s_waitcnt vmcnt(14)" ::: "memory");
@@ -210,10 +221,19 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
         x = frag16{y[0], y[1], z[0], z[1]};        // [16-k step][group of the pair]
       }
     const char* at = ring + set * kUnit;
-    const int have = min(4, groups - 4 * (ubeg + u));
+    const int have = groups - 4 * (ubeg + u);
+    if (have < 4) {                                // groups past the last are multiplied, and scaled to nothing
 #pragma unroll
-    for (int g = 0; g < 4; g++)
-      if (g < have) slab(at + g * kImage, set, g);
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int g = 1; g < 4; g++) s[set][j][g] = g < have ? s[set][j][g] : 0.f;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) fetch(at, 0, q);
+#pragma unroll
+    for (int j = 0; j < 2; j++) nibbles(set, 0, 0, j);
+#pragma unroll
+    for (int g = 0; g < 4; g++) slab(at + g * kImage, g < 3 ? at + (g + 1) * kImage : nullptr, set, g);
     barrier();                                     // everyone is done with this stage
     if (u + 2 < nu) {
       copy(u + 2, set);
@@ -233,6 +253,8 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
     if (u + 1 < nu) unit(1, u + 1);
   }
 
+#pragma unroll
+  for (int q = 0; q < 4; q++) scaled(1, q);        // the last half's
   // acc[v] of lane l: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32. The row's exponent comes back out, exactly.
   const int m0 = rb * kBM;
 #pragma unroll
