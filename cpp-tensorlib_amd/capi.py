@@ -41,6 +41,7 @@ SIGNATURES = {
     "tlhip_host_free": (cint, [P]),
     "tlhip_memcpy_h2d": (cint, [P, P, sz]),
     "tlhip_memcpy_d2h": (cint, [P, P, sz]),
+    "tlhip_copy_to_host": (cint, [P, P, sz]),
     "tlhip_memcpy_h2d_async": (cint, [P, P, sz]),
     "tlhip_memcpy_d2d_async": (cint, [P, P, sz]),
     "tlhip_fill_u32": (cint, [P, u32, sz]),

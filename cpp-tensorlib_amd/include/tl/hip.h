@@ -69,6 +69,7 @@ struct api {
   int (*host_free)(void*) = nullptr;
   int (*memcpy_h2d)(void*, const void*, size_t) = nullptr;
   int (*memcpy_d2h)(void*, const void*, size_t) = nullptr;
+  int (*copy_to_host)(void*, const void*, size_t) = nullptr;
   int (*memcpy_h2d_async)(void*, const void*, size_t) = nullptr;
   int (*memcpy_d2d_async)(void*, const void*, size_t) = nullptr;
   int (*fill_u32)(void*, uint32_t, size_t) = nullptr;
@@ -353,6 +354,7 @@ struct context {
               bind(f.free_, "tlhip_free") && bind(f.host_alloc, "tlhip_host_alloc") &&
               bind(f.host_free, "tlhip_host_free") && bind(f.memcpy_h2d, "tlhip_memcpy_h2d") &&
               bind(f.memcpy_d2h, "tlhip_memcpy_d2h") &&
+              bind(f.copy_to_host, "tlhip_copy_to_host") &&
               bind(f.memcpy_h2d_async, "tlhip_memcpy_h2d_async") &&
               bind(f.memcpy_d2d_async, "tlhip_memcpy_d2d_async") &&
               bind(f.fill_u32, "tlhip_fill_u32") && bind(f.sync, "tlhip_sync") &&
@@ -571,6 +573,15 @@ struct context {
     e->derived.push_back(d);
     return &e->derived.back();
   }
+  // device -> staging by a kernel behind the launches queued so far: true when it is queued, and the staging half holds
+  // the data once the stream has drained.
+  bool queue_pull(extent& e) {
+    if (capturing || e.size > kQueuedPull || f.copy_to_host(e.staging, e.base, e.size) != 0) return false;
+    e.live = extent::side::either;
+    return true;
+  }
+  // (bytes: the kernel saves 10-17 us up to 4 MB, 15 of 160 at 8, nothing from 16 on)
+  static constexpr size_t kQueuedPull = size_t(4) << 20;
   // device -> staging
   void pull(extent& e) {
     f.memcpy_d2h(e.staging, e.base, e.size);
@@ -706,6 +717,7 @@ inline void sync_to_host(void* native, bool for_write) {
   auto& c = context::get();
   extent* e = c.ready ? c.buffers.containing(native) : nullptr;
   if (!e) return;
+  if (e->staging && e->live == extent::side::device && c.queue_pull(*e)) c.pending = true;
   if (c.pending) flush();
   if (!e->staging) return;
   if (e->live == extent::side::device) c.pull(*e);

@@ -75,6 +75,8 @@ int tlhip_host_free(void* hptr);
 int tlhip_memcpy_h2d(void* dst, const void* src, size_t bytes);       /* blocking */
 int tlhip_memcpy_d2h(void* dst, const void* src, size_t bytes);       /* blocking, drains stream */
 int tlhip_memcpy_h2d_async(void* dst, const void* src, size_t bytes); /* src must stay valid */
+int tlhip_copy_to_host(void* dst_pinned, const void* src, size_t bytes); /* copy kernel, in order, not waited for, capturable;
+                                             dst_pinned from tlhip_host_alloc, both 16-byte aligned */
 int tlhip_memcpy_d2d_async(void* dst, const void* src, size_t bytes);
 int tlhip_fill_u32(void* dst, uint32_t value, size_t count);          /* fill kernel, capturable */
 int tlhip_sync(void);                     /* cuda.h:501-506 flush() */
