@@ -130,6 +130,9 @@ SIGNATURES = {
     "tlhip_linear_state_bytes": (i64, [i64, i64, i64]),
     "tlhip_mix_partials_bytes": (i64, [P]),
     "tlhip_mix_step": (cint, [P, P, P, P, P, i64, P, P, i64]),
+    "tlhip_mix_open": (cint, [P, i64]),
+    "tlhip_mix_step_open": (cint, [P, P, P, P, P, i64, P, P, i64]),
+    "tlhip_gemv_bf16_row_mix": (cint, [P, P, P, P, i64, P, P, i64, i64]),
     "tlhip_window_fill": (cint, [P, i64, P, i64, i64]),
     "tlhip_window_attn_chunk": (cint, [P, i64, P, i64, P, i64, i64, cint]),
     "tlhip_linear_attn_chunk": (cint, [P, i64, P, i64, P, i64, i64]),

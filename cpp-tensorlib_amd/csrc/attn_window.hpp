@@ -227,7 +227,8 @@ __device__ __forceinline__ void window_step_block(const tlhip_window_attn& a, co
 
 // The next splits of a window into a running merge: their weights w and the factor fo of what is merged so far (max M, sum
 // L); splits without a key (maximum -inf) and those past the last (s >= n) weigh nothing. One maximum over the group and one
-// weight a split: the running maximum that this replaced took two exponentials and the factors of a chain for each.
+// weight a split: the running maximum that this replaced took two exponentials and the factors of a chain for each. Written
+// out, so that the merge launch and the product that merges while it stages (gemv.hip) leave the same bits.
 constexpr int kMergeGroup = 8;
 __device__ __forceinline__ void merge_group(float& M, float& L, const float (&m)[kMergeGroup], const float (&l)[kMergeGroup],
                                             int n, float (&w)[kMergeGroup], float& fo) {
@@ -277,4 +278,6 @@ __device__ __forceinline__ void window_merge_head(const tlhip_window_attn& a, co
 
 // What the launchers check of a mixer description (host).
 int check_window_attn(const tlhip_window_attn* a, const char* who);
+// Splits the window of a decode step is cut into.
+int window_splits(const tlhip_window_attn* a);
 }  // namespace tlhip

@@ -18,6 +18,7 @@
 //     partials go to scratch and are summed in a fixed order by a second
 //     kernel.
 #include "common.hpp"
+#include "attn_window.hpp"
 #include "gemv_shared.hpp"
 
 #include <algorithm>
@@ -65,6 +66,42 @@ __device__ __forceinline__ void load_frag(RowFrag<Fmt, R>& f, const uint4* __res
       f.sc[r] = __builtin_nontemporal_load(reinterpret_cast<const float*>(sb + (idx << 2)));
   }
 }
+
+// Four values of a split window attention (kMixMerge): what the splits left for them, and their merge, which is
+// window_merge_head's arithmetic (attn_window.hpp) for each.
+struct MixSplits {
+  float m[kMergeGroup], l[kMergeGroup];
+  float2 a[kMergeGroup], b[kMergeGroup];
+  float4 g;
+  __device__ __forceinline__ void load(const Producer& pro, int e) {     // float4 e of [heads][D]
+    const int h = (int)__umulhi((uint32_t)e, (uint32_t)pro.parts), d = 4 * e - h * pro.D;
+    const float* p = pro.delta + (size_t)h * pro.S * pro.part_ld;        // (rows of an even number of floats)
+#pragma unroll
+    for (int s = 0; s < kMergeGroup; s++) {
+      const float* q = p + (size_t)min(s, pro.S - 1) * pro.part_ld;
+      const float2 ml = *reinterpret_cast<const float2*>(q);
+      m[s] = ml.x;
+      l[s] = ml.y;
+      a[s] = *reinterpret_cast<const float2*>(q + 2 + d);
+      b[s] = *reinterpret_cast<const float2*>(q + 4 + d);
+    }
+    g = pro.norm_w ? *reinterpret_cast<const float4*>(pro.norm_w + 4 * e) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __device__ __forceinline__ float4 merged(const Producer& pro) const {
+    float M = -INFINITY, L = 0.f, w[kMergeGroup], fo;
+    merge_group(M, L, m, l, pro.S, w, fo);
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int s = 0; s < kMergeGroup; s++) {
+      o.x = fmaf(w[s], a[s].x, o.x); o.y = fmaf(w[s], a[s].y, o.y);
+      o.z = fmaf(w[s], b[s].x, o.z); o.w = fmaf(w[s], b[s].y, o.w);
+    }
+    const float r = pro.eps / L;
+    o.x *= r; o.y *= r; o.z *= r; o.w *= r;
+    if (pro.norm_w) { o.x *= sigmoid_f(g.x); o.y *= sigmoid_f(g.y); o.z *= sigmoid_f(g.z); o.w *= sigmoid_f(g.w); }
+    return o;
+  }
+};
 
 // LPR = lanes that share a weight row: 64 (a row segment of 64 units per
 // wavefront step) or 16 (the wavefront works on 4 row groups at once, 16 units
@@ -144,10 +181,20 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     for (int k = 0; k < PL; k++) {
       const int i = min(tid + k * (int)blockDim.x, n4 - 1);
       if (PRO != kAttnMerge) px[k] = x4[i];
-      if (PRO != kPlain && PRO != kAttnMerge) pa[k] = aux4[i];
+      if (PRO != kPlain && PRO != kAttnMerge && PRO != kMixMerge) pa[k] = aux4[i];
       if (PRO == kRmsnorm || kPost) pn[k] = reinterpret_cast<const float4*>(pro.norm_w)[i];
       if (kPost && pro.bias) pb[k] = reinterpret_cast<const float4*>(pro.bias)[i];
     }
+  }
+  // split-window producer: the first float4 of the attention's columns that this thread stages
+  MixSplits mix;
+  int mix_i = 0;
+  if constexpr (PRO == kMixMerge) {
+    const int nt = (int)blockDim.x, n = pro.heads * (pro.D >> 2);
+    mix_i = tid;
+    if (pro.first4 > 0 && tid < pro.first4) mix_i += (pro.first4 - tid + nt - 1) / nt * nt;
+    // wavefronts whose columns are all other ones ask for nothing
+    if (__any(mix_i - pro.first4 < n)) mix.load(pro, min(mix_i - pro.first4, n - 1));
   }
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
@@ -271,6 +318,13 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
         for (int sp = kPre; sp < S; sp++) add(fh[sp], pacc[(size_t)sp * D4], false);
         const float L = fL[h];
         return make_float4(v.x / L, v.y / L, v.z / L, v.w / L);
+      }
+      if constexpr (PRO == kMixMerge) {
+        const int e = i - pro.first4;
+        if (e >= 0 && e < pro.heads * (pro.D >> 2)) {
+          if (i != mix_i) mix.load(pro, e);
+          return mix.merged(pro);
+        }
       }
       float4 v, aux, ab;
       bool have = false;
@@ -754,6 +808,7 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
   for (int64_t n0 = 0; n0 < N; n0 += max_rows) {
     const int64_t n = N - n0 < max_rows ? N - n0 : max_rows;
     const auto pick = [&](int producer) {
+      if (producer == kMixMerge) producer = kPlain;   // the plain product's shape, so that its sums are the same
       RowCfg g = pick_rows_cfg(n, upr, Fmt::E, producer, c.cus, c.lds_per_cu, tn);
       if (EPI != kStore && g.R == 1) {   // a lane group needs a gate row and its up row
         RowTune two = tn;
@@ -919,6 +974,31 @@ int tlhip_gemv_bf16_row_attn(const void* parts, int64_t n_parts, int64_t heads, 
   Producer pro{nullptr, nullptr, nullptr, 0.f, (int)n_parts, (int)heads, (int)head_dim};
   return launch_rows<FmtBf16, kAttnMerge>(static_cast<const float*>(parts), W, nullptr, static_cast<float*>(y), n, k,
                                           TLHIP_C_GEMV_BF16_ROW, RowTune{0, 0, 0, 0, 0}, pro);
+}
+
+int tlhip_gemv_bf16_row_mix(const void* a, const void* u, const tlhip_window_attn* at, const void* partials,
+                            int64_t partials_bytes, const void* W, void* y, int64_t n, int64_t k) {
+  TLHIP_REQUIRE_READY();
+  if (int rc = check_gemv_args(a, W, y, n, k, "tlhip_gemv_bf16_row_mix")) return rc;
+  if (!at || !u || !aligned16(u)) return fail(TLHIP_EINVAL, "tlhip_gemv_bf16_row_mix: bad operands");
+  if (int rc = check_window_attn(at, "tlhip_gemv_bf16_row_mix")) return rc;
+  if (!tlhip_mix_open(at, k)) return fail(TLHIP_EUNSUPPORTED, "tlhip_gemv_bf16_row_mix: this attention is merged by its own launch");
+  if (!partials || !aligned16(partials) || partials_bytes < tlhip_mix_partials_bytes(at))
+    return fail(TLHIP_EINVAL, "tlhip_gemv_bf16_row_mix: partials too small, null or not 16-byte aligned");
+  if (at->y_off + at->heads * at->dim > k) return fail(TLHIP_EINVAL, "tlhip_gemv_bf16_row_mix: the attention's columns end past K");
+  if ((k % 8) != 0) return fail(TLHIP_EUNSUPPORTED, "tlhip_gemv_bf16_row_mix: K %% 8 != 0");
+  if (!aligned16(W)) return fail(TLHIP_EINVAL, "tlhip_gemv_bf16_row_mix: weight pointer not 16-byte aligned");
+  const size_t xbytes = (size_t)((k / 8 + 63) / 64) * 72 * 8 * 4;
+  if (xbytes + 2048 > (size_t)ctx().lds_per_cu)
+    return fail(TLHIP_EUNSUPPORTED, "tlhip_gemv_bf16_row_mix: K too large for the LDS-staged kernel");
+  Producer pro{static_cast<const float*>(partials), at->gate_off >= 0 ? static_cast<const float*>(u) + at->gate_off : nullptr,
+               nullptr, at->out_scale, window_splits(at), (int)at->heads, (int)at->dim};
+  pro.part_ld = (int)at->ring_ld + 2;
+  pro.first4 = (int)(at->y_off / 4);
+  const int64_t d4 = at->dim / 4;                // e / d4 = umulhi(e, parts) for e d4^2 < 2^32: a row that fits LDS is far below
+  pro.parts = (int)(uint32_t)(((int64_t(1) << 32) + d4 - 1) / d4);
+  return launch_rows<FmtBf16, kMixMerge>(static_cast<const float*>(a), W, nullptr, static_cast<float*>(y), n, k,
+                                         TLHIP_C_GEMV_BF16_ROW, RowTune{0, 0, 0, 0, 0}, pro);
 }
 
 int tlhip_gemv_f32(const void* a, const void* B, void* y, int64_t n, int64_t k) {

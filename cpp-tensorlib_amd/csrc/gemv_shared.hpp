@@ -163,6 +163,12 @@ __device__ __forceinline__ float wave_sum_rows(float (&a)[R], int lane) {
 //             x[h*D + d] = sum_s e^(m_s - M) acc_s[d] / sum_s e^(m_s - M) l_s, at most 16 splits,
 //             in the summation order of the stand-alone merge kernel (same bits). The merge's
 //             launch goes; what it read (a few KB per head) every block now reads from L2.
+//   kMixMerge: x, but its columns of a window attention are merged here from the splits that the step's blocks left
+//             (attn_window.hpp): the merge's launch goes, and every block reads the partials (66 KB for 16 heads of 128,
+//             from L2) beside x. Step and product, cold weights, with the launch -> so: 16 heads of 128 into 2048 x 12288
+//             16.0 -> 15.4 us, 14 of 64 into 896 x 6656 11.3 -> 10.3, 8 of 64 into 1024 x 4096 10.4 -> 9.2; more in a
+//             layer's trace (the medium model's turn 6740 -> 6550). Rows longer than the threads hold keep the launch: 28
+//             heads into 3584 x 26112 36.6 with it, 37.3 so.
 //   kPostnorm: x = in (when there is one) + (delta + bias) / rms * norm_w, the norm over `parts` runs of part_len
 //             entries, each by its own root mean square; block 0 writes x to xout. The factor is needed before
 //             anything can be staged, so the block meets a barrier for it; the weights are on their way meanwhile.
@@ -176,8 +182,10 @@ __device__ __forceinline__ float wave_sum_rows(float (&a)[R], int lane) {
 //            activation in the GEMV that produces it, once per element, instead of in every
 //            block of the GEMV that consumes it.
 //   kGeglu:  as kGateUp with y[i] = gelu_tanh(g + gu_bias[i]) * (u + gu_bias[N/2 + i]).
-enum { kPlain = 0, kSwiglu = 1, kRmsnorm = 2, kAttnMerge = 3, kPostnorm = 4, kPostnormLong = 5 };
+enum { kPlain = 0, kSwiglu = 1, kRmsnorm = 2, kAttnMerge = 3, kPostnorm = 4, kPostnormLong = 5, kMixMerge = 6 };
 constexpr int kMergeMax = 16;  // splits the kAttnMerge producer takes (its lanes per head)
+constexpr int kMixMergeRow = 20480;   // columns of x that it takes: as many as 1024 threads ask for up front
+constexpr int kMixMergeMax = 8;  // splits the kMixMerge producer takes (one merge_group, its registers)
 enum { kStore = 0, kGateUp = 1, kGeglu = 2 };
 __device__ __forceinline__ float gated(float g, float u) { return (g * (1.0f / (1.0f + expf(-g)))) * u; }
 // z * Phi(z) in its tanh form: (1 + tanh(w)) / 2 = 1 / (1 + e^-2w)
@@ -194,6 +202,9 @@ struct Producer {
   // kPostnorm, kPostnormLong
   const float* bias = nullptr;
   int parts = 0, part_len = 0, add_x = 0;
+  // kMixMerge: delta = the partials, S splits of `heads` heads of D in rows of part_ld, norm_w = the gates' columns (nullptr:
+  // none), eps = what the result is multiplied by, parts = ceil(2^32 / (D / 4)); the attention's columns begin at float4 first4 of x
+  int part_ld = 0, first4 = 0;
   // kGeglu
   const float* gu_bias = nullptr;
 };

@@ -4,6 +4,7 @@
 // each writing its columns of y, the input of the layer's one output product. Where the window is
 // cut into splits a second launch merges them.
 #include "attn_window.hpp"
+#include "gemv_shared.hpp"
 #include "linear_attn.hpp"
 #include "polynorm.hpp"
 
@@ -20,7 +21,7 @@ struct MixPlan {
 constexpr int kPolySlice = 1024;   // ff values a polynorm block writes
 constexpr int kMaxSplits = 32;
 
-static int attn_splits(const tlhip_window_attn* a) {
+int window_splits(const tlhip_window_attn* a) {
   // What a block reads bounds it (a CU takes in some 100 bytes per ns): windows beyond 192 KB of keys are
   // cut into splits of about 64 KB, which costs the merge launch. The plan does not depend on the position.
   const int64_t bytes = a->window * tlhip_window_ring_ld(a->dim) * 4, S = bytes <= (192 << 10) ? 1 : (bytes + (64 << 10) - 1) / (64 << 10);
@@ -30,7 +31,7 @@ static MixPlan make_plan(const tlhip_window_attn* at, const tlhip_linear_attn* l
   MixPlan p{1, 0, 1, 0, 0, 0};
   if (at) {
     const int group = (int)(at->heads / at->kv_heads), cus = ctx().cus > 0 ? ctx().cus : 256;
-    p.S = attn_splits(at);
+    p.S = window_splits(at);
     // one query head per block while that fits the chip in one round; more share a block's key reads
     const auto blocks = [&](int nq) { return at->kv_heads * ((group + nq - 1) / nq) * p.S; };
     const int most = at->ring_ld > 128 ? 2 : 4;   // registers
@@ -102,7 +103,8 @@ int check_polynorm(const tlhip_polynorm* p, const char* who) {
 
 template <int NQ, int NF>
 static int launch_mix(const float* u, float* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
-                      const tlhip_polynorm* pn, int pos, const void* d_pos, float* partials, const MixPlan& plan) {
+                      const tlhip_polynorm* pn, int pos, const void* d_pos, float* partials, const MixPlan& plan,
+                      bool merge) {
   Context& c = ctx();
   const tlhip_window_attn a0{};
   const tlhip_linear_attn l0{};
@@ -119,7 +121,7 @@ static int launch_mix(const float* u, float* y, const tlhip_window_attn* at, con
   }
   hipLaunchKernelGGL(fn, dim3((unsigned)(plan.attn + plan.lin + plan.poly)), dim3(512), lds, c.stream, u, y,
                      at ? *at : a0, la ? *la : l0, pn ? *pn : p0, partials, pos, static_cast<const uint32_t*>(d_pos), plan);
-  if (at && plan.S > 1)
+  if (at && plan.S > 1 && merge)
     hipLaunchKernelGGL(mix_merge_kernel, dim3((unsigned)at->heads), dim3(256), 0, c.stream, u, y, *at, partials, plan.S);
   TLHIP_CHECK_LAUNCH(TLHIP_C_MIX_STEP);
 }
@@ -138,14 +140,21 @@ int64_t tlhip_window_ring_ld(int64_t dim) {
 int64_t tlhip_linear_state_bytes(int64_t heads, int64_t dim, int64_t vdim) {
   return 2 * heads * dim * linear_state_ld(vdim) * (int64_t)sizeof(float);
 }
+int tlhip_mix_open(const tlhip_window_attn* at, int64_t k) {
+  if (!at || at->heads <= 0 || tlhip_window_ring_ld(at->dim) == 0) return 0;
+  const int S = window_splits(at);
+  return S > 1 && S <= kMixMergeMax && k <= kMixMergeRow && at->dim % 4 == 0 && at->y_off >= 0 && at->y_off % 4 == 0 &&
+         (at->gate_off < 0 || at->gate_off % 4 == 0);
+}
 int64_t tlhip_mix_partials_bytes(const tlhip_window_attn* at) {
   if (!at || at->heads <= 0) return 0;
-  const int S = attn_splits(at);
+  const int S = window_splits(at);
   return S > 1 ? at->heads * S * (tlhip_window_ring_ld(at->dim) + 2) * (int64_t)sizeof(float) : 0;
 }
 
-int tlhip_mix_step(const void* u, void* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
-                   const tlhip_polynorm* pn, int64_t pos, const void* d_pos, void* partials, int64_t partials_bytes) {
+static int mix_step(const void* u, void* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
+                    const tlhip_polynorm* pn, int64_t pos, const void* d_pos, void* partials, int64_t partials_bytes,
+                    bool merge) {
   TLHIP_REQUIRE_READY();
   if (!u || !y || !aligned16(u) || (!at && !la && !pn)) return fail(TLHIP_EINVAL, "tlhip_mix_step: bad operands");
   if (pos < 0 || pos > (1 << 30)) return fail(TLHIP_EINVAL, "tlhip_mix_step: bad position");
@@ -164,7 +173,7 @@ int tlhip_mix_step(const void* u, void* y, const tlhip_window_attn* at, const tl
   const float* pu = static_cast<const float*>(u);
   float* py = static_cast<float*>(y);
   float* pp = static_cast<float*>(partials);
-#define TLHIP_MIX(NQ, NF) return launch_mix<NQ, NF>(pu, py, at, la, pn, (int)pos, d_pos, pp, plan)
+#define TLHIP_MIX(NQ, NF) return launch_mix<NQ, NF>(pu, py, at, la, pn, (int)pos, d_pos, pp, plan, merge)
   switch (plan.nq * 8 + nf) {
     case 8 + 1: TLHIP_MIX(1, 1);
     case 8 + 2: TLHIP_MIX(1, 2);
@@ -179,6 +188,18 @@ int tlhip_mix_step(const void* u, void* y, const tlhip_window_attn* at, const tl
     default: return fail(TLHIP_EUNSUPPORTED, "tlhip_mix_step: no kernel for this head size");
   }
 #undef TLHIP_MIX
+}
+
+int tlhip_mix_step(const void* u, void* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
+                   const tlhip_polynorm* pn, int64_t pos, const void* d_pos, void* partials, int64_t partials_bytes) {
+  return mix_step(u, y, at, la, pn, pos, d_pos, partials, partials_bytes, true);
+}
+
+int tlhip_mix_step_open(const void* u, void* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
+                        const tlhip_polynorm* pn, int64_t pos, const void* d_pos, void* partials, int64_t partials_bytes) {
+  TLHIP_REQUIRE_READY();
+  if (!at || !tlhip_mix_open(at, at->y_off + at->heads * at->dim)) return fail(TLHIP_EUNSUPPORTED, "tlhip_mix_step_open: no product merges the splits of this attention");
+  return mix_step(u, y, at, la, pn, pos, d_pos, partials, partials_bytes, false);
 }
 
 }  // extern "C"

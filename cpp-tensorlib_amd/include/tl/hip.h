@@ -192,6 +192,11 @@ struct api {
   int64_t (*mix_partials_bytes)(const void*) = nullptr;
   int (*mix_step)(const void*, void*, const void*, const void*, const void*, int64_t, const void*, void*,
                   int64_t) = nullptr;
+  int (*mix_open)(const void*, int64_t) = nullptr;
+  int (*mix_step_open)(const void*, void*, const void*, const void*, const void*, int64_t, const void*, void*,
+                       int64_t) = nullptr;
+  int (*gemv_bf16_row_mix)(const void*, const void*, const void*, const void*, int64_t, const void*, void*, int64_t,
+                           int64_t) = nullptr;
   int (*window_fill)(const void*, int64_t, const void*, int64_t, int64_t) = nullptr;
   int (*window_attn_chunk)(const void*, int64_t, void*, int64_t, const void*, int64_t, int64_t, int) = nullptr;
   int (*linear_attn_chunk)(const void*, int64_t, void*, int64_t, const void*, int64_t, int64_t) = nullptr;
@@ -417,6 +422,8 @@ struct context {
               bind(f.gemv_bf16_row_attn, "tlhip_gemv_bf16_row_attn") &&
               bind(f.window_ring_ld, "tlhip_window_ring_ld") && bind(f.linear_state_bytes, "tlhip_linear_state_bytes") &&
               bind(f.mix_partials_bytes, "tlhip_mix_partials_bytes") && bind(f.mix_step, "tlhip_mix_step") &&
+              bind(f.mix_open, "tlhip_mix_open") && bind(f.mix_step_open, "tlhip_mix_step_open") &&
+              bind(f.gemv_bf16_row_mix, "tlhip_gemv_bf16_row_mix") &&
               bind(f.window_fill, "tlhip_window_fill") && bind(f.window_attn_chunk, "tlhip_window_attn_chunk") &&
               bind(f.linear_attn_chunk, "tlhip_linear_attn_chunk") && bind(f.polynorm_rows, "tlhip_polynorm_rows") &&
               bind(f.embed_sinusoid, "tlhip_embed_sinusoid") && bind(f.residual_sum, "tlhip_residual_sum") &&
@@ -1673,9 +1680,14 @@ inline int64_t mix_partials_bytes(const window_attn* at) {
   auto& c = context::get();
   return c.ready ? c.f.mix_partials_bytes(at) : 0;
 }
-// One token through the sublayers given (nullptr: absent), one launch: u -> y, new key and state stored.
+inline bool mix_open(const window_attn& at, int64_t k) {
+  auto& c = context::get();
+  return c.ready && c.f.mix_open(&at, k) != 0;
+}
+// One token through the sublayers given (nullptr: absent), one launch: u -> y, new key and state stored. `open`: the splits
+// of a window are left for gemv_bf16_row_mix to merge (where mix_open allows it).
 inline bool mix_step(void* u, void* y, const window_attn* at, const linear_attn* la, const polynorm* pn, int64_t pos,
-                     void* d_pos, void* partials, int64_t partials_bytes) {
+                     void* d_pos, void* partials, int64_t partials_bytes, bool open = false) {
   launch L;
   if (!L.ok || !u || !y) return false;
   L.reads(u);
@@ -1685,7 +1697,15 @@ inline bool mix_step(void* u, void* y, const window_attn* at, const linear_attn*
   if (at) L.writes(at->ring);
   if (la) L.writes(la->state);
   if (partials) L.writes(partials);
-  return L.sent(L.lib.mix_step(u, y, at, la, pn, pos, d_pos, partials, partials_bytes));
+  return L.sent((open ? L.lib.mix_step_open : L.lib.mix_step)(u, y, at, la, pn, pos, d_pos, partials, partials_bytes));
+}
+inline bool gemv_bf16_row_mix(void* y, void* u, const window_attn& at, void* partials, int64_t partials_bytes, void* W,
+                              void* out, int64_t n, int64_t k) {
+  launch L;
+  if (!L.ok || !y || !u || !partials || !W || !out) return false;
+  L.reads(y, u, partials, W);
+  L.writes(out);
+  return L.sent(L.lib.gemv_bf16_row_mix(y, u, &at, partials, partials_bytes, W, out, n, k));
 }
 // The same for a chunk of T tokens at pos0, one mechanism per call.
 inline bool window_attn_chunk(void* u, int64_t ldu, void* y, int64_t ldy, const window_attn& at, int64_t T, int64_t pos0,

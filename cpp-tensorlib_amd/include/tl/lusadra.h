@@ -374,9 +374,10 @@ inline bool run_layers(model& M, int64_t pos, void* d_pos) {
       at ^= 1;
       d = nullptr;
     }
+    const bool open = M.fused && L.wout.fmt == wfmt::bf16_row && hip::mix_open(a, L.wout.K);   // the output product merges the splits
     if (M.fused) {
       ok = ok && gemv_rmsnorm(L.win, x, d, L.norm, d ? S.res[at] : nullptr, S.u, M.eps) &&
-           hip::mix_step(S.u, S.y, &a, &r, pn, pos, d_pos, S.partials, S.partials_bytes);
+           hip::mix_step(S.u, S.y, &a, &r, pn, pos, d_pos, S.partials, S.partials_bytes, open);
     } else {
       ok = ok && (d ? hip::rmsnorm_res(x, d, L.norm, S.res[at], S.h, WP, M.eps) : hip::rmsnorm(x, L.norm, S.h, WP, M.eps)) &&
            gemv(L.win, S.h, S.u) &&
@@ -388,7 +389,8 @@ inline bool run_layers(model& M, int64_t pos, void* d_pos) {
       x = S.res[at];
       at ^= 1;
     }
-    ok = ok && gemv(L.wout, S.y, S.delta);
+    ok = ok && (open ? hip::gemv_bf16_row_mix(S.y, S.u, a, S.partials, S.partials_bytes, L.wout.w, S.delta, L.wout.N, L.wout.K)
+                     : gemv(L.wout, S.y, S.delta));
     d = S.delta;
   }
   if (M.fused) return ok && gemv_rmsnorm(M.lm_head, x, d, M.onorm, nullptr, S.logitsb, M.eps);

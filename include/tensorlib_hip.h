@@ -521,6 +521,15 @@ int64_t tlhip_mix_partials_bytes(const tlhip_window_attn* at);
 int tlhip_mix_step(const void* u, void* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
                    const tlhip_polynorm* pn, int64_t pos, const void* d_pos, void* partials,
                    int64_t partials_bytes);
+/* The same with the merge left to the product that reads y: nonzero from tlhip_mix_open says that it can be (2 to 8 splits,
+ * dim, y_off and gate_off multiples of four, k up to 20480). y's columns of the attention are then not written; the product takes them from
+ * `partials` (and the gates from u), the other columns from y: y2[n] = y[k] . W, W bf16 [n][k]. */
+int tlhip_mix_open(const tlhip_window_attn* at, int64_t k);
+int tlhip_mix_step_open(const void* u, void* y, const tlhip_window_attn* at, const tlhip_linear_attn* la,
+                        const tlhip_polynorm* pn, int64_t pos, const void* d_pos, void* partials,
+                        int64_t partials_bytes);
+int tlhip_gemv_bf16_row_mix(const void* y, const void* u, const tlhip_window_attn* at, const void* partials,
+                            int64_t partials_bytes, const void* W, void* y2, int64_t n, int64_t k);
 /* A chunk of T tokens at positions pos0 .. pos0 + T - 1, u rows ldu and y rows ldy elements apart.
  * exact != 0: attention products in f32 on the fp32 matrix pipe; 0: chunks of 16 tokens up of heads up to
  * 128 cut every f32 operand into two bf16 terms (2^-17 relative) on the 16-bit matrix cores; scores,

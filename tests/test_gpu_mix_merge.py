@@ -32,14 +32,14 @@ def setting(lib, capi, H, G, dim, window, gate, first, tail):
 @pytest.mark.parametrize("H,G,dim,window,gate,first,tail,n", [
     (16, 4, 128, 1024, True, 0, 10240, 2048),     # 8 splits, one tile of rows a block
     (16, 4, 128, 1024, False, 8, 512, 300),       # columns ahead; no gate
-    (28, 4, 128, 1024, True, 0, 22528, 3584),
+    (28, 4, 128, 1024, True, 0, 16896, 3584),     # as many columns as it takes
     (6, 2, 128, 400, True, 4, 4, 40),             # 4 splits, short blocks: columns past what a thread asks for up front
     (40, 4, 64, 2048, True, 1004, 100, 5000),     # more columns than threads, K split
     (5, 5, 36, 1100, True, 0, 0, 17),             # heads of a width that no vector divides
 ])
 def test_same_bits(lib, capi, H, G, dim, window, gate, first, tail, n):
     at, ring, width, K = setting(lib, capi, H, G, dim, window, gate, first, tail)
-    assert lib.c.tlhip_mix_open(C.byref(at))
+    assert lib.c.tlhip_mix_open(C.byref(at), K)
     nb = lib.mix_partials_bytes(at)
     W = lib.to_device((rng(3).standard_normal((n, K)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16))
     y0 = rng(5).standard_normal(K).astype(np.float32)
@@ -81,6 +81,6 @@ def test_refused(lib, capi):
     for name, value in (("y_off", 2), ("gate_off", 2562), ("window", 4096), ("window", 100)):
         keep = getattr(at, name)
         setattr(at, name, value)
-        assert not lib.c.tlhip_mix_open(C.byref(at)) and rc(at) != 0        # its own merge launch, or none at all
+        assert not lib.c.tlhip_mix_open(C.byref(at), 4096) and rc(at) != 0        # its own merge launch, or none at all
         setattr(at, name, keep)
-    assert lib.c.tlhip_mix_open(C.byref(at)) and not lib.c.tlhip_mix_open(None)
+    assert lib.c.tlhip_mix_open(C.byref(at), 20480) and not lib.c.tlhip_mix_open(C.byref(at), 20488) and not lib.c.tlhip_mix_open(None, 4096)
