@@ -579,10 +579,10 @@ int tlhip_argmax(const void* in, int64_t n, int64_t* out_idx) {
   TLHIP_REQUIRE_READY();
   if (!out_idx) return fail(TLHIP_EINVAL, "tlhip_argmax: null out pointer");
   Context& c = ctx();
-  // the kernel stores the index into pinned memory itself (see copy_out_kernel)
-  if (int rc = tlhip_argmax_async(in, n, c.argmax_host)) return rc;
-  hipError_t e = hipStreamSynchronize(c.stream);
-  if (e != hipSuccess) return hip_fail(e, "argmax");
+  if (int rc = tlhip_argmax_async(in, n, c.argmax_dev)) return rc;
+  hipError_t e = hipMemcpyAsync(c.argmax_host, c.argmax_dev, sizeof(int), hipMemcpyDeviceToHost, c.stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+  if (e != hipSuccess) return hip_fail(e, "argmax result copy");
   *out_idx = *c.argmax_host;
   return TLHIP_OK;
 }
