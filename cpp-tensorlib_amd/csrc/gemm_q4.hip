@@ -13,9 +13,10 @@
 //     each half its k. Masked in place, a nibble is an f16 with its value (or 16 times that) in the last bits of 1024, so
 //     eight of them take nine instructions; the k order that gives (0 4 1 5 2 6 3 7) is the one the images are
 //     written in.
-// 102 vector instructions beside 16 MFMAs per slab and wavefront are left, 64 of them the scales'; they and the MFMAs of a
-// SIMD's two wavefronts add up (512 x 32768 x 3584: 235 us = 510 TFLOP/s; without the scales 192, without all of it and the
-// loads 148; wave priorities and a staggered start change nothing). Two blocks per CU, two barriers per 128 k.
+// 102 vector instructions beside 16 MFMAs per slab and wavefront are left, 64 of them the scales'. Behind the MFMAs they and
+// the MFMAs of a SIMD's two wavefronts add up (512 x 32768 x 3584: 235 us = 510 TFLOP/s; without the scales 192, without all
+// of it and the loads 148; wave priorities and a staggered start change nothing), so they go between them, six of which two
+// wavefronts hide behind one: 24 shapes 0.99 to 1.10 times as fast, 1.03 on average, 512 x 37888 x 3584 gated 1.06. Two blocks per CU, two barriers per 128 k.
 // Rows come in blocks of 64: 301 rows waste 6 % of the products, 128-row tiles waste 28 %. us, before -> now: 301 rows
 // gated 37888 x 3584 303 -> 209, 3584 x 18944 150 -> 113, 4608 x 3584 48 -> 42; 512 rows 393 -> 320, 207 -> 176, 61 -> 58.
 #include "gemm_shared.hpp"

@@ -12,7 +12,7 @@
 // mixers (hip::window_attn, hip::linear_attn, hip::polynorm), which read columns of u and write columns
 // of y, the mixer scales folded into y. A decode layer is three launches:
 //   [norm -> input product] , [attention | linear attention | polynorm] , [output product]
-// (four where the window is cut into splits), the residual add riding on the next layer's norm.
+// (four where a window's splits are too many for the output product to merge), the residual add riding on the next layer's norm.
 //
 // Residual, norms, scores, decays, state and sums are f32; weights stay the bf16 of the file.
 //
