@@ -74,7 +74,7 @@ struct MixSplits {
   float2 a[kMergeGroup], b[kMergeGroup];
   float4 g;
   __device__ __forceinline__ void load(const Producer& pro, int e) {     // float4 e of [heads][D]
-    const int h = (int)__umulhi((uint32_t)e, (uint32_t)pro.parts), d = 4 * e - h * pro.D;
+    const int h = (int)__umulhi(2u * (uint32_t)e, (uint32_t)pro.parts), d = 4 * e - h * pro.D;
     const float* p = pro.delta + (size_t)h * pro.S * pro.part_ld;        // (rows of an even number of floats)
 #pragma unroll
     for (int s = 0; s < kMergeGroup; s++) {
@@ -995,8 +995,9 @@ int tlhip_gemv_bf16_row_mix(const void* a, const void* u, const tlhip_window_att
                nullptr, at->out_scale, window_splits(at), (int)at->heads, (int)at->dim};
   pro.part_ld = (int)at->ring_ld + 2;
   pro.first4 = (int)(at->y_off / 4);
-  const int64_t d4 = at->dim / 4;                // e / d4 = umulhi(e, parts) for e d4^2 < 2^32: a row that fits LDS is far below
-  pro.parts = (int)(uint32_t)(((int64_t(1) << 32) + d4 - 1) / d4);
+  // e / d4 = umulhi(2 e, ceil(2^31 / d4)) while e d4 < 2^31, as all that fit a row in LDS do (2^32 would not fit for heads of 4)
+  const int64_t d4 = at->dim / 4;
+  pro.parts = (int)(uint32_t)(((int64_t(1) << 31) + d4 - 1) / d4);
   return launch_rows<FmtBf16, kMixMerge>(static_cast<const float*>(a), W, nullptr, static_cast<float*>(y), n, k,
                                          TLHIP_C_GEMV_BF16_ROW, RowTune{0, 0, 0, 0, 0}, pro);
 }

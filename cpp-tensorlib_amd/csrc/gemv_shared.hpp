@@ -203,7 +203,7 @@ struct Producer {
   const float* bias = nullptr;
   int parts = 0, part_len = 0, add_x = 0;
   // kMixMerge: delta = the partials, S splits of `heads` heads of D in rows of part_ld, norm_w = the gates' columns (nullptr:
-  // none), eps = what the result is multiplied by, parts = ceil(2^32 / (D / 4)); the attention's columns begin at float4 first4 of x
+  // none), eps = what the result is multiplied by, parts = ceil(2^31 / (D / 4)); the attention's columns begin at float4 first4 of x
   int part_ld = 0, first4 = 0;
   // kGeglu
   const float* gu_bias = nullptr;

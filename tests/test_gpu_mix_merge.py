@@ -36,6 +36,9 @@ def setting(lib, capi, H, G, dim, window, gate, first, tail):
     (6, 2, 128, 400, True, 4, 4, 40),             # 4 splits, short blocks: columns past what a thread asks for up front
     (40, 4, 64, 2048, True, 1004, 100, 5000),     # more columns than threads, K split
     (5, 5, 36, 1100, True, 0, 0, 17),             # heads of a width that no vector divides
+    (6, 3, 4, 2048, True, 4, 4, 40),              # heads of a single float4, and of two
+    (70, 7, 4, 1600, False, 0, 16, 300),
+    (6, 2, 8, 4096, True, 0, 0, 33),
 ])
 def test_same_bits(lib, capi, H, G, dim, window, gate, first, tail, n):
     at, ring, width, K = setting(lib, capi, H, G, dim, window, gate, first, tail)
