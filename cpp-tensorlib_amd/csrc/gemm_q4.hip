@@ -125,14 +125,22 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
     srow[j] = scales + r * groups;
   }
   const char* asrc = Aimg + ((size_t)rb * groups + 4 * ubeg) * kImage;
-  // my eighth of a unit's copy (past the last group: the images end, so the copy stops there)
+  // my quarter of a unit's copy. Groups past the last are zeros in LDS: they are multiplied too, by a scale of zero, and an
+  // infinity or NaN left there from another group would come through that.
   auto copy = [&](int u, int stage) {
     const int have = min(4, groups - 4 * (ubeg + u)) * (kImage / 1024);
+    const auto piece = [&](int p) {
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(asrc + (size_t)u * kUnit + p * 1024 + lane * 16),
+                                       (__attribute__((address_space(3))) void*)(ring + stage * kUnit + p * 1024), 16, 0, 0);
+    };
+    if (have == kUnit / 1024) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int piece = min(wave * 8 + i, have - 1);   // (a repeated piece lands in a slab whose scales are zero)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(asrc + (size_t)u * kUnit + piece * 1024 + lane * 16),
-                                       (__attribute__((address_space(3))) void*)(ring + stage * kUnit + (wave * 8 + i) * 1024), 16, 0, 0);
+      for (int i = 0; i < 8; i++) piece(wave * 8 + i);
+    } else {
+      for (int p = wave * 8; p < wave * 8 + 8; p++) {
+        if (p < have) piece(p);
+        else *reinterpret_cast<frag16*>(ring + stage * kUnit + p * 1024 + lane * 16) = frag16{0, 0, 0, 0};
+      }
     }
   };
   frag16 w[2][2][2];                               // [set][column tile][groups 0 1 | 2 3]
@@ -206,10 +214,10 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
     }
   };
   auto unit = [&](int set, int u) __attribute__((always_inline)) {
-    // my copies and loads of unit u have landed (those of u + 1 - eight copies, six loads - may be in flight); past the
-    // barrier that holds for every wavefront
+    // my copies and loads of unit u have landed (those of u + 1 - eight copies, six loads - may be in flight), and my zeros where
+    // it is the one that lacks groups; past the barrier that holds for every wavefront
     if (4 * (ubeg + u) + 8 <= groups && u + 1 < nu) asm volatile("s_waitcnt vmcnt(14)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     barrier();
     // words of groups (half) and 2 + (half): a half's k of both groups of a pair
 #pragma unroll
