@@ -77,8 +77,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void sgemm_split_kernel(const float
   // one contiguous run of tiles per XCD, row blocks fastest: they read the same columns of B
   const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int lid = xcd * q8 + min(xcd, r8) + within;
-  // (the last columns' tile is moved back to end with the matrix: its first columns are written twice, the same bits)
-  const int m0 = lid % row_blocks * BM, n0 = min(lid / row_blocks * kBN, N - kBN);
+  // (the last columns' tile is moved back to end with the matrix: it stores only the columns from `own` on, for those before them the
+  // tile ahead of it may have taken the other way through the range check below)
+  const int m0 = lid % row_blocks * BM, own = lid / row_blocks * kBN, n0 = min(own, N - kBN);
   const int kbeg = blockIdx.y * kchunk, kend = min(K, kbeg + kchunk);
   C += (size_t)blockIdx.y * M * N;                 // K-split parts are dense
   const int steps = (kend - kbeg) / kStep, mine = wave < steps ? (steps - wave + kWaves - 1) / kWaves : 0;
@@ -290,18 +291,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void sgemm_split_kernel(const float
   const bool wide = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
   for (int i = tid; i < BM * (kBN / 4); i += 64 * kWaves) {
     const int row = i / (kBN / 4), c = i % (kBN / 4) * 4, gm = m0 + row, gn = n0 + c;
-    if (gm >= M) continue;
+    if (gm >= M || gn + 3 < own) continue;
     const auto part = [&](int s) { return *reinterpret_cast<const f32x4*>(sums + (s * BM + row) * kLD + c); };
     f32x4 o = (part(0) + part(1)) + (part(2) + part(3));
     if (epi)
 #pragma unroll
       for (int e = 0; e < 4; e++) o[e] = add_rn(mul_rn(o[e], scale), offset);
     float* dst = C + (size_t)gm * N + gn;
-    if (wide) {
+    if (wide) {                                    // (N and with it n0 are multiples of four: all or none of them are own)
       *reinterpret_cast<f32x4*>(dst) = o;
-    } else {
+    } else if (gn >= own) {
 #pragma unroll
       for (int e = 0; e < 4; e++) dst[e] = o[e];
+    } else {
+      for (int e = own - gn; e < 4; e++) dst[e] = e == 1 ? o[1] : e == 2 ? o[2] : o[3];
     }
   }
 }

@@ -78,6 +78,22 @@ def test_infinities_and_nan_stay_where_they_are(lib, orc, tb):
     assert np.all(np.abs(got[np.ix_(rows, keep)] - (A64 @ B64)[:, keep]) <= ((K + 9) * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)))[:, keep])
 
 
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(193, 4865, 896), (333, 4861, 901), (700, 129, 4000), (500, 897, 4864)])
+def test_one_writer_for_each_column(lib, orc, M, N, K, tb):
+    """The last column tile is moved back to end with the matrix and reads columns that the one before it owns. A number that sends only
+    one of the two to the fp32 pipe leaves the other's columns their bits."""
+    print("case sgemm split overlap", M, N, K, tb, flush=True)
+    A, B = orc.normal(M * K, 81).reshape(M, K), orc.normal(N * K, 82).reshape((N, K) if tb else (K, N))
+    clean, first = _run(lib, A, B, tb), N // 128 * 128
+    for column, kept in ((N - 1, slice(0, first)), (first - 128, slice(first, N))):
+        for value in (2.0 ** -140, 2.0 ** 120):
+            Bx = B.copy()
+            (Bx.T if tb else Bx)[5, column] = value      # read by the last tile only, then by the one before it only
+            got = [_run(lib, A, Bx, tb) for _ in range(3)]
+            assert np.array_equal(got[0][:, kept], clean[:, kept]) and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
 def test_whole_numbers_are_exact(lib):
     """Products that fit 24 bits lose no term: 10 bits by 6, 15 by 2 and the other way round, each sum below 2^24."""
     g = np.random.default_rng(78)
