@@ -37,11 +37,7 @@ void* tlq_create(const qwen::dims* d) {
   return h;
 }
 
-void tlq_destroy(void* hv) {
-  auto* h = static_cast<handle*>(hv);
-  if (h && h->M.embed) hip::release(h->M.embed, 0, nullptr);
-  delete h;
-}
+void tlq_destroy(void* hv) { delete static_cast<handle*>(hv); }
 
 // ---- model files ------------------------------------------------------------------------------
 // The last error of tlq_gguf_* / tlq_create_from_gguf on this thread ("" when none).

@@ -28,6 +28,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -97,7 +98,8 @@ struct step_prof {
 struct model {
   dims d{};
   prefill_scratch ps;
-  void* embed = nullptr;        // [vocab, hidden] bf16 or f16 rows on the device (the reference gathers on the host, qm:530-535)
+  // [vocab, hidden] bf16 or f16 rows on the device (the reference gathers on the host, qm:530-535); goes with the model
+  std::shared_ptr<void> embed;
   bool embed_f16 = false;       // rows are IEEE half, as a model file stores token_embd (qm:297)
   void* onorm = nullptr;
   linear lm_head;
@@ -260,8 +262,7 @@ inline bool set_layer_bf16(model& M, int64_t li, const layer_blobs_bf16& b) {
 // runs at a fraction of the link's rate); the one before it is let go.
 inline bool set_embed(model& M, const void* rows, bool f16) {
   const int64_t bytes = M.d.vocab * M.d.hidden * 2, blk = std::min(bytes, int64_t(32) << 20);
-  if (M.embed) hip::release(M.embed, 0, nullptr);
-  M.embed = hip::alloc_device(bytes);
+  M.embed.reset(hip::alloc_device(bytes), [](void* p) { hip::release(p, 0, nullptr); });
   M.embed_f16 = f16;
   float* stage_host = nullptr;
   void* stage = M.embed ? hip::alloc(blk, &stage_host) : nullptr;
@@ -271,7 +272,7 @@ inline bool set_embed(model& M, const void* rows, bool f16) {
     const int64_t n = std::min(blk, bytes - o);
     std::memcpy(stage_host, static_cast<const char*>(rows) + o, (size_t)n);
     hip::upload(stage, stage_host, (n + 3) / 4);
-    ok = hip::copy_d2d(static_cast<char*>(M.embed) + o, stage, n);
+    ok = hip::copy_d2d(static_cast<char*>(M.embed.get()) + o, stage, n);
     hip::flush();   // the staging block is used again
   }
   hip::release(stage, blk, stage_host);
@@ -595,7 +596,7 @@ inline void set_cache_pos(model& M, int64_t p) {
 // The step's input: the token's embedding row, widened on the device. false for a token id outside [0, vocab): nothing is
 // read or launched.
 inline bool stage_embed(model& M, int64_t token) {
-  return hip::embed_rows(M.embed, M.embed_f16, &token, 1, M.s.embedb, M.d.hidden, M.d.vocab);
+  return hip::embed_rows(M.embed.get(), M.embed_f16, &token, 1, M.s.embedb, M.d.hidden, M.d.vocab);
 }
 
 // All layers + final norm + lm_head on the scratch buffers, no allocation, no
@@ -845,7 +846,7 @@ inline bool prefill_layers(model& M, int64_t T) {
 inline bool stage_chunk(model& M, const int64_t* tokens, int64_t T) {
   for (int64_t t = 0; t < T; t++)
     if (tokens[t] < 0 || tokens[t] >= M.d.vocab) return false;
-  return prefill_reserve(M, T) && hip::embed_rows(M.embed, M.embed_f16, tokens, T, M.ps.emb, M.d.hidden, M.d.vocab);
+  return prefill_reserve(M, T) && hip::embed_rows(M.embed.get(), M.embed_f16, tokens, T, M.ps.emb, M.d.hidden, M.d.vocab);
 }
 
 // ---- what the decode loops (decode_loop.h) ask of a model --------------------------------------
@@ -862,8 +863,8 @@ inline bool step_layers(model& M, int64_t pos, void* d_pos = nullptr, bool advan
 // The same with its input taken from a token id on the device.
 inline bool step_layers_from(model& M, void* d_tok, void* d_pos) {
   const dims& d = M.d;
-  const bool ok = M.embed_f16 ? hip::embed_gather_f16(M.embed, d_tok, M.s.embedb, d.hidden, d.vocab)
-                              : hip::embed_gather_bf16(M.embed, d_tok, M.s.embedb, d.hidden, d.vocab);
+  const bool ok = M.embed_f16 ? hip::embed_gather_f16(M.embed.get(), d_tok, M.s.embedb, d.hidden, d.vocab)
+                              : hip::embed_gather_bf16(M.embed.get(), d_tok, M.s.embedb, d.hidden, d.vocab);
   return ok && step_layers(M, 0, d_pos, /*advance=*/false);
 }
 // What steps with the position on the device need besides the model; false: this model has no such steps.
