@@ -100,6 +100,7 @@ struct model {
   prefill_scratch ps;
   // [vocab, hidden] bf16 or f16 rows on the device (the reference gathers on the host, qm:530-535); goes with the model
   std::shared_ptr<void> embed;
+  int64_t embed_bytes = 0;
   bool embed_f16 = false;       // rows are IEEE half, as a model file stores token_embd (qm:297)
   void* onorm = nullptr;
   linear lm_head;
@@ -259,10 +260,12 @@ inline bool set_layer_bf16(model& M, int64_t li, const layer_blobs_bf16& b) {
 }
 
 // The embedding table, [vocab, hidden] rows of 16 bits, onto the device through a pinned block (a copy from pageable memory
-// runs at a fraction of the link's rate); the one before it is let go.
+// runs at a fraction of the link's rate). Another table of the same size takes the place of the one before it: a recorded
+// token loop reads it there.
 inline bool set_embed(model& M, const void* rows, bool f16) {
   const int64_t bytes = M.d.vocab * M.d.hidden * 2, blk = std::min(bytes, int64_t(32) << 20);
-  M.embed.reset(hip::alloc_device(bytes), [](void* p) { hip::release(p, 0, nullptr); });
+  if (!M.embed || M.embed_bytes != bytes) M.embed.reset(hip::alloc_device(bytes), [](void* p) { hip::release(p, 0, nullptr); });
+  M.embed_bytes = bytes;
   M.embed_f16 = f16;
   float* stage_host = nullptr;
   void* stage = M.embed ? hip::alloc(blk, &stage_host) : nullptr;

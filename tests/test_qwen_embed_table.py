@@ -34,11 +34,17 @@ def stand_in(tmp_path_factory):
         #include <stdlib.h>
         #include <string.h>
         static struct { void* p; size_t n; } held[1 << 16];
-        static int count;
+        static int count, freed;
+        static size_t watched;
         static void* block(size_t n) { void* p = calloc(1, n + 64); held[count].p = p; held[count++].n = n; return p; }
         static int drop(void* p) {
-          for (int i = 0; i < count; i++) if (held[i].p == p) { held[i] = held[--count]; free(p); return 0; }
+          for (int i = 0; i < count; i++) if (held[i].p == p) { freed += held[i].n == watched; held[i] = held[--count]; free(p); return 0; }
           return -1;
+        }
+        int standin_freed(size_t n) { int k = freed; watched = n; freed = 0; return k; }   /* blocks of n bytes, since it was asked last */
+        int standin_holds(size_t n, const void* bytes) {
+          for (int i = 0; i < count; i++) if (held[i].n == n && !memcmp(held[i].p, bytes, n)) return 1;
+          return 0;
         }
         int standin_live(size_t n) { int k = 0; for (int i = 0; i < count; i++) k += held[i].n == n; return k; }
     """)
@@ -59,7 +65,7 @@ def _program(stand_in, body):
     """In a process of its own: the backend is chosen once per process."""
     head = "import sys, ctypes as C, importlib, numpy as np\nsys.path[:0] = [%r, %r]\n" % (ROOT, HERE)
     head += "q, models = (importlib.import_module('cpp-tensorlib_amd.' + m) for m in ('qwen', 'model'))\n"
-    head += "s = C.CDLL(%r)\ns.standin_live.argtypes = [C.c_size_t]\n" % stand_in
+    head += "s = C.CDLL(%r)\ns.standin_live.argtypes = s.standin_freed.argtypes = [C.c_size_t]\n" % stand_in
     r = subprocess.run([sys.executable, "-c", head + textwrap.dedent(body)], env=dict(os.environ, TENSORLIB_HIP_LIB=stand_in),
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=110)
     assert r.returncode == 0, r.stdout.decode(errors="replace")[-2000:]
@@ -81,3 +87,20 @@ def test_closing_a_model_lets_its_table_go(stand_in, tmp_path, api):
             live.append(s.standin_live(%d))
         assert live[1:] == live[:-1], live       # (a staging block of the same size stays for the next one)
     """ % (path, opener, TABLE))
+
+
+def test_another_table_takes_the_place_of_the_first(stand_in):
+    """A token loop recorded before reads the table where it was: the block must not be given back."""
+    _program(stand_in, """
+        d, table = %r, %d
+        g = q.QwenGPU(d)
+        onorm, head = np.ones(d["hidden"], np.float32), np.zeros(d["vocab"] * d["hidden"], np.uint8)
+        s.standin_freed(table)
+        for seed in (1, 2):
+            rows = np.random.default_rng(seed).integers(0, 1 << 16, (d["vocab"], d["hidden"]), np.uint16)
+            assert g.L.tlq_set_head_q4(g.h, q._p(rows), q._p(onorm), q._p(head)) == 0
+            assert s.standin_holds(C.c_size_t(table), q._p(rows))
+        assert s.standin_freed(table) == 0
+        g.close()
+        assert s.standin_freed(table) == 1
+    """ % (DIMS, TABLE))
