@@ -1,10 +1,16 @@
 // f32 products on the bf16 matrix pipe: C[M,N] = A[M,K] . op(B), operands cut into three bf16 terms.
 //
-// An f32 has 24 significant bits, a bf16 eight: rounding off one term after the other leaves a = a0 + a1 + a2 exactly, each
-// term at most 2^-9 of the one before. Of the nine products of a b the six with i + j <= 2 are summed; the others are below
-// 2^-26 of it, a quarter of what one fp32 rounding may lose, and vanish altogether where the product of a and b is itself a
-// 24-bit number (integers stay exact). v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of the fp32 pipe in a
-// clock, so six of them are 2.7 times as fast, with 6 roundings of the sum per 16 k where that one has 8.
+// An f32 has 24 significant bits, a bf16 eight: rounding off one term after the other leaves a = a0 + a1 + a2 exactly, with a1 at
+// most 2^-8 of a and a2 2^-17 (three bf16 terms for an f32 product: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", 2019). Of the nine products of a b the six with i + j <= 2 are summed. The
+// others are at most 2^-24 of it, what one fp32 rounding may lose, 6e-9 of a dense result, and vanish where the product is itself a
+// 24-bit number (integers stay exact, rows are selected exactly). v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of the
+// fp32 pipe in a clock, so six of them are 2.7 times as fast, with 6 roundings of the sum per 16 k where that one has 8; they lean
+// down where the fp32 pipe's do not (mean error -0.3e-7 to -0.7e-7 of a result's spread). Error against 64 bits beside the kernels that
+// ran before, five shapes of K 896 to 4864 (2-norm): normal numbers 0.5 to 0.8 of theirs, all positive 0.45 to 1.15, spread over
+// decades 0.4 to 0.8, rows with half their numbers zero 0.7 to 1.09. Sums of one product are the worst case: up to 1.43 units in the
+// last place, 0.5 there. With the two pairs a1 b2 and a2 b1 too they are 1.0, 333 x 4864 x 896 takes 31 us for 27 (event time) and dense
+// results are no nearer.
 //
 // Blocks and waves are those of sgemm_rows_kernel: the eight wavefronts of a block take the 16-k steps w, w + 8, ... of its
 // 32 TM x 128 tile, operands go from memory to the registers that cut them up (so every number is cut once per block, without
@@ -15,9 +21,9 @@
 // pipe's peak is 157, and 60 to 80 were reached). With a tile's matrix instructions after the next tile's cuts instead of between
 // them 333 x 4864 x 896 took 29.
 //
-// The cut is exact, and so is what the pipe makes of it, while no term is subnormal and none overflows. Each block keeps the
-// largest and the smallest magnitude (of what is not zero) it read, and where those leave that room - infinities too, which
-// must not meet the zeros of another number's lower terms - it does its tile again with the fp32 instruction.
+// The cut is exact while no term is subnormal and none overflows. Each block keeps the largest and the smallest magnitude (of what is
+// not zero) it read, and where those leave no room for that - infinities too, which must not meet the zeros of another number's
+// lower terms - it does its tile again with the fp32 instruction.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -227,7 +233,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void sgemm_split_kernel(const float
         most[i] = fmaxf(most[i], seen_most[i][w]);
         least[i] = min(least[i], seen_least[i][w]);
       }
-    // a third term is at least 2^-24 of its number, a product of two terms that are summed at least 2^-26 of theirs
+    // A term is at least the last place of its number, 2^-23 of its power of two, so from 2^-95 on none is subnormal. A product of two
+    // second terms can be 2^-46 of the whole; of a product of 2^-95 or more, what the pipe drops below 2^-126 is 2^-31 at most.
     const auto room = [&](uint32_t x) { return (int)(x >> 24) - 127; };   // exponent of the least magnitude (zeros only: 128)
     const bool fits = most[0] < 0x1p100f && most[1] < 0x1p100f && most[0] * most[1] < 0x1p100f && room(least[0]) > -96 && room(least[1]) > -96 &&
                       room(least[0]) + room(least[1]) > -96;
@@ -324,8 +331,10 @@ int launch_sgemm_split(const float* pa, int64_t lda, const float* pb, int64_t ld
   // (17 to 1000 rows, 128 to 16000 columns, K 32 .. 5000; error 12 %, the pick within 0.3 % of the best on average): blocks
   // run one to a CU, and a round of them starts and ends and takes its steps of 16 k; parts are written and read, and their sum
   // is a launch. It has to be 15 % less than the others' (their errors are 6 to 15 %): all of the shapes it is then given
-  // were faster, 1.03 to 2 times, 1.5 on average. A wavefront adds up no more than 1.4 times the
-  // other kernel's steps: for as many its error is 0.8 of theirs, and grows with their root.
+  // were faster, 1.03 to 2 times, 1.5 on average. At 10 % less it would also take 512 x 640 x 1001, a tenth faster, where one element
+  // of a test against the CPU path came to 1.04 of its tolerance (the 64-bit result itself is at 0.995 there): results of other
+  // bits are left alone where little is gained. A wavefront adds up no more than 1.4 times the
+  // other kernel's steps: for as many its error on normal numbers is 0.8 of theirs, and grows with their root.
   const int cus = ctx().cus;
   double least = 0.85 * other_us;
   int TM = 0, S = 1;

@@ -1,7 +1,8 @@
 """GPU parity: f32 products on the bf16 matrix pipe in three terms (sgemm_split_kernel of csrc/sgemm_split.hip) at the edges of its 32-row
 and 128-column tiles, its 16-k steps and its K splits, and over the whole range of f32, where it hands a tile to the fp32 pipe, against
 float64. A sum of K fp32 products is off by at most (K + 8) 2^-24 of the sum of its terms' magnitudes, whatever its order, and the terms
-left out add up to 2^-26 of each; a product below the least normal number may be lost. The sizes are such that the estimates choose it."""
+left out add up to 2^-24 of each; a product below the least normal number may be lost. That holds for any kernel and would hide a term
+gone missing, so the error over a whole result is compared with the fp32 pipe's too. The sizes are such that the estimates choose it."""
 import numpy as np
 import pytest
 
@@ -92,6 +93,45 @@ def test_one_writer_for_each_column(lib, orc, M, N, K, tb):
             (Bx.T if tb else Bx)[5, column] = value      # read by the last tile only, then by the one before it only
             got = [_run(lib, A, Bx, tb) for _ in range(3)]
             assert np.array_equal(got[0][:, kept], clean[:, kept]) and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(333, 4864, 896), (99, 4608, 3584), (500, 896, 4864), (700, 129, 4000), (320, 1152, 2049), (512, 2048, 1024)])
+def test_no_further_off_than_the_fp32_pipe(lib, orc, M, N, K, tb):
+    """The same numbers with A transposed go to the LDS-tiled fp32 kernel, which adds all of a block's K in one chain: 1.7 to 5.5 times this
+    kernel's error in these shapes (2-norm). Without the third terms of one operand the result would be
+    off by 2.4e-6, twice that kernel's error at its largest (1.1e-6)."""
+    print("case sgemm split error", M, N, K, tb, flush=True)
+    A, B = orc.normal(M * K, 85).reshape(M, K), orc.normal(N * K, 86).reshape((N, K) if tb else (K, N))
+    want = A.astype(np.float64) @ (B.T if tb else B).astype(np.float64)
+    err = lambda got: np.linalg.norm(got - want) / np.linalg.norm(want)
+    da, db, out = lib.to_device(np.ascontiguousarray(A.T)), lib.to_device(B), lib.empty((M, N))
+    lib.gemm(da, M, 1, db, K if tb else N, tb, out, M, N, K)
+    fp32, here = err(out.numpy()), err(_run(lib, A, B, tb))
+    assert here <= fp32, (here, fp32)
+    for b in (da, db, out):
+        b.free()
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+def test_sums_of_one_product(lib, orc, tb):
+    """Rows with a single element. Eight bits of it lose nothing, so that rows are selected and scaled by powers of two exactly. Of 24
+    bits the two pairs left out are at most 2^-24 of the product, half a unit in the last place of a result just above a power of two and one of
+    the largest, and the pipe's last addition is off by less than one: below 2 units (measured 1.43, and 0.5 on the fp32 pipe)."""
+    M, N, K = 333, 4864, 896
+    at, B = (np.arange(M) * 7) % K, orc.normal(N * K, 88).reshape((N, K) if tb else (K, N))
+    Bk = B.T if tb else B
+    for values in (np.ones(M), np.exp2(np.arange(M) % 9 - 4), 1 + np.arange(M) % 256):
+        A = np.zeros((M, K), np.float32)
+        A[np.arange(M), at] = values
+        got, want = _run(lib, A, B, tb), Bk[at].astype(np.float64) * values[:, None]
+        if values.max() < 100:
+            assert np.array_equal(got, want.astype(np.float32))
+        else:                                            # (32 bits: rounded, by the last addition)
+            assert np.all(np.abs(got - want) < np.spacing(np.abs(want).astype(np.float32)))
+    A[np.arange(M), at] = orc.normal(M, 89)
+    want = Bk[at].astype(np.float64) * A[np.arange(M), at].astype(np.float64)[:, None]
+    assert np.all(np.abs(_run(lib, A, B, tb) - want) < 2 * np.spacing(np.abs(want).astype(np.float32)))
 
 
 def test_whole_numbers_are_exact(lib):
