@@ -509,8 +509,18 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
   const int ltn = tn - tn0;                          // column tile within this launch
   const int nlim = N + (GU ? tn0 * 128 : tn0 * kTile);   // first unit of N past this launch, absolute
   const bool wide = (ldc & 3) == 0;
-  // exponents of the W rows behind tile columns c .. c + 3 of this block
+  // Exponents of the W rows behind tile columns c .. c + 3 of this block (c a multiple of four): neighbouring rows, so one
+  // load of four bytes where the up rows' offset keeps them aligned (the buffer is padded to whole 16 bytes; byte by byte they
+  // were 128 loads a lane: 512 x 3584 x 3584 in four parts 36.4 -> 35.0 us, 2560 gated columns 43.5 -> 42.0).
+  const bool by4 = !GU || (ff & 3) == 0;
   auto wexp4 = [&](int c, int e4[4]) {
+    if (by4) {
+      const int r = weight_row(GU, tn, c, nlim, ff);
+      const uint32_t w = r >= 0 ? *reinterpret_cast<const uint32_t*>(ew + r) : 0u;
+#pragma unroll
+      for (int e = 0; e < 4; e++) e4[e] = (int)(int8_t)(w >> (8 * e));
+      return;
+    }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int r = weight_row(GU, tn, c + e, nlim, ff);
