@@ -111,6 +111,7 @@ SIGNATURES = {
     "tlhip_attn_decode_qkv": (cint, [P, P, P, P, P, P, P, i64, i64, i64, P, i64, i64, f32, P, cint, P, i64]),
     "tlhip_embed_gather_bf16": (cint, [P, P, P, i64, i64]),
     "tlhip_token_advance": (cint, [P, P, P, i64]),
+    "tlhip_gemm_f16w_nt_geglu": (cint, [P, P, P, P, P, P, i64, i64, i64]),
     "tlhip_gemm_f16w_aimage_bytes": (i64, [i64, i64]),
     "tlhip_rmsnorm_res_parts_aimage": (cint, [P, P, i64, P, P, P, i64, f32, i64, P]),
     "tlhip_gemm_f16w_nt_aimage": (cint, [P, P, P, P, P, i64, i64, i64]),
@@ -428,6 +429,9 @@ class TlHip:
 
     def gemm_f16w_nt_swiglu(self, A, image, exps, act, M, ff, K):
         self._chk(self.c.tlhip_gemm_f16w_nt_swiglu(A.ptr, image.ptr, exps.ptr, act.ptr, M, ff, K))
+
+    def gemm_f16w_nt_geglu(self, A, image, exps, bias, act, M, ff, K, aimage=None):
+        self._chk(self.c.tlhip_gemm_f16w_nt_geglu(A.ptr, aimage.ptr if aimage else None, image.ptr, exps.ptr, bias.ptr, act.ptr, M, ff, K))
 
     def gemm_f16w_nt_parts(self, A, image, exps, parts, M, N, K):
         n = C.c_int(0)

@@ -27,6 +27,7 @@
 // error plus one fp32-rounding-sized term per product, as in the reference's fp32 FMA loop
 // (tensorlib_cuda.cu:509-519).
 #include "gemm_shared.hpp"
+#include "gemv_shared.hpp"
 
 namespace tlhip {
 namespace f16t {
@@ -316,17 +317,23 @@ __global__ __launch_bounds__(1024) void rmsnorm_aimage_kernel(const float* x, co
 // TM = 2: a 256 x 256 tile, 64 x 128 per wavefront. TM = 1: 128 x 256 (32 x 128 per wavefront, one
 // half of an activation image): twice the tiles for the products whose N is a few thousand, which
 // then need half the K splits and write half the parts.
-// GU: the result is the gated activation act[m][f] = swiglu(A . gate_f, A . up_f)
-// (array.h:2435-2439) when K is not split; under a split the raw parts are stored in tile column
-// order and splitk_sum_swiglu_kernel gates after the sum.
-template <int TM, bool GU>
+// ACT: the result is the gated activation act[m][f] = swiglu(A . gate_f, A . up_f)
+// (array.h:2435-2439), or gelu_tanh(A . gate_f + bias_f) (A . up_f + bias_(ff + f)), when K is not
+// split; under a split the raw parts are stored in tile column order and splitk_sum_swiglu_kernel or
+// splitk_sum_geglu_kernel gates after the sum. (The GELU gate was a launch over the [M, 2 ff]
+// products before: 20 us beside a product of 262 at 512 rows of 2 x 18944 columns over 3584, and
+// 39 MB more for the product to store.)
+enum Act { kPlain = 0, kSwiglu = 1, kGelu = 2 };
+template <int TM, int ACT>
 __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restrict__ Aimg,
                                                            const char* __restrict__ Wimg,
                                                            float* __restrict__ C, int M, int N, int nslab,
                                                            int part_slabs, int ldc, int tn0, int ff,
                                                            const int* __restrict__ ea,
                                                            const int8_t* __restrict__ ew, int wpad,
-                                                           const float* __restrict__ A) {
+                                                           const float* __restrict__ A,
+                                                           const float* __restrict__ bias) {
+  constexpr bool GU = ACT != kPlain;
   constexpr int BM = 128 * TM;
   constexpr int kAPlane = BM * kRowBytes;            // one plane of this block's rows in a stage
   constexpr int kStage = 2 * kAPlane + kWImage;
@@ -538,6 +545,7 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
   // stored that. Ordinary operands never get here: it takes an element 2^24 (of W: 2^31) below its
   // row's largest AND a row-times-column scale above 2^14. The pass is per lane and serial; the
   // kernel's time is not its concern.
+  auto gate = [](float g, float u, float bg, float bu) { return ACT == kGelu ? gelu_tanh(g + bg) * (u + bu) : gated(g, u); };
   const uint16_t* wcount = reinterpret_cast<const uint16_t*>(ew + wpad);
   const WHeader* whdr = reinterpret_cast<const WHeader*>(ew + 3 * (size_t)wpad);
   auto again = [&](bool gated_out) {
@@ -582,8 +590,8 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
           const int f = ltn * 128 + wn * 64 + j * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
           const int rg = weight_row(GU, tn, c, nlim, ff), ru = weight_row(GU, tn, c + 64, nlim, ff);
           if (f >= N || rg < 0 || ru < 0 || !(needs(rg) || needs(ru))) continue;
-          const float gt = chain(rg), sg = 1.0f / (1.0f + expf(-gt));
-          C[(size_t)gm * ldc + f] = (gt * sg) * chain(ru);
+          const int af = f + tn0 * 128;
+          C[(size_t)gm * ldc + f] = gate(chain(rg), chain(ru), ACT == kGelu ? bias[af] : 0.f, ACT == kGelu ? bias[ff + af] : 0.f);
         } else {
           const int gn = ltn * kTile + c;
           const int r = weight_row(GU, tn, c, nlim, ff);
@@ -609,12 +617,26 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
           int eg[4], eu[4];
           wexp4(c, eg);
           wexp4(c + 64, eu);
+          float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (ACT == kGelu) {
+            const float* b = bias + f + tn0 * 128;
+            if (by4 && f + 3 < N) {
+              const f32x4 g4 = *reinterpret_cast<const f32x4*>(b), u4 = *reinterpret_cast<const f32x4*>(b + ff);
+#pragma unroll
+              for (int e = 0; e < 4; e++) { bg[e] = g4[e]; bu[e] = u4[e]; }
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; e++) {
+                const int k = min(e, N - 1 - f);
+                bg[e] = b[k];
+                bu[e] = b[ff + k];
+              }
+            }
+          }
           f32x4 o;
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const float gt = ldexpf(acc[i][j][4 * g + e], -(em + eg[e])), sg = 1.0f / (1.0f + expf(-gt));
-            o[e] = (gt * sg) * ldexpf(acc[i][j + 2][4 * g + e], -(em + eu[e]));
-          }
+          for (int e = 0; e < 4; e++)
+            o[e] = gate(ldexpf(acc[i][j][4 * g + e], -(em + eg[e])), ldexpf(acc[i][j + 2][4 * g + e], -(em + eu[e])), bg[e], bu[e]);
           float* dst = C + (size_t)gm * ldc + f;
           if (wide && f + 3 < N) {
             *reinterpret_cast<f32x4*>(dst) = o;
@@ -672,8 +694,9 @@ int64_t cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // plain: C[M][N]; parts (S_out != nullptr): C is the caller's [S][M][N]; gated: N = features, C[M][N] the activation
 // aimg_in: the activation image of A made before (tlhip_rmsnorm_res_parts_aimage), or nullptr: made here
 int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, int64_t M, int64_t N, int64_t K,
-                   size_t parts_bytes, int* S_out, bool gu, const void* aimg_in = nullptr) {
+                   size_t parts_bytes, int* S_out, int act, const void* aimg_in = nullptr, const float* bias = nullptr) {
   TLHIP_REQUIRE_READY();
+  const bool gu = act != f16t::kPlain;
   const bool want_parts = S_out != nullptr;
   if (!A || !image || !exps || !C) return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt: null pointer");
   if (M <= 0 || N <= 0 || K <= 0 || (K % f16t::kBK) != 0 || K > 256 * 4 * f16t::kRowRegs)
@@ -768,10 +791,10 @@ int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, 
     const dim3 grid((unsigned)nblk, (unsigned)S);
     auto launch = [&](auto fn) -> hipError_t {
       // more than 64 KB of LDS per block has to be asked for once per kernel (and device); the
-      // four kernels share this one lambda instantiation (same function-pointer type), so the
-      // note of who has asked is kept per kernel: [gated][tile height - 1]
-      static int asked[2][2] = {{-1, -1}, {-1, -1}};
-      int& asked_on_ = asked[gu ? 1 : 0][P.tmh - 1];
+      // six kernels share this one lambda instantiation (same function-pointer type), so the
+      // note of who has asked is kept per kernel: [activation][tile height - 1]
+      static int asked[3][2] = {{-1, -1}, {-1, -1}, {-1, -1}};
+      int& asked_on_ = asked[act][P.tmh - 1];
       if (asked_on_ != c.device) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)((size_t)f16t::kRing * (2 * 128 * P.tmh * f16t::kRowBytes + f16t::kWImage)));
@@ -780,16 +803,22 @@ int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, 
       }
       fn<<<grid, dim3(512), lds, c.stream>>>(aimg, static_cast<const char*>(image), dst, (int)M, (int)pn, (int)nslab,
                                              part_slabs, ldc, (int)P.tn0, (int)N, ea, static_cast<const int8_t*>(exps),
-                                             (int)f16t::exps_pad(gu ? 2 * N : N), pa);
+                                             (int)f16t::exps_pad(gu ? 2 * N : N), pa, bias);
       return hipSuccess;
     };
-    const hipError_t e = P.tmh == 2 ? (gu ? launch(f16t::gemm_f16t_kernel<2, true>) : launch(f16t::gemm_f16t_kernel<2, false>))
-                                  : (gu ? launch(f16t::gemm_f16t_kernel<1, true>) : launch(f16t::gemm_f16t_kernel<1, false>));
+    const auto pick = [&](auto two, auto one) { return P.tmh == 2 ? launch(two) : launch(one); };
+    const hipError_t e = act == f16t::kPlain    ? pick(f16t::gemm_f16t_kernel<2, f16t::kPlain>, f16t::gemm_f16t_kernel<1, f16t::kPlain>)
+                         : act == f16t::kSwiglu ? pick(f16t::gemm_f16t_kernel<2, f16t::kSwiglu>, f16t::gemm_f16t_kernel<1, f16t::kSwiglu>)
+                                                : pick(f16t::gemm_f16t_kernel<2, f16t::kGelu>, f16t::gemm_f16t_kernel<1, f16t::kGelu>);
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(LDS)");
     if (S > 1 && !want_parts) {
       const size_t total4 = (size_t)M * pn / 4;
       const dim3 sgrid((unsigned)((total4 + 255) / 256));
-      if (gu)
+      if (act == f16t::kGelu)
+        splitk_sum_geglu_kernel<<<sgrid, dim3(256), 0, c.stream>>>(
+            reinterpret_cast<const float4*>(dst), reinterpret_cast<float4*>(pc + n0), (int)M, (int)(pn / 4), (int)(part_w / 4), (int)(N / 4), S,
+            64 / 4, reinterpret_cast<const float4*>(bias + n0), reinterpret_cast<const float4*>(bias + N + n0));
+      else if (gu)
         splitk_sum_swiglu_kernel<<<sgrid, dim3(256), 0, c.stream>>>(
             reinterpret_cast<const float4*>(dst), reinterpret_cast<float4*>(pc + n0), (int)M, (int)(pn / 4),
             (int)(part_w / 4), (int)(N / 4), S, 64 / 4);
@@ -844,12 +873,19 @@ int64_t tlhip_gemm_f16w_exps_bytes(int64_t N, int gated) {
 
 int tlhip_gemm_f16w_nt(const void* A, const void* image, const void* exps, void* C, int64_t M, int64_t N,
                        int64_t K) {
-  return gemm_f16w_impl(A, image, exps, C, M, N, K, 0, nullptr, false);
+  return gemm_f16w_impl(A, image, exps, C, M, N, K, 0, nullptr, f16t::kPlain);
 }
 
 int tlhip_gemm_f16w_nt_swiglu(const void* A, const void* image, const void* exps, void* act, int64_t M,
                               int64_t ff, int64_t K) {
-  return gemm_f16w_impl(A, image, exps, act, M, ff, K, 0, nullptr, true);
+  return gemm_f16w_impl(A, image, exps, act, M, ff, K, 0, nullptr, f16t::kSwiglu);
+}
+
+int tlhip_gemm_f16w_nt_geglu(const void* A, const void* aimage, const void* image, const void* exps, const void* bias, void* act, int64_t M,
+                             int64_t ff, int64_t K) {
+  if (!bias) return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt_geglu: null bias");
+  if (!aligned16(bias)) return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt_geglu: bias must be 16-byte aligned");
+  return gemm_f16w_impl(A, image, exps, act, M, ff, K, 0, nullptr, f16t::kGelu, aimage, static_cast<const float*>(bias));
 }
 
 int64_t tlhip_gemm_f16w_aimage_bytes(int64_t M, int64_t K) {
@@ -889,13 +925,13 @@ int tlhip_rmsnorm_res_parts_aimage(const void* x, const void* parts, int64_t S, 
 int tlhip_gemm_f16w_nt_aimage(const void* A, const void* aimage, const void* image, const void* exps, void* C,
                               int64_t M, int64_t N, int64_t K) {
   if (!aimage) return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt_aimage: null activation image");
-  return gemm_f16w_impl(A, image, exps, C, M, N, K, 0, nullptr, false, aimage);
+  return gemm_f16w_impl(A, image, exps, C, M, N, K, 0, nullptr, f16t::kPlain, aimage);
 }
 
 int tlhip_gemm_f16w_nt_swiglu_aimage(const void* A, const void* aimage, const void* image, const void* exps,
                                      void* act, int64_t M, int64_t ff, int64_t K) {
   if (!aimage) return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt_swiglu_aimage: null activation image");
-  return gemm_f16w_impl(A, image, exps, act, M, ff, K, 0, nullptr, true, aimage);
+  return gemm_f16w_impl(A, image, exps, act, M, ff, K, 0, nullptr, f16t::kSwiglu, aimage);
 }
 
 int tlhip_gemm_f16w_nt_parts_aimage(const void* A, const void* aimage, const void* image, const void* exps,
@@ -904,7 +940,7 @@ int tlhip_gemm_f16w_nt_parts_aimage(const void* A, const void* aimage, const voi
   if (M > 0 && N > 0 && parts_bytes < (int64_t)(M * N * sizeof(float)))
     return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt_parts_aimage: the buffer must hold at least one [M, N] part");
   *n_parts = 0;
-  return gemm_f16w_impl(A, image, exps, parts, M, N, K, (size_t)parts_bytes, n_parts, false, aimage);
+  return gemm_f16w_impl(A, image, exps, parts, M, N, K, (size_t)parts_bytes, n_parts, f16t::kPlain, aimage);
 }
 
 int tlhip_gemm_f16w_nt_parts(const void* A, const void* image, const void* exps, void* parts,
@@ -913,7 +949,7 @@ int tlhip_gemm_f16w_nt_parts(const void* A, const void* image, const void* exps,
   if (M > 0 && N > 0 && parts_bytes < (int64_t)(M * N * sizeof(float)))
     return fail(TLHIP_EINVAL, "tlhip_gemm_f16w_nt_parts: the buffer must hold at least one [M, N] part");
   *n_parts = 0;
-  return gemm_f16w_impl(A, image, exps, parts, M, N, K, (size_t)parts_bytes, n_parts, false);
+  return gemm_f16w_impl(A, image, exps, parts, M, N, K, (size_t)parts_bytes, n_parts, f16t::kPlain);
 }
 
 }  // extern "C"

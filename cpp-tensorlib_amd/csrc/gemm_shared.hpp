@@ -50,6 +50,8 @@ __global__ void splitk_sum_kernel(const float4* __restrict__ part, float4* __res
                                   int ldc4, int S);
 __global__ void splitk_sum_swiglu_kernel(const float4* __restrict__ part, float4* __restrict__ out, int M,
                                          int pf4, int nv4, int ldc4, int S, int hw4);
+__global__ void splitk_sum_geglu_kernel(const float4* __restrict__ part, float4* __restrict__ out, int M, int pf4, int nv4, int ldc4, int S,
+                                        int hw4, const float4* __restrict__ bg, const float4* __restrict__ bu);
 __global__ void row_exponent_f32_kernel(const float* __restrict__ A, int K, int* __restrict__ ea);
 __global__ void row_exponent_bf16_kernel(const uint16_t* __restrict__ W, int K, int8_t* __restrict__ ew);
 

@@ -20,6 +20,7 @@
 // fragment. Global loads of the next slab are in flight while the current one is
 // multiplied.
 #include "gemm_shared.hpp"
+#include "gemv_shared.hpp"
 
 namespace tlhip {
 
@@ -467,6 +468,20 @@ __global__ __launch_bounds__(256) void splitk_sum_swiglu_kernel(const float4* __
   o.z = (g.z * (1.0f / (1.0f + expf(-g.z)))) * u.z;
   o.w = (g.w * (1.0f / (1.0f + expf(-g.w)))) * u.w;
   out[m * ldc4 + f4] = o;
+}
+
+// The same with biases and the GELU gate: bg, bu = the biases of the piece's gate and up features.
+__global__ __launch_bounds__(256) void splitk_sum_geglu_kernel(const float4* __restrict__ part, float4* __restrict__ out, int M, int pf4, int nv4,
+                                                               int ldc4, int S, int hw4, const float4* __restrict__ bg,
+                                                               const float4* __restrict__ bu) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)M * pf4) return;
+  const size_t m = i / pf4;
+  const int f4 = (int)(i - m * pf4);
+  const size_t gi = m * nv4 + (size_t)(f4 / hw4) * 2 * hw4 + f4 % hw4, total = (size_t)M * nv4;
+  const GateUp4 gu = sum_parts(S, [&](int s) { return GateUp4{part[s * total + gi], part[s * total + gi + hw4]}; });
+  const float4 g = plus(gu.g, bg[f4]), u = plus(gu.u, bu[f4]);
+  out[m * ldc4 + f4] = make_float4(gelu_tanh(g.x) * u.x, gelu_tanh(g.y) * u.y, gelu_tanh(g.z) * u.z, gelu_tanh(g.w) * u.w);
 }
 
 void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t part_w, int64_t ldc, int S, int half) {

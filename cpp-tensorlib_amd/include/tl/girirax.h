@@ -469,7 +469,7 @@ inline bool chunk_layers(model& M, int64_t T, float* layer_out = nullptr) {
     ok = ok && gemm_parts(L.wout, P.y, P.parts, P.parts_bytes, T, &np) &&
          hip::postnorm_res_parts(P.res, P.parts, np, nullptr, L.norm1, P.res, WP, M.eps, T, L.mlp ? L.gate_up.N : next);
     if (L.mlp)
-      ok = ok && gemm(L.gate_up, P.res, P.gu, T) && hip::geglu_rows(P.gu, L.gate_up_b, P.act, L.down.K, T) &&
+      ok = ok && gemm_geglu(L.gate_up, P.res, L.gate_up_b, P.gu, P.act, T) &&
            gemm_parts(L.down, P.act, P.parts, P.parts_bytes, T, &np) &&
            hip::postnorm_res_parts(P.res, P.parts, np, L.down_b, L.norm2, P.res, WP, M.eps, T, next);
     if (ok && layer_out) {

@@ -169,6 +169,7 @@ struct api {
                                 void*, int64_t, int64_t, int64_t, float) = nullptr;
   int (*gemv_bf16_row_rmsnorm_gateup)(const void*, const void*, const void*, void*, const void*, void*,
                                       int64_t, int64_t, float) = nullptr;
+  int (*gemm_f16w_nt_geglu)(const void*, const void*, const void*, const void*, const void*, void*, int64_t, int64_t, int64_t) = nullptr;
   int64_t (*gemm_f16w_aimage_bytes)(int64_t, int64_t) = nullptr;
   int (*rmsnorm_res_parts_aimage)(const void*, const void*, int64_t, const void*, void*, void*, int64_t, float,
                                   int64_t, void*) = nullptr;
@@ -411,6 +412,7 @@ struct context {
               bind(f.gemv_bf16_row_rmsnorm, "tlhip_gemv_bf16_row_rmsnorm") &&
               bind(f.gemv_q4_rmsnorm_gateup, "tlhip_gemv_q4_rmsnorm_gateup") &&
               bind(f.gemv_bf16_row_rmsnorm_gateup, "tlhip_gemv_bf16_row_rmsnorm_gateup") &&
+              bind(f.gemm_f16w_nt_geglu, "tlhip_gemm_f16w_nt_geglu") &&
               bind(f.gemm_f16w_aimage_bytes, "tlhip_gemm_f16w_aimage_bytes") &&
               bind(f.rmsnorm_res_parts_aimage, "tlhip_rmsnorm_res_parts_aimage") &&
               bind(f.gemm_f16w_nt_aimage, "tlhip_gemm_f16w_nt_aimage") &&
@@ -1828,6 +1830,22 @@ inline bool geglu_rows(void* gu, void* bias, void* out, int64_t ff, int64_t rows
   L.reads(gu, bias);
   L.writes(out);
   return L.sent(L.lib.geglu_rows(gu, bias, out, ff, rows));
+}
+// act[m][f] = gelu_tanh(a_m . gate_f + bias[f]) (a_m . up_f + bias[ff + f]) for the fused [gate | up] bf16 weight B: in the product's
+// own epilogue where it runs over the weight's prepared form, else by a launch over the products in gu [m, 2 ff].
+inline bool gemm_bf16_nt_geglu(void* a, void* B, void* bias, void* gu, void* act, int64_t m, int64_t ff, int64_t k) {
+  if (prompt_product_is_large(m, 2 * ff, k) && m > 0 && ff > 0 && (k % 8) == 0) {
+    launch L;
+    if (!L.ok) return false;
+    L.reads(a, B);
+    L.reads(bias);
+    L.writes(act);
+    if (const auto* p = L.prepared(B, ff, k, true)) {
+      if (L.sent(L.lib.gemm_f16w_nt_geglu(a, L.act_of(a, m, k), p->image, p->exps, bias, act, m, ff, k))) return true;
+      L.refused(B, p);
+    }
+  }
+  return gemm_bf16_nt(a, B, gu, m, 2 * ff, k) && geglu_rows(gu, bias, act, ff, m);
 }
 inline bool embed_scaled(void* table, int64_t ldt, void* tokens, void* out, int64_t T, int64_t width, int64_t ld, int64_t vocab,
                          float scale) {

@@ -61,6 +61,11 @@ inline bool gemm_swiglu(const linear& L, void* a, void* act, int64_t T) {
   return hip::gemm_bf16_nt_swiglu(a, L.w, act, T, L.N / 2, L.K);
 }
 
+// The same with biases (f32 [N]) and the GELU gate, bf16 rows; gu: room for the [T, N] products
+inline bool gemm_geglu(const linear& L, void* a, void* bias, void* gu, void* act, int64_t T) {
+  return L.fmt == wfmt::bf16_row && hip::gemm_bf16_nt_geglu(a, L.w, bias, gu, act, T, L.N / 2, L.K);
+}
+
 // y = W . swiglu(gu)
 inline bool gemv_swiglu(const linear& L, void* gu, void* y) {
   if (L.fmt == wfmt::q4) {

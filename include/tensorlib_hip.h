@@ -402,8 +402,8 @@ int tlhip_gemm_bf16_nt_swiglu(const void* A, const void* W, void* act, int64_t M
  *     so each weight is exact unless it is one of the counted ones (then its absolute error is below
  *     2^-40 of the row's largest).
  * gated != 0: W = [gate rows | up rows], [2*N, K], N = features (the operand of
- * tlhip_gemm_bf16_nt_swiglu); the image then serves tlhip_gemm_f16w_nt_swiglu only, a plain image
- * the other two. K % 32 == 0.
+ * tlhip_gemm_bf16_nt_swiglu); the image then serves tlhip_gemm_f16w_nt_swiglu and _geglu only, a plain
+ * image the other two. K % 32 == 0.
  * The products cut every activation row, scaled the same way, into two f16 terms, both rounded to
  * nearest (2^-24 relative), and run two matrix-core products per weight instead of three, fp32
  * sums, the result scaled back exactly: the error is that of one fp32 rounding per product, as in
@@ -446,6 +446,10 @@ int tlhip_gemm_f16w_nt_parts_aimage(const void* A, const void* aimage, const voi
                                     int* n_parts);
 int tlhip_gemm_f16w_nt_swiglu_aimage(const void* A, const void* aimage, const void* image, const void* exps,
                                      void* act, int64_t M, int64_t ff, int64_t K);
+/* The gated product with biases and the GELU gate over a weight prepared with gated != 0: act[m][f] = gelu_tanh(A_m . gate_f + bias[f])
+ * (A_m . up_f + bias[ff + f]), what tlhip_geglu_rows makes of the plain product. aimage may be NULL. bias: f32 [2 ff], 16-byte aligned. */
+int tlhip_gemm_f16w_nt_geglu(const void* A, const void* aimage, const void* image, const void* exps, const void* bias, void* act,
+                             int64_t M, int64_t ff, int64_t K);
 /* The three prompt-chunk products over an int4 weight (qw = packed nibbles [N][K/2], scales
  * [N][K/32], group 32 - the operand of tlhip_gemv_q4): C = A . dequant(W)^T formed as
  * sum over groups of scale * (A . q) with exact products on the matrix pipe, fp32 sums - the decode

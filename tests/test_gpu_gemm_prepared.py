@@ -326,6 +326,41 @@ def test_gemm_f16w_swiglu_epilogue(lib, orc, M, ff, K):
     P.free()
 
 
+@pytest.mark.parametrize("M,ff,K,far", [
+    (512, 18944, 3584, False),    # 256 whole-round tiles + 40 split over K
+    (300, 1000, 256, False),      # split over K, ragged in M and in the last tile's features
+    (65, 130, 64, False),         # ff % 4 != 0: never split, biases one by one
+    (70, 4, 32, False),           # one group of columns
+    (130, 200, 64, True),         # rows whose results are worked out again
+])
+def test_gemm_f16w_geglu_epilogue(lib, orc, M, ff, K, far):
+    """gelu_tanh(A . Wg^T + bg) (A . Wu^T + bu) from the prepared weight against the oracle's products gated in float64, the GEMM's
+    tolerance on each product carried through the gate (|gelu'| < 1.13), and 4 ulp for the gate's own arithmetic."""
+    print("case gemm_f16w geglu", M, ff, K, flush=True)
+    A = orc.normal(M * K, 53).reshape(M, K).copy()
+    if far:
+        A[::3, 1] *= np.float32(2.0 ** 26)
+    Wb = orc.to_bf16(orc.normal(2 * ff * K, 54, std=0.05)).reshape(2 * ff, K)
+    bias = orc.normal(2 * ff, 55, std=0.5)
+    P = Prepared(lib, Wb, gated=True)
+    da, db, act = lib.to_device(A), lib.to_device(bias), lib.empty((M, ff))
+    rows = [0, 1, M // 2, M - 1]
+    p = orc.gemm_bf16_nt(np.ascontiguousarray(A[rows]), Wb)
+    g, u = p[:, :ff].astype(np.float64) + bias[:ff], p[:, ff:].astype(np.float64) + bias[ff:]
+    gelu = g / (1.0 + np.exp(np.minimum(-1.5957691216057308 * (g + 0.044715 * g ** 3), 700.0)))
+    dg, du = RTOL * np.abs(p[:, :ff]) + ATOL, RTOL * np.abs(p[:, ff:]) + ATOL
+    tol = 1.13 * np.abs(u) * dg + (np.abs(gelu) + 1.13 * dg) * du + 4 * 2.0 ** -23 * np.abs(gelu * u) + ATOL
+    lib.gemm_f16w_nt_geglu(da, P.image, P.exps, db, act, M, ff, K)
+    got = act.numpy()
+    assert np.all(np.isfinite(got)) and np.all(np.abs(got[rows] - gelu * u) <= tol), maxrel(got[rows], gelu * u)
+    assert lib.c.tlhip_gemm_f16w_nt_geglu(da.ptr, None, P.image.ptr, P.exps.ptr, None, act.ptr, M, ff, K) == -2
+    assert lib.c.tlhip_gemm_f16w_nt_geglu(da.ptr, None, P.image.ptr, P.exps.ptr, db.ptr + 4, act.ptr, M, ff, K) == -2
+    lib.last_error()
+    for b in (da, db, act):
+        b.free()
+    P.free()
+
+
 def test_gemm_f16w_swiglu_exact_cases(lib, orc):
     """A gate product large enough that sigmoid rounds to 1 gives act = g * up exactly; with a
     one-hot A row both products are weight entries, so every (row, feature) pair must land where its
