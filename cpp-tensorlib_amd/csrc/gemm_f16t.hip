@@ -21,7 +21,7 @@
 // The GEMM then has no vector ALU work and no address arithmetic in its loop: a slab is 48
 // contiguous kilobytes, copied by 48 global_load_lds_dwordx4 (1 KB each, whole cache lines, no
 // registers), six per wavefront. A block is eight wavefronts (4 x 2) on a 256 x 256 tile, 64 x 128
-// per wavefront (128 x 256 and 32 x 128 where N is small), one block per CU, a ring of three slabs
+// per wavefront (or 128 x 256 and 32 x 128: gemm_f16w_impl chooses), one block per CU, a ring of three slabs
 // in LDS (144 KB), one barrier per slab; a copy has two slab times to land. Products of f16 are exact in fp32, the MFMA sums in fp32, and
 // the result leaves as acc * 2^-(ea[m] + ew[n]), an exact scaling: the error is fp32 summation
 // error plus one fp32-rounding-sized term per product, as in the reference's fp32 FMA loop
@@ -712,35 +712,58 @@ int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, 
   const int64_t slots = c.cus;                      // one block per CU
   const int64_t tm256 = cdiv64(M, 256), tm128 = cdiv64(M, 128);
   const bool can_split = (N % 4) == 0;              // the part sums work on float4s
-  // Work is shaped to whole rounds of the block slots, as in tlhip_gemm_bf16_nt: fewer tiles than
-  // slots -> K split so that tiles * S comes close to the slots; more -> the columns that make
-  // whole rounds with full K, the remaining columns split over K in a second launch. A piece runs
-  // on 256-row tiles unless those would leave more than half of the CUs to K splits; then on
-  // 128-row tiles: twice the tiles, half the splits, half the parts to write and add up.
+  // A piece is a range of tile columns in tiles of one height, K split S ways. What a launch of one takes (us), fitted to 4079 runs of
+  // 100 to 1024 rows, 4 to 200 tile columns, K 1024 to 18944 (error 5 % and 3.5 %): a start, for every round of the CUs a block's own
+  // start and end and its slabs - slower the more CUs are busy: their clock falls - and the megabytes stored.
   struct Piece { int64_t tn0, tcols; int S; int tmh; };
+  struct Cost { double start, block, slab, busy, mb; };
+  static constexpr Cost kCost[2] = {{2.0, 8.7, 0.527, 0.335, 0.104}, {4.4, 11.9, 1.108, 0.545, 0.137}};   // tiles of 128 and of 256 rows
+  const auto piece_us = [&](int64_t tcols, int tmh, int64_t S) {
+    const Cost& k = kCost[tmh - 1];
+    const int64_t blocks = (tmh == 1 ? tm128 : tm256) * tcols * S;
+    const double slabs = (double)cdiv64(nslab, S), rest = (double)(blocks % slots) / (double)slots, mb = 4e-6 * (double)M * f16t::kTile * (double)tcols;
+    double us = k.start + (double)(blocks / slots) * (k.block + slabs * (k.slab + k.busy)) + k.mb * (double)S * mb;
+    if (rest > 0) us += k.block + slabs * (k.slab + k.busy * rest);
+    // parts are read by what adds them up: a launch of its own, or a norm that is there anyway, a few rows to a CU and less able
+    // to hide it (nine parts for four of 512 x 3584 cost it 14 us)
+    return us + (S > 1 ? (want_parts ? 0.35 * (double)S * mb : 2.5 + 0.12 * (double)(S + 1) * mb) : 0.0);
+  };
+  // The columns from tn0 on in one piece, as it takes least.
+  const auto best = [&](int64_t tn0, double& us) {
+    Piece P{tn0, tn - tn0, 1, 1};
+    us = piece_us(P.tcols, 1, 1);
+    for (int tmh = 1; tmh <= 2; tmh++)
+      for (int64_t want = 1; want <= (can_split ? 16 : 1) && (want == 1 || nslab / want >= 8); want++) {   // at least 256 k per part
+        const int64_t S = cdiv64(nslab, cdiv64(nslab, want));
+        if (want_parts && S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) break;
+        const double t = piece_us(P.tcols, tmh, S);
+        if (t < us) us = t, P.S = (int)S, P.tmh = tmh;
+      }
+    return P;
+  };
+  // One piece, or the columns that make whole rounds of the CUs without a split and the others as a second one: 512 x 16640 x 3584
+  // 64 columns of 128-row tiles and one split 14 ways (118 us) where 130 blocks of 256 rows took 159 to 176.
   Piece pieces[2];
-  int npieces = 0;
-  auto pick_S = [&](int64_t t) {
-    if (!can_split || t >= slots) return 1;
-    int64_t S = slots / t;
-    if (S > 16) S = 16;
-    while (S > 1 && nslab / S < 8) S--;             // at least 256 k per part
-    if (want_parts)
-      while (S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) S--;
-    return (int)S;
-  };
-  auto piece = [&](int64_t tn0, int64_t tcols, bool split) {
-    const int tmh = tm256 * tcols * 2 <= slots ? 1 : 2;
-    return Piece{tn0, tcols, split ? pick_S((tmh == 1 ? tm128 : tm256) * tcols) : 1, tmh};
-  };
-  const int64_t cols_per_round = slots / tm256;
-  if (tm256 * tn <= slots || cols_per_round == 0 || !can_split || want_parts) {
-    pieces[npieces++] = piece(0, tn, true);
-  } else {
-    const int64_t main_tn = tn / cols_per_round * cols_per_round;
-    pieces[npieces++] = Piece{0, main_tn, 1, 2};
-    if (main_tn < tn) pieces[npieces++] = piece(main_tn, tn - main_tn, true);
-  }
+  int npieces = 1;
+  double least;
+  pieces[0] = best(0, least);
+  if (!want_parts && can_split)
+    for (int tmh = 1; tmh <= 2; tmh++) {
+      const int64_t per_round = slots / (tmh == 1 ? tm128 : tm256);
+      if (per_round == 0) continue;
+      for (int64_t back = 0; back < 2; back++) {   // as many rounds as there are, or one fewer
+        const int64_t cols = (tn / per_round - back) * per_round;
+        if (cols <= 0 || cols >= tn) continue;
+        double rest;
+        const Piece tail = best(cols, rest);
+        if (piece_us(cols, tmh, 1) + rest < least) {
+          least = piece_us(cols, tmh, 1) + rest;
+          pieces[0] = Piece{0, cols, 1, tmh};
+          pieces[1] = tail;
+          npieces = 2;
+        }
+      }
+    }
   // scratch: exponents of A's rows, the slab images of A, room for the largest piece's parts
   const size_t ea_bytes = ((size_t)M * sizeof(int) + 1023) & ~(size_t)1023;
   const int64_t timg = cdiv64(M, f16t::kTile);      // activation images are 256 rows tall

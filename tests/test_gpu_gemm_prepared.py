@@ -45,6 +45,9 @@ class Prepared:
     (1, 64, 32),           # one row
     (65, 129, 96),         # N % 4 != 0: never split; ragged everywhere
     (1000, 256, 18944),    # long K at the 7B down shape's depth
+    (512, 16600, 896),     # a round of 128-row tiles with full K, one column tile split
+    (1000, 9000, 1024),    # the same, ragged in M and N, four column tiles split
+    (129, 37000, 1024),    # one row in the second row tile
 ])
 def test_gemm_f16w_matches_oracle(lib, orc, M, N, K):
     """out[M,N] = A[M,K] . W[N,K]^T with A ~ N(0,1), W ~ N(0,0.02) bf16: sampled rows against the
@@ -305,6 +308,7 @@ def test_gemm_f16w_parts_feed_the_residual_norm(lib, orc, M, N, K, room):
     (512, 4864, 896),      # 0.5B chunk
     (200, 1000, 256),      # ragged in M and in the last tile's features
     (65, 130, 64),         # ff % 4 != 0: never split
+    (512, 8300, 896),      # a round of 128-row tiles, one column tile split
 ])
 def test_gemm_f16w_swiglu_epilogue(lib, orc, M, ff, K):
     """act = swiglu(A . Wg^T, A . Wu^T) from the prepared [gate rows | up rows] weight: sampled rows
@@ -331,6 +335,7 @@ def test_gemm_f16w_swiglu_epilogue(lib, orc, M, ff, K):
     (300, 1000, 256, False),      # split over K, ragged in M and in the last tile's features
     (65, 130, 64, False),         # ff % 4 != 0: never split, biases one by one
     (70, 4, 32, False),           # one group of columns
+    (512, 8300, 896, False),      # a round of 128-row tiles, one column tile split
     (130, 200, 64, True),         # rows whose results are worked out again
 ])
 def test_gemm_f16w_geglu_epilogue(lib, orc, M, ff, K, far):
