@@ -4,8 +4,8 @@
 // chain of latencies of one block. gemm_bf16_nt_kernel (prefill.hip) walks K in slabs of 32 through LDS, two
 // barriers and one load round trip per slab: ten slabs were 20 us for weights that take 2 us to read. Here a
 // block has no barrier until its sums are complete: its eight wavefronts split the block's K range between
-// them (wavefront w takes the 32-k steps w, w + 8, ...), each with the WHOLE tile's accumulators, and loads
-// both operands straight into the registers of the MFMA that uses them, several steps ahead. The sums meet in
+// them (wavefront w takes the 32-k steps w, w + 8, ...), each with the WHOLE tile's accumulators; weights go straight
+// into the registers of the MFMA that uses them, activations through slots of LDS of the wavefront's own. The sums meet in
 // LDS once at the end, in a fixed order.
 //
 // Both operands of v_mfma_f32_16x16x32_bf16 are K-contiguous per lane: lane l supplies row l % 16 and k
@@ -35,10 +35,19 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 8, kStep = 32;
 constexpr int kMaxTM = 5;
 
-// Steps of activations in flight per wavefront (int4: a divisor of four): 2 KB of LDS per row tile each.
-__host__ __device__ constexpr int stages(int TM, bool q4) { return TM <= 2 ? 4 : TM == 3 && !q4 ? 3 : 2; }
-__host__ __device__ constexpr int lds_bytes(int TM, int TN, bool q4) {
-  const int ring = kWaves * stages(TM, q4) * TM * 2048, sums = 4 * 16 * TM * (16 * TN + 4) * 4;
+// int4: steps of activations in flight per wavefront (a divisor of four), 2 KB of LDS per row tile each
+__host__ __device__ constexpr int stages(int TM) { return TM <= 2 ? 4 : 2; }
+__host__ __device__ constexpr int lds_bytes_q4(int TM, int TN) {
+  const int ring = kWaves * stages(TM) * TM * 2048, sums = 4 * 16 * TM * (16 * TN + 4) * 4;
+  return ring > sums ? ring : sums;
+}
+// bf16: steps of activations in flight - one, or where a step's loads are few, two and four (8 x 446 x 12032 34.0 -> 28.5 us) -
+// and the sums of all wavefronts. Rows of four column tiles lie without padding, their 16-byte chunks XORed with the row (160 KB
+// at five row tiles).
+__host__ __device__ constexpr int steps_ahead(int TM, int TN) { return TM == 1 && TN <= 2 ? 4 / TN : 1; }
+__host__ __device__ constexpr int sum_stride(int TN) { return TN == 4 ? 16 * TN : 16 * TN + 4; }
+__host__ __device__ constexpr int lds_bytes_bf16(int TM, int TN) {
+  const int ring = kWaves * steps_ahead(TM, TN) * TM * 2048, sums = kWaves * 16 * TM * sum_stride(TN) * 4;
   return ring > sums ? ring : sums;
 }
 
@@ -76,27 +85,207 @@ __device__ __forceinline__ f32x4 mma(const frag16& a, const frag16& b, f32x4 c) 
 // Grid: x = row blocks (fastest) x column tiles, y = K-split parts of `part_units` units (bf16: steps of 32 k,
 // int4: 128 k); part y goes to C + y * M * ldc. N, ff, GU and the order of a gated tile's columns as in
 // gemm_bf16_nt_kernel: a tile's first 8 TN columns are gate features, the rest the same features' up rows.
-template <int TM, int TN, bool GU, bool Q4, bool RANGED>
-__global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* __restrict__ A, const void* __restrict__ W,
-                                                                  const float* __restrict__ scales, float* __restrict__ C,
-                                                                  int M, int N, int K, int part_units, int ldc, int ff,
-                                                                  int row_blocks) {
-  constexpr int BM = 16 * TM, BN = 16 * TN, LD = BN + 4;
-  constexpr int ST = stages(TM, Q4), kSlot = TM * 2048;
-  extern __shared__ __attribute__((aligned(1024))) float red[];   // activations in flight, then [4][BM][LD] sums
+//
+// What bounds the bf16 kernel: the CU returns loads in the order of their requests, so activations (from L2, read by every
+// block: 2.5 times the weights' bytes at five row tiles over four column tiles) wait behind weights from HBM. 77 x 9728 gated x 896
+// took 14.5 us, 10.0 without the weights' loads, 11.3 without the activations', 8.7 without both, and no less without the
+// matrix instructions. So little is in flight beyond what is needed next - one step of activations, each tile requested again
+// as soon as it is in registers, two steps of weights - and three column tiles (203 blocks instead of 152) are a choice too:
+// 12.3 us. With two steps of activations 13.2, all weights first 12.8. 227 shapes of 1 to 80 rows: 0.98 to 1.4 times as fast.
+template <int TM, int TN, bool GU>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const float* __restrict__ A, const void* __restrict__ W,
+                                                                       float* __restrict__ C, int M, int N, int K, int part_units,
+                                                                       int ldc, int ff, int row_blocks) {
+  constexpr int BM = 16 * TM, BN = 16 * TN, LD = sum_stride(TN), AS = steps_ahead(TM, TN), WS = AS + 1;
+  extern __shared__ __attribute__((aligned(1024))) float red[];   // activations in flight, then [8][BM][LD] sums
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, quarter = lane >> 4;
   // one contiguous run of tiles per XCD, row blocks fastest: those share a weight tile in one L2
   const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int lid = xcd * q8 + min(xcd, r8) + within;
   const int m0 = lid % row_blocks * BM, n0 = lid / row_blocks * BN;
   C += (size_t)blockIdx.y * M * ldc;
-  const int units = Q4 ? K / 128 : K / kStep, ubeg = blockIdx.y * part_units, uend = min(units, ubeg + part_units);
+  const int units = K / kStep, ubeg = blockIdx.y * part_units, uend = min(units, ubeg + part_units);
   const int first = ubeg + wave, mine = first < uend ? (uend - first + kWaves - 1) / kWaves : 0;
 
   // byte offsets of this lane's rows (clamped into the operands: what lies past an edge is not stored). A 1 KB copy
   // of activations is eight rows of 128 bytes, the 16-byte chunks of row r in the order c ^ (r & 7), which spreads
   // the fragment reads (16 rows, one chunk) over the LDS banks.
-  uint32_t aoff[TM][2], woff[TN], soff[Q4 ? TN : 1];
+  uint32_t aoff[TM][2], woff[TN];
+#pragma unroll
+  for (int j = 0; j < TN; j++) {
+    const int col = 16 * j + r16;
+    int r;
+    if (GU) {
+      const int f = min((n0 >> 1) + col % (BN / 2), N - 1);
+      r = f + (col >= BN / 2 ? ff : 0);
+    } else {
+      r = min(n0 + col, N - 1);
+    }
+    woff[j] = (uint32_t)r * (uint32_t)(K * 2) + quarter * 16;
+  }
+#pragma unroll
+  for (int t = 0; t < TM; t++)
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      aoff[t][h] = (uint32_t)min(m0 + 16 * t + 8 * h + (lane >> 3), M - 1) * (uint32_t)(K * 4) + ((lane & 7) ^ (lane >> 3)) * 16;
+  const int frag[2] = {r16 * 128 + ((2 * quarter) ^ (r16 & 7)) * 16, r16 * 128 + ((2 * quarter + 1) ^ (r16 & 7)) * 16};
+  char* slots = reinterpret_cast<char*>(red) + wave * (AS * TM * 2048);
+  const char* Ab = reinterpret_cast<const char*>(A) + (uint32_t)first * 128u;
+  const char* Wb = static_cast<const char*>(W) + (uint32_t)first * 64u;
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int t = 0; t < TM; t++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  frag16 w[WS][TN];
+  auto load_a = [&](char* slot, int t, uint32_t i) {   // row tile t of my i-th step
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(Ab + (aoff[t][h] + i * (kWaves * 128u))),
+                                       (__attribute__((address_space(3))) void*)(slot + t * 2048 + h * 1024), 16, 0, 0);
+  };
+  auto load_w = [&](int u, uint32_t i) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + i * (kWaves * 64u)));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // My i-th step, weights in slot U, activations in `slot`. R: later steps, capped at WS. Requests go out in the order W(0), A(0),
+  // W(1), .., W(AS), then in step i A(i + AS, t) as tile t leaves its slot and W(i + WS) at the end: what is younger than A(i, t)
+  // is counted, and W(i) is older (copies into LDS are waited for by count: the compiler does not see them).
+  auto step = [&](auto U, auto R_, uint32_t i, char* slot) {
+    constexpr int u = decltype(U)::value, R = decltype(R_)::value, ahead = R < AS - 1 ? R : AS - 1;
+    const auto tile = [&](auto T) {
+      constexpr int t = decltype(T)::value;
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (TM - 1 - t) + ahead * (TN + 2 * TM) + (R >= AS ? TN + 2 * t : 0)) : "memory");
+      const char* at = slot + t * 2048;
+      const f32x4 x0 = *reinterpret_cast<const f32x4*>(at + frag[0]), x1 = *reinterpret_cast<const f32x4*>(at + frag[1]);
+      if constexpr (R >= AS) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the copy that takes the slot goes out
+        load_a(slot, t, i + AS);
+      }
+      frag16 p[3];
+      split3(x0, x1, p);
+      // the weights are the first operand: the tile comes out transposed, four consecutive columns of a row to a lane
+#pragma unroll
+      for (int e = 0; e < 3; e++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[t][j] = mma(w[u][j], p[e], acc[t][j]);
+      if (TM * TN >= 12) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
+    };
+    tile(std::integral_constant<int, 0>{});
+    if constexpr (TM > 1) tile(std::integral_constant<int, 1>{});
+    if constexpr (TM > 2) tile(std::integral_constant<int, 2>{});
+    if constexpr (TM > 3) tile(std::integral_constant<int, 3>{});
+    if constexpr (TM > 4) tile(std::integral_constant<int, 4>{});
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (R >= WS) load_w(u, i + WS);
+  };
+  if (mine > 0) {
+    uint32_t i = 0, turn = 0;                      // turn: the slot of activations of step i
+    const auto go = [&](auto U, auto R_) {
+      step(U, R_, i, slots + turn * (TM * 2048));
+      i++;
+      turn = turn + 1 == AS ? 0 : turn + 1;
+    };
+    // N steps, the last ones
+    const auto rest = [&](auto N_, auto self, auto K_) {
+      constexpr int n = decltype(N_)::value, k = decltype(K_)::value;
+      if constexpr (k < n) {
+        go(std::integral_constant<int, k % WS>{}, std::integral_constant<int, (n - 1 - k < WS ? n - 1 - k : WS)>{});
+        self(N_, self, std::integral_constant<int, k + 1>{});
+      }
+    };
+    const auto last = [&](auto N_) { rest(N_, rest, std::integral_constant<int, 0>{}); };
+#pragma unroll
+    for (int q = 0; q < AS; q++)
+      if (q < mine) {
+        load_w(q, q);
+#pragma unroll
+        for (int t = 0; t < TM; t++) load_a(slots + q * (TM * 2048), t, q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    if (AS < mine) load_w(AS, AS);
+    while ((int)i + 2 * WS <= mine) {
+      go(std::integral_constant<int, 0>{}, std::integral_constant<int, WS>{});
+      go(std::integral_constant<int, 1>{}, std::integral_constant<int, WS>{});
+      if constexpr (WS > 2) go(std::integral_constant<int, 2>{}, std::integral_constant<int, WS>{});
+      if constexpr (WS > 3) go(std::integral_constant<int, 3>{}, std::integral_constant<int, WS>{});
+      if constexpr (WS > 4) go(std::integral_constant<int, 4>{}, std::integral_constant<int, WS>{});
+    }
+    static_assert(WS <= 5, "steps left below");
+    switch (mine - (int)i) {                       // 1 .. 2 WS - 1
+      case 1: last(std::integral_constant<int, 1>{}); break;
+      case 2: last(std::integral_constant<int, 2>{}); break;
+      case 3: last(std::integral_constant<int, 3>{}); break;
+      case 4: if constexpr (WS > 2) last(std::integral_constant<int, 4>{}); break;
+      case 5: if constexpr (WS > 2) last(std::integral_constant<int, 5>{}); break;
+      case 6: if constexpr (WS > 3) last(std::integral_constant<int, 6>{}); break;
+      case 7: if constexpr (WS > 3) last(std::integral_constant<int, 7>{}); break;
+      case 8: if constexpr (WS > 4) last(std::integral_constant<int, 8>{}); break;
+      case 9: if constexpr (WS > 4) last(std::integral_constant<int, 9>{}); break;
+    }
+  }
+
+  // acc[t][j] of lane l: row 16 t + l % 16, columns 16 j + 4 (l / 16) ..; every wavefront's into LDS, the eight added up
+  auto at = [&](int of, int row, int c4) { return red + ((size_t)of * BM + row) * LD + (TN == 4 ? c4 ^ (row & 7) : c4) * 4; };
+  __syncthreads();                                 // (the sums take the place of activations that other wavefronts read)
+#pragma unroll
+  for (int t = 0; t < TM; t++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) *reinterpret_cast<f32x4*>(at(wave, 16 * t + r16, 4 * j + quarter)) = acc[t][j];
+  __syncthreads();
+  const bool wide = (ldc & 3) == 0;
+  auto total = [&](int row, int c4) {
+    f32x4 x[kWaves];
+#pragma unroll
+    for (int v = 0; v < kWaves; v++) x[v] = *reinterpret_cast<const f32x4*>(at(v, row, c4));
+    return ((x[0] + x[4]) + (x[1] + x[5])) + ((x[2] + x[6]) + (x[3] + x[7]));
+  };
+  auto store = [&](float* dst, const f32x4& o, int left) {
+    if (wide && left >= 4) {
+      *reinterpret_cast<f32x4*>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (e < left) dst[e] = o[e];
+    }
+  };
+  if (GU && gridDim.y == 1) {
+    for (int i = tid; i < BM * (BN / 8); i += 64 * kWaves) {
+      const int row = i / (BN / 8), c4 = i % (BN / 8), gm = m0 + row, f = (n0 >> 1) + 4 * c4;
+      if (gm >= M || f >= N) continue;
+      const f32x4 g = total(row, c4), up = total(row, c4 + BN / 8);
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] = (g[e] * (1.0f / (1.0f + expf(-g[e])))) * up[e];   // swiglu_kernel's arithmetic
+      store(C + (size_t)gm * ldc + f, o, N - f);
+    }
+  } else {
+    for (int i = tid; i < BM * (BN / 4); i += 64 * kWaves) {
+      const int row = i / (BN / 4), c4 = i % (BN / 4), gm = m0 + row, gn = n0 + 4 * c4;
+      if (gm >= M || (!GU && gn >= N)) continue;   // gated parts are whole tiles wide
+      store(C + (size_t)gm * ldc + gn, total(row, c4), GU ? 4 : N - gn);
+    }
+  }
+}
+
+template <int TM, int TN, bool GU, bool RANGED>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_q4_kernel(const float* __restrict__ A, const void* __restrict__ W,
+                                                                     const float* __restrict__ scales, float* __restrict__ C, int M,
+                                                                     int N, int K, int part_units, int ldc, int ff, int row_blocks) {
+  constexpr int BM = 16 * TM, BN = 16 * TN, LD = BN + 4;
+  constexpr int ST = stages(TM), kSlot = TM * 2048;
+  extern __shared__ __attribute__((aligned(1024))) float red[];   // activations in flight, then [4][BM][LD] sums
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, quarter = lane >> 4;
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
+  const int lid = xcd * q8 + min(xcd, r8) + within;
+  const int m0 = lid % row_blocks * BM, n0 = lid / row_blocks * BN;
+  C += (size_t)blockIdx.y * M * ldc;
+  const int units = K / 128, ubeg = blockIdx.y * part_units, uend = min(units, ubeg + part_units);
+  const int first = ubeg + wave, mine = first < uend ? (uend - first + kWaves - 1) / kWaves : 0;
+
+  uint32_t aoff[TM][2], woff[TN], soff[TN];        // as above
 #pragma unroll
   for (int t = 0; t < TM; t++)
 #pragma unroll
@@ -114,8 +303,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
     } else {
       r = min(n0 + col, N - 1);
     }
-    woff[j] = (uint32_t)r * (uint32_t)(Q4 ? K / 2 : K * 2) + quarter * 16;
-    if (Q4) soff[j] = (uint32_t)r * (uint32_t)(K / 8);
+    woff[j] = (uint32_t)r * (uint32_t)(K / 2) + quarter * 16;
+    soff[j] = (uint32_t)r * (uint32_t)(K / 8);
   }
   const char* Ab = reinterpret_cast<const char*>(A);
   const char* Wb = static_cast<const char*>(W);
@@ -150,141 +339,95 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
       }
       split3(x0, x1, p);
     };
-    if constexpr (!Q4) {
-      frag16 w[ST][TN];
-      auto load = [&](int u, int i) {              // slot u takes my i-th step
-        const uint32_t step = (uint32_t)(first + kWaves * i);
-        load_a(u, step);
+    // a unit is four steps; W and the scales of the next unit and the activations of the next steps are on
+    // their way while one is multiplied
+    frag16 w[2][TN];
+    f32x4 s[2][TN];
+    auto load_w = [&](int u, int i) {
+      const uint32_t unit = (uint32_t)(first + kWaves * i);
 #pragma unroll
-        for (int j = 0; j < TN; j++) w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + step * 64u));
-        __builtin_amdgcn_sched_barrier(0);         // (else the compiler gathers the loads of all slots behind the last one's products)
-      };
-      auto compute = [&](int u) {
-#pragma unroll
-        for (int t = 0; t < TM; t++) {
-          frag16 p[3];
-          cut(u, t, p);
-#pragma unroll
-          for (int e = 0; e < 3; e++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) acc[t][j] = mma(p[e], w[u][j], acc[t][j]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      // every load is of a step that exists: one past the end would cost what a real one costs
-      int it = 0;
-#pragma unroll
-      for (int u = 0; u < ST; u++)
-        if (u < mine) load(u, u);
-      for (; it + 2 * ST <= mine; it += ST) {
-#pragma unroll
-        for (int u = 0; u < ST; u++) {
-          landed(std::integral_constant<int, (ST - 1) * (2 * TM + TN)>{});
-          compute(u);
-          load(u, it + u + ST);
-        }
+      for (int j = 0; j < TN; j++) {
+        w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + unit * 64u));
+        s[u][j] = *reinterpret_cast<const f32x4*>(Sb + (soff[j] + unit * 16u));
       }
-      landed(std::integral_constant<int, 0>{});
+    };
+    auto step_of = [&](int i) { return (uint32_t)(4 * (first + kWaves * (i >> 2)) + (i & 3)); };   // my i-th step: 4 per unit
+    // words of four groups -> one word of each of the four quarters' groups: afterwards w[u][j][g] is the eight
+    // weights of group g that this lane's quarter multiplies
+    auto trade = [&](int u) {
 #pragma unroll
-      for (int u = 0; u < ST; u++) {
-        if (it + u < mine) compute(u);
-        if (it + u + ST < mine) load(u, it + u + ST);
+      for (int j = 0; j < TN; j++) {
+        uint32_t x[4] = {w[u][j][0], w[u][j][1], w[u][j][2], w[u][j][3]};
+        auto y = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
+        x[0] = y[0]; x[2] = y[1];
+        y = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
+        x[1] = y[0]; x[3] = y[1];
+        y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+        x[0] = y[0]; x[1] = y[1];
+        y = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
+        x[2] = y[0]; x[3] = y[1];
+        w[u][j] = frag16{x[0], x[1], x[2], x[3]};
       }
-      landed(std::integral_constant<int, 0>{});
+    };
+    auto compute = [&](int u, int g) {           // group g of the unit in slot u
+      frag16 b[TN];
 #pragma unroll
-      for (int u = 0; u < ST; u++)
-        if (it + u + ST < mine) compute(u);
-    } else {
-      // a unit is four steps; W and the scales of the next unit and the activations of the next steps are on
-      // their way while one is multiplied
-      frag16 w[2][TN];
-      f32x4 s[2][TN];
-      auto load_w = [&](int u, int i) {
-        const uint32_t unit = (uint32_t)(first + kWaves * i);
+      for (int j = 0; j < TN; j++) b[j] = nib8(w[u][j][g]);
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-          w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + unit * 64u));
-          s[u][j] = *reinterpret_cast<const f32x4*>(Sb + (soff[j] + unit * 16u));
-        }
-      };
-      auto step_of = [&](int i) { return (uint32_t)(4 * (first + kWaves * (i >> 2)) + (i & 3)); };   // my i-th step: 4 per unit
-      // words of four groups -> one word of each of the four quarters' groups: afterwards w[u][j][g] is the eight
-      // weights of group g that this lane's quarter multiplies
-      auto trade = [&](int u) {
+      for (int t = 0; t < TM; t++) {
+        frag16 p[3];
+        cut(g % ST, t, p);
+        f32x4 grp[TN];
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-          uint32_t x[4] = {w[u][j][0], w[u][j][1], w[u][j][2], w[u][j][3]};
-          auto y = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
-          x[0] = y[0]; x[2] = y[1];
-          y = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
-          x[1] = y[0]; x[3] = y[1];
-          y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
-          x[0] = y[0]; x[1] = y[1];
-          y = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
-          x[2] = y[0]; x[3] = y[1];
-          w[u][j] = frag16{x[0], x[1], x[2], x[3]};
-        }
-      };
-      auto compute = [&](int u, int g) {           // group g of the unit in slot u
-        frag16 b[TN];
+        for (int e = 0; e < 3; e++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) b[j] = nib8(w[u][j][g]);
+          for (int j = 0; j < TN; j++) grp[j] = mma(p[e], b[j], e == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : grp[j]);
 #pragma unroll
-        for (int t = 0; t < TM; t++) {
-          frag16 p[3];
-          cut(g % ST, t, p);
-          f32x4 grp[TN];
+        for (int j = 0; j < TN; j++)
 #pragma unroll
-          for (int e = 0; e < 3; e++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) grp[j] = mma(p[e], b[j], e == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : grp[j]);
-#pragma unroll
-          for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[t][j][v] = fmaf(grp[j][v], s[u][j][g], acc[t][j][v]);
-          if (TM >= 3) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      // unit `it` in slot u; `more`: the next unit exists (its activations follow in), `far`: the one after it too
-      auto unit = [&](int u, int it, auto steady) {
-        const bool more = decltype(steady)::value || it + 1 < mine, far = decltype(steady)::value || it + 2 < mine;
-        trade(u);
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-          // younger than this step's activations: those of ST - 1 steps, and the unit of weights issued between
-          if (!decltype(steady)::value) landed(std::integral_constant<int, 0>{});
-          else if (g == 0) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
-          else if (g == 1) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
-          else if (ST == 4) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
-          else landed(std::integral_constant<int, (ST - 1) * 2 * TM>{});
-          compute(u, g);
-          if (g + ST < 4 || more) load_a(g % ST, step_of(4 * it + g + ST));
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (far) load_w(u, it + 2);
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      load_w(0, 0);
-      if (mine > 1) load_w(1, 1);
-#pragma unroll
-      for (int u = 0; u < ST; u++) load_a(u, step_of(u));
+          for (int v = 0; v < 4; v++) acc[t][j][v] = fmaf(grp[j][v], s[u][j][g], acc[t][j][v]);
+        if (TM >= 3) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
+      }
       __builtin_amdgcn_sched_barrier(0);
-      int it = 0;
-      if (mine > 3) {                              // (the first unit's weights were not issued between its activations: no count)
-        unit(0, 0, std::false_type{});
-        it = 1;
-        for (; it + 3 < mine; it += 2) {
-          unit(1, it, std::true_type{});
-          unit(0, it + 1, std::true_type{});
-        }
-        unit(1, it, std::false_type{});
-        it++;
+    };
+    // unit `it` in slot u; `more`: the next unit exists (its activations follow in), `far`: the one after it too
+    auto unit = [&](int u, int it, auto steady) {
+      const bool more = decltype(steady)::value || it + 1 < mine, far = decltype(steady)::value || it + 2 < mine;
+      trade(u);
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        // younger than this step's activations: those of ST - 1 steps, and the unit of weights issued between
+        if (!decltype(steady)::value) landed(std::integral_constant<int, 0>{});
+        else if (g == 0) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
+        else if (g == 1) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
+        else if (ST == 4) landed(std::integral_constant<int, (ST - 1) * 2 * TM + 2 * TN>{});
+        else landed(std::integral_constant<int, (ST - 1) * 2 * TM>{});
+        compute(u, g);
+        if (g + ST < 4 || more) load_a(g % ST, step_of(4 * it + g + ST));
+        __builtin_amdgcn_sched_barrier(0);
       }
-      for (; it < mine; it++) {
-        if ((it & 1) == 0) unit(0, it, std::false_type{});
-        else unit(1, it, std::false_type{});
+      if (far) load_w(u, it + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load_w(0, 0);
+    if (mine > 1) load_w(1, 1);
+#pragma unroll
+    for (int u = 0; u < ST; u++) load_a(u, step_of(u));
+    __builtin_amdgcn_sched_barrier(0);
+    int it = 0;
+    if (mine > 3) {                              // (the first unit's weights were not issued between its activations: no count)
+      unit(0, 0, std::false_type{});
+      it = 1;
+      for (; it + 3 < mine; it += 2) {
+        unit(1, it, std::true_type{});
+        unit(0, it + 1, std::true_type{});
       }
+      unit(1, it, std::false_type{});
+      it++;
+    }
+    for (; it < mine; it++) {
+      if ((it & 1) == 0) unit(0, it, std::false_type{});
+      else unit(1, it, std::false_type{});
     }
   };
 
@@ -321,7 +464,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
     return m < 0x1p-40f || z != 0.f;
   };
   int* found = reinterpret_cast<int*>(red + 4 * BM * LD);   // RANGED: two words behind the sums
-  static_assert(!RANGED || (4 * BM * LD + 2) * 4 <= lds_bytes(TM, TN, Q4), "room for the words");
+  static_assert(!RANGED || (4 * BM * LD + 2) * 4 <= lds_bytes_q4(TM, TN), "room for the words");
   auto any_of_block = [&](bool mine_too, int word) {
     if (mine_too) found[word] = 1;
     __syncthreads();
@@ -404,13 +547,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_kernel(const float* 
   }
 }
 
-template <int TM, int TN, bool GU, bool Q4, bool RANGED = false>
-int run(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int M, int N, int K, int ldc, int ff) {
-  constexpr int lds = lds_bytes(TM, TN, Q4);
-  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows_kernel<TM, TN, GU, Q4, RANGED>),
+template <int TM, int TN, bool GU>
+int run_bf16(const RowsPlan& P, const float* A, const void* W, float* C, int M, int N, int K, int ldc, int ff) {
+  constexpr int lds = lds_bytes_bf16(TM, TN);
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows_bf16_kernel<TM, TN, GU>),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
-  gemm_rows_kernel<TM, TN, GU, Q4, RANGED><<<dim3((unsigned)(P.tiles * P.row_blocks), (unsigned)P.S), dim3(64 * kWaves), lds, ctx().stream>>>(
+  gemm_rows_bf16_kernel<TM, TN, GU><<<dim3((unsigned)(P.tiles * P.row_blocks), (unsigned)P.S), dim3(64 * kWaves), lds, ctx().stream>>>(
+      A, W, C, M, N, K, P.part_units, ldc, ff, P.row_blocks);
+  return TLHIP_OK;
+}
+template <int TM, int TN, bool GU, bool RANGED = false>
+int run_q4(const RowsPlan& P, const float* A, const void* W, const float* scales, float* C, int M, int N, int K, int ldc, int ff) {
+  constexpr int lds = lds_bytes_q4(TM, TN);
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows_q4_kernel<TM, TN, GU, RANGED>),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
+  gemm_rows_q4_kernel<TM, TN, GU, RANGED><<<dim3((unsigned)(P.tiles * P.row_blocks), (unsigned)P.S), dim3(64 * kWaves), lds, ctx().stream>>>(
       A, W, scales, C, M, N, K, P.part_units, ldc, ff, P.row_blocks);
   return TLHIP_OK;
 }
@@ -421,33 +574,35 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
   if constexpr (TM >= 3) {                         // more than 64 rows are blocks of three to five row tiles
     if (q4 && M > 64) {
       switch (P.TN + (gu ? 16 : 0)) {
-        case 1: return run<TM, 1, false, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
-        case 2: return run<TM, 2, false, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
-        case 18: return run<TM, 2, true, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+        case 1: return run_q4<TM, 1, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+        case 2: return run_q4<TM, 2, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+        case 18: return run_q4<TM, 2, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
       }
       return fail(TLHIP_EUNSUPPORTED, "gemm_rows: no kernel for this plan");
     }
   }
   switch (P.TN + (gu ? 16 : 0) + (q4 ? 32 : 0)) {   // (int4 over four column tiles: the registers hold one row tile)
-    case 1: return run<TM, 1, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
-    case 2: return run<TM, 2, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
-    case 4: return run<TM, 4, false, false>(P, A, W, scales, C, M, N, K, ldc, ff);
-    case 18: return run<TM, 2, true, false>(P, A, W, scales, C, M, N, K, ldc, ff);
-    case 20: return run<TM, 4, true, false>(P, A, W, scales, C, M, N, K, ldc, ff);
+    case 1: return run_bf16<TM, 1, false>(P, A, W, C, M, N, K, ldc, ff);
+    case 2: return run_bf16<TM, 2, false>(P, A, W, C, M, N, K, ldc, ff);
+    case 3: return run_bf16<TM, 3, false>(P, A, W, C, M, N, K, ldc, ff);
+    case 4: return run_bf16<TM, 4, false>(P, A, W, C, M, N, K, ldc, ff);
+    case 18: return run_bf16<TM, 2, true>(P, A, W, C, M, N, K, ldc, ff);
+    case 19: return run_bf16<TM, 3, true>(P, A, W, C, M, N, K, ldc, ff);
+    case 20: return run_bf16<TM, 4, true>(P, A, W, C, M, N, K, ldc, ff);
     case 33:
-      if constexpr (TM <= 4) return run<TM, 1, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      if constexpr (TM <= 4) return run_q4<TM, 1, false>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;
     case 34:
-      if constexpr (TM <= 4) return run<TM, 2, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      if constexpr (TM <= 4) return run_q4<TM, 2, false>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;
     case 36:
-      if constexpr (TM == 1) return run<TM, 4, false, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      if constexpr (TM == 1) return run_q4<TM, 4, false>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;
     case 50:
-      if constexpr (TM <= 4) return run<TM, 2, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      if constexpr (TM <= 4) return run_q4<TM, 2, true>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;
     case 52:
-      if constexpr (TM == 1) return run<TM, 4, true, true>(P, A, W, scales, C, M, N, K, ldc, ff);
+      if constexpr (TM == 1) return run_q4<TM, 4, true>(P, A, W, scales, C, M, N, K, ldc, ff);
       break;
   }
   return fail(TLHIP_EUNSUPPORTED, "gemm_rows: no kernel for this plan");
@@ -456,57 +611,102 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 }  // namespace rows
 
 // Row tiles per block, columns per tile and K splits that an estimate of the time likes best; S == 0 where the shape is not
-// taken.
+// taken. `us` is the chosen plan's time, the launch that adds parts up not included: the caller weighs it against the time of the
+// kernel it would take instead.
 //
-// The estimate that chooses, fitted to 280 runs (K 384 .. 18944, N 384 .. 37888, M 8 .. 120): a step of a block's eight
+// bf16, fitted to 13980 runs (9 to 256 rows, 256 to 33000 columns, K 256 to 18944; error 8 to 13 %; the shape it chooses is 2 %
+// slower than the fastest one on average): a launch costs 2.1 us and its weights' way from HBM; a block starts and ends in
+// a time that grows with its sums; a step of its wavefronts takes the CU's loads of activations and weights, a little less where
+// CUs are idle; blocks that share a CU cost half again each, nearly twice where their steps are many.
+static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
+  // blocks of [row tiles][column tiles] that fit a CU (registers, LDS)
+  static constexpr int kFit[5][4] = {{4, 3, 2, 2}, {4, 2, 2, 1}, {3, 2, 1, 1}, {2, 2, 1, 1}, {2, 1, 1, 1}};
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  RowsPlan best;
+  const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / rows::kStep, t16 = cdiv(M, 16);
+  const double own_sum = gu || N > 8192 ? 5 : 0;   // a launch that adds up (a narrow product is planned as if left as parts, whose
+                                                   // sum its consumer forms: the two are the same bits)
+  double least = 0;
+  const int64_t few = cdiv(t16, rows::kMaxTM);
+  for (int64_t row_blocks = few; row_blocks <= std::min(few + 1, t16); row_blocks++)
+    for (int TN = 4; TN >= (gu ? 2 : 1); TN--) {
+      const int TM = (int)cdiv(t16, row_blocks);
+      const int64_t tiles = cdiv(rows_w, 16 * TN), fit = kFit[TM - 1][TN - 1], at_once = fit * cus;
+      if (row_blocks > few && t16 <= 4 && tiles * few > cus / 2) continue;   // (weights read twice for CUs that are busy anyway)
+      const int64_t unsplit = tiles * row_blocks;
+      const int most = unsplit >= cus ? 1 : (int)std::min<int64_t>(max_S, units);   // (K is split no further than keeps every CU busy)
+      for (int S = 1; S <= most && (S == 1 || unsplit * (S - 1) < cus); S++) {
+        const int64_t blocks = unsplit * S;
+        const int per = ((int)units + S - 1) / S;
+        if (((int)units + per - 1) / per != S) continue;
+        const double n = (double)((per + rows::kWaves - 1) / rows::kWaves);   // steps of a wavefront
+        const auto share = [&](int64_t on_a_cu) { return 1 + (0.424 + 0.593 * n / (n + 10)) * (double)(on_a_cu - 1); };
+        double rounds = 1;
+        if (blocks > cus) {
+          const int64_t rest = blocks % at_once;
+          const double fill = blocks > at_once ? 0.86 + 0.14 * (double)rest / (double)at_once : 1;   // of the last round
+          rounds = (double)(blocks / at_once) * share(fit) + (rest > 0 ? share(cdiv(rest, cus)) * fill : 0);
+        }
+        const double work = (0.086 * n + 0.914 * (double)per / rows::kWaves) * (0.194 * TM + 0.182 * TN) *
+                            (0.877 + 0.123 * std::min(1.0, (double)blocks / (double)cus));
+        const double parts = S > 1 ? (double)S * M * (gu ? tiles * 16 * TN : N) * 4e-6 : 0;   // MB
+        const double us = 2.08 + rounds * (0.144 * TM * TN + work) + 0.179 * parts + 0.103 * 2e-6 * (double)rows_w * (double)K;
+        const double all = us + 0.25 * parts + (S > 1 ? 0.4 + own_sum : 0);
+        if (best.S == 0 || all < least) {
+          least = all;
+          best.TM = TM;
+          best.TN = TN;
+          best.S = (int)S;
+          best.tiles = (int)tiles;
+          best.row_blocks = (int)row_blocks;
+          best.part_units = (int)per;
+          best.us = 1.05 * us;                     // (for the errors of both estimates it is weighed against)
+        }
+      }
+    }
+  return best;
+}
+
+// int4: the estimate that chooses, fitted to 280 runs (K 384 .. 18944, N 384 .. 37888, M 8 .. 120): a step of a block's eight
 // wavefronts takes the CU's vector memory path 35 clocks per KB of activations and 60 per KB of weights (whose lanes cover
 // 16 rows each), or its SIMDs, with two wavefronts each, the clocks of their matrix or vector instructions (5.5 per element
-// cut, 23 per eight nibbles; int4 measured 1.8 times that); a block starts and ends in 3500 clocks and 60 per accumulator
-// tile; bf16 blocks past the first round cost a fifth more; a launch costs 2 us. `us` is the chosen plan's time fitted again,
-// to 1000 runs (error 10 to 13 %) and 5 to 12 % up: the caller weighs it against the time of the kernel it would take instead.
-// Measured, us, other kernel -> this one: 896 x 896 at 5 / 37 / 77 rows 10.5 / 10.0 / 20.5 -> 3.6 / 3.7 / 4.4; 4864 x 896
-// gated 14.4 / 16.0 / 25.4 -> 7.8 / 11.1 / 13.4; 896 x 4864 11.0 / 11.4 / 21.7 -> 4.9 / 7.0 / 9.6; 9728 x 896 at 48 and 64
-// rows 16.8 / 17.8 -> 10.8 / 11.9; 18944 x 3584 gated 111 / 111 -> 63 / 92; int4 119 / 127 -> 53 / 93.
-static RowsPlan plan_row_blocks(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S, int64_t row_blocks) {
+// cut, 23 per eight nibbles; measured 1.8 times that); a block starts and ends in 3500 clocks and 60 per accumulator
+// tile; a launch costs 2 us. `us` is the chosen plan's time fitted again, to 1000 runs (error 10 to 13 %) and 5 to 12 % up.
+static RowsPlan plan_row_blocks_q4(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S, int64_t row_blocks) {
   RowsPlan best;
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / (q4 ? 128 : 32), steps = q4 ? 4 : 1;
+  const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / 128;
+  constexpr int steps = 4;
   best.row_blocks = (int)row_blocks;
   const int TM = best.TM = (int)cdiv(cdiv(M, 16), row_blocks);
   double least = 0;
-  const double own_sum = gu || (!q4 && N > 8192) ? 5 : 0;   // (18960 x 2048 at 32 rows: 33.6 us in two parts)
-  for (int TN = q4 && TM > 1 ? 2 : 4; TN >= (gu ? 2 : 1); TN /= 2) {   // (what the registers hold)
+  const double own_sum = gu ? 5 : 0;
+  for (int TN = TM > 1 ? 2 : 4; TN >= (gu ? 2 : 1); TN /= 2) {   // (what the registers hold)
     const int64_t tiles = cdiv(rows_w, 16 * TN);
     for (int64_t S = 1; S <= std::min<int64_t>(max_S, units); S++) {
       const int64_t per = cdiv(units, S), blocks = tiles * row_blocks * S;
       if (cdiv(units, per) != S) continue;
       const double n = (double)(cdiv(per, rows::kWaves) * steps);    // steps of a wavefront
-      const double mem = 8 * (70.0 * TM + (q4 ? 30.0 : 60.0) * TN);
-      const double math = 2 * (q4 ? 1.8 * std::max(48.0 * TM * TN, 176.0 * TM + TN * (92.0 + 16 * TM)) : std::max(48.0 * TM * TN, 176.0 * TM));
-      // (every CU is busy without a split, and the parts of more than a row tile cost more than the last round's gaps)
-      if (!q4 && S > 1 && M > 16 && tiles * row_blocks > cus) break;
-      const double rounds = blocks <= (q4 ? 2 : 4) * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus;
+      const double mem = 8 * (70.0 * TM + 30.0 * TN);
+      const double math = 2 * 1.8 * std::max(48.0 * TM * TN, 176.0 * TM + TN * (92.0 + 16 * TM));
+      const double rounds = blocks <= 2 * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus;
       const double parts = S > 1 ? (double)S * M * rows_w * 4 / 1e6 : 0;
-      // parts written and read, and their launch, which a gated product has and a wide one (a narrow one is planned as if
-      // left as parts, whose sum its consumer forms: the two are the same bits)
-      const double us = 2 + rounds * (!q4 && rounds > 1 ? 1.2 : 1.0) * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100 +
-                        (S > 1 ? parts / 4 + own_sum : 0);
+      // parts written and read, and their launch, which a gated product has
+      const double us = 2 + rounds * (n * std::max(math, mem) + 3500 + 60 * TM * TN) / 2100 + (S > 1 ? parts / 4 + own_sum : 0);
       if (best.S == 0 || us < least) {
         least = us;
         best.TN = TN;
         best.S = (int)S;
         best.tiles = (int)tiles;
         best.part_units = (int)per;
-        // fewer steps than wavefronts leave some idle; five row tiles of int4 spill, and int4 blocks in turn wait for what
+        // fewer steps than wavefronts leave some idle; five row tiles spill, and blocks in turn wait for what
         // they would have loaded ahead; over many blocks, wavefronts with a unit more than others even out (38 x 18088 gated x
         // 2560, 20 units over eight wavefronts: 64 us here, 89 in the 64-row tiles)
-        const double own = q4 && blocks > 2 * cus && per > rows::kWaves ? 1.05 * (double)per / rows::kWaves * steps : n;
+        const double own = blocks > 2 * cus && per > rows::kWaves ? 1.05 * (double)per / rows::kWaves * steps : n;
         const double work = rounds * own * std::max(mem * (double)std::min<int64_t>(rows::kWaves, per) / rows::kWaves, per > 4 ? math : math / 2) / 2100;
-        best.us = q4 ? 2 + work * (TM == 5 ? 1.3 : 1.0) * (rounds > 2 ? 1.2 : rounds > 1 ? 0.81 : 0.74) + rounds * (0.3 + 0.18 * TM * TN) + parts
-                     : 0.85 + 1.15 * work + rounds * (1.2 + 0.18 * TM * TN) + 0.75 * parts;
-        // many columns of a short K (14000 runs, N 20000 .. 160000): 24 x 21497 gated x 512 int4 24.8 us for an estimate of 20.3, 111 x
-        // 10540 gated x 256 bf16 15.3 for 19.9
-        if (blocks > 2 * cus) best.us *= q4 ? (per <= 4 ? 1.2 : 1.0) : M > 64 && K <= 384 ? 0.78 : 1.0;
+        best.us = 2 + work * (TM == 5 ? 1.3 : 1.0) * (rounds > 2 ? 1.2 : rounds > 1 ? 0.81 : 0.74) + rounds * (0.3 + 0.18 * TM * TN) + parts;
+        // many columns of a short K (14000 runs, N 20000 .. 160000): 24 x 21497 gated x 512 24.8 us for an estimate of 20.3
+        if (blocks > 2 * cus && per <= 4) best.us *= 1.2;
       }
     }
   }
@@ -515,15 +715,16 @@ static RowsPlan plan_row_blocks(int64_t M, int64_t N, int64_t K, bool gu, bool q
 
 RowsPlan plan_gemm_rows(int64_t M, int64_t N, int64_t K, bool gu, bool q4, int64_t max_S) {
   const int64_t rows_w = (gu ? 2 : 1) * N, t16 = (M + 15) / 16;
-  if (M > 128 || K % (q4 ? 128 : 32) != 0 || M * K * 4 >= (int64_t(1) << 32) || rows_w * K * (q4 ? 1 : 4) / 2 >= (int64_t(1) << 32))
+  if (M > (q4 ? 128 : kRowsMaxBf16) || K % (q4 ? 128 : 32) != 0 || M * K * 4 >= (int64_t(1) << 32) || rows_w * K * (q4 ? 1 : 4) / 2 >= (int64_t(1) << 32))
     return RowsPlan{};                             // (32-bit byte offsets)
-  // Up to 16 rows nothing else is as fast, save for int4 with so few units that most wavefronts of a block have none and so many
+  if (!q4) return plan_rows_bf16(M, N, K, gu, max_S);
+  // Up to 16 rows nothing else is as fast, save for so few units that most wavefronts of a block have none and so many
   // columns that blocks come in more rounds than that: up to 65000 columns x 128 twice what the 64-row tiles take, x 256 1.4 times;
   // up to 32768 x 256 0.9 times
-  if (q4 && M <= 16 && K < 512 && (rows_w + 63) / 64 > K / 128 * (int64_t)ctx().cus) return RowsPlan{};
-  const auto plan = [&](int64_t row_blocks) { return plan_row_blocks(M, N, K, gu, q4, max_S, row_blocks); };
-  if (!q4 || t16 != 5) return plan((t16 + rows::kMaxTM - 1) / rows::kMaxTM);
-  // int4 with 65 to 80 rows: one block of five row tiles, or two of three (77 x 640 x 768 7.8 us and 6.1; 74 x 4609 x 11008, whose
+  if (M <= 16 && K < 512 && (rows_w + 63) / 64 > K / 128 * (int64_t)ctx().cus) return RowsPlan{};
+  const auto plan = [&](int64_t row_blocks) { return plan_row_blocks_q4(M, N, K, gu, max_S, row_blocks); };
+  if (t16 != 5) return plan((t16 + rows::kMaxTM - 1) / rows::kMaxTM);
+  // 65 to 80 rows: one block of five row tiles, or two of three (77 x 640 x 768 7.8 us and 6.1; 74 x 4609 x 11008, whose
   // K cannot be split, 76 and 107)
   const RowsPlan one = plan(1), two = plan(2);
   const auto all = [](const RowsPlan& P) { return P.us + (P.S > 1 ? kPartSumUs : 0); };
