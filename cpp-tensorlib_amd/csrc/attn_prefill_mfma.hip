@@ -244,19 +244,153 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_mfma_kernel(const float* 
   }
 }
 
+// The same in tiles of 16 queries and 16 keys, for prompts so short that the tiles above leave the chip idle: three of a block's
+// wavefronts had a key tile each at 77 tokens, and a wavefront alone needs 2.8 us for the softmax of 32 x 32 scores. Both products are
+// formed transposed (S^T = K Q^T, O^T = V^T P^T): lane (g, c) = (l / 16, l % 16) then holds the scores of query c for the keys 4 g ..
+// 4 g + 3 of a tile, which are its operand of the second product as they are - one running maximum and sum to a lane, two register
+// swaps per statistic, no LDS until the wavefronts' states meet. All operands come from memory in 16-byte pieces: reduction step (m, j)
+// of the scores takes dims 16 m + 4 g + j, and output tile n of the second product holds the dims 64 (n / 4) + 4 c + n % 4, so
+// that a lane's piece of a V row is one element of each of four tiles. The next tile's rows are requested before this one's
+// arithmetic. 14 heads of 64, 77 tokens: 7.3 -> 4.9 us; error against 64 bits
+// 0.7 of the larger tiles' (shorter sums).
+template <int D, typename KT>
+__global__ __launch_bounds__(512, 1) void attn_prefill_small_kernel(const float* __restrict__ q, const KT* __restrict__ K,
+                                                                     const KT* __restrict__ V, float* __restrict__ out, int group, int T,
+                                                                     int pos0, int64_t kv_stride, float scale, int64_t o_head,
+                                                                     int64_t o_row) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int NM = D / 16, OS = D + 4;             // 16-byte pieces of a row per lane; row stride of the states in LDS
+  __shared__ __attribute__((aligned(16))) float states[8][16][OS];
+  __shared__ float ms[8][16], ls[8][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int h = blockIdx.x, p0 = ((T + 15) / 16 - 1 - (int)blockIdx.y) * 16;
+  const KT* Kh = K + (size_t)(h / group) * kv_stride;
+  const KT* Vh = V + (size_t)(h / group) * kv_stride;
+  const int kend = min(pos0 + p0 + 16, pos0 + T), nkt = (kend + 15) >> 4;
+  const int limit = pos0 + min(p0 + c, T - 1);       // the last key this lane's query sees (queries past T are not stored)
+
+  float4 kr[NM], vr[NM];                             // K: dims 16 m + 4 g .. of key c; V: dims 64 (m / 4) + 4 c .. of key 4 g + m % 4
+  const auto request = [&](int tile) {
+    const KT* kp = Kh + (size_t)min(tile * 16 + c, kend - 1) * D + 4 * g;
+#pragma unroll
+    for (int m = 0; m < NM; m++) kr[m] = load_kv4(kp + 16 * m);
+#pragma unroll
+    for (int m = 0; m < NM; m++)
+      vr[m] = load_kv4(Vh + (size_t)min(tile * 16 + 4 * g + (m & 3), kend - 1) * D + 64 * (m >> 2) + 4 * c);
+  };
+  float4 qr[NM];
+  const float* qp = q + ((size_t)h * T + min(p0 + c, T - 1)) * D + 4 * g;
+#pragma unroll
+  for (int m = 0; m < NM; m++) qr[m] = *reinterpret_cast<const float4*>(qp + 16 * m);
+  request(wave);
+
+  f32x4 o[NM];
+#pragma unroll
+  for (int n = 0; n < NM; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float mrow = -INFINITY, lrow = 0.f;
+  for (int kt = wave; kt < nkt; kt += 8) {
+    float4 kc[NM], vc[NM];
+#pragma unroll
+    for (int m = 0; m < NM; m++) { kc[m] = kr[m]; vc[m] = vr[m]; }
+    if (kt + 8 < nkt) request(kt + 8);
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[m].x, qr[m].x, s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[m].y, qr[m].y, s1, 0, 0, 0);
+      s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[m].z, qr[m].z, s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kc[m].w, qr[m].w, s1, 0, 0, 0);
+    }
+    float sv[4], mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      sv[v] = kt * 16 + 4 * g + v <= limit ? (s0[v] + s1[v]) * scale : -INFINITY;
+      mx = fmaxf(mx, sv[v]);
+    }
+    const auto over_groups = [](float x, auto op) {   // over the four lanes of a query
+      LanePair p = swap16(x, x);
+      x = op(p.first, p.second);
+      p = swap32(x, x);
+      return op(p.first, p.second);
+    };
+    mx = over_groups(mx, [](float x, float y) { return fmaxf(x, y); });
+    const float mnew = fmaxf(mrow, mx), mref = mnew == -INFINITY ? 0.f : mnew, corr = __expf(mrow - mref);
+    float p[4], sum = 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      p[v] = __expf(sv[v] - mref);
+      sum += p[v];
+    }
+    lrow = lrow * corr + sum;                        // of this lane's keys
+    mrow = mnew;
+    if (__any(corr != 1.f)) {
+#pragma unroll
+      for (int n = 0; n < NM; n++) o[n] *= corr;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+#pragma unroll
+      for (int half = 0; half < NM / 4; half++) {
+        const float4 x = vc[4 * half + v];
+        o[4 * half] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, p[v], o[4 * half], 0, 0, 0);
+        o[4 * half + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, p[v], o[4 * half + 1], 0, 0, 0);
+        o[4 * half + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, p[v], o[4 * half + 2], 0, 0, 0);
+        o[4 * half + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, p[v], o[4 * half + 3], 0, 0, 0);
+      }
+  }
+  // o[4 half + e][v]: query c, dim 64 half + 4 (4 g + v) + e
+#pragma unroll
+  for (int half = 0; half < NM / 4; half++)
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      *reinterpret_cast<f32x4*>(&states[wave][c][64 * half + 16 * g + 4 * v]) = f32x4{o[4 * half][v], o[4 * half + 1][v], o[4 * half + 2][v], o[4 * half + 3][v]};
+  {
+    LanePair p = swap16(lrow, lrow);
+    const float l = p.first + p.second;
+    p = swap32(l, l);
+    if (g == 0) { ms[wave][c] = mrow; ls[wave][c] = p.first + p.second; }
+  }
+  __syncthreads();
+  const int used = min(8, nkt);                      // wavefronts that had a tile
+  for (int i = tid; i < 16 * D / 4; i += 512) {
+    const int row = i / (D / 4), d = 4 * (i % (D / 4));
+    if (p0 + row >= T) continue;
+    float M = -INFINITY, L = 0.f;
+    for (int w = 0; w < used; w++) M = fmaxf(M, ms[w][row]);
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < used; w++) {
+      const float m = ms[w][row], f = m == -INFINITY ? 0.f : __expf(m - M);
+      L += f * ls[w][row];
+      a += f * *reinterpret_cast<const f32x4*>(&states[w][row][d]);
+    }
+    *reinterpret_cast<f32x4*>(out + (size_t)h * o_head + (size_t)(p0 + row) * o_row + d) = a * (1.0f / L);
+  }
+}
+
+// Which of the two: heads of 64 always the small tiles (58 shapes of 14 to 128 heads, 2 to 1000 keys: 1.01 to 1.95 times as fast);
+// heads of 128, whose states fill twice the LDS and whose K and V rows every 16 queries then read again, while their blocks
+// make one round of the CUs or the keys are few (28 heads, 77 tokens 10.8 -> 7.0 us, 150 15.7 -> 10.3, 77 after 400 27.6 -> 19.0; but 150
+// after 400, 280 blocks, 31.8 -> 33.3, 64 heads of 100 tokens after 150 17.3 -> 21.8).
 template <int D, typename KT>
 int launch_prefill_mfma(const float* q, const KT* K, const KT* V, float* out, int Hq, int Hkv, int T,
                         int64_t kv_max, float scale, int pos0, int token_major) {
   Context& c = ctx();
-  auto fn = attn_prefill_mfma_kernel<D, KT>;
-  const int lds = (int)PrefillLds<D>::kBytes;
-  if ((size_t)lds > (size_t)c.lds_per_cu) return fail(TLHIP_EUNSUPPORTED, "tlhip_attn_prefill: not enough LDS");
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(LDS)");
-  const dim3 grid((unsigned)Hq, (unsigned)((T + 31) / 32)), block(512);
   const int64_t o_head = token_major ? D : (int64_t)T * D, o_row = token_major ? (int64_t)Hq * D : D;
-  hipLaunchKernelGGL(fn, grid, block, (size_t)lds, c.stream, q, K, V, out, Hq / Hkv, T, pos0, kv_max * (int64_t)D, scale,
-                     o_head, o_row);
+  const int t16 = (T + 15) / 16;
+  if (D == 64 || (int64_t)Hq * t16 <= c.cus || pos0 + T <= 160) {
+    hipLaunchKernelGGL((attn_prefill_small_kernel<D, KT>), dim3((unsigned)Hq, (unsigned)t16), dim3(512), 0, c.stream, q, K, V, out, Hq / Hkv, T, pos0,
+                       kv_max * (int64_t)D, scale, o_head, o_row);
+    return 0;
+  }
+  if constexpr (D == 128) {
+    auto fn = attn_prefill_mfma_kernel<D, KT>;
+    const int lds = (int)PrefillLds<D>::kBytes;
+    if ((size_t)lds > (size_t)c.lds_per_cu) return fail(TLHIP_EUNSUPPORTED, "tlhip_attn_prefill: not enough LDS");
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(LDS)");
+    hipLaunchKernelGGL(fn, dim3((unsigned)Hq, (unsigned)((T + 31) / 32)), dim3(512), (size_t)lds, c.stream, q, K, V, out, Hq / Hkv, T, pos0,
+                       kv_max * (int64_t)D, scale, o_head, o_row);
+  }
   return 0;
 }
 

@@ -395,6 +395,41 @@ def test_attn_prefill_matches_oracle(lib, orc, D, Hq, Hkv, T, pos0, kernel):
     assert allclose(got, want, RTOL, ATOL), maxrel(got, want)
 
 
+@pytest.mark.parametrize("kv_bf16", [False, True])
+@pytest.mark.parametrize("D,Hq,Hkv,T,pos0", [
+    (64, 3, 1, 1, 0), (64, 2, 2, 15, 1), (64, 14, 2, 16, 0), (64, 14, 2, 17, 111), (128, 4, 4, 16, 127), (128, 2, 1, 33, 128),
+    (128, 28, 4, 144, 17), (128, 28, 4, 145, 16), (128, 40, 8, 112, 48),     # the last of 16-query tiles by blocks, the first of 32, and by keys
+])
+def test_attn_prefill_tile_sizes(lib, orc, D, Hq, Hkv, T, pos0, kv_bf16):
+    """The fp32 matrix-pipe kernels around the edges of their 16- and 32-wide tiles and on both sides of the choice between them,
+    in both output layouts; poison past the chunk."""
+    print("case attn_prefill tiles", D, Hq, Hkv, T, pos0, kv_bf16, flush=True)
+    kv_max = pos0 + T + 3
+    q = orc.normal(Hq * T * D, 34).reshape(Hq, T, D)
+    K = orc.normal(Hkv * kv_max * D, 35).reshape(Hkv, kv_max, D)
+    V = orc.normal(Hkv * kv_max * D, 36).reshape(Hkv, kv_max, D)
+    K[:, pos0 + T:, :] = 1e30
+    V[:, pos0 + T:, :] = np.nan
+    if kv_bf16:
+        Kd, Vd = orc.to_bf16(K.ravel()).reshape(K.shape), orc.to_bf16(V.ravel()).reshape(V.shape)
+        K, V = orc.bf16_widen(Kd.ravel()).reshape(K.shape), orc.bf16_widen(Vd.ravel()).reshape(V.shape)
+    else:
+        Kd, Vd = K, V
+    scale = 1.0 / np.sqrt(float(D))
+    got = _prefill(lib, q, Kd, Vd, scale, pos0, kv_bf16=kv_bf16, kernel="fp32pipe")
+    want = orc.attn_prefill(q, K, V, scale, pos0)
+    assert np.all(np.isfinite(got)) and allclose(got, want, RTOL, ATOL), maxrel(got, want)
+    dq, dk, dv, do = lib.to_device(q), lib.to_device(Kd), lib.to_device(Vd), lib.empty((T, Hq, D))
+    lib.tune_attn_prefill(KERNELS["fp32pipe"])
+    try:
+        lib.attn_prefill_tok(dq, dk, dv, do, Hq, Hkv, T, kv_max, D, scale, kv_bf16, pos0)
+    finally:
+        lib.tune_attn_prefill(0)
+    assert np.array_equal(do.numpy().transpose(1, 0, 2), got)
+    for b in (dq, dk, dv, do):
+        b.free()
+
+
 def _attn_f64(q, K, V, scale, pos0):
     """Causal attention in float64: what the arithmetic fixes, independent of any summation order."""
     Hq, T, D = q.shape
