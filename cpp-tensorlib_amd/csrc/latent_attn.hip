@@ -74,6 +74,15 @@ __device__ __forceinline__ size_t val_at(const Dims& d, int p, int e) {
   return (((size_t)(p >> 5) * d.NC * d.LT + (e >> 5)) * 2 + (a >> 1)) * 512 + (g * 32 + (e & 31)) * 8 + (a & 1) * 4 + (p & 3);
 }
 
+// How many of a decode step's S splits hold keys at position p: those past them write no partials and nobody reads any. The grid
+// is planned for the capacity, since the position may be on the device: at position 45 of 4096, 14 heads of 64 over 256 wrote and
+// read 64 splits' partials of which one held keys (attend 6.3, output 6.8 us; both about 0.8 us less, a chat turn of 18 such
+// layers and 37 + 16 tokens 7644 -> 7571 us).
+__device__ __forceinline__ int live_splits(const Dims& d, int p, int S) {
+  const int tiles = p / 32 + 1;
+  return min(S, d.NC == 1 ? (tiles + 1) / 2 : tiles);
+}
+
 // ---- new cache rows ------------------------------------------------------------------------------
 // One block of 256 threads per token.
 template <int NC>
@@ -349,6 +358,7 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_a
   const int row = rt * 32 + c;                       // this lane's query row
   const int limit = row < T * d.H ? p0 + row / d.H : -1;
   const int last = p0 + min(rt * 32 + 31, T * d.H - 1) / d.H, ntiles = last / 32 + 1, npairs = (ntiles + 1) / 2;
+  if (T == 1 && split >= live_splits(d, p0, S)) return;
   const u32x4* kc = reinterpret_cast<const u32x4*>(a.keys) + lane;
   const u32x4* vc = reinterpret_cast<const u32x4*>(a.values) + lane;
   const u32x4* qg = reinterpret_cast<const u32x4*>(qimg) + (size_t)rt * 2 * d.DS * 64 + lane;
@@ -482,6 +492,7 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const tlhip_la
   const int row = rt * 32 + c;                       // this lane's query row
   const int limit = row < T * d.H ? p0 + row / d.H : -1;
   const int last = p0 + min(rt * 32 + 31, T * d.H - 1) / d.H, ntiles = last / 32 + 1;   // key tiles the tile's last row sees
+  if (T == 1 && split >= live_splits(d, p0, S)) return;
   u32x4* qs = reinterpret_cast<u32x4*>(lds);         // [NQ][DS][64]
   f32x4* red = reinterpret_cast<f32x4*>(qs + NQ * d.DS * 64);   // [2][4 waves][4][64]
   const u32x4* qg = reinterpret_cast<const u32x4*>(qimg) + (size_t)rt * NQ * d.DS * 64;
@@ -599,7 +610,7 @@ __host__ __device__ inline int out_groups(int NT, int TQ, int LV) { const int n 
 template <int TQ, int NT, int ROWS>
 __global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict__ u, int64_t ldu, float* __restrict__ y, int64_t ldy,
                                                         const tlhip_latent_attn a, const float* __restrict__ part, int T, int S,
-                                                        int rows, int slices) {
+                                                        int rows, int slices, int pos0, const uint32_t* __restrict__ d_pos) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int NW = NT / 64;
   const Dims d = dims_of(a);
@@ -621,29 +632,31 @@ __global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict_
     pre[i] = uv[(size_t)v * n8 + min(lane, n8 - 1)];
     gate[i] = TQ == 1 && a.gate_off >= 0 ? u[(size_t)t0 * ldu + a.gate_off + h * d.V + v] : 0.f;
   }
+  const int live = TQ == 1 ? live_splits(d, d_pos ? (int)*d_pos : pos0, S) : S;
   f32x4 v[8];                          // eight splits' latents of this thread's item, the first ones before the weights are known
   const auto load_splits = [&](int i, int s0) {
     const int j = i % items, t = j / (LV / 4), e = 4 * (j - t * (LV / 4));
     const float* src = pa + ((size_t)(t0 + min(t, nt - 1)) * d.H + h) * LV + e;
 #pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = *reinterpret_cast<const f32x4*>(src + (size_t)min(s0 + k * G, S - 1) * R * LV);
+    for (int k = 0; k < 8; k++)
+      if (k * G < live) v[k] = *reinterpret_cast<const f32x4*>(src + (size_t)min(s0 + k * G, live - 1) * R * LV);
   };
-  load_splits(tid, tid / items);
+  if (tid / items < live) load_splits(tid, tid / items);
   if (wave < TQ) {                     // a wavefront weighs the (up to 64) splits of one token
     const int row = (t0 + min(wave, nt - 1)) * d.H + h;
-    const float m = lane < S ? pm[lane * R + row] : -INFINITY, l = lane < S ? pl[lane * R + row] : 0.f;
+    const float m = lane < live ? pm[lane * R + row] : -INFINITY, l = lane < live ? pl[lane * R + row] : 0.f;
     const float f = exp2f(m - wave_max(m)), tot = wave_sum(f * l);
-    if (lane < S) w[wave * S + lane] = f / tot;
+    if (lane < live) w[wave * S + lane] = f / tot;
   }
   __syncthreads();
   for (int i = tid; i < items * G; i += NT) {
     const int grp = i / items, j = i - grp * items, t = j / (LV / 4), e = 4 * (j - t * (LV / 4));
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = grp; s0 < S; s0 += 8 * G) {
+    for (int s0 = grp; s0 < live; s0 += 8 * G) {
       if (i != tid || s0 != grp) load_splits(i, s0);
 #pragma unroll
       for (int k = 0; k < 8; k++)
-        if (s0 + k * G < S) {
+        if (s0 + k * G < live) {
           const float f = w[t * S + s0 + k * G];
           acc += v[k] * f;
         }
@@ -899,7 +912,7 @@ static int launch(const float* u, int64_t ldu, const float* q, int64_t ldq, floa
   if (o_mfma)
     hipLaunchKernelGGL(fom, dim3((unsigned)(d.H * ((T + 31) / 32))), dim3(256), lo, c.stream, u, ldu, y, ldy, a, part, T, S, rows);
   else
-    hipLaunchKernelGGL(fo, dim3((unsigned)(oslices * d.H * tiles)), dim3((unsigned)ont), lo, c.stream, u, ldu, y, ldy, a, part, T, S, rows, oslices);
+    hipLaunchKernelGGL(fo, dim3((unsigned)(oslices * d.H * tiles)), dim3((unsigned)ont), lo, c.stream, u, ldu, y, ldy, a, part, T, S, rows, oslices, pos0, d_pos);
   TLHIP_CHECK_LAUNCH(TLHIP_C_LATENT_ATTN);
 }
 

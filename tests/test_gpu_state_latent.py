@@ -299,6 +299,30 @@ def test_long_context_in_chunks_and_steps(lib, capi, H, planes, tol):
         assert np.array_equal(a.run(u[p:p + 1], q[p:p + 1], p, d_pos), s)
 
 
+@pytest.mark.parametrize("planes,tol", PLANES)
+@pytest.mark.parametrize("H,capacity", [(4, 64), (4, 2048), (40, 512)])
+def test_steps_read_only_splits_with_keys(lib, capi, H, capacity, planes, tol):
+    """Steps at the edges of a split's first keys, each after a step at the far end that left every split's partials: by host and
+    by device position the same bits."""
+    a = Latent(lib, capi, H, 24, 8, 16, 72, capacity, planes, seed=4)
+    far = capacity - 1
+    uf, qf = a.rows(1, 5)
+    u, q = a.rows(min(far, 260), 6)
+    st = {}
+    a.run(u, q, 0)
+    a.want(u, np.zeros_like(q), 0, st)
+    d_pos = lib.to_device(np.zeros(1, np.uint32))
+    for p in (t for t in (0, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256) if t < len(u)):
+        want = a.want(u[p:p + 1], q[p:p + 1], p, {k: v[:p] for k, v in st.items()})
+        for dev in (False, True):
+            a.run(uf, 30 * qf, far)
+            d_pos.upload(np.array([p], np.uint32))
+            s = a.run(u[p:p + 1], q[p:p + 1], p, d_pos if dev else None)
+            close(s, want, tol)
+            assert not dev or np.array_equal(s, host)
+            host = s
+
+
 # ---- norms of what a sublayer wrote, activations, token rows ---------------------------------------
 
 @pytest.mark.parametrize("n,parts,K,N", [(96, 1, 96, 40), (60, 5, 64, 33), (105, 7, 128, 520), (2048, 8, 2048, 1000), (384, 96, 384, 16),
