@@ -166,9 +166,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
       }
       frag16 p[3];
       split3(x0, x1, p);
-      // the weights are the first operand: the tile comes out transposed, four consecutive columns of a row to a lane
+      // the weights are the first operand: the tile comes out transposed, four consecutive columns of a row to a lane.
+      // The small terms first: the matrix pipe truncates to the accumulator's size, so of a short chain's roundings two are small
+      // (error of 28 steps over eight wavefronts 1.32e-7 -> 1.12e-7, of 56 1.72e-7 -> 1.57e-7, no time)
 #pragma unroll
-      for (int e = 0; e < 3; e++)
+      for (int e = 2; e >= 0; e--)
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[t][j] = mma(w[u][j], p[e], acc[t][j]);
       if (TM * TN >= 12) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
@@ -615,7 +617,8 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 // kernel it would take instead.
 //
 // bf16, fitted to 13980 runs (9 to 256 rows, 256 to 33000 columns, K 256 to 18944; error 8 to 13 %; the shape it chooses is 2 %
-// slower than the fastest one on average): a launch costs 2.1 us and its weights' way from HBM; a block starts and ends in
+// slower than the fastest one on average; 150 shapes of 129 to 1024 rows 0.985 to 23 times as fast as the 128-row tiles, 2.2 on
+// average: 300 x 1152 x 896 20.9 -> 6.6 us, 300 x 4864 gated x 896 34.2 -> 27.4, 1024 x 896 x 4864 36.4 -> 36.2): a launch costs 2.1 us and its weights' way from HBM; a block starts and ends in
 // a time that grows with its sums; a step of its wavefronts takes the CU's loads of activations and weights, a little less where
 // CUs are idle; blocks that share a CU cost half again each, nearly twice where their steps are many.
 static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
@@ -626,6 +629,13 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
   const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / rows::kStep, t16 = cdiv(M, 16);
   const double own_sum = gu || N > 8192 ? 5 : 0;   // a launch that adds up (a narrow product is planned as if left as parts, whose
                                                    // sum its consumer forms: the two are the same bits)
+  // The error of a sum grows with a wavefront's chain of matrix instructions: 1.1e-7 of the result after 4 steps of 32 k, 1.6e-7
+  // after 7, 1.75e-7 after 9. The 128-row tiles, which split K up to 16 times, have 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192,
+  // 3.0e-7 at 12288, few rows in shorter chains 1.2e-7: no chain here is longer than gives that. (A gated product of 17 to 128
+  // rows that has a block for every CU is not split for it, the sum being a launch: the 64-row tiles do not either.)
+  const int64_t chain = M > 128 ? std::max<int64_t>(8, cdiv(units, 16)) : gu ? 8 : std::max<int64_t>(6, cdiv(units, 16));
+  const int most_S = (int)std::min<int64_t>(max_S, units), chain_S = (int)cdiv(units, rows::kWaves * chain);
+  if (M > 128 && chain_S > most_S) return best;
   double least = 0;
   const int64_t few = cdiv(t16, rows::kMaxTM);
   for (int64_t row_blocks = few; row_blocks <= std::min(few + 1, t16); row_blocks++)
@@ -634,8 +644,9 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
       const int64_t tiles = cdiv(rows_w, 16 * TN), fit = kFit[TM - 1][TN - 1], at_once = fit * cus;
       if (row_blocks > few && t16 <= 4 && tiles * few > cus / 2) continue;   // (weights read twice for CUs that are busy anyway)
       const int64_t unsplit = tiles * row_blocks;
-      const int most = unsplit >= cus ? 1 : (int)std::min<int64_t>(max_S, units);   // (K is split no further than keeps every CU busy)
-      for (int S = 1; S <= most && (S == 1 || unsplit * (S - 1) < cus); S++) {
+      // (K is split no further than keeps every CU busy)
+      const int least_S = gu && M > 16 && M <= 128 && tiles >= cus ? 1 : std::min(chain_S, most_S);
+      for (int S = least_S; S <= most_S && (S == least_S || unsplit * (S - 1) < cus); S++) {
         const int64_t blocks = unsplit * S;
         const int per = ((int)units + S - 1) / S;
         if (((int)units + per - 1) / per != S) continue;

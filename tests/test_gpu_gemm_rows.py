@@ -14,7 +14,8 @@ SHAPES = [(1, 16, 128), (2, 33, 128), (5, 200, 256), (16, 896, 896), (17, 130, 1
           (65, 100, 128), (77, 896, 4864), (80, 36, 2048), (81, 260, 384), (97, 128, 896), (128, 72, 640),
           (9, 18500, 128), (16, 18300, 128), (60, 33000, 128),
           # above 128 rows (bf16), three column tiles, one step of activations in flight and four (one row tile, few columns)
-          (129, 100, 896), (161, 48, 384), (255, 1200, 512), (256, 33, 4096), (7, 16, 12288), (11, 40, 9216)]
+          (129, 100, 896), (161, 48, 384), (255, 1200, 512), (256, 33, 4096), (7, 16, 12288), (11, 40, 9216),
+          (257, 1152, 896), (336, 100, 2560), (401, 36, 4864), (1024, 48, 384), (1025, 40, 128)]
 
 
 def _weights(orc, fmt, N, K, seed):
@@ -58,7 +59,7 @@ def test_plain_and_parts(lib, orc, fmt, M, N, K):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "q4"])
-@pytest.mark.parametrize("M,ff,K", [(1, 8, 128), (5, 4864, 896), (16, 100, 128), (33, 31, 256), (77, 4864, 896), (81, 200, 384), (128, 17, 128),
+@pytest.mark.parametrize("M,ff,K", [(1, 8, 128), (5, 4864, 896), (16, 100, 128), (33, 31, 256), (77, 4864, 896), (81, 200, 384), (128, 17, 128), (300, 200, 896), (16, 40, 4864), (40, 72, 4864),
                                     (150, 4864, 896), (200, 25, 1024)])
 def test_gated(lib, orc, fmt, M, ff, K):
     print("case gemm_rows gated", fmt, M, ff, K, flush=True)
