@@ -167,10 +167,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
       frag16 p[3];
       split3(x0, x1, p);
       // the weights are the first operand: the tile comes out transposed, four consecutive columns of a row to a lane.
-      // The small terms first: the matrix pipe truncates to the accumulator's size, so of a short chain's roundings two are small
-      // (error of 28 steps over eight wavefronts 1.32e-7 -> 1.12e-7, of 56 1.72e-7 -> 1.57e-7, no time)
+      // (The small terms first would have 0.85 of the spread, but rounding goes one way and three times the mean error adds up over
+      // the layers: a 0.5B prompt 2.2e-7 -> 2.8e-7.)
 #pragma unroll
-      for (int e = 2; e >= 0; e--)
+      for (int e = 0; e < 3; e++)
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[t][j] = mma(w[u][j], p[e], acc[t][j]);
       if (TM * TN >= 12) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
@@ -629,8 +629,8 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
   const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / rows::kStep, t16 = cdiv(M, 16);
   const double own_sum = gu || N > 8192 ? 5 : 0;   // a launch that adds up (a narrow product is planned as if left as parts, whose
                                                    // sum its consumer forms: the two are the same bits)
-  // The error of a sum grows with a wavefront's chain of matrix instructions: 1.1e-7 of the result after 4 steps of 32 k, 1.6e-7
-  // after 7, 1.75e-7 after 9. The 128-row tiles, which split K up to 16 times, have 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192,
+  // The error of a sum grows with a wavefront's chain of matrix instructions: 1.3e-7 of the result after 4 steps of 32 k, 1.7e-7
+  // after 7, 2.0e-7 after 10. The 128-row tiles, which split K up to 16 times, have 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192,
   // 3.0e-7 at 12288, few rows in shorter chains 1.2e-7: no chain here is longer than gives that. (A gated product of 17 to 128
   // rows that has a block for every CU is not split for it, the sum being a launch: the 64-row tiles do not either.)
   const int64_t chain = M > 128 ? std::max<int64_t>(8, cdiv(units, 16)) : gu ? 8 : std::max<int64_t>(6, cdiv(units, 16));
