@@ -633,7 +633,7 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
   // after 7, 2.0e-7 after 10. The 128-row tiles, which split K up to 16 times, have 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192,
   // 3.0e-7 at 12288, few rows in shorter chains 1.2e-7: no chain here is longer than gives that. (A gated product of 17 to 128
   // rows that has a block for every CU is not split for it, the sum being a launch: the 64-row tiles do not either.)
-  const int64_t chain = M > 128 ? std::max<int64_t>(8, cdiv(units, 16)) : gu ? 8 : std::max<int64_t>(6, cdiv(units, 16));
+  const int64_t chain = M > 128 ? std::max<int64_t>(7, units * 7 / 128) : gu ? 8 : std::max<int64_t>(6, cdiv(units, 16));
   const int most_S = (int)std::min<int64_t>(max_S, units), chain_S = (int)cdiv(units, rows::kWaves * chain);
   if (M > 128 && chain_S > most_S) return best;
   double least = 0;
