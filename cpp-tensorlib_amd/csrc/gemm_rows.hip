@@ -617,7 +617,7 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 // kernel it would take instead.
 //
 // bf16, fitted to 13980 runs (9 to 256 rows, 256 to 33000 columns, K 256 to 18944; error 8 to 13 %; the shape it chooses is 2 %
-// slower than the fastest one on average; 150 shapes of 129 to 1024 rows 0.985 to 23 times as fast as the 128-row tiles, 2.2 on
+// slower than the fastest one on average; 150 shapes of 129 to 1024 rows 0.85 (two) to 3.2 times as fast as the 128-row tiles, 1.7 on
 // average: 300 x 1152 x 896 20.9 -> 6.6 us, 300 x 4864 gated x 896 34.2 -> 27.4, 1024 x 896 x 4864 36.4 -> 36.2): a launch costs 2.1 us and its weights' way from HBM; a block starts and ends in
 // a time that grows with its sums; a step of its wavefronts takes the CU's loads of activations and weights, a little less where
 // CUs are idle; blocks that share a CU cost half again each, nearly twice where their steps are many.
