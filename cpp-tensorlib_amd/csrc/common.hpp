@@ -48,6 +48,8 @@ struct Context {
 };
 
 Context& ctx();
+// (plans can be asked for without a device)
+inline int cu_count() { return ctx().cus > 0 ? ctx().cus : 256; }
 int fail(int code, const char* fmt, ...);   // records the message, returns code
 int hip_fail(hipError_t e, const char* what);
 void* scratch(size_t bytes);                // nullptr on allocation failure

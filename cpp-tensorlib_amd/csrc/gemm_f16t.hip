@@ -28,6 +28,7 @@
 // (tensorlib_cuda.cu:509-519).
 #include "gemm_shared.hpp"
 #include "gemv_shared.hpp"
+#include "../../include/tensorlib_hip_bench.h"
 
 namespace tlhip {
 namespace f16t {
@@ -691,6 +692,84 @@ namespace {
 
 int64_t cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// A piece is a range of tile columns in tiles of one height (128 tmh rows), K split S ways.
+struct Piece { int64_t tn0, tcols; int S; int tmh; };
+struct Plan { Piece pieces[2]; int npieces; };
+
+// How a product of M rows is cut: N columns, or gated features (gu); want_parts: left as parts, in one piece.
+Plan plan_f16w(int64_t M, int64_t N, int64_t K, bool gu, bool want_parts, size_t parts_bytes) {
+  const int64_t nslab = K / f16t::kBK, tn = cdiv64(N, gu ? f16t::kTile / 2 : f16t::kTile);
+  const int64_t slots = cu_count();                 // one block per CU
+  const int64_t tm256 = cdiv64(M, 256), tm128 = cdiv64(M, 128);
+  const bool can_split = (N % 4) == 0;              // the part sums work on float4s
+  const auto room = [&](int64_t S) { return !want_parts || S == 1 || (size_t)S * M * N * sizeof(float) <= parts_bytes; };
+  // What a launch of a piece takes (us), fitted to 4079 runs of
+  // 100 to 1024 rows, 4 to 200 tile columns, K 1024 to 18944 (error 5 % and 3.5 %): a start, for every round of the CUs a block's own
+  // start and end and its slabs - slower the more CUs are busy: their clock falls - and the megabytes stored.
+  struct Cost { double start, block, slab, busy, mb; };
+  static constexpr Cost kCost[2] = {{2.0, 8.7, 0.527, 0.335, 0.104}, {4.4, 11.9, 1.108, 0.545, 0.137}};   // tiles of 128 and of 256 rows
+  const auto piece_us = [&](int64_t tcols, int tmh, int64_t S) {
+    const Cost& k = kCost[tmh - 1];
+    const int64_t blocks = (tmh == 1 ? tm128 : tm256) * tcols * S;
+    const double slabs = (double)cdiv64(nslab, S), rest = (double)(blocks % slots) / (double)slots, mb = 4e-6 * (double)M * f16t::kTile * (double)tcols;
+    double us = k.start + (double)(blocks / slots) * (k.block + slabs * (k.slab + k.busy)) + k.mb * (double)S * mb;
+    if (rest > 0) us += k.block + slabs * (k.slab + k.busy * rest);
+    // parts are read by what adds them up: a launch of its own, or a norm that is there anyway, a few rows to a CU and less able
+    // to hide it (nine parts for four of 512 x 3584 cost it 14 us)
+    return us + (S > 1 ? (want_parts ? 0.35 * (double)S * mb : 2.5 + 0.12 * (double)(S + 1) * mb) : 0.0);
+  };
+  // The error of a sum grows with its chain of slabs (512 x 4048 gated features x 1024: 3.2e-7 of the result in chains of 16, 4.5e-7 of
+  // 32), and the plan that takes least time would trade it. So no plan has longer chains, over its tile columns, than the one that
+  // only fills the CUs: whole rounds of 256-row tiles unsplit, the columns left over, or all if they make no round, split
+  // up to 16 ways. Most shapes take the same time so (744 x 4824 x 1408 in parts 46 us unbounded and 36 bounded, 384 x 3584 x 3584 39
+  // and 35); products of a round and a bit pay: 300 x 18944 gated x 3584 196 and 215, 309 x 39300 x 1056 73 and 95.
+  const auto filled = [&](int64_t tcols) {
+    const int64_t t = (tm256 * tcols * 2 <= slots ? tm128 : tm256) * tcols;
+    int64_t S = can_split && t < slots ? std::min<int64_t>(16, slots / t) : 1;
+    while (S > 1 && (nslab / S < 8 || !room(S))) S--;
+    return tcols * cdiv64(nslab, S);
+  };
+  int64_t chains = filled(tn);
+  if (const int64_t per_round = slots / tm256; tm256 * tn > slots && per_round > 0 && can_split && !want_parts) {
+    const int64_t whole = tn / per_round * per_round;
+    chains = whole * nslab + (whole < tn ? filled(tn - whole) : 0);
+  }
+  // The columns from tn0 on in one piece, as it takes least; S == 0: not in chains so short.
+  const auto best = [&](int64_t tn0, int64_t longest, double& us) {
+    Piece P{tn0, tn - tn0, 0, 1};
+    for (int tmh = 1; tmh <= 2; tmh++)
+      for (int64_t want = 1; want <= (can_split ? 16 : 1) && (want == 1 || nslab / want >= 8); want++) {   // at least 256 k per part
+        const int64_t S = cdiv64(nslab, cdiv64(nslab, want));
+        if (!room(S)) break;
+        if (P.tcols * cdiv64(nslab, S) > longest) continue;
+        const double t = piece_us(P.tcols, tmh, S);
+        if (P.S == 0 || t < us) us = t, P.S = (int)S, P.tmh = tmh;
+      }
+    return P;
+  };
+  // One piece, or the columns that make whole rounds of the CUs without a split and the others as a second one: 512 x 16640 x 3584
+  // 64 columns of 128-row tiles and one split 14 ways (118 us) where 130 blocks of 256 rows took 159 to 176.
+  double least = 0;
+  Plan plan{{best(0, chains, least), Piece{}}, 1};
+  if (!want_parts && can_split)
+    for (int tmh = 1; tmh <= 2; tmh++) {
+      const int64_t per_round = slots / (tmh == 1 ? tm128 : tm256);
+      if (per_round == 0) continue;
+      for (int64_t back = 0; back < 2; back++) {   // as many rounds as there are, or one fewer
+        const int64_t cols = (tn / per_round - back) * per_round;
+        if (cols <= 0 || cols >= tn) continue;
+        double rest = 0;
+        const Piece tail = best(cols, chains - cols * nslab, rest);
+        const double us = piece_us(cols, tmh, 1) + rest;
+        if (tail.S > 0 && (plan.pieces[0].S == 0 || us < least)) {
+          least = us;
+          plan = Plan{{Piece{0, cols, 1, tmh}, tail}, 2};
+        }
+      }
+    }
+  return plan;
+}
+
 // plain: C[M][N]; parts (S_out != nullptr): C is the caller's [S][M][N]; gated: N = features, C[M][N] the activation
 // aimg_in: the activation image of A made before (tlhip_rmsnorm_res_parts_aimage), or nullptr: made here
 int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, int64_t M, int64_t N, int64_t K,
@@ -708,62 +787,10 @@ int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, 
   Context& c = ctx();
   const int per = gu ? 2 : 1;                       // tile columns per unit of N
   const int64_t w = f16t::kTile / per;              // units of N per column tile
-  const int64_t nslab = K / f16t::kBK, tn = cdiv64(N, w);
-  const int64_t slots = c.cus;                      // one block per CU
-  const int64_t tm256 = cdiv64(M, 256), tm128 = cdiv64(M, 128);
-  const bool can_split = (N % 4) == 0;              // the part sums work on float4s
-  // A piece is a range of tile columns in tiles of one height, K split S ways. What a launch of one takes (us), fitted to 4079 runs of
-  // 100 to 1024 rows, 4 to 200 tile columns, K 1024 to 18944 (error 5 % and 3.5 %): a start, for every round of the CUs a block's own
-  // start and end and its slabs - slower the more CUs are busy: their clock falls - and the megabytes stored.
-  struct Piece { int64_t tn0, tcols; int S; int tmh; };
-  struct Cost { double start, block, slab, busy, mb; };
-  static constexpr Cost kCost[2] = {{2.0, 8.7, 0.527, 0.335, 0.104}, {4.4, 11.9, 1.108, 0.545, 0.137}};   // tiles of 128 and of 256 rows
-  const auto piece_us = [&](int64_t tcols, int tmh, int64_t S) {
-    const Cost& k = kCost[tmh - 1];
-    const int64_t blocks = (tmh == 1 ? tm128 : tm256) * tcols * S;
-    const double slabs = (double)cdiv64(nslab, S), rest = (double)(blocks % slots) / (double)slots, mb = 4e-6 * (double)M * f16t::kTile * (double)tcols;
-    double us = k.start + (double)(blocks / slots) * (k.block + slabs * (k.slab + k.busy)) + k.mb * (double)S * mb;
-    if (rest > 0) us += k.block + slabs * (k.slab + k.busy * rest);
-    // parts are read by what adds them up: a launch of its own, or a norm that is there anyway, a few rows to a CU and less able
-    // to hide it (nine parts for four of 512 x 3584 cost it 14 us)
-    return us + (S > 1 ? (want_parts ? 0.35 * (double)S * mb : 2.5 + 0.12 * (double)(S + 1) * mb) : 0.0);
-  };
-  // The columns from tn0 on in one piece, as it takes least.
-  const auto best = [&](int64_t tn0, double& us) {
-    Piece P{tn0, tn - tn0, 1, 1};
-    us = piece_us(P.tcols, 1, 1);
-    for (int tmh = 1; tmh <= 2; tmh++)
-      for (int64_t want = 1; want <= (can_split ? 16 : 1) && (want == 1 || nslab / want >= 8); want++) {   // at least 256 k per part
-        const int64_t S = cdiv64(nslab, cdiv64(nslab, want));
-        if (want_parts && S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) break;
-        const double t = piece_us(P.tcols, tmh, S);
-        if (t < us) us = t, P.S = (int)S, P.tmh = tmh;
-      }
-    return P;
-  };
-  // One piece, or the columns that make whole rounds of the CUs without a split and the others as a second one: 512 x 16640 x 3584
-  // 64 columns of 128-row tiles and one split 14 ways (118 us) where 130 blocks of 256 rows took 159 to 176.
-  Piece pieces[2];
-  int npieces = 1;
-  double least;
-  pieces[0] = best(0, least);
-  if (!want_parts && can_split)
-    for (int tmh = 1; tmh <= 2; tmh++) {
-      const int64_t per_round = slots / (tmh == 1 ? tm128 : tm256);
-      if (per_round == 0) continue;
-      for (int64_t back = 0; back < 2; back++) {   // as many rounds as there are, or one fewer
-        const int64_t cols = (tn / per_round - back) * per_round;
-        if (cols <= 0 || cols >= tn) continue;
-        double rest;
-        const Piece tail = best(cols, rest);
-        if (piece_us(cols, tmh, 1) + rest < least) {
-          least = piece_us(cols, tmh, 1) + rest;
-          pieces[0] = Piece{0, cols, 1, tmh};
-          pieces[1] = tail;
-          npieces = 2;
-        }
-      }
-    }
+  const int64_t nslab = K / f16t::kBK, tm256 = cdiv64(M, 256), tm128 = cdiv64(M, 128);
+  const Plan plan = plan_f16w(M, N, K, gu, want_parts, parts_bytes);
+  const int npieces = plan.npieces;
+  const Piece* const pieces = plan.pieces;
   // scratch: exponents of A's rows, the slab images of A, room for the largest piece's parts
   const size_t ea_bytes = ((size_t)M * sizeof(int) + 1023) & ~(size_t)1023;
   const int64_t timg = cdiv64(M, f16t::kTile);      // activation images are 256 rows tall
@@ -857,6 +884,18 @@ int gemm_f16w_impl(const void* A, const void* image, const void* exps, void* C, 
 }  // namespace
 
 extern "C" {
+
+int tlhip_plan_gemm_f16w(int64_t M, int64_t N, int64_t K, int gated, int parts, int64_t pieces[8]) {
+  if (!pieces || M <= 0 || N <= 0 || K <= 0 || K % f16t::kBK != 0 || parts < 0)
+    return fail(TLHIP_EINVAL, "tlhip_plan_gemm_f16w: bad arguments");
+  const Plan P = plan_f16w(M, N, K, gated != 0, parts > 0, (size_t)parts * M * N * sizeof(float));
+  for (int i = 0; i < 2; i++) {
+    const Piece p = i < P.npieces ? P.pieces[i] : Piece{0, 0, 0, 0};
+    const int64_t v[4] = {p.tcols, p.S, p.S > 0 ? cdiv64(K / f16t::kBK, p.S) : 0, 128 * p.tmh};
+    std::copy(v, v + 4, pieces + 4 * i);
+  }
+  return TLHIP_OK;
+}
 
 int64_t tlhip_gemm_f16w_bytes(int64_t N, int64_t K, int gated) {
   if (N <= 0 || K <= 0 || (K % f16t::kBK) != 0) return 0;

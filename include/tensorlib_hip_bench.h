@@ -62,6 +62,10 @@ int tlhip_tune_attn_decode(int kernel);
  * choice (two f16 terms), 3 = three bf16 terms. Same results within fp32 summation order; for A/B
  * timing and tests. */
 int tlhip_tune_gemm_planes(int planes);
+/* How a product over a prepared weight (tlhip_gemm_f16w_nt, or gated its _swiglu and _geglu forms with N features; parts > 0: the
+ * _parts form with room for so many) is cut: of each of up to two pieces its tile columns, K splits, the 32-k slabs that are
+ * summed in a row and the tiles' rows. On the host alone, also without a device (then as for 256 CUs). */
+int tlhip_plan_gemm_f16w(int64_t M, int64_t N, int64_t K, int gated, int parts, int64_t pieces[8]);
 /* Every override back to the built-in choice (tlhip_tune_gemv_cols included). */
 int tlhip_tune_reset(void);
 
