@@ -158,6 +158,7 @@ SIGNATURES = {
     "tlhip_tune_gemv_cols": (cint, [cint]),
     "tlhip_tune_attn_prefill": (cint, [cint]),
     "tlhip_tune_gemm_planes": (cint, [cint]),
+    "tlhip_plan_gemm_bf16": (cint, [i64, i64, i64, cint, cint, C.POINTER(cint)]),
     "tlhip_plan_gemm_f16w": (cint, [i64, i64, i64, cint, cint, P]),
     "tlhip_tune_reset": (cint, []),
     "tlhip_bench_copy": (cint, [P, P, sz, cint]),
@@ -689,6 +690,12 @@ class TlHip:
     def tune_gemm_planes(self, planes):
         """3: the int4 prompt GEMMs cut activations into three bf16 terms; 0: built-in choice (two f16)."""
         self._chk(self.c.tlhip_tune_gemm_planes(int(planes)))
+
+    def plan_gemm_bf16(self, M, N, K, gated=False, parts=0):
+        """(the kernel of few rows?, its row tiles, its column tiles, K splits, longest chain of 32-k steps)"""
+        v = (cint * 5)()
+        self._chk(self.c.tlhip_plan_gemm_bf16(M, N, K, int(gated), parts, v))
+        return tuple(v)
 
     def plan_gemm_f16w(self, M, N, K, gated=False, parts=0):
         """The pieces of a product over a prepared weight: (tile columns, K splits, slabs in a row, rows of a tile) of each."""

@@ -612,30 +612,66 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 
 }  // namespace rows
 
+// The longest chain of matrix instructions, in steps of 32 k, that a wavefront may form a sum of bf16 products by. The error of a sum
+// grows with it (1.0e-7 of the result after a step, 1.3e-7 after 4, 1.7e-7 after 7, 2.0e-7 after 10), and the plan that takes
+// least time would trade it: few rows' products of K 896 run as fast unsplit on narrow column tiles, in chains of 4 (24 x 1152 x 896
+// 1.3e-7 of error for 0.9e-7). So K is split at least as far as fills the CUs by blocks of wide tiles, where that does not cost more
+// than it gives. Up to 128 rows that is what an estimate fitted to 280 runs says (K 384 .. 18944, N 384 .. 37888, M 8 .. 120: clocks
+// of a step by the CU's vector memory path or its matrix or vector instructions, 3500 and 60 per accumulator tile for a block, parts
+// written and read, a launch that adds them up); wide products, which have a block for every CU, stay whole: 18960 x 2048 at 32 rows takes
+// 33.6 us in two parts. Above, the 128-row tiles, which run what does not come here, split K up to 16 times and have
+// 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192, 3.0e-7 at 12288.
+static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t rows_w = (gu ? 2 : 1) * N, cus = cu_count(), units = K / rows::kStep, t16 = cdiv(M, 16), row_blocks = cdiv(t16, rows::kMaxTM);
+  if (M > 128) return std::max<int64_t>(7, units * 7 / 128);
+  const int TM = (int)cdiv(t16, row_blocks);
+  double least = 0;
+  int64_t chain = 0;
+  for (int TN = 4; TN >= (gu ? 2 : 1); TN /= 2) {
+    const int64_t blocks1 = cdiv(rows_w, 16 * TN) * row_blocks;
+    for (int64_t S = 1; S <= std::min<int64_t>(max_S, units); S++) {
+      const int64_t per = cdiv(units, S), blocks = blocks1 * S, n = cdiv(per, rows::kWaves);
+      if (cdiv(units, per) != S) continue;
+      if (S > 1 && M > 16 && blocks1 > cus) break;
+      const double clocks = (double)n * std::max(96.0 * TM * TN, std::max(352.0 * TM, 8 * (70.0 * TM + 60.0 * TN))) + 3500 + 60 * TM * TN;
+      const double rounds = blocks <= cus ? 1 : 1.2 * (blocks <= 4 * cus ? (double)cdiv(blocks, cus) : (double)blocks / cus);
+      const double us = rounds * clocks / 2100 + (S > 1 ? 1e-6 * (double)(S * M * rows_w) + (gu || N > 8192 ? 5 : 0) : 0);
+      if (chain == 0 || us < least) {
+        least = us;
+        chain = n;
+      }
+    }
+  }
+  return chain;
+}
+
 // Row tiles per block, columns per tile and K splits that an estimate of the time likes best; S == 0 where the shape is not
 // taken. `us` is the chosen plan's time, the launch that adds parts up not included: the caller weighs it against the time of the
 // kernel it would take instead.
 //
-// bf16, fitted to 13980 runs (9 to 256 rows, 256 to 33000 columns, K 256 to 18944; error 8 to 13 %; the shape it chooses is 2 %
-// slower than the fastest one on average; 150 shapes of 129 to 1024 rows 0.85 (two) to 3.2 times as fast as the 128-row tiles, 1.7 on
-// average: 300 x 1152 x 896 20.9 -> 6.6 us, 300 x 4864 gated x 896 34.2 -> 27.4, 1024 x 896 x 4864 36.4 -> 36.2): a launch costs 2.1 us and its weights' way from HBM; a block starts and ends in
-// a time that grows with its sums; a step of its wavefronts takes the CU's loads of activations and weights, a little less where
-// CUs are idle; blocks that share a CU cost half again each, nearly twice where their steps are many.
+// bf16: a launch costs a start and its weights' way from HBM; a block starts and ends in a time that grows with its sums, and each
+// costs a little for its dispatch; a step of its wavefronts takes the CU's loads of activations and weights, a little less where
+// CUs are idle; blocks that share a CU cost half again each, more where their steps are many. Fitted up to 128 rows to 25000
+// runs in the chains allowed (2 to 128 rows, 256 to 16000 columns, K 256 to 18944: error 8 %, the shape it chooses 1.1 % slower than the
+// fastest one on average and 1.15 times at most), above to 13980 others, all of it times 1.1 (12800 runs of 129 to 1024 rows: error 9 %, 1.1 %).
 static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
   // blocks of [row tiles][column tiles] that fit a CU (registers, LDS)
   static constexpr int kFit[5][4] = {{4, 3, 2, 2}, {4, 2, 2, 1}, {3, 2, 1, 1}, {2, 2, 1, 1}, {2, 1, 1, 1}};
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   RowsPlan best;
-  const int64_t rows_w = (gu ? 2 : 1) * N, cus = ctx().cus, units = K / rows::kStep, t16 = cdiv(M, 16);
-  const double own_sum = gu || N > 8192 ? 5 : 0;   // a launch that adds up (a narrow product is planned as if left as parts, whose
-                                                   // sum its consumer forms: the two are the same bits)
-  // The error of a sum grows with a wavefront's chain of matrix instructions: 1.3e-7 of the result after 4 steps of 32 k, 1.7e-7
-  // after 7, 2.0e-7 after 10. The 128-row tiles, which split K up to 16 times, have 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192,
-  // 3.0e-7 at 12288, few rows in shorter chains 1.2e-7: no chain here is longer than gives that. (A gated product of 17 to 128
-  // rows that has a block for every CU is not split for it, the sum being a launch: the 64-row tiles do not either.)
-  const int64_t chain = M > 128 ? std::max<int64_t>(7, units * 7 / 128) : gu ? 8 : std::max<int64_t>(6, cdiv(units, 16));
+  const int64_t rows_w = (gu ? 2 : 1) * N, cus = cu_count(), units = K / rows::kStep, t16 = cdiv(M, 16);
+  struct Cost { double start, share, share_n, steps, fill, whole, rows, cols, idle, sums, dispatch, parts, weights, all; };
+  static constexpr Cost kFew = {2.33, 0.40, 0.35, 20, 0.77, 0, 0.229, 0.184, 0.827, 0.165, 0.317, 0, 0.051, 1};
+  static constexpr Cost kMany = {2.08, 0.424, 0.593, 10, 0.86, 0.086, 0.194, 0.182, 0.877, 0.144, 0, 0.179, 0.103, 1.1};
+  const Cost& k = M > 128 ? kMany : kFew;
+  // What adds the parts up beside reading them: a launch, or where a narrow product is left as parts their consumer. (Both
+  // forms of a narrow product take one plan: two products of this kernel with room for as many parts are the same bits.)
+  const double own_sum = gu || N > 8192 ? 5.4 : M > 128 ? 0.4 : 1.3;
+  const int64_t chain = longest_chain(M, N, K, gu, max_S);
   const int most_S = (int)std::min<int64_t>(max_S, units), chain_S = (int)cdiv(units, rows::kWaves * chain);
-  if (M > 128 && chain_S > most_S) return best;
+  // (where K cannot be split so far, the tiles cannot split it either, and their chains are eight times as long)
+  const int least_S = (int)cdiv(units, cdiv(units, std::min(chain_S, most_S)));
   double least = 0;
   const int64_t few = cdiv(t16, rows::kMaxTM);
   for (int64_t row_blocks = few; row_blocks <= std::min(few + 1, t16); row_blocks++)
@@ -645,24 +681,28 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
       if (row_blocks > few && t16 <= 4 && tiles * few > cus / 2) continue;   // (weights read twice for CUs that are busy anyway)
       const int64_t unsplit = tiles * row_blocks;
       // (K is split no further than keeps every CU busy)
-      const int least_S = gu && M > 16 && M <= 128 && tiles >= cus ? 1 : std::min(chain_S, most_S);
       for (int S = least_S; S <= most_S && (S == least_S || unsplit * (S - 1) < cus); S++) {
         const int64_t blocks = unsplit * S;
         const int per = ((int)units + S - 1) / S;
         if (((int)units + per - 1) / per != S) continue;
-        const double n = (double)((per + rows::kWaves - 1) / rows::kWaves);   // steps of a wavefront
-        const auto share = [&](int64_t on_a_cu) { return 1 + (0.424 + 0.593 * n / (n + 10)) * (double)(on_a_cu - 1); };
+        const int steps = (per + rows::kWaves - 1) / rows::kWaves;   // of a wavefront
+        // (up to 128 rows no split that leaves them as many: parts are added one after the other, which costs a rounding each - 22 x 68
+        // gated x 1600, 50 steps, 1.75e-7 of error in 13 parts and 1.51e-7 in 7)
+        if (M <= 128 && S > least_S && ((int)units + rows::kWaves * steps - 1) / (rows::kWaves * steps) != S) continue;
+        const double n = (double)steps;
+        const auto share = [&](int64_t on_a_cu) { return 1 + (k.share + k.share_n * n / (n + k.steps)) * (double)(on_a_cu - 1); };
         double rounds = 1;
         if (blocks > cus) {
           const int64_t rest = blocks % at_once;
-          const double fill = blocks > at_once ? 0.86 + 0.14 * (double)rest / (double)at_once : 1;   // of the last round
+          const double fill = blocks > at_once ? k.fill + (1 - k.fill) * (double)rest / (double)at_once : 1;   // of the last round
           rounds = (double)(blocks / at_once) * share(fit) + (rest > 0 ? share(cdiv(rest, cus)) * fill : 0);
         }
-        const double work = (0.086 * n + 0.914 * (double)per / rows::kWaves) * (0.194 * TM + 0.182 * TN) *
-                            (0.877 + 0.123 * std::min(1.0, (double)blocks / (double)cus));
+        const double work = (k.whole * n + (1 - k.whole) * (double)per / rows::kWaves) * (k.rows * TM + k.cols * TN) *
+                            (k.idle + (1 - k.idle) * std::min(1.0, (double)blocks / (double)cus));
         const double parts = S > 1 ? (double)S * M * (gu ? tiles * 16 * TN : N) * 4e-6 : 0;   // MB
-        const double us = 2.08 + rounds * (0.144 * TM * TN + work) + 0.179 * parts + 0.103 * 2e-6 * (double)rows_w * (double)K;
-        const double all = us + 0.25 * parts + (S > 1 ? 0.4 + own_sum : 0);
+        const double us = k.start + rounds * (k.sums * TM * TN + work) + k.dispatch * (double)blocks / (double)cus + k.parts * parts +
+                          k.weights * 2e-6 * (double)rows_w * (double)K;
+        const double all = us + 0.25 * parts + (S > 1 ? own_sum : 0);
         if (best.S == 0 || all < least) {
           least = all;
           best.TM = TM;
@@ -671,7 +711,7 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
           best.tiles = (int)tiles;
           best.row_blocks = (int)row_blocks;
           best.part_units = (int)per;
-          best.us = 1.05 * us;                     // (for the errors of both estimates it is weighed against)
+          best.us = 1.05 * k.all * us;             // (5 % for the errors of both estimates it is weighed against)
         }
       }
     }

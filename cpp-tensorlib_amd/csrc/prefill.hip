@@ -21,6 +21,7 @@
 // multiplied.
 #include "gemm_shared.hpp"
 #include "gemv_shared.hpp"
+#include "../../include/tensorlib_hip_bench.h"
 
 namespace tlhip {
 
@@ -494,6 +495,117 @@ void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t
                                                             (int)(n / 4), (int)(ldc / 4), S);
 }
 
+// Columns (features) [n0, n0 + n) in tiles of one variant, K split S ways.
+struct Piece { int64_t n0, n; int S; int variant; };
+static const int kBm[4] = {128, 64, 64, 128}, kBn[4] = {256, 128, 64, 128};   // rows and columns of a variant's tile
+// Which kernel forms a product: the rows kernel where rows.S > 0, else the images' where `images`, else the tiles here in pieces.
+struct Choice {
+  Piece pieces[2];
+  int npieces = 0;
+  bool half = false;                   // int4 rows as two f16 planes
+  bool images_fit = false, images = false;
+  Q4Plan q4;
+  RowsPlan rows;
+};
+// aligned: the result is 16-byte aligned.
+static Choice choose_gemm(int64_t M, int64_t N, int64_t K, bool gu, bool q4, bool aligned, bool want_parts, size_t parts_bytes) {
+  // Tile variants {MFMA tiles per wavefront in M, in N}, 2 x 2 wavefronts each. The wide one
+  // (128 x 256 block tile, 64 x 128 per wavefront) needs fewest LDS reads per MFMA - the three
+  // A planes make LDS, not the matrix pipe, the first limit - and runs 2 blocks per CU.
+  // Work is shaped to fill those 2 * CUs block slots in whole rounds:
+  //   * fewer tiles than slots: K is split over gridDim.y so that tiles * S comes close to
+  //     the slots; parts go to scratch and are summed in a fixed order (no atomics);
+  //   * more tiles than slots: the columns that make whole rounds run with full K, the
+  //     remaining columns (less than one round of tiles) are split over K the same way.
+  // gu: a tile column of bn is bn / 2 features wide (gate and up of each), so all widths below
+  // are in units of N - columns, or features.
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t cus = cu_count(), slots = cus * 2;
+  const int per = gu ? 2 : 1;                             // tile columns per unit of N
+  const bool can_split = (N % 4) == 0 && aligned;        // the part sum works on float4s
+  Choice ch;
+  ch.half = q4 && M > 64 && ctx().tune_gemm_planes != 3;
+  auto& pieces = ch.pieces;
+  int& npieces = ch.npieces;
+  auto pick_S = [&](int64_t tiles) {   // K splits that bring `tiles` blocks up to the slots
+    if (!can_split || tiles >= slots) return 1;
+    int64_t S = slots / tiles;   // never past the slots: a few blocks left for a second round double the launch
+    if (S > 16) S = 16;
+    while (S > 1 && K / S < 256) S--;
+    if (want_parts)   // the caller's buffer bounds the parts
+      while (S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) S--;
+    return (int)S;
+  };
+  if (M > 64) {
+    // int4: two accumulator sets per wavefront, so 64 x 64 wavefront tiles (128 x 128 per block)
+    const int64_t w = (q4 ? 128 : 256) / per;
+    const int wide = q4 ? 3 : 0;
+    const int64_t tm = cdiv(M, 128), tn = cdiv(N, w), tiles = tm * tn;
+    const int64_t cols_per_round = slots / tm;            // whole tile columns in one round
+    if (tiles <= slots || cols_per_round == 0 || !can_split || want_parts) {
+      pieces[npieces++] = Piece{0, N, pick_S(tiles), wide};
+    } else {
+      const int64_t main_tn = tn / cols_per_round * cols_per_round;   // whole rounds
+      const int64_t n_main = main_tn * w;
+      pieces[npieces++] = Piece{0, n_main, 1, wide};
+      if (n_main < N) pieces[npieces++] = Piece{n_main, N - n_main, pick_S(tm * (tn - main_tn)), wide};
+    }
+  } else {
+    // short prompts: 64-row tiles; narrow ones when that is what fills the chip (a gated
+    // tile needs two MFMA tiles per wavefront in N, so the narrow one is not for gu)
+    const int64_t t128 = cdiv(N, 128 / per), t64 = cdiv(N, 64 / per);
+    if (gu || q4 || t128 >= slots || pick_S(t128) > 1) pieces[npieces++] = Piece{0, N, pick_S(t128), 1};
+    else pieces[npieces++] = Piece{0, N, pick_S(t64), 2};
+  }
+  // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
+  // against 50, 301 x 37888 x 3584 209 against 303)
+  ch.images_fit = ch.half && K <= 32768 && (per * N >= 2048 || K <= 1024);
+  bool& images = ch.images;
+  Q4Plan& q4_plan = ch.q4;
+  images = ch.images_fit;
+  if (images) q4_plan = plan_gemm_q4(M, N, K, parts_bytes, want_parts, gu, can_split);
+  const auto part_slabs = [&](const Piece& O) { return cdiv(cdiv(K, O.S), kBK); };
+  const auto part_blocks = [&](const Piece& O) {
+    return cdiv(M, kBm[O.variant]) * cdiv(O.n, kBn[O.variant] / per) * cdiv(cdiv(K, kBK), part_slabs(O));
+  };
+  // Above 128 rows also by what the two take, where the images' tiles are a round and a bit and these are one (us, images and here:
+  // 613 x 6528 x 5248 169 and 134, 705 x 10880 x 3584 in parts 195 and 161, 847 x 9344 x 256 33 and 26). This kernel's time is fitted
+  // to the 11000 runs of plan_gemm_q4 (error 5 %); 5 % are the images', for the errors of both.
+  if (images && M > 128) {
+    double here = 10.1 + 0.9e-6 * (double)M * (double)(per * N) + 7.3 * (npieces - 1);
+    for (int pi = 0; pi < npieces; pi++) {
+      const Piece& O = pieces[pi];
+      here += (double)part_slabs(O) * rounds_us(part_blocks(O), cus, 0.98, 1.22);
+      if (O.S > 1) here += 1.2e-6 * O.S * M * per * O.n + (want_parts ? 0 : 2.7);
+    }
+    images = 0.95 * q4_plan.us < here;
+  }
+  // A few rows: a kernel of their own, above 16 where it is the faster one. What the others take, fitted to 1000 runs (17 to
+  // 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 to 9 %): a start, and a time per 32-k slab with one and two blocks on a CU.
+  if (aligned) {
+    int64_t max_S = can_split ? 16 : 1;
+    if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
+    RowsPlan& P = ch.rows;
+    P = plan_gemm_rows(M, N, K, gu, q4, max_S);
+    if (M > 16 && P.S > 0) {
+      double other = images ? q4_plan.us : 0;
+      for (int pi = 0; !images && pi < npieces; pi++) {
+        const Piece& O = pieces[pi];
+        const int bn = kBn[O.variant];
+        const int64_t slabs = part_slabs(O), blocks = part_blocks(O);
+        if (M <= 64 && q4) other += 2.4 + (double)slabs * slab_us(blocks, cus, 0.965, 1.13);
+        else if (M <= 64) other += 2.2 + (double)slabs * (bn > 64 ? slab_us(blocks, cus, 0.9, 1.12) : slab_us(blocks, cus, 0.65, 0.95)) *
+                                             (bn == 64 && O.S == 1 && blocks > 3 * cus ? 0.85 : 1);   // (four blocks to a CU: 60 x 64982 x 768 32 us, 43 by rows)
+        else if (q4) other += 12.1 + (double)slabs * slab_us(blocks, cus, 1.03, 1.03);
+        else other += (gu && K <= 256 ? 9 : 7) + (double)slabs * slab_us(blocks, cus, 1.5, 2.18);   // (67 x 10732 gated x 128: 16.2 us, 10.8 by rows)
+        if (O.S > 1) other += (M <= 64 ? 0.65e-6 : 0.36e-6) * O.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
+      }
+      if (P.us + (P.S > 1 && !want_parts ? kPartSumUs : 0) > other) P.S = 0;
+    }
+  }
+  return ch;
+}
+
 }  // namespace tlhip
 
 using namespace tlhip;
@@ -528,99 +640,13 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   const float* pa = static_cast<const float*>(A);
   const uint16_t* pw = static_cast<const uint16_t*>(W);
   float* pc = static_cast<float*>(C);
-  // Tile variants {MFMA tiles per wavefront in M, in N}, 2 x 2 wavefronts each. The wide one
-  // (128 x 256 block tile, 64 x 128 per wavefront) needs fewest LDS reads per MFMA - the three
-  // A planes make LDS, not the matrix pipe, the first limit - and runs 2 blocks per CU.
-  // Work is shaped to fill those 2 * CUs block slots in whole rounds:
-  //   * fewer tiles than slots: K is split over gridDim.y so that tiles * S comes close to
-  //     the slots; parts go to scratch and are summed in a fixed order (no atomics);
-  //   * more tiles than slots: the columns that make whole rounds run with full K, the
-  //     remaining columns (less than one round of tiles) are split over K the same way.
-  // gu: a tile column of bn is bn / 2 features wide (gate and up of each), so all widths below
-  // are in units of N - columns, or features.
-  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  const int64_t slots = (int64_t)c.cus * 2;
   const int per = gu ? 2 : 1;                             // tile columns per unit of N
-  const bool can_split = (N % 4) == 0 && aligned16(C);   // the part sum works on float4s
-  const bool half = q4 && M > 64 && c.tune_gemm_planes != 3;
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const Choice ch = choose_gemm(M, N, K, gu, q4, aligned16(C), want_parts, parts_bytes);
+  const bool half = ch.half;
   const size_t ea_bytes = half ? (((size_t)M * sizeof(int) + 255) & ~(size_t)255) : 0;
-  struct Piece { int64_t n0, n; int S; int variant; };    // columns (features) [n0, n0 + n)
-  Piece pieces[2];
-  int npieces = 0;
-  auto pick_S = [&](int64_t tiles) {   // K splits that bring `tiles` blocks up to the slots
-    if (!can_split || tiles >= slots) return 1;
-    int64_t S = slots / tiles;   // never past the slots: a few blocks left for a second round double the launch
-    if (S > 16) S = 16;
-    while (S > 1 && K / S < 256) S--;
-    if (want_parts)   // the caller's buffer bounds the parts
-      while (S > 1 && (size_t)S * M * N * sizeof(float) > parts_bytes) S--;
-    return (int)S;
-  };
-  if (M > 64) {
-    // int4: two accumulator sets per wavefront, so 64 x 64 wavefront tiles (128 x 128 per block)
-    const int64_t w = (q4 ? 128 : 256) / per;
-    const int wide = q4 ? 3 : 0;
-    const int64_t tm = cdiv(M, 128), tn = cdiv(N, w), tiles = tm * tn;
-    const int64_t cols_per_round = slots / tm;            // whole tile columns in one round
-    if (tiles <= slots || cols_per_round == 0 || !can_split || want_parts) {
-      pieces[npieces++] = Piece{0, N, pick_S(tiles), wide};
-    } else {
-      const int64_t main_tn = tn / cols_per_round * cols_per_round;   // whole rounds
-      const int64_t n_main = main_tn * w;
-      pieces[npieces++] = Piece{0, n_main, 1, wide};
-      if (n_main < N) pieces[npieces++] = Piece{n_main, N - n_main, pick_S(tm * (tn - main_tn)), wide};
-    }
-  } else {
-    // short prompts: 64-row tiles; narrow ones when that is what fills the chip (a gated
-    // tile needs two MFMA tiles per wavefront in N, so the narrow one is not for gu)
-    const int64_t t128 = cdiv(N, 128 / per), t64 = cdiv(N, 64 / per);
-    if (gu || q4 || t128 >= slots || pick_S(t128) > 1) pieces[npieces++] = Piece{0, N, pick_S(t128), 1};
-    else pieces[npieces++] = Piece{0, N, pick_S(t64), 2};
-  }
-  static const int kBm[4] = {128, 64, 64, 128}, kBn[4] = {256, 128, 64, 128};
-  // (few columns of a long K do not pay for the images of A: 512 x 896 x 4864 35 us against 29 here, 512 x 3584 x 3584 48
-  // against 50, 301 x 37888 x 3584 209 against 303)
-  const bool images_fit = half && K <= 32768 && (per * N >= 2048 || K <= 1024);
-  bool images = images_fit;
-  Q4Plan q4_plan;
-  if (images) q4_plan = plan_gemm_q4(M, N, K, parts_bytes, want_parts, gu, can_split);
-  const auto part_slabs = [&](const Piece& O) { return cdiv(cdiv(K, O.S), kBK); };
-  const auto part_blocks = [&](const Piece& O) {
-    return cdiv(M, kBm[O.variant]) * cdiv(O.n, kBn[O.variant] / per) * cdiv(cdiv(K, kBK), part_slabs(O));
-  };
-  // Above 128 rows also by what the two take, where the images' tiles are a round and a bit and these are one (us, images and here:
-  // 613 x 6528 x 5248 169 and 134, 705 x 10880 x 3584 in parts 195 and 161, 847 x 9344 x 256 33 and 26). This kernel's time is fitted
-  // to the 11000 runs of plan_gemm_q4 (error 5 %); 5 % are the images', for the errors of both.
-  if (images && M > 128) {
-    double here = 10.1 + 0.9e-6 * (double)M * (double)(per * N) + 7.3 * (npieces - 1);
-    for (int pi = 0; pi < npieces; pi++) {
-      const Piece& O = pieces[pi];
-      here += (double)part_slabs(O) * rounds_us(part_blocks(O), c.cus, 0.98, 1.22);
-      if (O.S > 1) here += 1.2e-6 * O.S * M * per * O.n + (want_parts ? 0 : 2.7);
-    }
-    images = 0.95 * q4_plan.us < here;
-  }
-  // A few rows: a kernel of their own, above 16 where it is the faster one. What the others take, fitted to 1000 runs (17 to
-  // 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 to 9 %): a start, and a time per 32-k slab with one and two blocks on a CU.
-  if (aligned16(C)) {
-    int64_t max_S = can_split ? 16 : 1;
-    if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
-    RowsPlan P = plan_gemm_rows(M, N, K, gu, q4, max_S);
-    if (M > 16 && P.S > 0) {
-      double other = images ? q4_plan.us : 0;
-      for (int pi = 0; !images && pi < npieces; pi++) {
-        const Piece& O = pieces[pi];
-        const int bn = kBn[O.variant];
-        const int64_t slabs = part_slabs(O), blocks = part_blocks(O);
-        if (M <= 64 && q4) other += 2.4 + (double)slabs * slab_us(blocks, c.cus, 0.965, 1.13);
-        else if (M <= 64) other += 2.2 + (double)slabs * (bn > 64 ? slab_us(blocks, c.cus, 0.9, 1.12) : slab_us(blocks, c.cus, 0.65, 0.95)) *
-                                             (bn == 64 && O.S == 1 && blocks > 3 * c.cus ? 0.85 : 1);   // (four blocks to a CU: 60 x 64982 x 768 32 us, 43 by rows)
-        else if (q4) other += 12.1 + (double)slabs * slab_us(blocks, c.cus, 1.03, 1.03);
-        else other += (gu && K <= 256 ? 9 : 7) + (double)slabs * slab_us(blocks, c.cus, 1.5, 2.18);   // (67 x 10732 gated x 128: 16.2 us, 10.8 by rows)
-        if (O.S > 1) other += (M <= 64 ? 0.65e-6 : 0.36e-6) * O.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
-      }
-      if (P.us + (P.S > 1 && !want_parts ? kPartSumUs : 0) > other) P.S = 0;
-    }
+  RowsPlan P = ch.rows;
+  if (P.S > 0) {
     const auto part_width = [&] { return gu ? (int64_t)P.tiles * 16 * P.TN : N; };
     char* parts = nullptr;
     if (P.S > 1 && !want_parts) {
@@ -637,8 +663,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
       TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
     }
   }
-  if (images) {
-    const int rc = gemm_q4_prompt(q4_plan, pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, S_out, gu);
+  if (ch.images) {
+    const int rc = gemm_q4_prompt(ch.q4, pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, S_out, gu);
     if (rc < 0) return rc;
     if (rc != kNoScratch) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
   }
@@ -646,8 +672,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   // exponents of A's rows first, then room for the largest piece's K-split parts.
   size_t parts_need = 0;
   if (!want_parts)
-    for (int pi = 0; pi < npieces; pi++) {
-      const Piece& P = pieces[pi];
+    for (int pi = 0; pi < ch.npieces; pi++) {
+      const Piece& P = ch.pieces[pi];
       const int bn = kBn[P.variant];
       const int64_t part_w = gu ? cdiv(P.n, bn / per) * bn : P.n;
       if (P.S > 1) parts_need = std::max(parts_need, (size_t)P.S * M * part_w * sizeof(float));
@@ -662,8 +688,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
         if (int rc = launch_gemm_rows(P, pa, W, static_cast<const float*>(scales), pc, M, N, K, N, gu)) return rc;
         TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
       }
-      if (images_fit && !images) {
-        const int rc = gemm_q4_prompt(q4_plan, pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, S_out, gu);
+      if (ch.images_fit && !ch.images) {
+        const int rc = gemm_q4_prompt(ch.q4, pa, static_cast<const uint8_t*>(W), static_cast<const float*>(scales), pc, M, N, K, S_out, gu);
         if (rc < 0) return rc;
         if (rc != kNoScratch) TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
       }
@@ -672,8 +698,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
   }
   int* ea = reinterpret_cast<int*>(sbase);
   if (half) row_exponent_f32_kernel<<<dim3((unsigned)M), dim3(256), 0, c.stream>>>(pa, (int)K, ea);
-  for (int pi = 0; pi < npieces; pi++) {
-    const Piece& P = pieces[pi];
+  for (int pi = 0; pi < ch.npieces; pi++) {
+    const Piece& P = ch.pieces[pi];
     const int bm = kBm[P.variant], bn = kBn[P.variant];
     const int64_t tcols = cdiv(P.n, bn / per);            // tile columns of this piece
     const int64_t part_w = gu ? tcols * bn : P.n;         // row width of a K-split part
@@ -722,6 +748,20 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
     if (S > 1 && !want_parts) launch_part_sum(dst, pc + P.n0, M, P.n, part_w, N, S, gu ? bn / 4 : 0);
   }
   TLHIP_CHECK_LAUNCH(TLHIP_C_GEMM_BF16_NT);
+}
+
+int tlhip_plan_gemm_bf16(int64_t M, int64_t N, int64_t K, int gated, int parts, int plan[5]) {
+  if (!plan || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || parts < 0) return fail(TLHIP_EINVAL, "tlhip_plan_gemm_bf16: bad arguments");
+  const Choice ch = choose_gemm(M, N, K, gated != 0, false, true, parts > 0, (size_t)parts * M * N * sizeof(float));
+  const RowsPlan& P = ch.rows;
+  int chain = P.S > 0 ? (P.part_units + 7) / 8 : 0, S = P.S;
+  for (int i = 0; P.S == 0 && i < ch.npieces; i++) {
+    chain = std::max(chain, (int)(((K + ch.pieces[i].S - 1) / ch.pieces[i].S + kBK - 1) / kBK));
+    S = std::max(S, ch.pieces[i].S);
+  }
+  const int v[5] = {P.S > 0, P.S > 0 ? P.TM : 0, P.S > 0 ? P.TN : 0, S, chain};
+  std::copy(v, v + 5, plan);
+  return TLHIP_OK;
 }
 
 int tlhip_gemm_bf16_nt(const void* A, const void* W, void* C, int64_t M, int64_t N, int64_t K) {

@@ -64,3 +64,30 @@ def test_prepared_products_keep_their_chains_over_drawn_shapes(plans):
         gated, parts = rng.choice([(False, 0), (True, 0), (False, 16), (False, 3)])
         pieces = plans.plan_gemm_f16w(M, N, K, gated, parts)
         assert sum(p[0] * p[2] for p in pieces) <= _filled(M, N, K, gated, parts), (M, N, K, gated, parts)
+
+
+# M, N, K, gated, room for parts; steps of 32 k in a row and K splits at most
+FEW_ROWS = [(24, 1152, 896, False, 16, 1, 4), (100, 1152, 896, False, 16, 1, 4), (24, 896, 896, False, 16, 1, 4), (77, 896, 896, False, 0, 1, 4),
+            (40, 896, 4864, False, 16, 2, 16), (77, 896, 4864, False, 16, 2, 16), (16, 4864, 896, True, 0, 4, 1), (77, 4864, 896, True, 0, 4, 1),
+            (22, 68, 1600, True, 0, 1, 7), (37, 2048, 8192, False, 16, 4, 16), (127, 248, 1856, True, 0, 1, 8),
+            # a block for every CU: no launch to add parts up
+            (8, 9000, 2048, False, 0, 8, 1), (32, 9000, 2048, False, 0, 8, 1), (64, 9000, 2048, False, 0, 8, 1), (100, 9000, 2048, False, 0, 8, 1),
+            (8, 18960, 2048, False, 0, 8, 1), (32, 18960, 2048, False, 0, 8, 1), (8, 32000, 2048, False, 0, 8, 1), (77, 32000, 2048, False, 0, 8, 1)]
+
+
+@pytest.mark.parametrize("M,N,K,gated,parts,chain,S", FEW_ROWS)
+def test_few_rows_are_split_for_the_error_and_no_further(plans, M, N, K, gated, parts, chain, S):
+    got = plans.plan_gemm_bf16(M, N, K, gated, parts)
+    assert got[0] == 1 and got[4] <= chain and got[3] <= S, got
+
+
+def test_few_rows_keep_parts_and_room(plans):
+    """A plan's parts are no more than there is room for, and none where N is no multiple of four."""
+    rng = random.Random(4)
+    for _ in range(4000):
+        M, N, K = _draw(rng, 2, 1024), _draw(rng, 16, 40000), 32 * _draw(rng, 4, 592)
+        gated, parts = rng.choice([(False, 0), (True, 0), (False, 16), (False, 2), (False, 1)])
+        rows, TM, TN, S, chain = plans.plan_gemm_bf16(M, N, K, gated, parts)
+        assert 1 <= S <= (1 if N % 4 else min(16, parts or 16)) and chain >= 1, (M, N, K, gated, parts)
+        if rows:
+            assert 1 <= TM <= 5 and (2 if gated else 1) <= TN <= 4 and chain == _ceil(_ceil(K // 32, S), 8)
