@@ -619,7 +619,7 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 // than it gives. Up to 128 rows that is what an estimate fitted to 280 runs says (K 384 .. 18944, N 384 .. 37888, M 8 .. 120: clocks
 // of a step by the CU's vector memory path or its matrix or vector instructions, 3500 and 60 per accumulator tile for a block, parts
 // written and read, a launch that adds them up); wide products, which have a block for every CU, stay whole: 18960 x 2048 at 32 rows takes
-// 33.6 us in two parts. Above, the 128-row tiles, which run what does not come here, split K up to 16 times and have
+// 19.3 us, in two parts 22.9. Above, the 128-row tiles, which run what does not come here, split K up to 16 times and have
 // 1.73e-7 at K 3584, 1.9e-7 at 4864, 2.5e-7 at 8192, 3.0e-7 at 12288.
 static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
@@ -654,7 +654,10 @@ static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t m
 // costs a little for its dispatch; a step of its wavefronts takes the CU's loads of activations and weights, a little less where
 // CUs are idle; blocks that share a CU cost half again each, more where their steps are many. Fitted up to 128 rows to 25000
 // runs in the chains allowed (2 to 128 rows, 256 to 16000 columns, K 256 to 18944: error 8 %, the shape it chooses 1.1 % slower than the
-// fastest one on average and 1.15 times at most), above to 13980 others, all of it times 1.1 (12800 runs of 129 to 1024 rows: error 9 %, 1.1 %).
+// fastest one on average), above to 13980 others (12800 runs of 129 to 1024 rows take 1.1 times as much, error 9 %, the shape 1.1 %).
+// Measured, us, tiles -> this kernel: 896 x 896 at 37 / 77 / 512 rows 10.3 / 20.9 / 21.7 -> 3.8 / 4.4 / 7.7; 4864 x 896 gated at 37 / 77 / 256
+// 15.0 / 25.2 / 28.3 -> 8.3 / 10.7 / 24.4; 896 x 4864 at 37 / 77 / 150 10.9 / 21.4 / 22.5 -> 6.5 / 8.7 / 10.6; 1152 x 896 at 77 / 300 20.9 / 21.4 -> 5.1 / 7.3;
+// 18944 x 3584 gated at 37 / 64 104 / 105 -> 73 / 89.
 static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
   // blocks of [row tiles][column tiles] that fit a CU (registers, LDS)
   static constexpr int kFit[5][4] = {{4, 3, 2, 2}, {4, 2, 2, 1}, {3, 2, 1, 1}, {2, 2, 1, 1}, {2, 1, 1, 1}};
@@ -711,7 +714,7 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
           best.tiles = (int)tiles;
           best.row_blocks = (int)row_blocks;
           best.part_units = (int)per;
-          best.us = 1.05 * k.all * us;             // (5 % for the errors of both estimates it is weighed against)
+          best.us = k.all * us;
         }
       }
     }

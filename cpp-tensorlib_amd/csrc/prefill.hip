@@ -580,27 +580,46 @@ static Choice choose_gemm(int64_t M, int64_t N, int64_t K, bool gu, bool q4, boo
     }
     images = 0.95 * q4_plan.us < here;
   }
-  // A few rows: a kernel of their own, above 16 where it is the faster one. What the others take, fitted to 1000 runs (17 to
-  // 128 rows, N 256 .. 33000, K 256 .. 18944; error 6 to 9 %): a start, and a time per 32-k slab with one and two blocks on a CU.
+  // A few rows: a kernel of their own, above 16 where it is the faster one. What the others take: int4 fitted to 1000 runs (17 to 128 rows,
+  // N 256 .. 33000, K 256 .. 18944; error 6 to 9 %), bf16 to 3000 (17 to 1024 rows, N 256 .. 40000, K 256 .. 18944; error 6 to 7 %): a start, for
+  // every launch, a time per 32-k slab with one and two blocks on a CU, the megabytes stored as result and as parts, a launch that adds
+  // parts up. A gated product of 128-row tiles over up to 256 k starts later (67 x 10732 gated x 128: 16.2 us, 10.8 by rows).
   if (aligned) {
     int64_t max_S = can_split ? 16 : 1;
     if (want_parts) max_S = std::min<int64_t>(max_S, (int64_t)(parts_bytes / ((size_t)M * N * sizeof(float))));
     RowsPlan& P = ch.rows;
     P = plan_gemm_rows(M, N, K, gu, q4, max_S);
     if (M > 16 && P.S > 0) {
-      double other = images ? q4_plan.us : 0;
+      const double mb = 4e-6 * (double)M * (double)N;
+      double other = images ? q4_plan.us : 0, own = P.us;
+      int64_t chain = 0;               // the tiles' longest, in slabs
       for (int pi = 0; !images && pi < npieces; pi++) {
         const Piece& O = pieces[pi];
         const int bn = kBn[O.variant];
         const int64_t slabs = part_slabs(O), blocks = part_blocks(O);
-        if (M <= 64 && q4) other += 2.4 + (double)slabs * slab_us(blocks, cus, 0.965, 1.13);
-        else if (M <= 64) other += 2.2 + (double)slabs * (bn > 64 ? slab_us(blocks, cus, 0.9, 1.12) : slab_us(blocks, cus, 0.65, 0.95)) *
-                                             (bn == 64 && O.S == 1 && blocks > 3 * cus ? 0.85 : 1);   // (four blocks to a CU: 60 x 64982 x 768 32 us, 43 by rows)
-        else if (q4) other += 12.1 + (double)slabs * slab_us(blocks, cus, 1.03, 1.03);
-        else other += (gu && K <= 256 ? 9 : 7) + (double)slabs * slab_us(blocks, cus, 1.5, 2.18);   // (67 x 10732 gated x 128: 16.2 us, 10.8 by rows)
-        if (O.S > 1) other += (M <= 64 ? 0.65e-6 : 0.36e-6) * O.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
+        const double parts = O.S > 1 ? 4e-6 * (double)O.S * (double)M * (double)(per * O.n) : 0;
+        const bool sum = O.S > 1 && !want_parts;
+        chain = std::max(chain, slabs);
+        if (q4) {
+          other += M <= 64 ? 2.4 + (double)slabs * slab_us(blocks, cus, 0.965, 1.13) : 12.1 + (double)slabs * slab_us(blocks, cus, 1.03, 1.03);
+          if (O.S > 1) other += (M <= 64 ? 0.65e-6 : 0.36e-6) * O.S * M * per * N * 4 + (want_parts ? 0 : kPartSumUs);
+        } else if (M <= 64 && bn > 64) {
+          other += 2.5 + (double)slabs * slab_us(blocks, cus, 0.77, 0.92) + 0.41 * mb + 0.32 * parts + (sum ? 2.8 : 0);
+        } else if (M <= 64) {
+          const double four_to_a_cu = O.S == 1 && blocks > 3 * cus ? 0.85 : 1;   // (60 x 64982 x 768 32 us, 43 by rows)
+          other += 1.5 + (double)slabs * slab_us(blocks, cus, 0.64, 0.755) * four_to_a_cu + 0.42 * mb + 0.2 * parts + (sum ? 2 : 0);
+        } else {
+          const int64_t rest = blocks % (2 * cus);
+          const double slab = (double)(blocks / (2 * cus)) * 2.13 + (rest == 0 ? 0 : rest <= cus ? 1.435 : 2.13);
+          other += (pi > 0 ? 22.2 : gu && K <= 256 ? 8.7 : 6.7) + (double)slabs * slab + 0.147 * parts + (sum ? 3.4 : 0);
+          if (pi == 0) other += 0.122 * mb;
+        }
       }
-      if (P.us + (P.S > 1 && !want_parts ? kPartSumUs : 0) > other) P.S = 0;
+      if (P.S > 1 && !want_parts) own += q4 ? kPartSumUs : 2.3 + 0.29e-6 * 4 * (double)P.S * (double)M * (double)(gu ? (int64_t)P.tiles * 16 * P.TN : N);
+      // Of two that are about as fast the more accurate one: the rows kernel's chains are mostly the shorter ones, and the error of a
+      // 0.5B prompt of 420 tokens is 3.65e-7 with its gated products there and 3.9e-7 with them in tiles (43.2 us each and 42.1).
+      if (!q4) own *= (P.part_units + 7) / 8 > chain ? 1.08 : (P.part_units + 7) / 4 > chain ? 0.96 : 0.9;
+      if (own > other) P.S = 0;
     }
   }
   return ch;

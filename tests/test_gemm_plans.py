@@ -91,3 +91,17 @@ def test_few_rows_keep_parts_and_room(plans):
         assert 1 <= S <= (1 if N % 4 else min(16, parts or 16)) and chain >= 1, (M, N, K, gated, parts)
         if rows:
             assert 1 <= TM <= 5 and (2 if gated else 1) <= TN <= 4 and chain == _ceil(_ceil(K // 32, S), 8)
+
+
+# M, N, K, gated, room for parts; us measured in tiles and by the kernel of few rows
+MEASURED = [(626, 13780, 640, True, 0, 87.5, 132.2), (270, 18820, 512, False, 16, 26.9, 37.8), (921, 1268, 8128, False, 16, 63.5, 81.9),
+            (366, 4728, 3456, False, 16, 43.5, 57.3), (242, 4608, 3584, False, 16, 33.1, 44.6), (476, 2048, 4096, False, 16, 34.0, 43.7),
+            (108, 21844, 1344, False, 16, 31.7, 41.9), (512, 896, 6656, False, 16, 29.3, 34.3),
+            (300, 1152, 896, False, 16, 21.3, 7.2), (202, 5886, 384, False, 16, 24.2, 11.5), (150, 896, 4864, False, 16, 22.3, 10.5),
+            (256, 4864, 896, True, 0, 28.4, 24.8), (77, 4864, 896, True, 0, 24.9, 10.6), (64, 18944, 3584, True, 0, 106.9, 88.7),
+            (77, 32000, 2048, False, 0, 56.1, 46.6), (32, 9000, 2048, False, 0, 18.8, 14.8)]
+
+
+@pytest.mark.parametrize("M,N,K,gated,parts,tiles,rows", MEASURED)
+def test_the_faster_kernel_is_chosen(plans, M, N, K, gated, parts, tiles, rows):
+    assert plans.plan_gemm_bf16(M, N, K, gated, parts)[0] == (rows < tiles)
