@@ -496,7 +496,7 @@ void launch_part_sum(const float* parts, float* C, int64_t M, int64_t n, int64_t
 }
 
 // Columns (features) [n0, n0 + n) in tiles of one variant, K split S ways.
-struct Piece { int64_t n0, n; int S; int variant; };
+struct Piece { int64_t n0 = 0, n = 0; int S = 0; int variant = 0; };
 static const int kBm[4] = {128, 64, 64, 128}, kBn[4] = {256, 128, 64, 128};   // rows and columns of a variant's tile
 // Which kernel forms a product: the rows kernel where rows.S > 0, else the images' where `images`, else the tiles here in pieces.
 struct Choice {
@@ -670,7 +670,9 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
     char* parts = nullptr;
     if (P.S > 1 && !want_parts) {
       parts = static_cast<char*>(scratch((size_t)P.S * M * part_width() * sizeof(float)));
-      if (!parts) P = plan_gemm_rows(M, N, K, gu, q4, 1);   // no scratch to be had (a recording may not grow it): no parts
+      // No scratch to be had (a recording may not grow it): no parts. Above 128 rows tiles with a split of their own are tried
+      // first, whose parts may be fewer; what finds no room there either comes back to this kernel below.
+      if (!parts) P = M > 128 && (ch.pieces[0].S > 1 || ch.pieces[1].S > 1) ? RowsPlan{} : plan_gemm_rows(M, N, K, gu, q4, 1);
     }
     if (P.S > 0) {
       const bool sum = P.S > 1 && !want_parts;

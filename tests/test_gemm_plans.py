@@ -105,3 +105,10 @@ MEASURED = [(626, 13780, 640, True, 0, 87.5, 132.2), (270, 18820, 512, False, 16
 @pytest.mark.parametrize("M,N,K,gated,parts,tiles,rows", MEASURED)
 def test_the_faster_kernel_is_chosen(plans, M, N, K, gated, parts, tiles, rows):
     assert plans.plan_gemm_bf16(M, N, K, gated, parts)[0] == (rows < tiles)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 999, 8192), (200, 1151, 4864), (150, 3585, 3584), (1000, 301, 12288)])
+def test_a_k_that_cannot_be_split_has_no_longer_chains_above_128_rows(plans, M, N, K):
+    """The tiles cannot split it either: theirs would be all of K (129 x 999 x 8192 369 us, 26 here)."""
+    rows, _, _, S, chain = plans.plan_gemm_bf16(M, N, K)
+    assert (rows, S) == (1, 1) and chain == _ceil(K // 32, 8)

@@ -15,7 +15,8 @@ SHAPES = [(1, 16, 128), (2, 33, 128), (5, 200, 256), (16, 896, 896), (17, 130, 1
           (9, 18500, 128), (16, 18300, 128), (60, 33000, 128),
           # above 128 rows (bf16), three column tiles, one step of activations in flight and four (one row tile, few columns)
           (129, 100, 896), (161, 48, 384), (255, 1200, 512), (256, 33, 4096), (7, 16, 12288), (11, 40, 9216),
-          (257, 1152, 896), (336, 100, 2560), (401, 36, 4864), (1024, 48, 384), (1025, 40, 128)]
+          (257, 1152, 896), (336, 100, 2560), (401, 36, 4864), (1024, 48, 384), (1025, 40, 128),
+          (129, 999, 8192), (200, 1151, 4864)]     # K cannot be split
 
 
 def _weights(orc, fmt, N, K, seed):
@@ -141,10 +142,11 @@ def test_infinities_and_nan_stay_in_their_rows(lib, orc, fmt, M, N, K):
 
 
 @pytest.mark.parametrize("fmt,M,N,K", [("bf16", 37, 896, 4864), ("bf16", 77, 896, 4864), ("q4", 20, 896, 4864), ("q4", 77, 896, 4864),
-                                         ("bf16", 64, 4608, 3584), ("q4", 128, 4608, 3584)])
+                                         ("bf16", 64, 4608, 3584), ("q4", 128, 4608, 3584),
+                                         ("bf16", 200, 896, 4864), ("bf16", 300, 2048, 4096), ("bf16", 130, 5000, 3584)])
 def test_recorded_without_scratch(fresh_lib, recorded, orc, fmt, M, N, K):
     """Where the parts of a split K have no room the product is formed in one part, also one that another kernel would have formed
-    in parts (the last two)."""
+    in parts (the fifth and sixth), and above 128 rows (the last three)."""
     print("case gemm_rows recorded", fmt, M, N, K, flush=True)
     A = orc.normal(M * K, 35).reshape(M, K)
     w, W = _weights(orc, fmt, N, K, 36)
