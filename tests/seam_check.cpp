@@ -378,6 +378,51 @@ int main() {
     check("a prompt product deeper than the prepared form runs on the bf16 rows", ok);
   }
 
+  {  // the GELU gate with its biases: in the epilogue of the product over the prepared weight, on the bf16 rows where that
+     // form is off or refused (a bias that is not 16-byte aligned), and on a weight edited in between
+    const int64_t m = 200, ff = 5120, k = 2048;      // m * 2 ff * k = 4.2e9: large enough to be prepared
+    buf a(m * k), w(2 * ff * k / 2), bias(2 * ff + 1), gu(m * 2 * ff), act(m * ff);
+    fill(a); fill(bias, 0.5f);
+    uint16_t* pw = reinterpret_cast<uint16_t*>(w.write());
+    for (int64_t i = 0; i < 2 * ff * k; i++) { const float v = 0.05f * rnd(); uint32_t u; std::memcpy(&u, &v, 4); pw[i] = (uint16_t)(u >> 16); }
+    auto rows_match = [&](int64_t off, const char* what) {
+      const float* got = act.read();
+      auto product = [&](int64_t r, int64_t c) {
+        double s = 0;
+        for (int64_t i = 0; i < k; i++) {
+          const uint32_t u = (uint32_t)reinterpret_cast<const uint16_t*>(w.host)[c * k + i] << 16;
+          float f; std::memcpy(&f, &u, 4);
+          s += (double)a.host[r * k + i] * (double)f;
+        }
+        return s + (double)bias.host[off + c];
+      };
+      for (int64_t r : {int64_t(0), m / 2, m - 1})
+        for (int64_t f : {int64_t(0), int64_t(130), ff - 1}) {
+          const double g = product(r, f), want = 0.5 * g * (1 + std::tanh(0.7978845608028654 * (g + 0.044715 * g * g * g))) * product(r, ff + f);
+          if (!close(got[r * ff + f], want)) {
+            std::printf("  %s at (%lld, %lld): got %.9g want %.9g\n", what, (long long)r, (long long)f, got[r * ff + f], want);
+            return false;
+          }
+        }
+      return true;
+    };
+    auto run = [&](int64_t off) {
+      { float* p = act.write(); for (int64_t i = 0; i < act.n; i++) p[i] = NAN; }
+      return hip::gemm_bf16_nt_geglu(a.native, w.native, static_cast<char*>(bias.native) + 4 * off, gu.native, act.native, m, ff, k);
+    };
+    const float mark = -777.0f;                      // the products' room stays as it is where the epilogue gates
+    { float* p = gu.write(); for (int64_t i = 0; i < gu.n; i++) p[i] = mark; }
+    bool ok = run(0) && rows_match(0, "first product") && run(0) && rows_match(0, "second product (cached form)");
+    ok = ok && gu.read()[0] == mark && gu.host[gu.n - 1] == mark;
+    reinterpret_cast<uint16_t*>(w.write())[130 * k + 5] = 0x4080;
+    ok = ok && run(0) && rows_match(0, "after a host edit") && gu.read()[0] == mark;
+    ok = ok && run(1) && rows_match(1, "a bias at an odd offset") && gu.read()[0] != mark;
+    hip::set_prompt_f16(false);
+    ok = ok && run(0) && rows_match(0, "on the bf16 rows");
+    hip::set_prompt_f16(true);
+    check("gated product with biases and the GELU gate, prepared and on the bf16 rows", ok);
+  }
+
   {  // pool: a released buffer comes back for the same size, contents pointer included
     float* h1 = nullptr;
     void* n1 = hip::alloc(4096, &h1);

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(1, 16, 128), (2, 33, 128), (5, 200, 256), (16, 896, 896), (17, 130, 128), (37, 1152, 896), (64, 64, 3584),
           (65, 100, 128), (77, 896, 4864), (80, 36, 2048), (81, 260, 384), (97, 128, 896), (128, 72, 640),
           (9, 18500, 128), (16, 18300, 128), (60, 33000, 128),
-          # above 128 rows (bf16), three column tiles, one step of activations in flight and four (one row tile, few columns)
+          # above 128 rows (bf16), few rows and columns of a long K; 1025 rows run in the tiles
           (129, 100, 896), (161, 48, 384), (255, 1200, 512), (256, 33, 4096), (7, 16, 12288), (11, 40, 9216),
           (257, 1152, 896), (336, 100, 2560), (401, 36, 4864), (1024, 48, 384), (1025, 40, 128),
           (129, 999, 8192), (200, 1151, 4864)]     # K cannot be split
@@ -80,9 +80,9 @@ def test_gated(lib, orc, fmt, M, ff, K):
 @pytest.mark.parametrize("fmt,K", [("bf16", 2048), ("bf16", 9216), ("q4", 4096), ("q4", 4736), ("q4", 9216)])
 def test_many_steps_to_a_wavefront(lib, orc, fmt, K):
     """Columns that are no multiple of four keep K in one part: a wavefront's steps go through its slots several times (bf16: 8 and
-    36 steps in two to four slots; int4: four, five and nine units in two), for every number of row tiles. The sums' order
-    does not depend on the tiles, so the first five rows of every product are the bits of the five-row product, which only
-    this kernel forms: the others are formed by it too."""
+    36 steps in one slot, or four where a block has one row tile; int4: four, five and nine units in two), for one to five (bf16:
+    three) row tiles. The sums' order does not depend on the tiles, so the first five rows of every product are the bits of the
+    five-row product, which only this kernel forms: the others are formed by it too."""
     N = 33
     A = orc.normal(128 * K, 27).reshape(128, K)
     w, W = _weights(orc, fmt, N, K, 28)
@@ -122,7 +122,45 @@ def test_many_steps_of_wide_gated_tiles(lib, orc, fmt):
     dw.free()
 
 
-@pytest.mark.parametrize("fmt,M,N,K", [("bf16", 40, 130, 896), ("q4", 40, 130, 896), ("q4", 77, 896, 896), ("q4", 128, 900, 384)])
+# Every block of row tiles and column tiles of the bf16 kernel (1: gated), its wavefronts with more steps than the loop that keeps
+# loads in flight needs, some one more than others, in one, two (one row tile, two column tiles) and four slots
+TILES = {(0, 1, 1): (3, 17, 2592), (0, 1, 2): (3, 4194, 1568), (0, 1, 3): (3, 8289, 1056), (0, 1, 4): (3, 12664, 3360),
+         (0, 2, 1): (33, 17, 1056), (0, 2, 2): (33, 2053, 1056), (0, 2, 3): (17, 8265, 1056), (0, 2, 4): (17, 4120, 3104),
+         (0, 3, 1): (65, 17, 1056), (0, 3, 2): (33, 4119, 1056), (0, 3, 3): (65, 4107, 1056), (0, 3, 4): (65, 6165, 1056),
+         (0, 4, 1): (150, 17, 1056), (0, 4, 2): (257, 1027, 1056), (0, 4, 3): (49, 8237, 1056), (0, 4, 4): (49, 12386, 1056),
+         (0, 5, 1): (200, 1025, 1056), (0, 5, 2): (150, 2726, 1056), (0, 5, 3): (65, 8361, 1056), (0, 5, 4): (65, 4148, 3104),
+         (1, 1, 2): (3, 16, 1568), (1, 1, 3): (3, 4134, 1056), (1, 1, 4): (3, 12380, 1056), (1, 2, 2): (33, 17, 1056),
+         (1, 2, 3): (17, 4117, 1056), (1, 2, 4): (17, 6223, 1056), (1, 3, 2): (65, 17, 1056), (1, 3, 3): (100, 1367, 1056),
+         (1, 3, 4): (65, 3103, 1056), (1, 4, 2): (150, 16, 1056), (1, 4, 3): (49, 4101, 1056), (1, 4, 4): (49, 2088, 3104),
+         (1, 5, 2): (150, 1363, 1056), (1, 5, 3): (65, 4137, 1056), (1, 5, 4): (129, 3085, 1056)}
+
+
+@pytest.mark.parametrize("tile", sorted(TILES))
+def test_every_tile(lib, orc, tile):
+    """The plan is asked for, so that another estimate cannot move a shape to another tile unseen."""
+    gated, TM, TN = tile
+    M, N, K = TILES[tile]
+    print("case gemm_rows tile", tile, M, N, K, flush=True)
+    rows, tm, tn, S, chain = lib.plan_gemm_bf16(M, N, K, bool(gated))
+    slots = 4 // TN if TM == 1 and TN <= 2 else 1
+    assert (rows, tm, tn) == (1, TM, TN) and chain > 2 * (slots + 1) and -(-K // 32 // S) % 8 != 0
+    A = orc.normal(M * K, 37).reshape(M, K)
+    w, W = _weights(orc, "bf16", (1 + gated) * N, K, 38)
+    p, s = A.astype(np.float64) @ W.T, _slack(A.astype(np.float64), W, K)
+    da, dw, out = lib.to_device(A), lib.to_device(w), lib.to_device(np.full((M, N), np.nan, np.float32))
+    if gated:
+        lib.gemm_bf16_nt_swiglu(da, dw, out, M, N, K)
+        g, u, sg, su = p[:, :N], p[:, N:], s[:, :N], s[:, N:]
+        act = g / (1 + np.exp(-g))
+        assert np.all(np.abs(out.numpy() - act * u) <= 1.1 * sg * (np.abs(u) + su) + np.abs(act) * su + 1e-6 * np.abs(act * u))
+    else:
+        lib.gemm_bf16_nt(da, dw, out, M, N, K)
+        assert np.all(np.abs(out.numpy() - p) <= s)
+    for b in (da, dw, out):
+        b.free()
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [("bf16", 40, 130, 896), ("bf16", 150, 130, 896), ("bf16", 300, 1152, 896), ("q4", 40, 130, 896), ("q4", 77, 896, 896), ("q4", 128, 900, 384)])
 def test_infinities_and_nan_stay_in_their_rows(lib, orc, fmt, M, N, K):
     """An infinity and a NaN make their rows NaN (an infinity's lower terms are); the other rows keep their bits, also where
     a block multiplies once more for them."""

@@ -23,12 +23,17 @@ def _gemm(lib, A, Wb):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (512, 512, 3584),      # a prompt chunk against a kv-sized projection: 8 wide tiles, K split 14 ways
-    (512, 4608, 896),      # 72 wide tiles, K split 3 ways
-    (1024, 4864, 896),     # 152 wide tiles, K split 3 ways
+    (512, 512, 3584),      # a prompt chunk against a kv-sized projection: the kernel of few rows, K split 4 ways
+    (512, 4608, 896),      # the same kernel, unsplit
+    (1024, 4864, 896),
+    (512, 512, 3592),      # K % 32 != 0 is for the tiles: 8 wide ones, K split 14 ways
+    (512, 4608, 904),      # 72 wide tiles, K split 3 ways
+    (1024, 4864, 904),     # 152 wide tiles, K split 3 ways
+    (1040, 512, 3584),     # more rows than the kernel of few takes
     (128, 1152, 896),      # 0.5B fused q|k|v
     (33, 200, 40),         # short prompt: 64-row tiles; ragged in M, N and K (K % 32 != 0)
     (64, 4608, 896),       # short prompt, K split
+    (64, 4608, 904),       # in tiles of 64 rows
     (1, 64, 8),            # smallest legal
     (257, 129, 264),       # N % 4 != 0: no K split possible
 ])
@@ -108,14 +113,14 @@ def test_gemm_bf16_nt_random_shapes_exact(lib, orc):
     (512, 3584, 3584, 4),     # the caller's buffer holds 4 parts: the split stops there
     (512, 3584, 3584, 1),     # room for the product only: one part
     (200, 896, 4864, 16),     # 0.5B down, ragged M
-    (33, 896, 896, 16),       # short prompt: 64-row tiles
+    (33, 896, 896, 16),       # short prompt: the kernel of few rows
     (257, 130, 264, 16),      # N % 4 != 0: never split
 ])
 def test_gemm_parts_then_residual_norm_is_gemm_then_residual_norm(lib, orc, M, N, K, room):
     """The product left as its K-split parts and summed by the residual norm while it reads them
     is, bit for bit, the product summed by the GEMM's own part-sum launch and then normalised:
-    same parts, same order of addition (when the caller's buffer has room for the split the plain
-    GEMM picks - 16 parts always is). Checked on the residual stream and on the normalised rows."""
+    same parts, same order of addition (when both take the same kernel, as they do here, and the
+    caller's buffer has room for the split the plain GEMM picks - 16 parts always is). Checked on the residual stream and on the normalised rows."""
     print("case gemm parts", M, N, K, room, flush=True)
     A = orc.normal(M * K, 41).reshape(M, K)
     Wb = orc.to_bf16(orc.normal(N * K, 42, std=0.02)).reshape(N, K)
@@ -153,9 +158,11 @@ def test_gemm_parts_then_residual_norm_is_gemm_then_residual_norm(lib, orc, M, N
 
 @pytest.mark.parametrize("M,ff,K", [
     (512, 18944, 3584),    # 7B chunk: 128 whole-round tile columns + 20 split over K
-    (512, 4864, 896),      # 0.5B chunk: 152 tiles, split over K
+    (512, 4864, 896),      # 0.5B chunk: the kernel of few rows
+    (300, 4864, 904),      # K % 32 != 0: 128-row tiles, K split 3 ways
     (200, 1000, 264),      # ragged in M and in the last tile's features
-    (64, 4864, 896),       # short prompt: 64-row tiles
+    (64, 4864, 896),       # short prompt
+    (64, 4864, 904),       # in 64-row tiles
     (7, 36, 40),           # less than one tile
     (130, 130, 64),        # ff % 4 != 0: never split
 ])
