@@ -5,6 +5,10 @@
 // v_mfma_f32_32x32x2_f32 multiplies f32 by f32 exactly and accumulates in fp32, so scores and
 // outputs differ from the reference's loops in summation order only.
 //
+// Two kernels: attn_prefill_small_kernel in tiles of 16 queries and 16 keys for head size 64, and for head size 128 where prompt and
+// context are short; attn_prefill_mfma_kernel in tiles of 32 for the rest of head size 128. What follows is the second; the first
+// has its own remarks.
+//
 // A block owns one query head and 32 consecutive query positions; its 8 wavefronts deal the
 // 32-key tiles of the causal range round-robin and each keeps a running (max, sum, output) state
 // for all 32 queries (online softmax), merged through LDS at the end. Per key tile a wavefront
@@ -61,23 +65,23 @@ __device__ __forceinline__ float4 load_kv4(const uint16_t* p) {   // 4 bf16, wid
 
 // LDS: the Q tile (shared by the block) and one 32 x (D+4) region per wavefront that holds the K
 // tile, then P, then the V tile.
-template <int D>
 struct PrefillLds {
+  static constexpr int D = 128;
   static constexpr int KS = D + 4;
   static constexpr int PS = 36;
   static constexpr int kRegion = 32 * KS;                 // floats: Q, and one region per wavefront
   static constexpr size_t kBytes = (size_t)9 * kRegion * sizeof(float);
 };
 
-template <int D, typename KT>
+template <typename KT>
 __global__ __launch_bounds__(512, 1) void attn_prefill_mfma_kernel(const float* __restrict__ q,
                                                                     const KT* __restrict__ K,
                                                                     const KT* __restrict__ V,
                                                                     float* __restrict__ out, int group, int T,
                                                                     int pos0, int64_t kv_stride, float scale,
                                                                     int64_t o_head, int64_t o_row) {
-  using L = PrefillLds<D>;
-  constexpr int KS = L::KS, PS = L::PS;
+  using L = PrefillLds;
+  constexpr int D = L::D, KS = L::KS, PS = L::PS;
   constexpr int kLoads = 32 * D / 4 / 64;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -383,8 +387,8 @@ int launch_prefill_mfma(const float* q, const KT* K, const KT* V, float* out, in
     return 0;
   }
   if constexpr (D == 128) {
-    auto fn = attn_prefill_mfma_kernel<D, KT>;
-    const int lds = (int)PrefillLds<D>::kBytes;
+    auto fn = attn_prefill_mfma_kernel<KT>;
+    const int lds = (int)PrefillLds::kBytes;
     if ((size_t)lds > (size_t)c.lds_per_cu) return fail(TLHIP_EUNSUPPORTED, "tlhip_attn_prefill: not enough LDS");
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(LDS)");
