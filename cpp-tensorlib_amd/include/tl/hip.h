@@ -873,8 +873,10 @@ inline bool gemv_q4(void* a, void* qw, void* scales, void* y, int64_t N, int64_t
 }
 
 // The prepared-weight products pay one more launch (the activation planes) and win it back on the
-// matrix cores only when the product is large: measured, from about 4 * 10^9 multiply-adds on
-// (512 x 4608 x 3584 gains 13 %, 512 x 896 x 4864 loses 10 %).
+// matrix cores only when the product is large: from about 4 * 10^9 multiply-adds on. Measured, us, prepared with
+// that launch and on the bf16 rows: 512 x 4864 gated x 896 34.6 and 45.1, 512 x 9488 x 896 34.9 and 44.1, 320 x 2048 x 8192
+// 41.8 and 47.5, 320 x 3584 x 3584 35.3 and 36.1, 256 x 2048 x 8192 38.3 and 38.1; below the line 512 x 896 x 4864 31.0 and
+// 27.5, 400 x 4864 gated x 896 34.3 and 33.5, but 450 x 4864 gated x 896 35.0 and 43.2.
 inline bool prompt_product_is_large(int64_t m, int64_t n, int64_t k) {
   return m > 64 && (double)m * (double)n * (double)k >= 4e9;
 }

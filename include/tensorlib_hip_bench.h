@@ -1,8 +1,8 @@
 /* Benchmark and tuning entry points of libtensorlib_hip.so.
  *
  * Not part of the backend boundary: a backend header binds include/tensorlib_hip.h only.
- * These serve bench.py, the profiles and the tests that force a launch shape. They set
- * process-wide state: a caller that changes a launch shape restores it with the same call
+ * These serve bench.py, the profiles and the tests that force a launch shape or ask for a plan. The
+ * tune calls set process-wide state: a caller that changes a launch shape restores it with the same call
  * (zeros) or with tlhip_tune_reset(). None has a counterpart in the reference.
  */
 #ifndef TENSORLIB_HIP_BENCH_H
