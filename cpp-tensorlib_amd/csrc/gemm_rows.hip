@@ -613,7 +613,7 @@ int run_tm(const RowsPlan& P, const float* A, const void* W, const float* scales
 }  // namespace rows
 
 // The longest chain of matrix instructions, in steps of 32 k, that a wavefront may form a sum of bf16 products by. The error of a sum
-// grows with it (1.0e-7 of the result after a step, 1.3e-7 after 4, 1.7e-7 after 7, 2.0e-7 after 10), and the plan that takes
+// grows with it (0.9e-7 of the result after a step, 1.3e-7 after 4, 1.7e-7 after 7, 2.0e-7 after 10), and the plan that takes
 // least time would trade it: few rows' products of K 896 run as fast unsplit on narrow column tiles, in chains of 4 (24 x 1152 x 896
 // 1.3e-7 of error for 0.9e-7). So K is split at least as far as fills the CUs by blocks of wide tiles, where that does not cost more
 // than it gives. Up to 128 rows that is what an estimate fitted to 280 runs says (K 384 .. 18944, N 384 .. 37888, M 8 .. 120: clocks
