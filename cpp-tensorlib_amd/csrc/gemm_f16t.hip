@@ -888,7 +888,8 @@ extern "C" {
 int tlhip_plan_gemm_f16w(int64_t M, int64_t N, int64_t K, int gated, int parts, int64_t pieces[8]) {
   if (!pieces || M <= 0 || N <= 0 || K <= 0 || K % f16t::kBK != 0 || parts < 0)
     return fail(TLHIP_EINVAL, "tlhip_plan_gemm_f16w: bad arguments");
-  const Plan P = plan_f16w(M, N, K, gated != 0, parts > 0, (size_t)parts * M * N * sizeof(float));
+  if (!plan_bytes_fit(M, N) || K > 256 * 4 * f16t::kRowRegs) return fail(TLHIP_EUNSUPPORTED, "tlhip_plan_gemm_f16w: dimension too large");
+  const Plan P = plan_f16w(M, N, K, gated != 0, parts > 0, (size_t)std::min(parts, 16) * M * N * sizeof(float));
   for (int i = 0; i < 2; i++) {
     const Piece p = i < P.npieces ? P.pieces[i] : Piece{0, 0, 0, 0};
     const int64_t v[4] = {p.tcols, p.S, p.S > 0 ? cdiv64(K / f16t::kBK, p.S) : 0, 128 * p.tmh};

@@ -10,6 +10,11 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t frag16 __attribute__((ext_vector_type(4)));   // eight 16-bit operands of one lane
 
+// What a plan may be asked for without a product's own checks: rows and columns as there, sixteen parts' bytes within 64 bits.
+inline bool plan_bytes_fit(int64_t M, int64_t N) {
+  return M <= 0x3fffffff && N <= 0x3fffffff && M * N <= (int64_t)1 << 56;
+}
+
 // gemm_rows.hip: products of a few rows. S == 0: not a shape it takes.
 struct RowsPlan {
   int TM = 0, TN = 0, S = 0, tiles = 0, row_blocks = 0, part_units = 0;

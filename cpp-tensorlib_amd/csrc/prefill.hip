@@ -773,7 +773,8 @@ static int gemm_bf16_nt_impl(const void* A, const void* W, void* C, int64_t M, i
 
 int tlhip_plan_gemm_bf16(int64_t M, int64_t N, int64_t K, int gated, int parts, int plan[5]) {
   if (!plan || M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || parts < 0) return fail(TLHIP_EINVAL, "tlhip_plan_gemm_bf16: bad arguments");
-  const Choice ch = choose_gemm(M, N, K, gated != 0, false, true, parts > 0, (size_t)parts * M * N * sizeof(float));
+  if (!plan_bytes_fit(M, N) || K > 0x3fffffff) return fail(TLHIP_EUNSUPPORTED, "tlhip_plan_gemm_bf16: dimension too large");
+  const Choice ch = choose_gemm(M, N, K, gated != 0, false, true, parts > 0, (size_t)std::min(parts, 16) * M * N * sizeof(float));
   const RowsPlan& P = ch.rows;
   int chain = P.S > 0 ? (P.part_units + 7) / 8 : 0, S = P.S;
   for (int i = 0; P.S == 0 && i < ch.npieces; i++) {

@@ -69,7 +69,7 @@ int tlhip_plan_gemm_f16w(int64_t M, int64_t N, int64_t K, int gated, int parts, 
 /* Which kernel forms a bf16 product (tlhip_gemm_bf16_nt, or gated its _swiglu form with N features; parts > 0: the _parts form with
  * room for so many), its result 16-byte aligned, and how: plan[0] 1 = the kernel of few rows (plan[1], [2]: its row and column tiles
  * of 16 to a block), 0 = tiles of 64 or 128 rows; [3] K splits; [4] the longest chain of 32-k steps that one accumulator sums. On the
- * host alone, as above. */
+ * host alone, as above. Both refuse sizes that the products refuse. */
 int tlhip_plan_gemm_bf16(int64_t M, int64_t N, int64_t K, int gated, int parts, int plan[5]);
 /* Every override back to the built-in choice (tlhip_tune_gemv_cols included). */
 int tlhip_tune_reset(void);

@@ -112,3 +112,12 @@ def test_a_k_that_cannot_be_split_has_no_longer_chains_above_128_rows(plans, M, 
     """The tiles cannot split it either: theirs would be all of K (129 x 999 x 8192 369 us, 26 here)."""
     rows, _, _, S, chain = plans.plan_gemm_bf16(M, N, K)
     assert (rows, S) == (1, 1) and chain == _ceil(K // 32, 8)
+
+
+@pytest.mark.parametrize("M,N,K", [(1 << 31, 1 << 31, 128), (1 << 30, 64, 128), (64, 1 << 30, 128), (1 << 29, 1 << 29, 128), (64, 64, 1 << 40)])
+def test_plans_refuse_what_no_product_takes(plans, M, N, K):
+    """With an error: the bytes of the first wrap to none, by which the room for parts was divided."""
+    for ask in (plans.plan_gemm_bf16, plans.plan_gemm_f16w):
+        for parts in (0, 16):
+            with pytest.raises(Exception, match="dimension too large"):
+                ask(M, N, K, False, parts)
