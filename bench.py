@@ -733,8 +733,7 @@ def main():
                     help="also launch the plain 1 GiB copy kernel 3 times (scale for --pmc runs)")
     a = ap.parse_args()
     if a.gpus != 1:
-        print("bench.py: this build runs on ONE GPU; every GPU box of this run has one. "
-              "Run with --gpus 1.", file=sys.stderr)
+        print("bench.py: the framework runs on ONE GPU. Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
 
     pkg = importlib.import_module("cpp-tensorlib_amd")

@@ -72,7 +72,7 @@ enum class kernel_class { elementwise, reduction, matmul };
 
 // auto_ mode: the op size from which GPU-total (single op + flush) beats the CPU path.
 // MI355X census with the reference's own tool (misc/census.cpp compiled against this backend,
-// host = the GPU box's Xeon cores, CPU side = the reference's blocked SGEMM / loops); a
+// host = Xeon cores, CPU side = the reference's blocked SGEMM / loops); a
 // launch plus a flush costs ~12 us here:
 //   matmul      64^3 = 2.6e5 already GPU (0.022 vs cpu 0.035 ms), 512^3 0.091 vs 0.446 ms:
 //               the crossover lies at or below the smallest measured size.
