@@ -20,8 +20,8 @@ SOURCES = ["runtime.hip", "gemv.hip", "elementwise.hip", "modelops.hip", "attn.h
 # -packed-fp32-ops off: some forms of v_pk_*_f32 have given wrong results now and then; hipcc must not form them.
 # Preloaded kernel arguments: the command processor puts a kernel's first 14 dwords of arguments into scalar registers while the
 # launch before it still runs, where a load of them is the first thing that a block waits for (a chain of kernels of 4 us each, with
-# LDS and 16 arguments: 4.69 us a launch without, 4.29 with; recorded in a graph 4.30 and 4.08). Arguments that the first
-# loads need stand first for that.
+# LDS and 16 arguments: 4.69 us a launch without, 4.29 with; recorded in a graph 4.30 and 4.08). What a
+# kernel needs first is to be among them.
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-fno-gpu-rdc",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-mllvm", "-amdgpu-kernarg-preload-count=16",

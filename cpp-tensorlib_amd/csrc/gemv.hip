@@ -32,10 +32,11 @@ namespace tlhip {
 // Block = nw wavefronts arranged as (nw/KW row groups) x (KW K-splits).
 // LDS: x as float4 xs[(chunk*J + j)*XS + lane], J = E/4, XS = LPR + a few (see the kernel), so that lane l's j-th
 // fragment of chunk c is one conflict-free ds_read_b128; then KW*rows floats.
-template <typename Fmt, int R>
+template <typename Fmt, int R, int EPI = kStore>
 struct RowFrag {          // one (row tile, chunk) work item of a lane: R weight units in flight
   uint4 w[R];
   float sc[R];
+  float bg, bu;           // kGeglu: the biases of the row pair that this lane may write
 };
 
 // Weight and scale addresses are formed as a uniform base plus a 32-bit byte
@@ -45,13 +46,14 @@ struct RowFrag {          // one (row tile, chunk) work item of a lane: R weight
 // PAIR: the matrix is two stacked halves of N/2 rows (gate rows, then up rows) and the R
 // fragments are R/2 consecutive rows of the first half followed by the same rows of the
 // second; row0 counts rows of a half.
-template <typename Fmt, int R, bool PAIR = false>
-__device__ __forceinline__ void load_frag(RowFrag<Fmt, R>& f, const uint4* __restrict__ W,
+template <typename Fmt, int R, int EPI>
+__device__ __forceinline__ void load_frag(RowFrag<Fmt, R, EPI>& f, const uint4* __restrict__ W,
                                           const float* __restrict__ scales, int N, int upr,
                                           int row0, int u) {
   // Branch-free: a lane past the end of the row re-reads the row's last unit (its result is
   // never used). Loads under a condition would make the compiler's wait counters
   // conservative - every wait would also cover the loads issued after the ones it needs.
+  constexpr bool PAIR = EPI != kStore;
   u = min(u, upr - 1);
   const char* wb = reinterpret_cast<const char*>(W);
   const char* sb = reinterpret_cast<const char*>(scales);
@@ -73,9 +75,9 @@ struct MixSplits {
   float m[kMergeGroup], l[kMergeGroup];
   float2 a[kMergeGroup], b[kMergeGroup];
   float4 g;
-  __device__ __forceinline__ void load(const Producer& pro, int e) {     // float4 e of [heads][D]
+  __device__ __forceinline__ void load(const ProducerArgs& pro, const float* parts, const float* gates, int e) {     // float4 e of [heads][D]
     const int h = (int)__umulhi(2u * (uint32_t)e, (uint32_t)pro.parts), d = 4 * e - h * pro.D;
-    const float* p = pro.delta + (size_t)h * pro.S * pro.part_ld;        // (rows of an even number of floats)
+    const float* p = parts + (size_t)h * pro.S * pro.part_ld;        // (rows of an even number of floats)
 #pragma unroll
     for (int s = 0; s < kMergeGroup; s++) {
       const float* q = p + (size_t)min(s, pro.S - 1) * pro.part_ld;
@@ -85,9 +87,9 @@ struct MixSplits {
       a[s] = *reinterpret_cast<const float2*>(q + 2 + d);
       b[s] = *reinterpret_cast<const float2*>(q + 4 + d);
     }
-    g = pro.norm_w ? *reinterpret_cast<const float4*>(pro.norm_w + 4 * e) : make_float4(0.f, 0.f, 0.f, 0.f);
+    g = gates ? *reinterpret_cast<const float4*>(gates + 4 * e) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  __device__ __forceinline__ float4 merged(const Producer& pro) const {
+  __device__ __forceinline__ float4 merged(const ProducerArgs& pro, bool gated) const {
     float M = -INFINITY, L = 0.f, w[kMergeGroup], fo;
     merge_group(M, L, m, l, pro.S, w, fo);
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -98,7 +100,7 @@ struct MixSplits {
     }
     const float r = pro.eps / L;
     o.x *= r; o.y *= r; o.z *= r; o.w *= r;
-    if (pro.norm_w) { o.x *= sigmoid_f(g.x); o.y *= sigmoid_f(g.y); o.z *= sigmoid_f(g.z); o.w *= sigmoid_f(g.w); }
+    if (gated) { o.x *= sigmoid_f(g.x); o.y *= sigmoid_f(g.y); o.z *= sigmoid_f(g.z); o.w *= sigmoid_f(g.w); }
     return o;
   }
 };
@@ -109,10 +111,20 @@ struct MixSplits {
 // lanes idle in the 64-lane form (K = 3584 is 112 units: 12.5 % idle; K = 896 is
 // 28 units: 56 % idle); the 16-lane form wastes at most 15 units per row and
 // finishes a row sum inside one DPP row.
+//
+// The arguments up to `block` are the 14 dwords that arrive in scalar registers with the block; what the first loads need is among
+// them, and the launcher has done their divisions. Loaded from memory in the order of their use they were three loads one after the other
+// (of lines that no cache holds yet), with two integer divisions between them, before the first weight was asked for, and two divisions
+// an item in the loop (0.5B int4 step 681 -> 623 us, 7B at 4095 1626 -> 1548, a small Girirax turn 7550 -> 7260).
+//   scales   of an int4 weight; the bias of the post-norm producers (bf16: kernels without scales)
+//   delta    Producer::delta; kAttnMerge: splits | heads << 8 | head size << 24
+//   len      16-byte units of a row | chunks / KW << 13 | chunks % KW << 22
+//   tiles    ntiles / blocks | ntiles % blocks << 19: a block's row tiles, one more for the first ones
+//   block    KW | wavefronts << 5 | blocks << 10 | (ceil(256 / KW) - 1) << 24
 template <typename Fmt, int R, int PRO, int LPR, int EPI = kStore>
 __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
-    const float* x, const uint4* __restrict__ W, const float* __restrict__ scales,
-    float* __restrict__ y, int N, int upr, int KW, int ntiles, const Producer pro) {
+    const float* x, const uint4* __restrict__ W, const float* __restrict__ scales, const float* delta, const float* norm_w,
+    int N, uint32_t len, uint32_t tiles, uint32_t block, float* __restrict__ y, const ProducerArgs pro) {
   constexpr int J = Fmt::E / 4;
   constexpr int QN = 64 / LPR;       // row groups a wavefront works on at once
   extern __shared__ float4 smem4[];
@@ -121,7 +133,8 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   // branches, which also keeps the compiler's wait counters exact
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & (LPR - 1), q = lane / LPR;
-  const int nw = blockDim.x >> 6;
+  const int KW = block & 31, nw = (block >> 5) & 31, grid = (block >> 10) & 0x3fff, threads = nw * 64;
+  const int upr = len & 0x1fff;
   const int chunks = (upr + LPR - 1) / LPR;
   // Row stride of the staged x: LPR float4s plus padding chosen so that the staging writes
   // spread over all banks as well (the J threads of a unit write J rows at the same column:
@@ -132,17 +145,20 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   float* red = xsum + (Fmt::kScaled ? chunks * LPR : 0);   // [nw * QN * 8] K-split partials
   float* nsum = red + nw * QN * 8;                          // [16] per-wavefront sums of squares (norm producer)
   float* fw = nsum + 16;                                    // [heads * 8] split weights (attention-merge producer)
-  float* fL = fw + (PRO == kAttnMerge ? pro.heads * kMergeMax : 0);   // [heads] the heads' sums
+  const uint64_t am = reinterpret_cast<uint64_t>(delta);
+  const int am_S = am & 255, am_heads = (int)(am >> 8) & 0xffff, am_shift = (am >> 24) == 64 ? 4 : 5;   // (float4s of a head: 16 or 32)
+  float* fL = fw + (PRO == kAttnMerge ? am_heads * kMergeMax : 0);    // [heads] the heads' sums
 
-  const int kw = wave % KW;          // which K split this wavefront takes
-  const int wn = wave / KW;          // which row group of the block tile
-  const int groups = nw / KW;        // wavefront row groups per block tile
+  const int inv_kw = (int)(block >> 24) + 1;             // n / KW = n inv_kw >> 8 for the 0 to 16 wavefronts of a block
+  const int wn = wave * inv_kw >> 8; // which row group of the block tile
+  const int kw = wave - wn * KW;     // which K split this wavefront takes
+  const int groups = nw * inv_kw >> 8;   // wavefront row groups per block tile
   const int rows_per_tile = groups * QN * R;
   const int wrow = (wn * QN + q) * R;  // this lane's first row inside a tile
   float* psum = fw;                                         // sums of squares (kPostnormLong: then 1 / rms): post-norm producers
   constexpr bool kPair = EPI != kStore;
-  const auto act = [&](float g, float u, int i) {
-    return EPI == kGeglu ? gelu_tanh(g + pro.gu_bias[i]) * (u + pro.gu_bias[N / 2 + i]) : gated(g, u);
+  const auto act = [&](const RowFrag<Fmt, R, EPI>& f, float g, float u) {
+    return EPI == kGeglu ? gelu_tanh(g + f.bg) * (u + f.bu) : gated(g, u);
   };
   static_assert(!kPair || R >= 2, "a gate/up pair needs two rows per lane group");
   // first row of work item (tile tt): a row of W, or with kPair a row of each half
@@ -154,7 +170,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   TLHIP_MARK(0);
   const float4* x4 = reinterpret_cast<const float4*>(x);
   const int n4 = upr * J;
-  const float4* d4 = reinterpret_cast<const float4*>(pro.delta);
+  const float4* d4 = reinterpret_cast<const float4*>(delta);
   // float4s a thread requests up front: all of x up to 20 floats per thread (K = 18944 on 1024
   // threads), 8 per thread in the norm form, whose vector is the hidden size (registers)
   constexpr bool kPost = PRO == kPostnorm || PRO == kPostnormLong;
@@ -166,80 +182,95 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   float4 pre[kPre];
   float pre_m = -INFINITY, pre_l = 0.f;
   if constexpr (PRO == kAttnMerge) {
-    const int S = pro.S, D4 = pro.D >> 2;
-    const int i = min(tid, n4 - 1), h = i / D4;
-    const float4* pacc = reinterpret_cast<const float4*>(x + 2 * pro.heads * S) + (size_t)h * S * D4 + (i - h * D4);
+    const int S = am_S, D4 = 1 << am_shift;
+    const int i = min(tid, n4 - 1), h = i >> am_shift;
+    const float4* pacc = reinterpret_cast<const float4*>(x + 2 * am_heads * S) + (size_t)h * S * D4 + (i - h * D4);
 #pragma unroll
     for (int sp = 0; sp < kPre; sp++)
       if (sp < S) pre[sp] = pacc[(size_t)sp * D4];
     const int hh = tid / kMergeMax, sp = tid % kMergeMax;
-    if (hh < pro.heads && sp < S) { pre_m = x[hh * S + sp]; pre_l = x[pro.heads * S + hh * S + sp]; }
+    if (hh < am_heads && sp < S) { pre_m = x[hh * S + sp]; pre_l = x[am_heads * S + hh * S + sp]; }
   }
   {
     const float4* aux4 = PRO == kSwiglu ? x4 + n4 : (d4 ? d4 : x4);   // up half, or delta (x when none: ignored)
 #pragma unroll
     for (int k = 0; k < PL; k++) {
-      const int i = min(tid + k * (int)blockDim.x, n4 - 1);
+      const int i = min(tid + k * threads, n4 - 1);
       if (PRO != kAttnMerge) px[k] = x4[i];
       if (PRO != kPlain && PRO != kAttnMerge && PRO != kMixMerge) pa[k] = aux4[i];
-      if (PRO == kRmsnorm || kPost) pn[k] = reinterpret_cast<const float4*>(pro.norm_w)[i];
-      if (kPost && pro.bias) pb[k] = reinterpret_cast<const float4*>(pro.bias)[i];
+      if (PRO == kRmsnorm || kPost) pn[k] = reinterpret_cast<const float4*>(norm_w)[i];
+      if (kPost && scales) pb[k] = reinterpret_cast<const float4*>(scales)[i];
     }
   }
   // split-window producer: the first float4 of the attention's columns that this thread stages
   MixSplits mix;
   int mix_i = 0;
   if constexpr (PRO == kMixMerge) {
-    const int nt = (int)blockDim.x, n = pro.heads * (pro.D >> 2);
+    const int nt = threads, n = pro.heads * (pro.D >> 2);
     mix_i = tid;
     if (pro.first4 > 0 && tid < pro.first4) mix_i += (pro.first4 - tid + nt - 1) / nt * nt;
     // wavefronts whose columns are all other ones ask for nothing
-    if (__any(mix_i - pro.first4 < n)) mix.load(pro, min(mix_i - pro.first4, n - 1));
+    if (__any(mix_i - pro.first4 < n)) mix.load(pro, delta, norm_w, min(mix_i - pro.first4, n - 1));
   }
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  // This wavefront's work items, numbered i = 0, 1, ...: item i is chunk kw + (i % cpw) * KW of
-  // the block's tile number i / cpw. Two items are kept in flight (NS).
+  // This wavefront's work items: the chunks kw, kw + KW, ... of the block's first tile, then those of its next one, and so on.
+  // Two items are kept in flight (NS).
   constexpr int NS = 2;
   // chunks per tile for this wavefront; one (idle) when KW exceeds the chunk count, so that
   // the wavefront still meets the block's barriers at every tile end
-  const int cpw = max((chunks - kw + KW - 1) / KW, 1);
-  const int my_tiles = (int)blockIdx.x < ntiles ? (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x : 0;
+  const int cpw = max((int)((len >> 13) & 0x1ff) + (kw < (int)((len >> 22) & 15) ? 1 : 0), 1);
+  const int my_tiles = (int)(tiles & 0x7ffff) + ((int)blockIdx.x < (int)(tiles >> 19) ? 1 : 0);
   const int n_items = my_tiles * cpw;
-  const auto load_item = [&](RowFrag<Fmt, R>& f, int i) {
-    const int ti = i / cpw, ci = i - ti * cpw;
-    const int tt = min((int)blockIdx.x + ti * (int)gridDim.x, ntiles - 1);
-    load_frag<Fmt, R, kPair>(f, W, scales, N, upr, item_row(tt), (kw + ci * KW) * LPR + li);
+  // the item to ask for next and the one to compute next: tile and chunk; an item's last chunk is number cpw - 1
+  int lt = (int)blockIdx.x, lc = 0, t = (int)blockIdx.x, c = 0;
+  const auto load_item = [&](RowFrag<Fmt, R, EPI>& f) {
+    const int row0 = item_row(lt);
+    load_frag<Fmt, R, EPI>(f, W, scales, N, upr, row0, (kw + lc * KW) * LPR + li);
+    if constexpr (EPI == kGeglu) {     // behind the weights, whose request must not wait for this pointer; asked for with every item: after the last one they would be a round trip of their own
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      const int r = min(row0 + min(LPR == 64 && KW == 1 ? (lane * R) >> 6 : li, R / 2 - 1), N / 2 - 1);
+      f.bg = pro.gu_bias[r];
+      f.bu = pro.gu_bias[N / 2 + r];
+    }
+    const bool end = lc == cpw - 1;
+    lc = end ? 0 : lc + 1;
+    lt += end ? grid : 0;
   };
-  RowFrag<Fmt, R> frag[NS];
-  load_item(frag[0], 0);
+  RowFrag<Fmt, R, EPI> frag[NS];
+  load_item(frag[0]);
   TLHIP_MARK(1);
 
   if constexpr (PRO == kAttnMerge) {
     // The splits' weights e^(m_s - M) and each head's sum, once per block into LDS: sixteen adjacent
     // lanes hold the (up to) sixteen splits of a head. Sums in the order of attn_combine_kernel's
     // wavefront sum over its first sixteen lanes: partners 8, 4, 2 and 1 lanes away in turn.
-    const int S = pro.S, hs = pro.heads * S;
-    const int nl = (pro.heads * kMergeMax + 63) & ~63;
-    for (int e = tid; e < nl; e += blockDim.x) {
+    const int S = am_S, hs = am_heads * S;
+    const auto weigh = [&](int e, float m, float l) {
       const int h = e / kMergeMax, sp = e % kMergeMax;
-      const bool live = h < pro.heads && sp < S;
-      const float m = e == tid ? pre_m : (live ? x[h * S + sp] : -INFINITY);
-      const float l = e == tid ? pre_l : (live ? x[hs + h * S + sp] : 0.f);
-      float M = fmaxf(m, __shfl_xor(m, 8, kWave));
-      M = fmaxf(M, __shfl_xor(M, 4, kWave));
-      M = fmaxf(M, __shfl_xor(M, 2, kWave));
-      M = fmaxf(M, __shfl_xor(M, 1, kWave));
-      const float w = live ? __expf(m - M) : 0.f;
+      float M = fmaxf(m, dpp_read<0x128>(m));     // row_ror:8, 4, 2, 1: partners 8, 4, 2 and 1 lanes away, of lanes alike so far
+      M = fmaxf(M, dpp_read<0x124>(M));
+      M = fmaxf(M, dpp_read<0x122>(M));
+      M = fmaxf(M, dpp_read<0x121>(M));
+      const float w = h < am_heads && sp < S ? __expf(m - M) : 0.f;
       float t = mul_rn(l, w);   // (a product left to the compiler could fuse with the first sum)
-      t = add_rn(t, __shfl_xor(t, 8, kWave));
-      t += __shfl_xor(t, 4, kWave);
-      t += __shfl_xor(t, 2, kWave);
-      t += __shfl_xor(t, 1, kWave);
-      if (h < pro.heads) {
+      t = add_rn(t, dpp_read<0x128>(t));
+      t += dpp_read<0x124>(t);
+      t += dpp_read<0x122>(t);
+      t += dpp_read<0x121>(t);
+      if (h < am_heads) {
         fw[e] = w;
         if (sp == 0) fL[h] = t;
       }
+    };
+    // The pairs requested above, then any that are more than the threads: with loads of its own in this first pass the block
+    // waited for its first weights before it weighed a split.
+    weigh(tid, pre_m, pre_l);
+    for (int e = tid + threads; e < ((am_heads * kMergeMax + 63) & ~63); e += threads) {
+      const int h = e / kMergeMax, sp = e % kMergeMax;
+      const bool live = h < am_heads && sp < S;
+      weigh(e, live ? x[h * S + sp] : -INFINITY, live ? x[hs + h * S + sp] : 0.f);
     }
     __syncthreads();
   }
@@ -252,9 +283,9 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     const int n = pro.parts * pro.part_len;
 #pragma unroll
     for (int k = 0; k < PL; k++) {
-      const int e = 4 * (tid + k * (int)blockDim.x);
+      const int e = 4 * (tid + k * threads);
       float4 v = pa[k];
-      if (pro.bias) { v.x += pb[k].x; v.y += pb[k].y; v.z += pb[k].z; v.w += pb[k].w; }
+      if (scales) { v.x += pb[k].x; v.y += pb[k].y; v.z += pb[k].z; v.w += pb[k].w; }
       float ss = e < n ? v.x * v.x : 0.f;
       ss = e + 1 < n ? fmaf(v.y, v.y, ss) : ss;
       ss = e + 2 < n ? fmaf(v.z, v.z, ss) : ss;
@@ -278,7 +309,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       const int p = s / seg, b = p * len;
       float ss = 0.f;
       for (int i = (s - p * seg) * 64 + lane; i < len; i += 64 * seg) {
-        const float v = pro.delta[b + i] + (pro.bias ? pro.bias[b + i] : 0.f);
+        const float v = delta[b + i] + (scales ? scales[b + i] : 0.f);
         ss = fmaf(v, v, ss);
       }
       ss = wave_sum(ss);
@@ -286,7 +317,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     }
     __syncthreads();
     float* pinv = psum + sums;
-    for (int p = tid; p < pro.parts; p += blockDim.x) {
+    for (int p = tid; p < pro.parts; p += threads) {
       float t = psum[p * seg];
       for (int k = 1; k < seg; k++) t += psum[p * seg + k];
       pinv[p] = 1.0f / sqrtf(t / (float)len + pro.eps);
@@ -303,8 +334,8 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     // nv receives its norm weights. The first PL come from the registers requested above.
     const auto raw = [&](int k, int i, float4& nv) -> float4 {
       if constexpr (PRO == kAttnMerge) {
-        const int D4 = pro.D >> 2, h = i / D4, d4i = i - h * D4, S = pro.S;
-        const float4* pacc = reinterpret_cast<const float4*>(x + 2 * pro.heads * S) + (size_t)h * S * D4 + d4i;
+        const int D4 = 1 << am_shift, h = i >> am_shift, d4i = i - h * D4, S = am_S;
+        const float4* pacc = reinterpret_cast<const float4*>(x + 2 * am_heads * S) + (size_t)h * S * D4 + d4i;
         const float* fh = fw + h * kMergeMax;
         // split 0's product, then the others' added one by one: the merge kernel's order
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -322,8 +353,8 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       if constexpr (PRO == kMixMerge) {
         const int e = i - pro.first4;
         if (e >= 0 && e < pro.heads * (pro.D >> 2)) {
-          if (i != mix_i) mix.load(pro, e);
-          return mix.merged(pro);
+          if (i != mix_i) mix.load(pro, delta, norm_w, e);
+          return mix.merged(pro, norm_w != nullptr);
         }
       }
       float4 v, aux, ab;
@@ -334,11 +365,11 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       if (!have) {
         v = x4[i];
         if (PRO == kSwiglu) aux = x4[n4 + i];
-        if (PRO == kRmsnorm || kPost) { nv = reinterpret_cast<const float4*>(pro.norm_w)[i]; if (d4) aux = d4[i]; }
-        if (kPost && pro.bias) ab = reinterpret_cast<const float4*>(pro.bias)[i];
+        if (PRO == kRmsnorm || kPost) { nv = reinterpret_cast<const float4*>(norm_w)[i]; if (d4) aux = d4[i]; }
+        if (kPost && scales) ab = reinterpret_cast<const float4*>(scales)[i];
       }
       if constexpr (kPost) {
-        if (pro.bias) { aux.x += ab.x; aux.y += ab.y; aux.z += ab.z; aux.w += ab.w; }
+        if (scales) { aux.x += ab.x; aux.y += ab.y; aux.z += ab.z; aux.w += ab.w; }
         const int last = pro.parts - 1;
         float i0 = inv_all, i1 = inv_all, i2 = inv_all, i3 = inv_all;
         if constexpr (PRO == kPostnormLong) {
@@ -366,7 +397,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       // not wait for this sum and the block needs no barrier of its own for it.
       float ss = 0.f;
       int k = 0;
-      for (int i = tid; i < n4; i += blockDim.x, k++) {
+      for (int i = tid; i < n4; i += threads, k++) {
         float4 nv;
         const float4 v = raw(k, i, nv);
         ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
@@ -375,7 +406,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       if (lane == 0) nsum[wave] = ss;
     }
     int k2 = 0;
-    for (int i = tid; i < n4_padded; i += blockDim.x, k2++) {
+    for (int i = tid; i < n4_padded; i += threads, k2++) {
       const bool live = i < n4;
       float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
       if (live) {
@@ -419,13 +450,12 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   // Software pipeline over the items: NS fragments in flight, each requested again right after
   // it has been consumed. Loads are branch-free in the steady-state loop, so the waits of a
   // compute cover exactly its own fragment.
-  int t = 0, c = 0, nt = 0;   // the item being computed: tile, chunk; nt != t at a tile's last chunk
-  const auto compute = [&](const RowFrag<Fmt, R>& cur) {   // item (t, c); nt != t ends its tile
-    const int u = c * LPR + li;
+  const auto compute_item = [&](const RowFrag<Fmt, R, EPI>& cur) {
+    const int ch = kw + c * KW, u = ch * LPR + li;
     if (u < upr) {
       float4 xv[J];
 #pragma unroll
-      for (int j = 0; j < J; j++) xv[j] = xs[(c * J + j) * XS + li];
+      for (int j = 0; j < J; j++) xv[j] = xs[(ch * J + j) * XS + li];
       if (Fmt::kScaled) {
         const float bias = xsum[u];
 #pragma unroll
@@ -436,7 +466,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       }
     }
 
-    if (nt != t) {  // last chunk of tile t for this wavefront: reduce and store
+    if (c == cpw - 1) {  // last chunk of tile t for this wavefront: reduce and store
       const int row0 = item_row(t);
       float v;
       int r;
@@ -461,7 +491,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
         if constexpr (kPair) {
           // the up row's total sits half a wavefront (64-lane form) or R/2 lanes (16-lane form) away
           const float up = LPR == 64 ? swap32(v, v).second : __shfl_down(v, R / 2, kWave);   // .second: the upper half's value in the lower lanes
-          if (writer && r < R / 2 && row0 + r < N / 2) y[row0 + r] = act(v, up, row0 + r);
+          if (writer && r < R / 2 && row0 + r < N / 2) y[row0 + r] = act(cur, v, up);
         } else {
           if (writer && row0 + r < N) y[row0 + r] = v;
         }
@@ -474,7 +504,7 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
           if (kw == 0 && li < R)
             for (int sidx = 0; sidx < KW; sidx++) sum += red[(wrow / R * KW + sidx) * R + li];
           const float up = __shfl_down(sum, R / 2, kWave);
-          if (kw == 0 && li < R / 2 && row0 + li < N / 2) y[row0 + li] = act(sum, up, row0 + li);
+          if (kw == 0 && li < R / 2 && row0 + li < N / 2) y[row0 + li] = act(cur, sum, up);
         } else if (kw == 0 && li < R && row0 + li < N) {
           float sum = 0.f;
           for (int sidx = 0; sidx < KW; sidx++) sum += red[(wrow / R * KW + sidx) * R + li];
@@ -484,24 +514,21 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       }
 #pragma unroll
       for (int r2 = 0; r2 < R; r2++) acc[r2] = 0.f;
+      c = 0;
+      t += grid;
+    } else {
+      c++;
     }
-  };
-  const auto compute_item = [&](const RowFrag<Fmt, R>& f, int i) {
-    const int ti = i / cpw, ci = i - ti * cpw;
-    t = (int)blockIdx.x + ti * (int)gridDim.x;
-    c = kw + ci * KW;
-    nt = ci == cpw - 1 ? -1 : t;
-    compute(f);
   };
   if (n_items >= NS) {
 #pragma unroll
-    for (int k = 1; k < NS; k++) load_item(frag[k], k);
+    for (int k = 1; k < NS; k++) load_item(frag[k]);
     int it = 0;
     for (; it + 2 * NS <= n_items; it += NS) {
 #pragma unroll
       for (int k = 0; k < NS; k++) {
-        compute_item(frag[k], it + k);
-        load_item(frag[k], it + k + NS);
+        compute_item(frag[k]);
+        load_item(frag[k]);
       }
     }
     TLHIP_MARK(3);
@@ -509,16 +536,16 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     // its waits stay exact
     static_assert(NS == 2, "the tail below is written for two fragments");
     if (n_items - it == 2) {
-      compute_item(frag[0], it);
-      compute_item(frag[1], it + 1);
+      compute_item(frag[0]);
+      compute_item(frag[1]);
     } else {
-      compute_item(frag[0], it);
-      load_item(frag[0], it + 2);
-      compute_item(frag[1], it + 1);
-      compute_item(frag[0], it + 2);
+      compute_item(frag[0]);
+      load_item(frag[0]);
+      compute_item(frag[1]);
+      compute_item(frag[0]);
     }
   } else if (n_items == 1) {   // a single item: nothing more to request
-    compute_item(frag[0], 0);
+    compute_item(frag[0]);
   }
   TLHIP_MARK(4);
 }
@@ -777,8 +804,8 @@ static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int pro, int cus, int lds
 }
 
 template <typename Fmt, int PRO, int LPR, int EPI>
-static auto pick_rows_fn(int R) -> void (*)(const float*, const uint4*, const float*, float*, int, int,
-                                            int, int, const Producer) {
+static auto pick_rows_fn(int R) -> void (*)(const float*, const uint4*, const float*, const float*, const float*, int, uint32_t,
+                                            uint32_t, uint32_t, float*, const ProducerArgs) {
   switch (R) {
     case 1:
       if constexpr (EPI == kStore) return gemv_rows_kernel<Fmt, 1, PRO, LPR, EPI>;   // (a pair needs two rows)
@@ -841,8 +868,20 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
     }
     const uint4* Wn = static_cast<const uint4*>(W) + (size_t)n0 * upr;
     const float* sn = scales ? scales + (size_t)n0 * upr : nullptr;
-    hipLaunchKernelGGL(fn, dim3(cfg.blocks), dim3(cfg.nw * 64), cfg.lds, c.stream, x, Wn, sn, y + n0,
-                       (int)n, upr, cfg.KW, ntiles, pro);
+    const int chunks = (upr + cfg.lpr - 1) / cfg.lpr;
+    if (upr > 0x1fff || chunks / cfg.KW > 0x1ff || cfg.KW > 16 || cfg.nw > 16 || cfg.blocks > 0x2000 || ntiles / cfg.blocks > 0x7ffff)
+      return fail(TLHIP_EUNSUPPORTED, "gemv: launch shape out of range");   // (rows that LDS holds end far below)
+    const uint32_t len = (uint32_t)upr | (uint32_t)(chunks / cfg.KW) << 13 | (uint32_t)(chunks % cfg.KW) << 22;
+    const uint32_t tiles = (uint32_t)(ntiles / cfg.blocks) | (uint32_t)(ntiles % cfg.blocks) << 19;
+    const uint32_t block = (uint32_t)cfg.KW | (uint32_t)cfg.nw << 5 | (uint32_t)cfg.blocks << 10 |
+                           (uint32_t)((256 + cfg.KW - 1) / cfg.KW - 1) << 24;
+    const float* third = PRO == kPostnorm ? pro.bias : sn;
+    const float* fourth = pro.delta;
+    if (PRO == kAttnMerge) fourth = reinterpret_cast<const float*>((uint64_t)pro.S | (uint64_t)pro.heads << 8 | (uint64_t)pro.D << 24);
+    hipLaunchKernelGGL(fn, dim3(cfg.blocks), dim3(cfg.nw * 64), cfg.lds, c.stream, x, Wn, third, fourth, pro.norm_w, (int)n, len, tiles,
+                       block, y + n0,
+                       ProducerArgs{pro.parts, pro.part_len, pro.add_x, pro.eps, pro.xout, pro.gu_bias, pro.S, pro.heads, pro.D,
+                                    pro.part_ld, pro.first4});
   }
   TLHIP_CHECK_LAUNCH(census_id);
 }

@@ -208,5 +208,14 @@ struct Producer {
   // kGeglu
   const float* gu_bias = nullptr;
 };
+// What of it the kernel loads from memory, in whole aligned groups: a scalar register that a wider load leaves unused
+// is given to something else, which then waits for the load.
+struct ProducerArgs {
+  int parts, part_len, add_x;
+  float eps;
+  float* xout;
+  const float* gu_bias;
+  int S, heads, D, part_ld, first4;
+};
 
 }  // namespace tlhip
