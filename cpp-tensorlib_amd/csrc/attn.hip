@@ -692,16 +692,27 @@ template <int D> struct Geo {
   static constexpr int COPIES = 2 * kKeys / RPI; // 1 KB copies per tile (K and V)
 };
 
-template <int D> inline size_t lds_bytes(int group, int stages) {
-  return (size_t)stages * 2 * Geo<D>::TILE + (size_t)(2 * D + 2 * group * D + D + group * 64) * sizeof(float);
+// tiles, the new row, the query rows, a tile's probabilities; QKV: the rows' parts as they were copied, 3 KB for each wavefront
+// of query rows and 5 KB for the new row
+template <int D> inline size_t lds_bytes(int group, int stages, bool qkv) {
+  return (size_t)stages * 2 * Geo<D>::TILE + (size_t)(2 * D + group * D + group * 64) * sizeof(float) +
+         (qkv ? ((group * Geo<D>::CH + 63) / 64 * 3 + 5) * 1024 : 0);
 }
 
+// LDS is read and written as f32x4, never as float4: the compiler takes a float4 for something that any copy into LDS may write, and waited
+// before each such access for every copy in flight - the scores for the V rows and for the next tile.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Grid: x = kv heads, y = splits (S). The arguments up to `shape` arrive in scalar registers with the block: what the first requests need.
+// shape = S | stages << 10 | kv heads << 12.
+// Nothing is loaded into vector registers: query rows, biases, table and the new row's parts are copied into LDS like the tiles, all
+// in one go, and a wavefront rotates what it copied itself. A register load would be waited for with every copy in flight (the compiler
+// takes the two kinds to return out of order), so the rows were rotated when the tile had landed and the first scores waited for V.
 template <int D, int GRP, bool QKV>
 __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
-    const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V,
-    float* __restrict__ out, float* __restrict__ part_m, float* __restrict__ part_l,
-    float* __restrict__ part_acc, int ctx, int64_t kv_stride, float scale, int S,
-    const uint32_t* __restrict__ dpos, QkvFuse fz, int kv_rows, int n_kv_heads, int stages) {
+    const float* __restrict__ q, const float* __restrict__ K, const float* __restrict__ V, const float2* __restrict__ table,
+    const float* __restrict__ bq, int64_t kv_stride, int ctx, uint32_t shape, const float* __restrict__ bk, const float* __restrict__ bv,
+    float scale, const uint32_t* __restrict__ dpos, void* Kw, void* Vw, float* __restrict__ out, float* __restrict__ part_m,
+    float* __restrict__ part_l, float* __restrict__ part_acc) {
   using Gm = Geo<D>;
   constexpr int CH = Gm::CH, RB = Gm::RB, KG = Gm::KG, TILE = Gm::TILE, RPI = Gm::RPI;
   constexpr int NW = GRP + 1;
@@ -709,14 +720,15 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, tq = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kvh = blockIdx.x % n_kv_heads, split = blockIdx.x / n_kv_heads;
+  const int S = shape & 0x3ff, stages = (shape >> 10) & 3, n_kv_heads = shape >> 12;
+  const int kvh = blockIdx.x, split = blockIdx.y;
+  const int64_t kv_max = kv_stride / D;                      // rows of the cache
+  const int last_row = (int)min(kv_max - 1, (int64_t)0x7fffffff);
   char* extra = smem + (size_t)stages * 2 * TILE;
   float* newk = reinterpret_cast<float*>(extra);             // the step's own key / value row (QKV)
   float* newv = newk + D;
-  float* qs = newv + D;                                      // QKV: the query rows with bias, not yet rotated
-  float* qrot = qs + GRP * D;                                // the query rows the scores use
-  float* tabs = qrot + GRP * D;                              // QKV: (cos, sin) pairs of the step
-  float* pb = tabs + D;                                      // [GRP][64] probabilities of the current tile
+  float* qrot = newv + D;                                    // the query rows the scores use
+  float* pb = qrot + GRP * D;                                // [GRP][64] probabilities of the current tile
   const float* Kh = K + (size_t)kvh * kv_stride;
   const float* Vh = V + (size_t)kvh * kv_stride;
 
@@ -739,7 +751,7 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
         const int rp = min(wave + i * NW, Gm::COPIES / 2 - 1);   // (a spare slot repeats the last copy)
         const int r = rp * RPI + lane / CH;                      // row of the tile
         const int j = (lane % CH) ^ (r & (CH - 1));              // the chunk that belongs at this lane's position
-        const int key = min(t * kKeys + r, kv_rows - 1);
+        const int key = min(t * kKeys + r, last_row);
         const float* src = (half ? Vh : Kh) + (size_t)key * D + j * 4;
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                          (__attribute__((address_space(3))) void*)(stage + half * TILE + rp * 1024),
@@ -748,32 +760,31 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
   };
 
   // ---- requests, oldest first: the query rows (a few), then the first tile -----------------------
+  // QKV: with bias and table, and what the step's own key/value row is made of, by the wavefront that serves no head (in
+  // every block: which block needs it depends on the position, which may live on the device and is not known yet).
   TLHIP_MARK(0);
-  constexpr int QT = GRP * CH;                               // float4s of the block's query rows
-  float4 q_own = make_float4(0.f, 0.f, 0.f, 0.f), q_bias = q_own;
-  if (tq < QT) {
-    const size_t r = ((size_t)kvh * GRP + tq / CH) * D + (tq % CH) * 4;
-    q_own = *reinterpret_cast<const float4*>(q + r);
-    if (QKV && fz.bq) q_bias = *reinterpret_cast<const float4*>(fz.bq + r);
-  } else if (QKV && tq < QT + D / 4) {
-    q_own = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(fz.table) + (tq - QT) * 4);
-  }
-  // QKV: what the step's own key/value row is made of, requested now by the wavefront that serves
-  // no head (in every block: which block needs it depends on the position, which may live on the
-  // device and is not known yet)
-  float4 nk_own = q_own, nk_oth = q_own, nv_own = q_own, nt0 = q_own, nt1 = q_own;
-  const int nd0 = (lane % CH) * 4;
-  const bool nlo = nd0 < D / 2;
-  if (QKV && wave == GRP) {
-    const int Hq = n_kv_heads * GRP;
-    const float* kraw = q + (size_t)(Hq + kvh) * D;
-    const float* vraw = q + (size_t)(Hq + n_kv_heads + kvh) * D;
-    const int j0 = nlo ? nd0 : nd0 - D / 2;
-    nk_own = load_biased4(kraw, fz.bk ? fz.bk + (size_t)kvh * D : nullptr, nd0);
-    nk_oth = load_biased4(kraw, fz.bk ? fz.bk + (size_t)kvh * D : nullptr, nlo ? nd0 + D / 2 : nd0 - D / 2);
-    nv_own = load_biased4(vraw, fz.bv ? fz.bv + (size_t)kvh * D : nullptr, nd0);
-    nt0 = *reinterpret_cast<const float4*>(fz.table + j0);
-    nt1 = *reinterpret_cast<const float4*>(fz.table + j0 + 2);
+  constexpr int QT = GRP * CH;                               // float4s of the block's query rows (in the heads' wavefronts)
+  constexpr int QW = (QT + 63) / 64;
+  const int d0 = (lane % CH) * 4;                            // this thread's values of its row
+  char* pre = reinterpret_cast<char*>(pb + GRP * 64) + min(wave, QW) * 3072;   // this wavefront's 1 KB slots
+  const auto copy16 = [](const float* src, void* dst) {      // 16 bytes a lane, lane after lane
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst,
+                                     16, 0, 0);
+  };
+  if (wave < QW) {
+    const size_t row = ((size_t)kvh * GRP + min(tq / CH, GRP - 1)) * D;
+    copy16(q + row + d0, QKV ? pre : reinterpret_cast<char*>(qrot) + wave * 1024);   // (lanes past the rows: into pb, not in use yet)
+    if constexpr (QKV) {
+      copy16(reinterpret_cast<const float*>(table) + d0, pre + 1024);
+      if (bq) copy16(bq + row + d0, pre + 2048);
+    }
+  } else if (QKV && wave == GRP) {
+    const float* kraw = q + (size_t)(n_kv_heads * GRP + kvh) * D;
+    copy16(kraw + d0, pre);
+    copy16(reinterpret_cast<const float*>(table) + d0, pre + 1024);
+    copy16(kraw + (size_t)n_kv_heads * D + d0, pre + 3072);
+    if (bk) copy16(bk + (size_t)kvh * D + d0, pre + 2048);
+    if (bv) copy16(bv + (size_t)kvh * D + d0, pre + 4096);
   }
   __builtin_amdgcn_sched_barrier(0);
   copy_tile(split, smem);
@@ -785,49 +796,43 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
   bool has_new = false;
   if constexpr (QKV) {
     new_pos = dpos ? (int64_t)*dpos : (int64_t)ctx - 1;
-    has_new = new_pos < fz.kv_max;
-    ctx = (int)min(new_pos, fz.kv_max) + (has_new ? 1 : 0);  // keys [0, pos) of the cache and the new one
+    has_new = new_pos < kv_max;
+    ctx = (int)min(new_pos, kv_max) + (has_new ? 1 : 0);     // keys [0, pos) of the cache and the new one
   } else if (dpos) {
     ctx = min(ctx, (int)*dpos + 1);
   }
   const int newt = (int)(new_pos / kKeys), newj = (int)(new_pos % kKeys);
   const bool owner = QKV && has_new && newt % S == split;    // this block's tiles include the step's position
 
-  // ---- query rows into LDS (the copies stay in flight: wait for what is older than them) ----------
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CPW) : "memory");
-  if (tq < QT) {
-    if constexpr (QKV) {
-      q_own.x += q_bias.x; q_own.y += q_bias.y; q_own.z += q_bias.z; q_own.w += q_bias.w;
-      *reinterpret_cast<float4*>(qs + (tq / CH) * D + (tq % CH) * 4) = q_own;
-    } else {
-      *reinterpret_cast<float4*>(qrot + (tq / CH) * D + (tq % CH) * 4) = q_own;
+  // ---- the query rows and the new row, rotated (the tile's copies stay in flight: wait for what is older than them) ------------
+  if (QKV && (wave < QW || (owner && wave == GRP))) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CPW) : "memory");
+    const auto got = [&](int slot, int l) { return *reinterpret_cast<const f32x4*>(pre + slot * 1024 + l * 16); };
+    const bool lo = d0 < D / 2;
+    const int j0 = lo ? d0 : d0 - D / 2, other = lane ^ (CH / 2);   // where the rotation partners lie
+    f32x4 own = got(0, lane), oth = got(0, other);
+    const f32x4 t0 = got(1, j0 / 2), t1 = got(1, j0 / 2 + 1);
+    if (wave < QW ? bq : bk) {
+      own += got(2, lane);
+      oth += got(2, other);
     }
-  } else if (QKV && tq < QT + D / 4) {
-    *reinterpret_cast<float4*>(tabs + (tq - QT) * 4) = q_own;
-  }
-  if constexpr (QKV) {
-    barrier();
-    if (tq < QT) {
-      const int g = tq / CH, d0 = (tq % CH) * 4;
-      const bool lo = d0 < D / 2;
-      const int j0 = lo ? d0 : d0 - D / 2;
-      const float4 own = *reinterpret_cast<const float4*>(qs + g * D + d0);
-      const float4 oth = *reinterpret_cast<const float4*>(qs + g * D + (lo ? d0 + D / 2 : d0 - D / 2));
-      const float4 t0 = *reinterpret_cast<const float4*>(tabs + 2 * j0);        // (c0, s0, c1, s1)
-      const float4 t1 = *reinterpret_cast<const float4*>(tabs + 2 * j0 + 4);    // (c2, s2, c3, s3)
-      *reinterpret_cast<float4*>(qrot + g * D + d0) = rope4_pair(own, oth, t0, t1, lo);
+    const auto f4 = [](f32x4 v) { return make_float4(v[0], v[1], v[2], v[3]); };
+    const float4 r = rope4_pair(f4(own), f4(oth), f4(t0), f4(t1), lo);
+    const f32x4 rot = {r.x, r.y, r.z, r.w};
+    if (wave < QW) {
+      if (tq < QT) *reinterpret_cast<f32x4*>(qrot + tq * 4) = rot;
+    } else if (lane < CH) {
+      // kept in LDS for this block's scores and stored into the cache (rows of other tiles belong to other blocks)
+      f32x4 v = got(3, lane);
+      if (bv) v += got(4, lane);
+      const size_t at = (size_t)kvh * kv_stride + (size_t)new_pos * D + d0;
+      *reinterpret_cast<f32x4*>(newk + d0) = rot;
+      *reinterpret_cast<f32x4*>(newv + d0) = v;
+      *reinterpret_cast<f32x4*>(static_cast<float*>(Kw) + at) = rot;
+      *reinterpret_cast<f32x4*>(static_cast<float*>(Vw) + at) = v;
     }
-    // the step's own key/value row: formed by the wavefront that serves no head, kept in LDS for
-    // this block's scores and stored into the cache (rows of other tiles belong to other blocks)
-    if (owner && wave == GRP && lane < CH) {
-      float* krow = static_cast<float*>(fz.Kw) + (size_t)kvh * kv_stride + (size_t)new_pos * D;
-      float* vrow = static_cast<float*>(fz.Vw) + (size_t)kvh * kv_stride + (size_t)new_pos * D;
-      const float4 kr = rope4_pair(nk_own, nk_oth, nt0, nt1, nlo);
-      *reinterpret_cast<float4*>(krow + nd0) = kr;
-      *reinterpret_cast<float4*>(vrow + nd0) = nv_own;
-      *reinterpret_cast<float4*>(newk + nd0) = kr;
-      *reinterpret_cast<float4*>(newv + nd0) = nv_own;
-    }
+  } else if (!QKV && wave < QW) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CPW) : "memory");
   }
   // ---- the tiles of this split ---------------------------------------------------------------------
   const int h = wave;                                        // the query head this wavefront serves (wave GRP: none)
@@ -838,11 +843,11 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
   // of more than eight wavefronts leave a lane fewer registers than the row needs at head size
   // 128; they read the row from LDS as they go.)
   constexpr bool QREG = D == 64 || NW <= 8;
-  float4 qreg[QREG ? CH : 1];
+  f32x4 qreg[QREG ? CH : 1];
   barrier();                                                 // the rotated query rows (and the new row) are in LDS
   if (QREG && h < GRP) {
 #pragma unroll
-    for (int j = 0; j < CH; j++) qreg[j] = *reinterpret_cast<const float4*>(qrot + h * D + j * 4);
+    for (int j = 0; j < CH; j++) qreg[j] = *reinterpret_cast<const f32x4*>(qrot + h * D + j * 4);
   }
   TLHIP_MARK(1);
   float m = -INFINITY, l = 0.f;
@@ -877,14 +882,14 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
       float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
 #pragma unroll
       for (int j = 0; j < CH; j += 4) {
-        const float4 k0 = *reinterpret_cast<const float4*>(smem + (kx ^ ((j + 0) << 4)));
-        const float4 k1 = *reinterpret_cast<const float4*>(smem + (kx ^ ((j + 1) << 4)));
-        const float4 k2 = *reinterpret_cast<const float4*>(smem + (kx ^ ((j + 2) << 4)));
-        const float4 k3 = *reinterpret_cast<const float4*>(smem + (kx ^ ((j + 3) << 4)));
-        const float4 q0 = QREG ? qreg[QREG ? j + 0 : 0] : *reinterpret_cast<const float4*>(qh + (j + 0) * 4);
-        const float4 q1 = QREG ? qreg[QREG ? j + 1 : 0] : *reinterpret_cast<const float4*>(qh + (j + 1) * 4);
-        const float4 q2 = QREG ? qreg[QREG ? j + 2 : 0] : *reinterpret_cast<const float4*>(qh + (j + 2) * 4);
-        const float4 q3 = QREG ? qreg[QREG ? j + 3 : 0] : *reinterpret_cast<const float4*>(qh + (j + 3) * 4);
+        const f32x4 k0 = *reinterpret_cast<const f32x4*>(smem + (kx ^ ((j + 0) << 4)));
+        const f32x4 k1 = *reinterpret_cast<const f32x4*>(smem + (kx ^ ((j + 1) << 4)));
+        const f32x4 k2 = *reinterpret_cast<const f32x4*>(smem + (kx ^ ((j + 2) << 4)));
+        const f32x4 k3 = *reinterpret_cast<const f32x4*>(smem + (kx ^ ((j + 3) << 4)));
+        const f32x4 q0 = QREG ? qreg[QREG ? j + 0 : 0] : *reinterpret_cast<const f32x4*>(qh + (j + 0) * 4);
+        const f32x4 q1 = QREG ? qreg[QREG ? j + 1 : 0] : *reinterpret_cast<const f32x4*>(qh + (j + 1) * 4);
+        const f32x4 q2 = QREG ? qreg[QREG ? j + 2 : 0] : *reinterpret_cast<const f32x4*>(qh + (j + 2) * 4);
+        const f32x4 q3 = QREG ? qreg[QREG ? j + 3 : 0] : *reinterpret_cast<const f32x4*>(qh + (j + 3) * 4);
         s0 = fmaf(q0.x, k0.x, s0); s0 = fmaf(q0.y, k0.y, s0); s0 = fmaf(q0.z, k0.z, s0); s0 = fmaf(q0.w, k0.w, s0);
         s1 = fmaf(q1.x, k1.x, s1); s1 = fmaf(q1.y, k1.y, s1); s1 = fmaf(q1.z, k1.z, s1); s1 = fmaf(q1.w, k1.w, s1);
         s2 = fmaf(q2.x, k2.x, s2); s2 = fmaf(q2.y, k2.y, s2); s2 = fmaf(q2.z, k2.z, s2); s2 = fmaf(q2.w, k2.w, s2);
@@ -916,11 +921,11 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
         const uint32_t vx = ((uint32_t)(vt - smem) + kg * CH * RB) ^ (cg << 4);   // the group's first row, this lane's chunk
 #pragma unroll
         for (int i = 0; i < CH; i += 4) {
-          const float4 p4 = *reinterpret_cast<const float4*>(ph + i);
+          const f32x4 p4 = *reinterpret_cast<const f32x4*>(ph + i);
           const float pp[4] = {p4.x, p4.y, p4.z, p4.w};
 #pragma unroll
           for (int u = 0; u < 4; u++) {
-            const float4 v = *reinterpret_cast<const float4*>(smem + (vx ^ ((i + u) << 4)) + (i + u) * RB);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(smem + (vx ^ ((i + u) << 4)) + (i + u) * RB);
             acc.x = fmaf(pp[u], v.x, acc.x); acc.y = fmaf(pp[u], v.y, acc.y);
             acc.z = fmaf(pp[u], v.z, acc.z); acc.w = fmaf(pp[u], v.w, acc.w);
           }
@@ -933,7 +938,7 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
           const int row = min(kg * CH + i, nvalid - 1);
           const char* vrow = with_new && row == newj ? reinterpret_cast<const char*>(newv) + (cg << 4)
                                                      : vt + row * RB + ((cg ^ (row & (CH - 1))) << 4);
-          const float4 v = *reinterpret_cast<const float4*>(vrow);
+          const f32x4 v = *reinterpret_cast<const f32x4*>(vrow);
           const float pp = ph[i];
           acc.x = fmaf(pp, v.x, acc.x); acc.y = fmaf(pp, v.y, acc.y);
           acc.z = fmaf(pp, v.z, acc.z); acc.w = fmaf(pp, v.w, acc.w);
@@ -1083,8 +1088,8 @@ static int launch_gqa(const float* q, const float* K, const float* V, float* out
     pl = pm + hs;
     pacc = pl + hs;
   }
-  const size_t lds = gqa::lds_bytes<D>(group, p.stages);
-  const dim3 grid((unsigned)(Hkv * S)), block(64 * (group + 1));
+  const size_t lds = gqa::lds_bytes<D>(group, p.stages, fuse != nullptr);
+  const dim3 grid((unsigned)Hkv, (unsigned)S), block(64 * (group + 1));
   const int64_t kv_stride = kv_max * D;
   const QkvFuse fz = fuse ? *fuse : QkvFuse{};
   hipError_t e = hipSuccess;
@@ -1093,8 +1098,8 @@ static int launch_gqa(const float* q, const float* K, const float* V, float* out
     if (lds > 64 * 1024)
       e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess)
-      hipLaunchKernelGGL(kernel, grid, block, lds, c.stream, q, K, V, out, pm, pl, pacc, ctx, kv_stride, scale, S, dpos,
-                         fz, (int)kv_max, Hkv, p.stages);
+      hipLaunchKernelGGL(kernel, grid, block, lds, c.stream, q, K, V, fz.table, fz.bq, kv_stride, ctx,
+                         (uint32_t)S | (uint32_t)p.stages << 10 | (uint32_t)Hkv << 12, fz.bk, fz.bv, scale, dpos, fz.Kw, fz.Vw, out, pm, pl, pacc);
   };
 #define TLHIP_GQA(GG) \
   if (fuse) go(gqa::attn_gqa_kernel<D, GG, true>); else go(gqa::attn_gqa_kernel<D, GG, false>)

@@ -61,6 +61,20 @@ def test_attn_gqa_and_split_boundaries(lib, orc, D, Hq, Hkv, ctx, kernel):
     assert allclose(got, want, RTOL, ATOL), maxrel(got, want)
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,ctx", [(64, 14, 2, 16421), (128, 24, 8, 6153), (128, 32, 4, 8192), (64, 6, 2, 8193), (64, 40, 40 // 5, 4200)])
+def test_attn_several_tiles_a_split(lib, orc, D, Hq, Hkv, ctx):
+    """Splits of two to four 64-key tiles, the last one whole or not: a tile is copied while the one before it is used."""
+    print("case attn tiles", D, Hq, Hkv, ctx, flush=True)
+    q = orc.normal(Hq * D, 31).reshape(Hq, D)
+    K = orc.normal(Hkv * ctx * D, 32).reshape(Hkv, ctx, D)
+    V = orc.normal(Hkv * ctx * D, 33).reshape(Hkv, ctx, D)
+    scale = 1.0 / np.sqrt(float(D))
+    want = orc.attn_decode(q, K, V, scale, ctx=ctx)
+    got = _run(lib, q, K, V, ctx, scale)
+    assert allclose(got, want, RTOL, ATOL), maxrel(got, want)
+    assert np.array_equal(_run(lib, q, K, V, ctx, scale), got)
+
+
 def test_attn_closed_forms(lib, orc):
     H, D, ctx = 4, 128, 300
     q = orc.normal(H * D, 1).reshape(H, D)
