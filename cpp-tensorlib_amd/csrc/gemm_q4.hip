@@ -16,7 +16,7 @@
 // 102 vector instructions beside 16 MFMAs per slab and wavefront are left, 64 of them the scales'. Behind the MFMAs they and
 // the MFMAs of a SIMD's two wavefronts add up (512 x 32768 x 3584: 235 us = 510 TFLOP/s; without the scales 192, without all
 // of it and the loads 148; wave priorities and a staggered start change nothing), so they go between them, six of which two
-// wavefronts hide behind one: 24 shapes 0.99 to 1.10 times as fast, 1.03 on average, 512 x 37888 x 3584 gated 1.06. Two blocks per CU, two barriers per 128 k.
+// wavefronts hide behind one: 24 shapes 0.99 to 1.10 times as fast, 1.03 on average, 512 x 37888 x 3584 gated 1.06. Two blocks per CU, one barrier per 128 k.
 // Rows come in blocks of 64: 301 rows waste 6 % of the products, 128-row tiles waste 28 %. us, before -> now: 301 rows
 // gated 37888 x 3584 303 -> 209, 3584 x 18944 150 -> 113, 4608 x 3584 48 -> 42; 512 rows 393 -> 320, 207 -> 176, 61 -> 58.
 #include "gemm_shared.hpp"
@@ -143,22 +143,23 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
       }
     }
   };
-  frag16 w[2][2][2];                               // [set][column tile][groups 0 1 | 2 3]
-  f32x4u s[2][2];
-  auto load_w = [&](int set, int u) {
+  struct Words { frag16 w[2][2]; f32x4u s[2]; };   // of a unit: [column tile][groups 0 1 | 2 3], the scales
+  auto load_w = [&](Words& x, int u) __attribute__((always_inline)) {
     const int g0 = 4 * (ubeg + u);
 #pragma unroll
     for (int j = 0; j < 2; j++) {
 #pragma unroll
-      for (int p = 0; p < 2; p++) w[set][j][p] = *reinterpret_cast<const frag16*>(wrow[j] + 16 * min(g0 + 2 * p + half, groups - 1));
+      for (int p = 0; p < 2; p++) x.w[j][p] = *reinterpret_cast<const frag16*>(wrow[j] + 16 * min(g0 + 2 * p + half, groups - 1));
       if (g0 + 4 <= groups) {
-        s[set][j] = *reinterpret_cast<const f32x4u*>(srow[j] + g0);
+        x.s[j] = *reinterpret_cast<const f32x4u*>(srow[j] + g0);
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++) s[set][j][e] = srow[j][min(g0 + e, groups - 1)];
+        for (int e = 0; e < 4; e++) x.s[j][e] = srow[j][min(g0 + e, groups - 1)];
       }
     }
   };
+  frag16 w[2][2];                                  // of the unit in hand: [column tile][16-k step][group of the pair]
+  f32x4u s[2];
   auto barrier = [] {                              // without the fence that would wait for every copy in flight
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -187,14 +188,14 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
 #pragma unroll
     for (int v = 0; v < 16; v++) grp[1][j][v] = 0.f;
   auto fetch = [&](const char* at, int i, int q) __attribute__((always_inline)) { a[q] = *reinterpret_cast<const frag16*>(at + aoff[q >> 1] + (q & 1) * kPlane + i * 32 * kSlab * 2); };
-  auto nibbles = [&](int set, int g, int ks, int j) __attribute__((always_inline)) { b[ks][j] = nib8(w[set][j][g >> 1][2 * ks + (g & 1)]); };
+  auto nibbles = [&](int g, int ks, int j) __attribute__((always_inline)) { b[ks][j] = nib8(w[j][g >> 1][2 * ks + (g & 1)]); };
   auto scaled = [&](int i, int q) __attribute__((always_inline)) {   // a quarter of half i's sums
 #pragma unroll
     for (int v = 8 * (q & 1); v < 8 * (q & 1) + 8; v++) acc[i][q >> 1][v] = fmaf(grp[i][q >> 1][v], ps[q >> 1], acc[i][q >> 1][v]);
     asm volatile("" : "+v"(acc[i][q >> 1]));       // (here: the compiler would gather the slabs' scales, and spill their sums)
   };
   // next: where the slab after this one lies (nullptr: the unit ends)
-  auto slab = [&](const char* at, const char* next, int set, int g) __attribute__((always_inline)) {
+  auto slab = [&](const char* at, const char* next, int g) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
 #pragma unroll
@@ -205,74 +206,85 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_kernel(const char* __restrict_
         if (i == 0) fetch(at, 1, q);
         else if (next) fetch(next, 0, q);
         scaled(1 - i, q);
-        if (i == 0 && q < 2) nibbles(set, g, 1, q);
-        if (i == 1 && q >= 2 && next) nibbles(set, g + 1, 0, q - 2);
+        if (i == 0 && q < 2) nibbles(g, 1, q);
+        if (i == 1 && q >= 2 && next) nibbles(g + 1, 0, q - 2);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int j = 0; j < 2; j++) ps[j] = s[set][j][g];
+      for (int j = 0; j < 2; j++) ps[j] = s[j][g];
     }
   };
-  auto unit = [&](int set, int u) __attribute__((always_inline)) {
-    // my copies and loads of unit u have landed (those of u + 1 - eight copies, six loads - may be in flight), and my zeros where
-    // it is the one that lacks groups; past the barrier that holds for every wavefront
-    if (4 * (ubeg + u) + 8 <= groups && u + 1 < nu) asm volatile("s_waitcnt vmcnt(14)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  // What was asked for of unit u has landed - my copies and loads, and my zeros where it lacks groups - and my reads of the unit
+  // before it are done; past the barrier that holds for every wavefront. This stands where nothing younger is in flight, and names
+  // the words' registers: the compiler takes copies and register loads to return out of order, so at the first use of a word it waits
+  // for everything. With two units asked for ahead that was the whole latency of the second, once per unit (so, and with the rows' exponents
+  // below asked for at once, a 301-token prompt of eight 7B layers 3912 -> 3746 us).
+  auto landed = [&](Words& x, int u) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 2; j++) asm volatile("" : "+v"(x.w[j][0]), "+v"(x.w[j][1]), "+v"(x.s[j]));
     barrier();
     // words of groups (half) and 2 + (half): a half's k of both groups of a pair
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
       for (int p = 0; p < 2; p++) {
-        frag16& x = w[set][j][p];
-        const auto y = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
-        const auto z = __builtin_amdgcn_permlane32_swap(x[2], x[3], false, false);
-        x = frag16{y[0], y[1], z[0], z[1]};        // [16-k step][group of the pair]
+        const auto y = __builtin_amdgcn_permlane32_swap(x.w[j][p][0], x.w[j][p][1], false, false);
+        const auto z = __builtin_amdgcn_permlane32_swap(x.w[j][p][2], x.w[j][p][3], false, false);
+        w[j][p] = frag16{y[0], y[1], z[0], z[1]};  // [16-k step][group of the pair]
       }
-    const char* at = ring + set * kUnit;
-    const int have = groups - 4 * (ubeg + u);
-    if (have < 4) {                                // groups past the last are multiplied, and scaled to nothing
+    const int have = groups - 4 * (ubeg + u);      // groups past the last are multiplied, and scaled to nothing
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+    for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int g = 1; g < 4; g++) s[set][j][g] = g < have ? s[set][j][g] : 0.f;
+      for (int g = 0; g < 4; g++) s[j][g] = g < have ? x.s[j][g] : 0.f;
+  };
+  {
+    Words x;
+    copy(0, 0);
+    load_w(x, 0);
+    landed(x, 0);
+  }
+  for (int u = 0;; u++) {
+    Words x;
+    const bool more = u + 1 < nu;
+    if (more) {                                    // (everyone is done with that stage)
+      copy(u + 1, (u + 1) & 1);
+      load_w(x, u + 1);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    const char* at = ring + (u & 1) * kUnit;
 #pragma unroll
     for (int q = 0; q < 4; q++) fetch(at, 0, q);
 #pragma unroll
-    for (int j = 0; j < 2; j++) nibbles(set, 0, 0, j);
+    for (int j = 0; j < 2; j++) nibbles(0, 0, j);
 #pragma unroll
-    for (int g = 0; g < 4; g++) slab(at + g * kImage, g < 3 ? at + (g + 1) * kImage : nullptr, set, g);
-    barrier();                                     // everyone is done with this stage
-    if (u + 2 < nu) {
-      copy(u + 2, set);
-      load_w(set, u + 2);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  copy(0, 0);
-  load_w(0, 0);
-  if (nu > 1) {
-    copy(1, 1);
-    load_w(1, 1);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  for (int u = 0; u < nu; u += 2) {
-    unit(0, u);
-    if (u + 1 < nu) unit(1, u + 1);
+    for (int g = 0; g < 4; g++) slab(at + g * kImage, g < 3 ? at + (g + 1) * kImage : nullptr, g);
+    if (!more) break;
+    landed(x, u + 1);
   }
 
 #pragma unroll
   for (int q = 0; q < 4; q++) scaled(1, q);        // the last half's
   // acc[v] of lane l: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32. The row's exponent comes back out, exactly.
   const int m0 = rb * kBM;
+  int4 e4[2][4];                                   // four rows each; (past M: into the images behind the exponents, not used). Asked for one
+#pragma unroll                                     // by one between the stores they were 32 round trips, each behind a store
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) e4[i][g] = *reinterpret_cast<const int4*>(ea + m0 + i * 32 + 8 * g + 4 * half);
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) asm volatile("" : "+v"(e4[i][g].x), "+v"(e4[i][g].y), "+v"(e4[i][g].z), "+v"(e4[i][g].w));   // (here, once)
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       const int gm = m0 + i * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
       if (gm >= M) continue;
-      const int e = ea[gm];
+      const int4 q4 = e4[i][v >> 2];
+      const int e = (v & 3) == 0 ? q4.x : (v & 3) == 1 ? q4.y : (v & 3) == 2 ? q4.z : q4.w;
       if (GU && gridDim.y == 1) {
         const int f = (n0 >> 1) + wave * 32 + l32;
         if (f >= N) continue;
