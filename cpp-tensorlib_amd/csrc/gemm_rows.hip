@@ -4,8 +4,8 @@
 // chain of latencies of one block. gemm_bf16_nt_kernel (prefill.hip) walks K in slabs of 32 through LDS, two
 // barriers and one load round trip per slab: ten slabs were 20 us for weights that take 2 us to read. Here a
 // block has no barrier until its sums are complete: its eight wavefronts split the block's K range between
-// them (wavefront w takes the 32-k steps w, w + 8, ...), each with the WHOLE tile's accumulators; weights go straight
-// into the registers of the MFMA that uses them, activations through slots of LDS of the wavefront's own. The sums meet in
+// them (wavefront w takes the 32-k steps w, w + 8, ...), each with the WHOLE tile's accumulators; both operands come
+// through slots of LDS of the wavefront's own (int4 weights straight into registers). The sums meet in
 // LDS once at the end, in a fixed order.
 //
 // Both operands of v_mfma_f32_16x16x32_bf16 are K-contiguous per lane: lane l supplies row l % 16 and k
@@ -46,8 +46,16 @@ __host__ __device__ constexpr int lds_bytes_q4(int TM, int TN) {
 // at five row tiles).
 __host__ __device__ constexpr int steps_ahead(int TM, int TN) { return TM == 1 && TN <= 2 ? 4 / TN : 1; }
 __host__ __device__ constexpr int sum_stride(int TN) { return TN == 4 ? 16 * TN : 16 * TN + 4; }
+// Steps of weights in LDS: one more than of activations, or one where only so two blocks fit a CU (128 x 4864 gated x 896, four row tiles
+// over two column tiles: 19.0 us so, 21.0 with one block and two steps).
+__host__ __device__ constexpr int ring_bf16(int TM, int TN, int WS) { return kWaves * (steps_ahead(TM, TN) * TM * 2048 + WS * TN * 1024); }
+__host__ __device__ constexpr int sums_bf16(int TM, int TN) { return kWaves * 16 * TM * sum_stride(TN) * 4; }
+__host__ __device__ constexpr int weight_steps(int TM, int TN) {
+  const int AS = steps_ahead(TM, TN), half = 80 * 1024;
+  return AS == 1 && ring_bf16(TM, TN, 2) > half && ring_bf16(TM, TN, 1) <= half && sums_bf16(TM, TN) <= half ? 1 : AS + 1;
+}
 __host__ __device__ constexpr int lds_bytes_bf16(int TM, int TN) {
-  const int ring = kWaves * steps_ahead(TM, TN) * TM * 2048, sums = kWaves * 16 * TM * sum_stride(TN) * 4;
+  const int ring = ring_bf16(TM, TN, weight_steps(TM, TN)), sums = sums_bf16(TM, TN);
   return ring > sums ? ring : sums;
 }
 
@@ -92,28 +100,33 @@ __device__ __forceinline__ f32x4 mma(const frag16& a, const frag16& b, f32x4 c) 
 // matrix instructions. So little is in flight beyond what is needed next - one step of activations, each tile requested again
 // as soon as it is in registers, two steps of weights - and three column tiles (203 blocks instead of 152) are a choice too:
 // 12.3 us. With two steps of activations 13.2, all weights first 12.8. 227 shapes of 1 to 80 rows: 0.98 to 1.4 times as fast.
+// Weights in LDS like the activations, and what the first copies need from registers and without a division: 145 shapes of 2 to 300
+// rows 1.08 times as fast, 0.98 to 1.18 (37 x 4608 x 3584 16.0 -> 14.4 us, 77 x 4864 gated x 896 12.2 -> 11.4).
 template <int TM, int TN, bool GU>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const float* __restrict__ A, const void* __restrict__ W,
                                                                        float* __restrict__ C, int M, int N, int K, int part_units,
                                                                        int ldc, int ff, int row_blocks) {
-  constexpr int BM = 16 * TM, BN = 16 * TN, LD = sum_stride(TN), AS = steps_ahead(TM, TN), WS = AS + 1;
-  extern __shared__ __attribute__((aligned(1024))) float red[];   // activations in flight, then [8][BM][LD] sums
+  constexpr int BM = 16 * TM, BN = 16 * TN, LD = sum_stride(TN), AS = steps_ahead(TM, TN), WS = weight_steps(TM, TN);
+  extern __shared__ __attribute__((aligned(1024))) float red[];   // operands in flight, then [8][BM][LD] sums
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, quarter = lane >> 4;
   // one contiguous run of tiles per XCD, row blocks fastest: those share a weight tile in one L2
-  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
+  // (the grid's size from the arguments, which are in registers already, and no division where one block holds all rows)
+  constexpr int TW = GU ? BN / 2 : BN;
+  const int nb = row_blocks * ((N + TW - 1) / TW), xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
   const int lid = xcd * q8 + min(xcd, r8) + within;
-  const int m0 = lid % row_blocks * BM, n0 = lid / row_blocks * BN;
+  const int tile = row_blocks == 1 ? lid : lid / row_blocks;
+  const int m0 = (lid - tile * row_blocks) * BM, n0 = tile * BN;
   C += (size_t)blockIdx.y * M * ldc;
   const int units = K / kStep, ubeg = blockIdx.y * part_units, uend = min(units, ubeg + part_units);
   const int first = ubeg + wave, mine = first < uend ? (uend - first + kWaves - 1) / kWaves : 0;
 
   // byte offsets of this lane's rows (clamped into the operands: what lies past an edge is not stored). A 1 KB copy
   // of activations is eight rows of 128 bytes, the 16-byte chunks of row r in the order c ^ (r & 7), which spreads
-  // the fragment reads (16 rows, one chunk) over the LDS banks.
+  // the fragment reads (16 rows, one chunk) over the LDS banks; of weights sixteen rows of 64, in the order c ^ (r / 2 & 3).
   uint32_t aoff[TM][2], woff[TN];
 #pragma unroll
   for (int j = 0; j < TN; j++) {
-    const int col = 16 * j + r16;
+    const int col = 16 * j + (lane >> 2);
     int r;
     if (GU) {
       const int f = min((n0 >> 1) + col % (BN / 2), N - 1);
@@ -121,7 +134,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
     } else {
       r = min(n0 + col, N - 1);
     }
-    woff[j] = (uint32_t)r * (uint32_t)(K * 2) + quarter * 16;
+    woff[j] = (uint32_t)r * (uint32_t)(K * 2) + ((lane & 3) ^ (lane >> 3 & 3)) * 16;
   }
 #pragma unroll
   for (int t = 0; t < TM; t++)
@@ -129,7 +142,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
     for (int h = 0; h < 2; h++)
       aoff[t][h] = (uint32_t)min(m0 + 16 * t + 8 * h + (lane >> 3), M - 1) * (uint32_t)(K * 4) + ((lane & 7) ^ (lane >> 3)) * 16;
   const int frag[2] = {r16 * 128 + ((2 * quarter) ^ (r16 & 7)) * 16, r16 * 128 + ((2 * quarter + 1) ^ (r16 & 7)) * 16};
-  char* slots = reinterpret_cast<char*>(red) + wave * (AS * TM * 2048);
+  const int wfrag = r16 * 64 + (quarter ^ (r16 >> 1 & 3)) * 16;
+  char* slots = reinterpret_cast<char*>(red) + wave * (AS * TM * 2048 + WS * TN * 1024);
+  char* wslots = slots + AS * TM * 2048;
   const char* Ab = reinterpret_cast<const char*>(A) + (uint32_t)first * 128u;
   const char* Wb = static_cast<const char*>(W) + (uint32_t)first * 64u;
 
@@ -138,7 +153,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
   for (int t = 0; t < TM; t++)
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  frag16 w[WS][TN];
+  // Both operands are copied into LDS: weights loaded into registers, beside the activations' copies, were taken by the compiler to
+  // return out of order with those, and at the first use of every second step's it waited for all that was in flight.
   auto load_a = [&](char* slot, int t, uint32_t i) {   // row tile t of my i-th step
 #pragma unroll
     for (int h = 0; h < 2; h++)
@@ -147,21 +163,30 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
   };
   auto load_w = [&](int u, uint32_t i) {
 #pragma unroll
-    for (int j = 0; j < TN; j++) w[u][j] = *reinterpret_cast<const frag16*>(Wb + (woff[j] + i * (kWaves * 64u)));
+    for (int j = 0; j < TN; j++)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(Wb + (woff[j] + i * (kWaves * 64u))),
+                                       (__attribute__((address_space(3))) void*)(wslots + (u * TN + j) * 1024), 16, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
   // My i-th step, weights in slot U, activations in `slot`. R: later steps, capped at WS. Requests go out in the order W(0), A(0),
-  // W(1), .., W(AS), then in step i A(i + AS, t) as tile t leaves its slot and W(i + WS) at the end: what is younger than A(i, t)
-  // is counted, and W(i) is older (copies into LDS are waited for by count: the compiler does not see them).
+  // W(1), .., W(AS), then in step i A(i + AS, t) as tile t leaves its slot and W(i + WS) at the end (of one slot W(i + 1) as it
+  // is read): what is younger than A(i, t) is counted, and W(i) is older (copies into LDS are waited for by count). W(i + WS) takes the
+  // slot that W(i) was read from, by fragments that have arrived.
   auto step = [&](auto U, auto R_, uint32_t i, char* slot) {
     constexpr int u = decltype(U)::value, R = decltype(R_)::value, ahead = R < AS - 1 ? R : AS - 1;
+    frag16 w[TN];
     const auto tile = [&](auto T) {
       constexpr int t = decltype(T)::value;
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (TM - 1 - t) + ahead * (TN + 2 * TM) + (R >= AS ? TN + 2 * t : 0)) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (TM - 1 - t) + ahead * (TN + 2 * TM) + (R >= AS ? (WS == 1 && t == 0 ? 0 : TN) + 2 * t : 0)) : "memory");
       const char* at = slot + t * 2048;
       const f32x4 x0 = *reinterpret_cast<const f32x4*>(at + frag[0]), x1 = *reinterpret_cast<const f32x4*>(at + frag[1]);
+      if constexpr (t == 0) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) w[j] = *reinterpret_cast<const frag16*>(wslots + (u * TN + j) * 1024 + wfrag);
+      }
       if constexpr (R >= AS) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the copy that takes the slot goes out
+        if constexpr (WS == 1 && t == 0) load_w(0, i + 1);
         load_a(slot, t, i + AS);
       }
       frag16 p[3];
@@ -172,7 +197,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
 #pragma unroll
       for (int e = 0; e < 3; e++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[t][j] = mma(w[u][j], p[e], acc[t][j]);
+        for (int j = 0; j < TN; j++) acc[t][j] = mma(w[j], p[e], acc[t][j]);
       if (TM * TN >= 12) __builtin_amdgcn_sched_barrier(0);   // (the registers do not hold two row tiles' terms)
     };
     tile(std::integral_constant<int, 0>{});
@@ -181,7 +206,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
     if constexpr (TM > 3) tile(std::integral_constant<int, 3>{});
     if constexpr (TM > 4) tile(std::integral_constant<int, 4>{});
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (R >= WS) load_w(u, i + WS);
+    if constexpr (WS > 1 && R >= WS) load_w(u, i + WS);
   };
   if (mine > 0) {
     uint32_t i = 0, turn = 0;                      // turn: the slot of activations of step i
@@ -207,10 +232,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
         for (int t = 0; t < TM; t++) load_a(slots + q * (TM * 2048), t, q);
         __builtin_amdgcn_sched_barrier(0);
       }
-    if (AS < mine) load_w(AS, AS);
+    if (WS > 1 && AS < mine) load_w(AS, AS);
     while ((int)i + 2 * WS <= mine) {
       go(std::integral_constant<int, 0>{}, std::integral_constant<int, WS>{});
-      go(std::integral_constant<int, 1>{}, std::integral_constant<int, WS>{});
+      if constexpr (WS > 1) go(std::integral_constant<int, 1>{}, std::integral_constant<int, WS>{});
       if constexpr (WS > 2) go(std::integral_constant<int, 2>{}, std::integral_constant<int, WS>{});
       if constexpr (WS > 3) go(std::integral_constant<int, 3>{}, std::integral_constant<int, WS>{});
       if constexpr (WS > 4) go(std::integral_constant<int, 4>{}, std::integral_constant<int, WS>{});
@@ -218,8 +243,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_rows_bf16_kernel(const fl
     static_assert(WS <= 5, "steps left below");
     switch (mine - (int)i) {                       // 1 .. 2 WS - 1
       case 1: last(std::integral_constant<int, 1>{}); break;
-      case 2: last(std::integral_constant<int, 2>{}); break;
-      case 3: last(std::integral_constant<int, 3>{}); break;
+      case 2: if constexpr (WS > 1) last(std::integral_constant<int, 2>{}); break;
+      case 3: if constexpr (WS > 1) last(std::integral_constant<int, 3>{}); break;
       case 4: if constexpr (WS > 2) last(std::integral_constant<int, 4>{}); break;
       case 5: if constexpr (WS > 2) last(std::integral_constant<int, 5>{}); break;
       case 6: if constexpr (WS > 3) last(std::integral_constant<int, 6>{}); break;
