@@ -58,48 +58,42 @@ __device__ __forceinline__ float conv_step(const tlhip_ssm& a, const SsmDims& d,
   return fmaf(w[(size_t)(d.taps - 1) * d.ch + c], now, s) + static_cast<const float*>(a.conv_b)[c];
 }
 
-// Decode step, 512 threads: a thread owns one float4 column of every ng-th state row. SLICED: a block takes 16 of a head's
-// columns, else all of them. The step is a chain of round trips (position, state and convolution inputs, sums), so the
-// slices are there to shorten it: four times the blocks, one state row to a thread, the sum over the rows by shuffles
-// instead of 32 LDS reads in turn (28 heads of 128 x 64: 6.6 us whole, 5.1 in slices). Each slice convolves its
-// group's B and C again.
-template <bool SLICED>
+// Decode step, a block to a head, 512 threads: a thread owns one float4 column of every ng-th state row.
 __global__ __launch_bounds__(512) void ssm_step_kernel(const float* __restrict__ u, float* __restrict__ y, const tlhip_ssm a,
                                                        int pos, const uint32_t* __restrict__ d_pos) {
   extern __shared__ __attribute__((aligned(16))) float ssm_lds[];
   const SsmDims d = ssm_dims(a);
-  const int slices = SLICED ? d.V >> 4 : 1, tid = threadIdx.x, h = blockIdx.x / slices, slice = blockIdx.x - h * slices, col0 = 16 * slice;
+  const int tid = threadIdx.x, h = blockIdx.x;
   const int per = d.H / d.G, g = h / per;
   const int p = d_pos ? (int)*d_pos : pos;
-  const int ld = ssm_ld(d.V), cols = SLICED ? 16 : ld, nv4 = cols >> 2, ng = 512 / nv4, v4 = tid % nv4, ng0 = tid / nv4;
+  const int ld = ssm_ld(d.V), nv4 = ld >> 2, ng = 512 / nv4, v4 = tid % nv4, ng0 = tid / nv4;
   const bool live = ng0 < ng;
-  float* xs = ssm_lds;                 // [cols] convolved x of the block's columns
-  float* Bs = xs + cols;               // [N]
+  float* xs = ssm_lds;                 // [ld] convolved x
+  float* Bs = xs + ld;                 // [N]
   float* Cs = Bs + d.N;                // [N]
-  float* red = Cs + d.N + ((4 - (cols + 2 * d.N) % 4) & 3);   // [ng][ld], sliced: [wavefronts][16]
-  const size_t slot = (size_t)d.H * d.N * ld, at = (size_t)h * d.N * ld + col0 + 4 * v4;
+  float* red = Cs + d.N + ((4 - (ld + 2 * d.N) % 4) & 3);   // [ng][ld]
+  const size_t slot = (size_t)d.H * d.N * ld, at = (size_t)h * d.N * ld + 4 * v4;
   const float* src = static_cast<const float*>(a.ssm_state) + (size_t)(p & 1) * slot + at;
   float* dst = static_cast<float*>(a.ssm_state) + (size_t)((p + 1) & 1) * slot + at;
-  constexpr int PRE = SLICED ? 2 : 8;  // rows of this thread requested up front
+  constexpr int PRE = 8;               // rows of this thread requested up front
   float4 st[PRE];
 #pragma unroll
   for (int i = 0; i < PRE; i++) {
     const int n = ng0 + i * ng;
     st[i] = live && p > 0 && n < d.N ? *reinterpret_cast<const float4*>(src + (size_t)n * ld) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  const float z = SLICED && tid < 16 ? u[a.z_off + h * d.V + col0 + tid] : 0.f;
   float* ring = static_cast<float*>(a.conv_state);
   const float dt = softplus_f(u[a.dt_off + h] + static_cast<const float*>(a.dt_bias)[h]);
   const float w = exp2f(static_cast<const float*>(a.decay)[h] * dt);
   // the block's x and its group's B and C; the input row is kept for the coming tokens (B, C: by the group's first block)
-  for (int i = tid; i < cols + 2 * d.N; i += 512) {
+  for (int i = tid; i < ld + 2 * d.N; i += 512) {
     int c;
     bool keep = true;
-    if (i < cols) c = col0 + i < d.V ? h * d.V + col0 + i : -1;
+    if (i < ld) c = i < d.V ? h * d.V + i : -1;
     else {
-      const int n = i - cols;
+      const int n = i - ld;
       c = d.inner + (n < d.N ? g * d.N + n : (d.G + g) * d.N + n - d.N);
-      keep = h == g * per && slice == 0;
+      keep = h == g * per;
     }
     float v = 0.f;
     if (c >= 0) {
@@ -124,38 +118,149 @@ __global__ __launch_bounds__(512) void ssm_step_kernel(const float* __restrict__
       if (ng0 + i * ng < d.N) row(ng0 + i * ng, st[i]);
     for (int n = ng0 + PRE * ng; n < d.N; n += ng)
       row(n, p > 0 ? *reinterpret_cast<const float4*>(src + (size_t)n * ld) : make_float4(0.f, 0.f, 0.f, 0.f));
+    *reinterpret_cast<float4*>(red + ng0 * ld + 4 * v4) = o;
   }
-  const auto finish = [&](int v, float t, float zv) {
+  __syncthreads();
+  for (int v = tid; v < d.V; v += 512) {
+    float t = 0.f;
+    for (int k = 0; k < ng; k++) t += red[k * ld + v];
     t = fmaf(static_cast<const float*>(a.skip)[h], xs[v], t);
-    y[a.y_off + h * d.V + col0 + v] = t * silu_f(zv);
+    y[a.y_off + h * d.V + v] = t * silu_f(u[a.z_off + h * d.V + v]);
+  }
+}
+
+// The same by slices: a block takes 16 of a head's columns (grid: slices, heads), a thread one float4 column of ROWS state rows and of
+// every 128th after those. The step is a chain of round trips, which this is there to shorten: four times the blocks, the sum
+// over the rows across lanes instead of 32 LDS reads in turn (28 heads of 128 x 64: 6.6 us whole, 5.1 in slices). Each slice convolves
+// its group's B and C again. Nothing waits for another load before it is asked for: what the requests need are the 14
+// dwords of arguments that arrive with the block, the state is read in both slots and the convolution's ring (four taps) whole, and
+// the position, which may have to be loaded itself, only picks among what came (TAPS4 false: other taps wait for it).
+// (28 heads of 128 x 64, a small Girirax turn of six such layers: 7263 -> 7174 us.)
+// dims = state rows | taps << 10 | heads << 17, vper = head size | heads per group << 16; inv: ceil(2^32 / heads per group), 0 for one.
+struct SsmRest {
+  const float *conv_b, *dt_bias, *decay, *skip;
+  int z_off, dt_off, y_off, pos;
+};
+template <int ROWS, bool TAPS4>
+__global__ __launch_bounds__(512) void ssm_step_sliced_kernel(const float* __restrict__ u, float* state, float* ring,
+                                                              const float* __restrict__ conv_w, const uint32_t* __restrict__ d_pos,
+                                                              uint32_t dims, uint32_t vper, uint32_t inv, int x_off, float* __restrict__ y,
+                                                              const SsmRest a) {
+  extern __shared__ __attribute__((aligned(16))) float ssm_lds[];
+  const int N = dims & 0x3ff, taps = (dims >> 10) & 127, H = dims >> 17, V = vper & 0xffff, per = vper >> 16;
+  const int tid = threadIdx.x, lane = tid & 63, h = blockIdx.y, col0 = 16 * blockIdx.x, v4 = tid & 3, row0 = tid >> 2;
+  const int g = inv ? (int)__umulhi((uint32_t)h, inv) : h, G = inv ? (int)__umulhi((uint32_t)H + per - 1, inv) : H;
+  const int inner = H * V, ch = inner + 2 * G * N, chans = 16 + 2 * N;
+  const bool first_block = h == g * per && blockIdx.x == 0;
+  float* xs = ssm_lds;                 // [16] convolved x of the block's columns
+  float* Bs = xs + 16;                 // [N]
+  float* Cs = Bs + N;                  // [N]
+  float* red = Cs + N + ((4 - (2 * N) % 4) & 3);            // [wavefronts][16]
+  const size_t slot = (size_t)H * N * V;
+  const uint32_t at = (uint32_t)h * (uint32_t)(N * V) + col0 + 4 * v4;       // (a head's rows: below 2^32 floats by the sizes taken)
+  const auto channel = [&](int i) { return i < 16 ? h * V + col0 + i : i - 16 < N ? inner + g * N + i - 16 : inner + (G + g) * N + i - 16 - N; };
+  f32x4 st[2][ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; i++)
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      st[k][i] = *reinterpret_cast<const f32x4*>(state + k * slot + at + (size_t)min(row0 + 128 * i, N - 1) * V);
+  const int c0 = channel(min(tid, chans - 1));
+  float now = u[x_off + c0], x[4], f[4];
+  if constexpr (TAPS4) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      x[k] = ring[(uint32_t)(k * ch + c0)];
+      f[k] = conv_w[(uint32_t)(k * ch + c0)];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const float bias0 = a.conv_b[c0], z = u[a.z_off + h * V + col0 + (tid & 15)];
+  const float dt = softplus_f(u[a.dt_off + h] + a.dt_bias[h]), w = exp2f(a.decay[h] * dt), skip = a.skip[h];
+  const int p = d_pos ? (int)*d_pos : a.pos;
+  // sum over the taps of channel c for the token at position p; `now` is the token's own input
+  const auto conv4 = [&](const float r[4], const float f[4], float now, float bias) {
+    float q[4] = {r[0], r[1], r[2], r[3]};           // the ring from slot (p + 1) % 4 on: positions p - 3, p - 2, p - 1
+    const bool odd = (p + 1) & 1, two = (p + 1) & 2;
+    const float o0 = odd ? q[1] : q[0], o1 = odd ? q[2] : q[1], o2 = odd ? q[3] : q[2], o3 = odd ? q[0] : q[3];
+    q[0] = two ? o2 : o0; q[1] = two ? o3 : o1; q[2] = two ? o0 : o2;
+    float s = fmaf(f[0], p >= 3 ? q[0] : 0.f, 0.f);
+    s = fmaf(f[1], p >= 2 ? q[1] : 0.f, s);
+    s = fmaf(f[2], p >= 1 ? q[2] : 0.f, s);
+    return fmaf(f[3], now, s) + bias;
   };
-  if constexpr (SLICED) {
+  const auto conv_any = [&](int c, float now) {
+    const int first = (p + 1) % taps;                // slot of position p - (taps - 1)
+    float s = 0.f;
+    for (int j = 0; j < taps - 1; j++) {
+      const int from = first + j < taps ? first + j : first + j - taps;
+      s = fmaf(conv_w[(size_t)j * ch + c], p - (taps - 1) + j >= 0 ? ring[(size_t)from * ch + c] : 0.f, s);
+    }
+    return fmaf(conv_w[(size_t)(taps - 1) * ch + c], now, s) + a.conv_b[c];
+  };
+  const int mine = TAPS4 ? p & 3 : p % taps;
+  // the block's x and its group's B and C; the input row is kept for the coming tokens (B, C: by the group's first block)
+  if (tid < chans) {
+    ssm_lds[tid] = silu_f(TAPS4 ? conv4(x, f, now, bias0) : conv_any(c0, now));
+    if (tid < 16 || first_block) ring[(size_t)mine * ch + c0] = now;
+  }
+  for (int i = tid + 512; i < chans; i += 512) {
+    const int c = channel(i);
+    const float n = u[x_off + c];
+    float v;
+    if constexpr (TAPS4) {
+      float r[4], q[4];
 #pragma unroll
-    for (int m = 4; m < 64; m *= 2) {
-      o.x += __shfl_xor(o.x, m, kWave); o.y += __shfl_xor(o.y, m, kWave);
-      o.z += __shfl_xor(o.z, m, kWave); o.w += __shfl_xor(o.w, m, kWave);
+      for (int k = 0; k < 4; k++) { r[k] = ring[(size_t)k * ch + c]; q[k] = conv_w[(size_t)k * ch + c]; }
+      v = conv4(r, q, n, a.conv_b[c]);
+    } else {
+      v = conv_any(c, n);
     }
-    if ((tid & 63) < 4) *reinterpret_cast<float4*>(red + (tid >> 6) * 16 + 4 * (tid & 63)) = o;
-    __syncthreads();
-    if (tid < 16) {
-      float t = red[tid];
+    ssm_lds[i] = silu_f(v);
+    if (first_block) ring[(size_t)mine * ch + c] = n;
+  }
+  __syncthreads();
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  const f32x4 x4 = *reinterpret_cast<const f32x4*>(xs + 4 * v4) * dt;
+  float* dst = state + (size_t)((p + 1) & 1) * slot + at;
+  const auto row = [&](int n, f32x4 s) {
+    const float b = Bs[n], c = Cs[n];
 #pragma unroll
-      for (int k = 1; k < 8; k++) t += red[16 * k + tid];
-      finish(tid, t, z);
-    }
-  } else {
-    if (live) *reinterpret_cast<float4*>(red + ng0 * ld + 4 * v4) = o;
-    __syncthreads();
-    for (int v = tid; v < d.V; v += 512) {
-      float t = 0.f;
-      for (int k = 0; k < ng; k++) t += red[k * ld + v];
-      finish(v, t, u[a.z_off + h * d.V + v]);
-    }
+    for (int e = 0; e < 4; e++) s[e] = fmaf(w, s[e], b * x4[e]);
+    *reinterpret_cast<f32x4*>(dst + (size_t)n * V) = s;
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = fmaf(c, s[e], o[e]);
+  };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < ROWS; i++)
+    if (row0 + 128 * i < N) row(row0 + 128 * i, p > 0 ? ((p & 1) ? st[1][i] : st[0][i]) : zero);
+  for (int n = row0 + 128 * ROWS; n < N; n += 128)
+    row(n, p > 0 ? *reinterpret_cast<const f32x4*>(state + (size_t)(p & 1) * slot + at + (size_t)n * V) : zero);
+#pragma unroll
+  for (int e = 0; e < 4; e++) {        // over the lanes of one column: 32, 16, 8 and 4 apart
+    LanePair t = swap32(o[e], o[e]);
+    t = swap16(t.first + t.second, t.first + t.second);
+    o[e] = t.first + t.second;
+    o[e] += dpp_read<0x128>(o[e]);
+    o[e] += dpp_read<0x124>(o[e]);
+  }
+  if (lane < 4) *reinterpret_cast<f32x4*>(red + (tid >> 6) * 16 + 4 * lane) = o;
+  __syncthreads();
+  if (tid < 16) {
+    float t = red[tid];
+#pragma unroll
+    for (int k = 1; k < 8; k++) t += red[16 * k + tid];
+    t = fmaf(skip, xs[tid], t);
+    y[a.y_off + h * V + col0 + tid] = t * silu_f(z);
   }
 }
 // up to two blocks per CU, and whole slices (heads of 64 and 128 state rows, us, whole -> slices: 28 6.6 -> 5.1, 112 (448
 // slices) 6.1 -> 6.1, 160 6.4 -> 7.2; 256 heads of 16 state rows 4.9 -> 7.3)
-static bool ssm_sliced(const tlhip_ssm& a) { return a.vdim % 16 == 0 && a.heads * (a.vdim / 16) <= 2 * (int64_t)ctx().cus; }
+static bool ssm_sliced(const tlhip_ssm& a) {
+  const int64_t far = std::max(std::max(a.x_off, a.z_off), std::max(a.dt_off, a.y_off));
+  return a.vdim % 16 == 0 && a.heads * (a.vdim / 16) <= std::min<int64_t>(2 * (int64_t)ctx().cus, 8192) && far < (1 << 30);   // (its arguments' widths)
+}
 static size_t ssm_step_lds(const tlhip_ssm& a) {
   const bool sliced = ssm_sliced(a);
   const int ld = ssm_ld((int)a.vdim), ng = 512 / (ld >> 2);
@@ -517,9 +622,22 @@ int tlhip_ssm_step(const void* u, void* y, const tlhip_ssm* a, int64_t pos, cons
   const size_t lds = ssm_step_lds(*a);
   if (lds > (size_t)c.lds_per_cu) return fail(TLHIP_EUNSUPPORTED, "tlhip_ssm_step: not enough LDS");
   const bool sliced = ssm_sliced(*a);
-  hipLaunchKernelGGL(sliced ? ssm_step_kernel<true> : ssm_step_kernel<false>, dim3((unsigned)(a->heads * (sliced ? a->vdim / 16 : 1))),
-                     dim3(512), lds, c.stream, static_cast<const float*>(u), static_cast<float*>(y), *a, (int)pos,
-                     static_cast<const uint32_t*>(d_pos));
+  const float* pu = static_cast<const float*>(u);
+  const uint32_t* dp = static_cast<const uint32_t*>(d_pos);
+  if (sliced) {
+    const auto f = [](const void* p) { return static_cast<const float*>(p); };
+    const uint32_t per = (uint32_t)(a->heads / a->groups);
+    const SsmRest rest{f(a->conv_b), f(a->dt_bias), f(a->decay), f(a->skip), (int)a->z_off, (int)a->dt_off, (int)a->y_off, (int)pos};
+    const bool four = a->taps == 4, one = a->state <= 128;
+    auto fn = four ? (one ? ssm_step_sliced_kernel<1, true> : ssm_step_sliced_kernel<2, true>)
+                   : (one ? ssm_step_sliced_kernel<1, false> : ssm_step_sliced_kernel<2, false>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(a->vdim / 16), (unsigned)a->heads), dim3(512), lds, c.stream, pu, static_cast<float*>(a->ssm_state),
+                       static_cast<float*>(a->conv_state), f(a->conv_w), dp,
+                       (uint32_t)a->state | (uint32_t)a->taps << 10 | (uint32_t)a->heads << 17, (uint32_t)a->vdim | per << 16,
+                       per == 1 ? 0u : (uint32_t)(((uint64_t(1) << 32) + per - 1) / per), (int)a->x_off, static_cast<float*>(y), rest);
+    TLHIP_CHECK_LAUNCH(TLHIP_C_SSM);
+  }
+  hipLaunchKernelGGL(ssm_step_kernel, dim3((unsigned)a->heads), dim3(512), lds, c.stream, pu, static_cast<float*>(y), *a, (int)pos, dp);
   TLHIP_CHECK_LAUNCH(TLHIP_C_SSM);
 }
 
