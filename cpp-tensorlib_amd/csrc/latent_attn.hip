@@ -78,9 +78,9 @@ __device__ __forceinline__ size_t val_at(const Dims& d, int p, int e) {
 // is planned for the capacity, since the position may be on the device: at position 45 of 4096, 14 heads of 64 over 256 wrote and
 // read 64 splits' partials of which one held keys (attend 6.3, output 6.8 us; both about 0.8 us less, a chat turn of 18 such
 // layers and 37 + 16 tokens 7644 -> 7571 us).
-__device__ __forceinline__ int live_splits(const Dims& d, int p, int S) {
-  const int tiles = p / 32 + 1;
-  return min(S, d.NC == 1 ? (tiles + 1) / 2 : tiles);
+__device__ __forceinline__ int live_splits(int planes, int p, int S) {
+  const int tiles = (p >> 5) + 1;
+  return min(S, planes == 1 ? (tiles + 1) / 2 : tiles);
 }
 
 // ---- new cache rows ------------------------------------------------------------------------------
@@ -90,30 +90,39 @@ __device__ __forceinline__ void fill_row(const float* __restrict__ u, const tlhi
   const Dims d = dims_of(a);
   const int tid = threadIdx.x;
   const float* x = u + a.kv_off;
-  float ss = 0.f;
-  for (int i = tid; i < d.L; i += 256) ss = fmaf(x[i], x[i], ss);
-  const float inv = 1.0f / sqrtf(block_sum<4>(ss, red) / (float)d.L + a.eps);
   uint16_t* kc = static_cast<uint16_t*>(a.keys);
   uint16_t* vc = static_cast<uint16_t*>(a.values);
   const float2* tab = static_cast<const float2*>(a.angles) + (size_t)p * (d.R / 2);
+  const int half = d.R / 2;
+  // number i of the row before its scaling (latents) or rotation, and what that takes
+  struct Num { float lo, hi; float2 c; };
+  const auto load = [&](int i) {
+    Num n;
+    const bool latent = i < d.L;
+    const int r = latent ? 0 : i - d.L, j = r < half ? r : r - half;
+    n.lo = x[latent ? i : d.L + j];
+    n.hi = latent ? 0.f : x[d.L + half + j];
+    n.c = latent ? make_float2(static_cast<const float*>(a.kv_norm)[i], 0.f) : tab[j];
+    return n;
+  };
+  const Num first = load(min(tid, d.L + d.R - 1));         // (asked for ahead of the sum, not behind it)
+  float ss = tid < d.L ? first.lo * first.lo : 0.f;
+  for (int i = tid + 256; i < d.L; i += 256) ss = fmaf(x[i], x[i], ss);
+  const float inv = 1.0f / sqrtf(block_sum<4>(ss, red) / (float)d.L + a.eps);
   for (int i = tid; i < d.L + d.R; i += 256) {
+    const Num n = i == tid ? first : load(i);
     float v;
-    if (i < d.L) v = x[i] * inv * static_cast<const float*>(a.kv_norm)[i];
-    else {
-      const int r = i - d.L, half = d.R / 2, j = r < half ? r : r - half;
-      const float2 cs = tab[j];
-      const float lo = x[d.L + j], hi = x[d.L + half + j];
-      v = r < half ? lo * cs.x - hi * cs.y : hi * cs.x + lo * cs.y;
-    }
+    if (i < d.L) v = n.lo * inv * n.c.x;
+    else v = i - d.L < half ? n.lo * n.c.x - n.hi * n.c.y : n.hi * n.c.x + n.lo * n.c.y;
     uint16_t t[NC];
     cut<NC>(v, t);
     const size_t k = key_at(d, p, i);
 #pragma unroll
-    for (int n = 0; n < NC; n++) kc[k + (size_t)n * d.DS * 512] = t[n];
+    for (int n2 = 0; n2 < NC; n2++) kc[k + (size_t)n2 * d.DS * 512] = t[n2];
     if (i < d.L) {
       const size_t w = val_at(d, p, i);
 #pragma unroll
-      for (int n = 0; n < NC; n++) vc[w + (size_t)n * d.LT * 1024] = t[n];
+      for (int n2 = 0; n2 < NC; n2++) vc[w + (size_t)n2 * d.LT * 1024] = t[n2];
     }
   }
 }
@@ -123,26 +132,54 @@ __device__ __forceinline__ void fill_row(const float* __restrict__ u, const tlhi
 // scale * log2 e before it is cut. Block (slice of 128 dims, head, TQ tokens), 256 threads: 16 dim units of 8 x
 // 16 groups of query dims. Blocks past the slices fill the cache rows (one per token).
 constexpr int kSliceDims = 128;
+// A single token: grid (slices, 1 + heads), row 0 fills the cache, and what a block asks for first - its query, eight rows of
+// weights - needs only the arguments up to `slices`, which arrive with it (hd = heads | dim << 16, lr = latents | rotated << 16).
 template <int TQ, int NC, int NQ>
-__global__ __launch_bounds__(256) void latent_query_kernel(const float* __restrict__ u, int64_t ldu, const float* __restrict__ q,
-                                                           int64_t ldq, const tlhip_latent_attn a, uint16_t* __restrict__ qimg,
-                                                           int T, int pos0, const uint32_t* __restrict__ d_pos, int slices) {
+__global__ __launch_bounds__(256) void latent_query_kernel(const float* __restrict__ q, const uint16_t* __restrict__ uk,
+                                                           const uint32_t* __restrict__ d_pos, const float* __restrict__ u, uint32_t hd,
+                                                           uint32_t lr, int T, int slices, uint16_t* __restrict__ qimg, int64_t ldu,
+                                                           int64_t ldq, int pos0, const tlhip_latent_attn a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const Dims d = dims_of(a);
+  Dims d;
+  d.H = hd & 0xffff; d.D = hd >> 16; d.L = lr & 0xffff; d.R = lr >> 16;
+  d.DS = (d.L + d.R + 15) / 16;
   const int tid = threadIdx.x, p0 = d_pos ? (int)*d_pos : pos0;
-  const int tiles = (T + TQ - 1) / TQ, work = slices * d.H * tiles;
-  if ((int)blockIdx.x >= work) {
-    const int t = (int)blockIdx.x - work;
-    fill_row<NC>(u + (size_t)t * ldu, a, p0 + t, lds);
-    return;
+  int slice, h, t0 = 0;
+  if constexpr (TQ == 1) {
+    slice = blockIdx.x;
+    h = (int)blockIdx.y - 1;
+    if (h < 0) {
+      if (slice == 0) fill_row<NC>(u, a, p0, lds);
+      return;
+    }
+  } else {
+    const int tiles = (T + TQ - 1) / TQ, work = slices * d.H * tiles;
+    if ((int)blockIdx.x >= work) {
+      const int t = (int)blockIdx.x - work;
+      fill_row<NC>(u + (size_t)t * ldu, a, p0 + t, lds);
+      return;
+    }
+    slice = blockIdx.x % slices, h = blockIdx.x / slices % d.H, t0 = blockIdx.x / slices / d.H * TQ;
   }
-  const int slice = blockIdx.x % slices, h = blockIdx.x / slices % d.H, t0 = blockIdx.x / slices / d.H * TQ;
   const int nt = min(TQ, T - t0), unit = slice * (kSliceDims / 8) + (tid & 15), dg = tid >> 4, ldk = up8(d.L);
   float* qs = lds;                     // [TQ][D] unrotated query dims
   float* red = lds + TQ * d.D;         // [16 groups][16 units][8] per token
-  for (int i = tid; i < TQ * d.D; i += 256) {
-    const int t = i / d.D;
-    qs[i] = q[(size_t)(t0 + min(t, nt - 1)) * ldq + h * (d.D + d.R) + i % d.D];
+  const u32x4* w = reinterpret_cast<const u32x4*>(uk + (size_t)h * d.D * ldk) + min(unit, ldk / 8 - 1);
+  const int n8 = ldk / 8;
+  constexpr int PRE = TQ == 1 ? 8 : 1;
+  u32x4 pre[PRE];
+  if constexpr (TQ == 1) {
+    const float mine = q[h * (d.D + d.R) + min(tid, d.D - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < PRE; i++) pre[i] = w[(size_t)min(dg + 16 * i, d.D - 1) * n8];
+    qs[min(tid, d.D - 1)] = mine;      // (threads past the last write its value once more)
+    for (int i = tid + 256; i < d.D; i += 256) qs[i] = q[h * (d.D + d.R) + i];
+  } else {
+    for (int i = tid; i < TQ * d.D; i += 256) {
+      const int t = i / d.D;
+      qs[i] = q[(size_t)(t0 + min(t, nt - 1)) * ldq + h * (d.D + d.R) + i % d.D];
+    }
   }
   __syncthreads();
   float acc[TQ][8];
@@ -151,11 +188,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(const float* __restri
 #pragma unroll
     for (int j = 0; j < 8; j++) acc[t][j] = 0.f;
   if (unit * 8 < ldk) {
-    const u32x4* w = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.uk) + (size_t)h * d.D * ldk) + unit;
-    const int n8 = ldk / 8;
-#pragma unroll 4
-    for (int k = dg; k < d.D; k += 16) {
-      const u32x4 x = w[(size_t)k * n8];
+    const auto add = [&](int k, const u32x4 x) {
 #pragma unroll
       for (int t = 0; t < TQ; t++) {
         const float f = qs[t * d.D + k];
@@ -165,7 +198,15 @@ __global__ __launch_bounds__(256) void latent_query_kernel(const float* __restri
           acc[t][2 * j + 1] = fmaf(bf16_hi(x[j]), f, acc[t][2 * j + 1]);
         }
       }
+    };
+    int k = dg;
+    if constexpr (TQ == 1) {
+#pragma unroll
+      for (int i = 0; i < PRE; i++, k += 16)
+        if (k < d.D) add(k, pre[i]);
     }
+#pragma unroll 4
+    for (; k < d.D; k += 16) add(k, w[(size_t)k * n8]);
   }
   const float sc = a.scale * 1.4426950408889634f;
   for (int t = 0; t < TQ; t++) {
@@ -343,40 +384,59 @@ __global__ __launch_bounds__(256) void latent_query_mfma_kernel(const float* __r
 // Scores: wavefront (k, d) takes key tile k and every fourth dim step from d, its queries in registers; the four
 // partial tiles meet in LDS and d's owner keeps eight keys of a lane pair: maximum, weights (two bf16 terms, half an
 // operand fragment) and sum are formed once. Values: wavefront w takes value tiles w, w + 8, ... (NL of them).
+// Grid: splits, query tiles (65535 to a z). The arguments up to `rows` arrive with the block (steps = DS | LT << 16, hs = heads |
+// S << 16), and with them alone keys, queries and values of the first pair are asked for: which keys there are is known only when the
+// position, which may be on the device, has come. Until then tiles are bound by the cache; a value tile past the last is taken as zeros.
 template <int KS, int NL>
-__global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_attn a, const uint16_t* __restrict__ qimg,
-                                                            float* __restrict__ part, int T, int pos0,
-                                                            const uint32_t* __restrict__ d_pos, int S, int rows) {
+__global__ __launch_bounds__(512) void latent_attend_kernel(const uint16_t* __restrict__ qimg, const void* __restrict__ keys,
+                                                            const void* __restrict__ values, const uint32_t* __restrict__ d_pos,
+                                                            uint32_t steps, uint32_t hs, int T, int pos0, int cap_tiles, int rows,
+                                                            float* __restrict__ part) {
   __shared__ f32x4 ex[8][4][64];       // partial scores of (wavefront, eight keys)
   __shared__ u32x4 pb[4][2][64];       // weights of (16 keys, term)
   __shared__ float mx[8][32];
-  const Dims d = dims_of(a);
+  const int DS = steps & 0xffff, LT = steps >> 16, H = hs & 0xffff, S = hs >> 16;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kt = wave & 1, dq = wave >> 1;
-  const int rt = blockIdx.x / S, split = blockIdx.x % S;
-  const int p0 = d_pos ? (int)*d_pos : pos0;
+  const int rt = (int)blockIdx.z * 65535 + (int)blockIdx.y, split = blockIdx.x;
+  if (rt * 32 >= rows) return;
   const int row = rt * 32 + c;                       // this lane's query row
-  const int limit = row < T * d.H ? p0 + row / d.H : -1;
-  const int last = p0 + min(rt * 32 + 31, T * d.H - 1) / d.H, ntiles = last / 32 + 1, npairs = (ntiles + 1) / 2;
-  if (T == 1 && split >= live_splits(d, p0, S)) return;
-  const u32x4* kc = reinterpret_cast<const u32x4*>(a.keys) + lane;
-  const u32x4* vc = reinterpret_cast<const u32x4*>(a.values) + lane;
-  const u32x4* qg = reinterpret_cast<const u32x4*>(qimg) + (size_t)rt * 2 * d.DS * 64 + lane;
+  const u32x4* kc = reinterpret_cast<const u32x4*>(keys) + lane;
+  const u32x4* vc = reinterpret_cast<const u32x4*>(values) + lane;
+  const u32x4* qg = reinterpret_cast<const u32x4*>(qimg) + (size_t)rt * 2 * DS * 64 + lane;
 
-  u32x4 kr[KS], qr[KS][2];
-  const auto load_keys = [&](int pair) {             // (steps past the last: any key meets a zero query)
-    const u32x4* k = kc + (size_t)min(2 * pair + kt, ntiles - 1) * d.DS * 64;
+  u32x4 kr[KS], qr[KS][2], vr[NL][4];
+  const auto load_keys = [&](int pair, int top) {    // (steps past the last: any key meets a zero query)
+    const u32x4* k = kc + (size_t)min(2 * pair + kt, top) * DS * 64;
 #pragma unroll
-    for (int i = 0; i < KS; i++) kr[i] = k[min(dq + 4 * i, d.DS - 1) * 64];
+    for (int i = 0; i < KS; i++) kr[i] = k[min(dq + 4 * i, DS - 1) * 64];
   };
-  load_keys(split);
+  const auto load_values = [&](int pair, int top) {
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        vr[i][k] = vc[(((size_t)min(2 * pair + (k >> 1), top) * LT + min(wave + 8 * i, LT - 1)) * 2 + (k & 1)) * 64];
+  };
+  load_keys(split, cap_tiles - 1);
 #pragma unroll
   for (int i = 0; i < KS; i++)
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-      const u32x4 x = qg[(n * d.DS + min(dq + 4 * i, d.DS - 1)) * 64];
-      qr[i][n] = dq + 4 * i < d.DS ? x : u32x4{0, 0, 0, 0};
-    }
+    for (int n = 0; n < 2; n++) qr[i][n] = qg[(n * DS + min(dq + 4 * i, DS - 1)) * 64];
+  load_values(split, cap_tiles - 1);
+  __builtin_amdgcn_sched_barrier(0);
+  const int p0 = d_pos ? (int)*d_pos : pos0;
+  const int token = T == 1 ? 0 : row / H, last_row = min(rt * 32 + 31, T * H - 1);
+  const int limit = row < T * H ? p0 + token : -1;
+  const int last = p0 + (T == 1 ? 0 : last_row / H), ntiles = last / 32 + 1, npairs = (ntiles + 1) / 2;
+  if (T == 1 && split >= live_splits(1, p0, S)) return;
+#pragma unroll
+  for (int i = 0; i < KS; i++)
+#pragma unroll
+    for (int n = 0; n < 2; n++) qr[i][n] = dq + 4 * i < DS ? qr[i][n] : u32x4{0, 0, 0, 0};
+  if (2 * split + 1 >= ntiles)
+#pragma unroll
+    for (int i = 0; i < NL; i++) vr[i][2] = vr[i][3] = u32x4{0, 0, 0, 0};
   f32x16 o[NL];
 #pragma unroll
   for (int i = 0; i < NL; i++)
@@ -384,12 +444,6 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_a
     for (int v = 0; v < 16; v++) o[i][v] = 0.f;
   float m = -INFINITY, l = 0.f;
   for (int pair = split; pair < npairs; pair += S) {
-    u32x4 vr[NL][4];                   // values of these keys, requested before the scores are formed
-#pragma unroll
-    for (int i = 0; i < NL; i++)
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-        vr[i][k] = vc[(((size_t)min(2 * pair + (k >> 1), ntiles - 1) * d.LT + min(wave + 8 * i, d.LT - 1)) * 2 + (k & 1)) * 64];
     f32x16 s[2];
 #pragma unroll
     for (int n = 0; n < 2; n++)
@@ -400,7 +454,7 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_a
 #pragma unroll
       for (int n = 1; n >= 0; n--)
         s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kr[i]), __builtin_bit_cast(bf16x8, qr[i][n]), s[n], 0, 0, 0);
-    load_keys(min(pair + S, npairs - 1));
+    load_keys(min(pair + S, npairs - 1), ntiles - 1);
 #pragma unroll
     for (int i = 0; i < 4; i++)
       ex[wave][i][lane] = f32x4{s[0][4 * i] + s[1][4 * i], s[0][4 * i + 1] + s[1][4 * i + 1], s[0][4 * i + 2] + s[1][4 * i + 2],
@@ -450,6 +504,7 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_a
         for (int i = 0; i < NL; i++)
           o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vr[i][k]), pf, o[i], 0, 0, 0);
       }
+    if (pair + S < npairs) load_values(pair + S, ntiles - 1);   // requested before the next scores are formed
   }
   const LanePair lp = swap32(l, l);
   __syncthreads();                     // mx has been read
@@ -469,10 +524,10 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_a
 #pragma unroll
   for (int i = 0; i < NL; i++) {
     const int lt = wave + 8 * i;
-    if (lt < d.LT)
+    if (lt < LT)
 #pragma unroll
       for (int k = 0; k < 4; k++)
-        *reinterpret_cast<f32x4*>(pa + at * (32 * d.LT) + 32 * lt + 8 * k + 4 * g) = f32x4{o[i][4 * k], o[i][4 * k + 1], o[i][4 * k + 2], o[i][4 * k + 3]};
+        *reinterpret_cast<f32x4*>(pa + at * (32 * LT) + 32 * lt + 8 * k + 4 * g) = f32x4{o[i][4 * k], o[i][4 * k + 1], o[i][4 * k + 2], o[i][4 * k + 3]};
   }
 }
 
@@ -480,25 +535,28 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const tlhip_latent_a
 // fourth dim step, the four partial sums meet in LDS and every wavefront adds them in the same order. Values:
 // wavefront w takes value tiles w, w + 4, ... (NL of them).
 template <int NL, int NC, int NQ>
-__global__ __launch_bounds__(256) void latent_attend_exact_kernel(const tlhip_latent_attn a, const uint16_t* __restrict__ qimg,
-                                                            float* __restrict__ part, int T, int pos0,
-                                                            const uint32_t* __restrict__ d_pos, int S, int rows) {
+__global__ __launch_bounds__(256) void latent_attend_exact_kernel(const uint16_t* __restrict__ qimg, const void* __restrict__ keys,
+                                                                  const void* __restrict__ values, const uint32_t* __restrict__ d_pos,
+                                                                  uint32_t steps, uint32_t hs, int T, int pos0, int, int rows,
+                                                                  float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const Dims d = dims_of(a);
+  struct { int DS, LT, H; } d = {(int)(steps & 0xffff), (int)(steps >> 16), (int)(hs & 0xffff)};
+  const int S = hs >> 16;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rt = blockIdx.x / S, split = blockIdx.x % S;
+  const int rt = (int)blockIdx.z * 65535 + (int)blockIdx.y, split = blockIdx.x;
+  if (rt * 32 >= rows) return;
   const int p0 = d_pos ? (int)*d_pos : pos0;
   const int row = rt * 32 + c;                       // this lane's query row
   const int limit = row < T * d.H ? p0 + row / d.H : -1;
   const int last = p0 + min(rt * 32 + 31, T * d.H - 1) / d.H, ntiles = last / 32 + 1;   // key tiles the tile's last row sees
-  if (T == 1 && split >= live_splits(d, p0, S)) return;
+  if (T == 1 && split >= live_splits(NC, p0, S)) return;
   u32x4* qs = reinterpret_cast<u32x4*>(lds);         // [NQ][DS][64]
   f32x4* red = reinterpret_cast<f32x4*>(qs + NQ * d.DS * 64);   // [2][4 waves][4][64]
   const u32x4* qg = reinterpret_cast<const u32x4*>(qimg) + (size_t)rt * NQ * d.DS * 64;
   for (int i = tid; i < NQ * d.DS * 64; i += 256) qs[i] = qg[i];
-  const u32x4* kc = reinterpret_cast<const u32x4*>(a.keys) + lane;
-  const u32x4* vc = reinterpret_cast<const u32x4*>(a.values) + lane;
+  const u32x4* kc = reinterpret_cast<const u32x4*>(keys) + lane;
+  const u32x4* vc = reinterpret_cast<const u32x4*>(values) + lane;
 
   f32x16 o[NL];
 #pragma unroll
@@ -607,53 +665,80 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const tlhip_la
 // Block (slice of ROWS value rows, head, TQ <= 4 tokens) of NT threads; G groups of threads share the splits.
 constexpr int kMaxSplits = 64;
 __host__ __device__ inline int out_groups(int NT, int TQ, int LV) { const int n = TQ * (LV / 4); return n >= NT ? 1 : NT / n; }
+// Grid: slices, heads, token tiles. The arguments up to `inv` arrive with the block (hs = heads | S << 16, vl = V | L << 16, inv =
+// ceil(2^20 / items)); of a single token the weights, every split's maximum and sum and the first splits' latents are asked for with
+// them alone: how many splits hold keys is known when the position has come, and only what they left is used.
 template <int TQ, int NT, int ROWS>
-__global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict__ u, int64_t ldu, float* __restrict__ y, int64_t ldy,
-                                                        const tlhip_latent_attn a, const float* __restrict__ part, int T, int S,
-                                                        int rows, int slices, int pos0, const uint32_t* __restrict__ d_pos) {
+__global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict__ part, const uint16_t* __restrict__ uvp,
+                                                        const float* __restrict__ gates, const uint32_t* __restrict__ d_pos, uint32_t hs,
+                                                        uint32_t vl, int rows, int T, uint32_t inv, int pos0, int planes,
+                                                        int64_t ldu, float* __restrict__ y, int64_t ldy, int64_t y_off) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int NW = NT / 64;
-  const Dims d = dims_of(a);
+  struct { int H, V, L, LT; } d = {(int)(hs & 0xffff), (int)(vl & 0xffff), (int)(vl >> 16), 0};
+  d.LT = (d.L + 31) / 32;
+  const int S = hs >> 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int slice = blockIdx.x % slices, h = blockIdx.x / slices % d.H, t0 = blockIdx.x / slices / d.H * TQ;
-  const int nt = min(TQ, T - t0), LV = 32 * d.LT, ldv = up8(d.L), n8 = ldv / 8, G = out_groups(NT, TQ, LV), items = TQ * (LV / 4);
+  const int slice = blockIdx.x, h = blockIdx.y, t0 = blockIdx.z * TQ;
+  const int nt = min(TQ, T - t0), LV = 32 * d.LT, ldv = up8(d.L), n8 = ldv / 8, items = TQ * (LV / 4);
+  const auto by_items = [&](int i) { return (int)((uint32_t)i * inv >> 20); };   // (i up to 1024)
+  const int G = max(by_items(NT), 1);
   float* oc = lds;                     // [G][TQ][LV] sums of latents, normalised
   float* w = oc + G * TQ * LV;         // [TQ][S] the splits' weights
   const size_t R = (size_t)rows;
   const float *pm = part, *pl = part + (size_t)S * R, *pa = pl + (size_t)S * R;
   const int v1 = min(d.V, (slice + 1) * ROWS), vw = slice * ROWS + wave;
-  const u32x4* uv = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.uv)) + (size_t)h * d.V * n8;
+  const u32x4* uv = reinterpret_cast<const u32x4*>(uvp) + (size_t)h * d.V * n8;
   constexpr int PRE = ROWS / NW < 2 ? 1 : 2;     // rows whose weights are requested up front
   u32x4 pre[PRE];
   float gate[PRE];                     // (of a single token)
+  f32x4 v[8];                          // eight splits' latents of this thread's item, the first ones before the weights are known
+  const auto from = [&](int i) {       // (TQ == 1: i below 2 items)
+    const int j = TQ == 1 ? i - by_items(i) * items : i % items, t = TQ == 1 ? 0 : j / (LV / 4), e = 4 * (j - t * (LV / 4));
+    return pa + ((size_t)(t0 + min(t, nt - 1)) * d.H + h) * LV + e;
+  };
+  int live = S;
+  float m1 = -INFINITY, l1 = 0.f;      // lane's split, of a single token
+  if constexpr (TQ == 1) {
+    v[0] = *reinterpret_cast<const f32x4*>(from(min(tid, G * items - 1)) + (size_t)min(by_items(tid), S - 1) * R * LV);
+    if (wave == 0) {
+      m1 = pm[(size_t)min(lane, S - 1) * R + h];
+      l1 = pl[(size_t)min(lane, S - 1) * R + h];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < PRE; i++) {
     const int v = min(vw + i * NW, d.V - 1);
     pre[i] = uv[(size_t)v * n8 + min(lane, n8 - 1)];
-    gate[i] = TQ == 1 && a.gate_off >= 0 ? u[(size_t)t0 * ldu + a.gate_off + h * d.V + v] : 0.f;
+    if (TQ == 1) gate[i] = (gates ? gates : part)[gates ? h * d.V + v : 0];   // (no gate: any number, not used)
   }
-  const int live = TQ == 1 ? live_splits(d, d_pos ? (int)*d_pos : pos0, S) : S;
-  f32x4 v[8];                          // eight splits' latents of this thread's item, the first ones before the weights are known
-  const auto load_splits = [&](int i, int s0) {
-    const int j = i % items, t = j / (LV / 4), e = 4 * (j - t * (LV / 4));
-    const float* src = pa + ((size_t)(t0 + min(t, nt - 1)) * d.H + h) * LV + e;
+  if constexpr (TQ == 1) {
+    __builtin_amdgcn_sched_barrier(0);
+    live = live_splits(planes, d_pos ? (int)*d_pos : pos0, S);
+  }
+  const auto load_splits = [&](int i, int s0, int k0) {
+    const float* src = from(i);
 #pragma unroll
     for (int k = 0; k < 8; k++)
-      if (k * G < live) v[k] = *reinterpret_cast<const f32x4*>(src + (size_t)min(s0 + k * G, live - 1) * R * LV);
+      if (k >= k0 && k * G < live) v[k] = *reinterpret_cast<const f32x4*>(src + (size_t)min(s0 + k * G, live - 1) * R * LV);
   };
-  if (tid / items < live) load_splits(tid, tid / items);
+  const int grp0 = TQ == 1 ? by_items(tid) : tid / items;
+  if (grp0 < live && (TQ > 1 || G < live)) load_splits(tid, grp0, TQ == 1 ? 1 : 0);
   if (wave < TQ) {                     // a wavefront weighs the (up to 64) splits of one token
     const int row = (t0 + min(wave, nt - 1)) * d.H + h;
-    const float m = lane < live ? pm[lane * R + row] : -INFINITY, l = lane < live ? pl[lane * R + row] : 0.f;
+    float m = m1, l = l1;
+    if (TQ > 1 && lane < live) m = pm[lane * R + row], l = pl[lane * R + row];
+    m = lane < live ? m : -INFINITY;
+    l = lane < live ? l : 0.f;
     const float f = exp2f(m - wave_max(m)), tot = wave_sum(f * l);
     if (lane < live) w[wave * S + lane] = f / tot;
   }
   __syncthreads();
   for (int i = tid; i < items * G; i += NT) {
-    const int grp = i / items, j = i - grp * items, t = j / (LV / 4), e = 4 * (j - t * (LV / 4));
+    const int grp = i < NT ? grp0 : i / items, j = i - grp * items, t = TQ == 1 ? 0 : j / (LV / 4), e = 4 * (j - t * (LV / 4));
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = grp; s0 < live; s0 += 8 * G) {
-      if (i != tid || s0 != grp) load_splits(i, s0);
+      if (i != tid || s0 != grp) load_splits(i, s0, 0);
 #pragma unroll
       for (int k = 0; k < 8; k++)
         if (s0 + k * G < live) {
@@ -709,13 +794,13 @@ __global__ __launch_bounds__(NT) void latent_out_kernel(const float* __restrict_
       const float s = wave_sum(acc[t]);
       if (lane == 0 && t < nt) {
         float o = s;
-        if (a.gate_off >= 0) {
+        if (gates) {
           float z;
           if (TQ == 1 && i < PRE) z = i == 0 ? gate[0] : gate[PRE - 1];
-          else z = u[(size_t)(t0 + t) * ldu + a.gate_off + h * d.V + v];
+          else z = gates[(size_t)(t0 + t) * ldu + h * d.V + v];
           o = s / (1.f + expf(-z));
         }
-        y[(size_t)(t0 + t) * ldy + a.y_off + h * d.V + v] = o;
+        y[(size_t)(t0 + t) * ldy + y_off + h * d.V + v] = o;
       }
     }
   }
@@ -840,7 +925,7 @@ static int splits(const tlhip_latent_attn* a, int64_t T, int64_t pos0) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({S, runs, kMaxSplits}));
 }
 
-typedef void (*attend_fn)(const tlhip_latent_attn, const uint16_t*, float*, int, int, const uint32_t*, int, int);
+typedef void (*attend_fn)(const uint16_t*, const void*, const void*, const uint32_t*, uint32_t, uint32_t, int, int, int, int, float*);
 template <int KS>
 static attend_fn pick_values(int nl) {
   return nl <= 1 ? latent_attend_kernel<KS, 1> : nl <= 2 ? latent_attend_kernel<KS, 2> : latent_attend_kernel<KS, 4>;
@@ -906,13 +991,19 @@ static int launch(const float* u, int64_t ldu, const float* q, int64_t ldq, floa
     const int tail = (int)((items + 255) / 256);
     hipLaunchKernelGGL(fqm, dim3((unsigned)(work + tail + T)), dim3(256), lq, c.stream, u, ldu, q, ldq, a, qimg, T, pos0, slices, tail);
   } else {
-    hipLaunchKernelGGL(fq, dim3((unsigned)(slices * d.H * tiles + T)), dim3(256), lq, c.stream, u, ldu, q, ldq, a, qimg, T, pos0, d_pos, slices);
+    hipLaunchKernelGGL(fq, TQ == 1 ? dim3((unsigned)slices, (unsigned)d.H + 1) : dim3((unsigned)(slices * d.H * tiles + T)), dim3(256), lq,
+                       c.stream, q, static_cast<const uint16_t*>(a.uk), d_pos, u, (uint32_t)d.H | (uint32_t)d.D << 16,
+                       (uint32_t)d.L | (uint32_t)d.R << 16, T, slices, qimg, ldu, ldq, pos0, a);
   }
-  hipLaunchKernelGGL(fa, dim3((unsigned)(rts * S)), dim3(kExact ? 256 : 512), la, c.stream, a, qimg, part, T, pos0, d_pos, S, rows);
+  hipLaunchKernelGGL(fa, dim3((unsigned)S, (unsigned)std::min(rts, 65535), (unsigned)((rts + 65534) / 65535)), dim3(kExact ? 256 : 512), la,
+                     c.stream, qimg, a.keys, a.values, d_pos, (uint32_t)d.DS | (uint32_t)d.LT << 16, (uint32_t)d.H | (uint32_t)S << 16, T, pos0,
+                     (int)(a.capacity / 32), rows, part);
   if (o_mfma)
     hipLaunchKernelGGL(fom, dim3((unsigned)(d.H * ((T + 31) / 32))), dim3(256), lo, c.stream, u, ldu, y, ldy, a, part, T, S, rows);
   else
-    hipLaunchKernelGGL(fo, dim3((unsigned)(oslices * d.H * tiles)), dim3((unsigned)ont), lo, c.stream, u, ldu, y, ldy, a, part, T, S, rows, oslices, pos0, d_pos);
+    hipLaunchKernelGGL(fo, dim3((unsigned)oslices, (unsigned)d.H, (unsigned)tiles), dim3((unsigned)ont), lo, c.stream, part,
+                       static_cast<const uint16_t*>(a.uv), a.gate_off >= 0 ? u + a.gate_off : nullptr, d_pos, (uint32_t)d.H | (uint32_t)S << 16,
+                       (uint32_t)d.V | (uint32_t)d.L << 16, rows, T, (uint32_t)(((1 << 20) + TQ * (LV / 4) - 1) / (TQ * (LV / 4))), pos0, d.NC, ldu, y, ldy, a.y_off);
   TLHIP_CHECK_LAUNCH(TLHIP_C_LATENT_ATTN);
 }
 
