@@ -17,6 +17,15 @@ constexpr float kLog2e = 1.4426950408889634f;
 __device__ __forceinline__ float exp2_native(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float log2_native(float x) { return __builtin_amdgcn_logf(x); }
 
+// p % rows for 0 <= p <= 2^30: quotients by a reciprocal, twice (the first is off by up to 2^-22 of itself), then the last unit.
+__device__ __forceinline__ int ring_row(int p, int rows) {
+  const float inv = __builtin_amdgcn_rcpf((float)rows);
+  int r = p - (int)((float)p * inv) * rows;
+  r -= (int)floorf((float)r * inv) * rows;
+  r = r < 0 ? r + rows : r;
+  return r >= rows ? r - rows : r;
+}
+
 // Query multiplier at position p.
 __device__ __forceinline__ float query_temperature(int p, float coef, float every) {
   if (every <= 0.f) return 1.f;
@@ -66,7 +75,7 @@ __device__ __forceinline__ void window_step_block(const tlhip_window_attn& a, co
   float* ring = static_cast<float*>(a.ring) + (size_t)kvh * R * ld;
   const int lo = max(0, pos - (int)a.window + 1), n = pos - lo;    // keys [lo, pos) are in the ring
   const int nb = (n + KB - 1) / KB, streams = 32 * S, sid = split * 32 + wave * 4 + row;
-  const int lo_row = lo % R, last = min(n, R) - 1;     // key lo + j is in ring row lo_row + j, once round
+  const int lo_row = ring_row(lo, R), last = min(n, R) - 1;     // key lo + j is in ring row lo_row + j, once round
   const auto load = [&](float4 (&k)[KB][NF], int b) {
 #pragma unroll
     for (int i = 0; i < KB; i++) {
@@ -79,10 +88,10 @@ __device__ __forceinline__ void window_step_block(const tlhip_window_attn& a, co
       }
     }
   };
+  float4 k[KB][NF];
+  load(k, sid);                        // (they need the position only: asked for ahead of the query; a stream without keys reads a row again)
   // every lane of the wavefront makes the same number of turns (row sums are exchanged across lanes)
   const int turns = (max(nb - (split * 32 + wave * 4), 0) + streams - 1) / streams;
-  float4 k[KB][NF];
-  if (turns > 0) load(k, sid);         // (they need the position only: asked for ahead of the query)
   float* qs = smem;                    // [NQ][64 * NF], zeros past dim
   float* ks = smem + NQ * 64 * NF;     // [64 * NF] the new key
   const float temp = query_temperature(pos, a.temp_coef, a.temp_every);
@@ -97,7 +106,7 @@ __device__ __forceinline__ void window_step_block(const tlhip_window_attn& a, co
   }
   __syncthreads();
   if (h0 == 0 && split == 0)
-    for (int d = tid; d < dim; d += 512) ring[(size_t)(pos % R) * ld + d] = ks[d];
+    for (int d = tid; d < dim; d += 512) ring[(size_t)ring_row(pos, R) * ld + d] = ks[d];
   float4 q[NQ][NF], acc[NQ][NF];
   float m[NQ], l[NQ], sl2[NQ];
   const float sc2 = a.scale * kLog2e;
@@ -179,13 +188,17 @@ __device__ __forceinline__ void window_step_block(const tlhip_window_attn& a, co
   float* wl = smem;                    // [8][NQ][max, sum, out[64 * NF]]
 #pragma unroll
   for (int h = 0; h < NQ; h++) {
-    float M = fmaxf(m[h], __shfl_xor(m[h], 16, kWave));
-    M = fmaxf(M, __shfl_xor(M, 32, kWave));
+    LanePair t = swap16(m[h], m[h]);
+    float M = fmaxf(t.first, t.second);
+    t = swap32(M, M);
+    M = fmaxf(t.first, t.second);
     const float f0 = m[h] == -INFINITY ? 0.f : exp2_native(m[h] - M);
     const auto rows = [&](float v) {
-      v *= f0;
-      v += __shfl_xor(v, 16, kWave);
-      return v + __shfl_xor(v, 32, kWave);
+      v = mul_rn(v, f0);
+      LanePair p = swap16(v, v);
+      v = p.first + p.second;
+      p = swap32(v, v);
+      return p.first + p.second;
     };
     const float Ls = rows(l[h]);
     float* o = wl + (wave * NQ + h) * WS;

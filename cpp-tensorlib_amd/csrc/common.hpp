@@ -163,6 +163,11 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// a / n and a % n for 0 <= a < 2^20, n > 0, by a reciprocal that is off by an ulp (a / n + 1 / 2n is never that close to a whole
+// number): six instructions where the compiler's division is a chain of thirty, at the head of kernels that wait for its result.
+__device__ __forceinline__ int small_div(int a, int n) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)n)); }
+__device__ __forceinline__ int small_mod(int a, int n) { return a - small_div(a, n) * n; }
+
 // Block-wide sum for blocks of NW wavefronts; `red` is NW floats of LDS.
 // Every thread gets the result. Summation order is fixed (wave 0..NW-1).
 template <int NW>

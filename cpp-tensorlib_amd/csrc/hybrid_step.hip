@@ -45,26 +45,27 @@ static MixPlan make_plan(const tlhip_window_attn* at, const tlhip_linear_attn* l
   return p;
 }
 
+// The plan and what every kind of block reads first arrive in registers with the block.
 template <int NQ, int NF>
-__global__ __launch_bounds__(512) void mix_step_kernel(const float* __restrict__ u, float* __restrict__ y,
-                                                       const tlhip_window_attn at, const tlhip_linear_attn la,
-                                                       const tlhip_polynorm pn, float* __restrict__ partials, int pos,
-                                                       const uint32_t* __restrict__ d_pos, const MixPlan plan) {
+__global__ __launch_bounds__(512) void mix_step_kernel(const float* __restrict__ u, const uint32_t* __restrict__ d_pos,
+                                                       float* __restrict__ y, float* __restrict__ partials, int pos, int S, int subs,
+                                                       int attn, int lin, const tlhip_window_attn at, const tlhip_linear_attn la,
+                                                       const tlhip_polynorm pn) {
   extern __shared__ __attribute__((aligned(16))) float mix_lds[];
   int b = blockIdx.x;
   const int p = d_pos ? (int)*d_pos : pos;
-  if (b < plan.attn) {
-    const int split = b % plan.S, r = b / plan.S, sub = r % plan.subs, kvh = r / plan.subs;
-    const int group = (int)(at.heads / at.kv_heads), h0 = sub * NQ;
-    window_step_block<NQ, NF>(at, u, y, partials, p, kvh, h0, min(NQ, group - h0), split, plan.S, mix_lds);
+  if (b < attn) {
+    const int r = small_div(b, S), split = b - r * S, kvh = small_div(r, subs), sub = r - kvh * subs;
+    const int group = small_div((int)at.heads, (int)at.kv_heads), h0 = sub * NQ;
+    window_step_block<NQ, NF>(at, u, y, partials, p, kvh, h0, min(NQ, group - h0), split, S, mix_lds);
     return;
   }
-  b -= plan.attn;
-  if (b < plan.lin) {
+  b -= attn;
+  if (b < lin) {
     linear_step_block(la, u, y, p, b, mix_lds);
     return;
   }
-  b -= plan.lin;
+  b -= lin;
   const int i0 = b * kPolySlice;
   polynorm_block<512>(pn, u + pn.z_off, y + pn.y_off, i0, min(i0 + kPolySlice, (int)pn.ff), mix_lds);
 }
@@ -119,8 +120,8 @@ static int launch_mix(const float* u, float* y, const tlhip_window_attn* at, con
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(LDS)");
   }
-  hipLaunchKernelGGL(fn, dim3((unsigned)(plan.attn + plan.lin + plan.poly)), dim3(512), lds, c.stream, u, y,
-                     at ? *at : a0, la ? *la : l0, pn ? *pn : p0, partials, pos, static_cast<const uint32_t*>(d_pos), plan);
+  hipLaunchKernelGGL(fn, dim3((unsigned)(plan.attn + plan.lin + plan.poly)), dim3(512), lds, c.stream, u, static_cast<const uint32_t*>(d_pos),
+                     y, partials, pos, plan.S, plan.subs, plan.attn, plan.lin, at ? *at : a0, la ? *la : l0, pn ? *pn : p0);
   if (at && plan.S > 1 && merge)
     hipLaunchKernelGGL(mix_merge_kernel, dim3((unsigned)at->heads), dim3(256), 0, c.stream, u, y, *at, partials, plan.S);
   TLHIP_CHECK_LAUNCH(TLHIP_C_MIX_STEP);

@@ -20,19 +20,30 @@ __device__ __forceinline__ float log2_decay(float z, float inv_tau) {
 // z of channel `ch` (head * dim + d): the low-rank product and its bias
 __device__ __forceinline__ float decay_logit(const tlhip_linear_attn& a, const float* __restrict__ low, int ch) {
   const uint16_t* w = static_cast<const uint16_t*>(a.a2) + (size_t)ch * a.rank;
+  const int rank = (int)a.rank;
+  const float bias = static_cast<const float*>(a.bias)[ch];
   float z = 0.f;
-  for (int r = 0; r < (int)a.rank; r++) z = fmaf(__uint_as_float((uint32_t)w[r] << 16), low[r], z);
-  return z + static_cast<const float*>(a.bias)[ch];
+  for (int r0 = 0; r0 < rank; r0 += 16) {          // sixteen at once, not in turn
+    uint16_t x[16];
+    float l[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) x[r] = w[min(r0 + r, rank - 1)], l[r] = low[min(r0 + r, rank - 1)];
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+      if (r0 + r < rank) z = fmaf(__uint_as_float((uint32_t)x[r] << 16), l[r], z);
+  }
+  return z + bias;
 }
 __host__ __device__ inline int64_t linear_state_ld(int64_t vdim) { return (vdim + 3) & ~(int64_t)3; }
 
 // Decode step of head h, one block of 512 threads. The state is read from the slot of `pos` and
-// written to the other one; a thread owns one float4 column of every ng-th row.
+// written to the other one; a thread owns one float4 column of every ng-th row. Of its first rows both slots are asked for: the
+// position may be on the device, and what depends on it would be asked for a round trip later.
 __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, const float* __restrict__ u,
                                                   float* __restrict__ y, int pos, int h, float* smem) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int dim = (int)a.dim, vdim = (int)a.vdim, ld = (int)linear_state_ld(vdim), nv4 = ld >> 2;
-  const int ng = 512 / nv4, v4 = tid % nv4, dg = tid / nv4;
+  const int ng = small_div(512, nv4), dg = small_div(tid, nv4), v4 = tid - dg * nv4;
   const bool live = dg < ng;
   float* qs = smem;               // [dim]
   float* ks = qs + dim;
@@ -41,24 +52,27 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
   float* red = vs + ld + ((4 - (3 * dim + ld) % 4) & 3);   // [ng][ld], 16-byte aligned
   float* sums = red + 2048;       // [8]
   const size_t slot = (size_t)a.heads * dim * ld;
-  const float* src = static_cast<const float*>(a.state) + (size_t)(pos & 1) * slot + (size_t)h * dim * ld;
-  float* dst = static_cast<float*>(a.state) + (size_t)((pos + 1) & 1) * slot + (size_t)h * dim * ld;
-  constexpr int PRE = 8;          // rows of this thread requested up front
-  float4 st[PRE];
+  const float* both = static_cast<const float*>(a.state) + (size_t)h * dim * ld;
+  constexpr int PRE = 4;          // rows of this thread requested up front
+  float4 st[2][PRE];
 #pragma unroll
-  for (int i = 0; i < PRE; i++) {
-    const int d = dg + i * ng;
-    st[i] = live && pos > 0 && d < dim ? *reinterpret_cast<const float4*>(src + (size_t)d * ld + 4 * v4)
-                                       : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+  for (int i = 0; i < PRE; i++)
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      st[k][i] = *reinterpret_cast<const float4*>(both + k * slot + (size_t)min(dg + i * ng, dim - 1) * ld + 4 * v4);
+  const int64_t ch0 = (int64_t)h * vdim + min(tid, vdim - 1);
+  const float gate0 = u[a.gate_off + ch0], norm0 = static_cast<const float*>(a.norm)[min(tid, vdim - 1)];   // of what this thread writes first
   for (int d = tid; d < dim; d += 512) {
     const int ch = h * dim + d;
-    qs[d] = u[a.q_off + ch] * a.q_scale;
-    ks[d] = u[a.k_off + ch];
+    const float q = u[a.q_off + ch], k = u[a.k_off + ch];
     al[d] = exp2_native(log2_decay(decay_logit(a, u + a.low_off, ch), 1.0f / a.tau));
+    qs[d] = q * a.q_scale;
+    ks[d] = k;
   }
   for (int v = tid; v < ld; v += 512) vs[v] = v < vdim ? u[a.v_off + (int64_t)h * vdim + v] : 0.f;
   __syncthreads();
+  const float* src = both + (size_t)(pos & 1) * slot;
+  float* dst = static_cast<float*>(a.state) + (size_t)((pos + 1) & 1) * slot + (size_t)h * dim * ld;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   if (live) {
     const float v0 = vs[4 * v4], v1 = vs[4 * v4 + 1], v2 = vs[4 * v4 + 2], v3 = vs[4 * v4 + 3];
@@ -70,7 +84,7 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
     };
 #pragma unroll
     for (int i = 0; i < PRE; i++)
-      if (dg + i * ng < dim) row(dg + i * ng, st[i]);
+      if (dg + i * ng < dim) row(dg + i * ng, pos > 0 ? ((pos & 1) ? st[1][i] : st[0][i]) : make_float4(0.f, 0.f, 0.f, 0.f));
     for (int d = dg + PRE * ng; d < dim; d += ng)
       row(d, pos > 0 ? *reinterpret_cast<const float4*>(src + (size_t)d * ld + 4 * v4) : make_float4(0.f, 0.f, 0.f, 0.f));
     *reinterpret_cast<float4*>(red + dg * ld + 4 * v4) = o;
@@ -80,7 +94,14 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
   float ss = 0.f;
   for (int v = tid; v < vdim; v += 512) {
     float t = 0.f;
-    for (int g = 0; g < ng; g++) t += red[g * ld + v];
+    for (int g0 = 0; g0 < ng; g0 += 8) {           // (eight LDS reads at once)
+      float x[8];
+#pragma unroll
+      for (int g = 0; g < 8; g++) x[g] = red[min(g0 + g, ng - 1) * ld + v];
+#pragma unroll
+      for (int g = 0; g < 8; g++)
+        if (g0 + g < ng) t += x[g];
+    }
     vs[v] = t;
     ss = fmaf(t, t, ss);
   }
@@ -93,8 +114,8 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
   const float inv = 1.0f / sqrtf(tot / (float)vdim + a.eps);
   for (int v = tid; v < vdim; v += 512) {
     const int64_t ch = (int64_t)h * vdim + v;
-    const float g = u[a.gate_off + ch];
-    y[a.y_off + ch] = vs[v] * inv * static_cast<const float*>(a.norm)[v] * (g * sigmoid_f(g)) * a.out_scale;
+    const float g = v == tid ? gate0 : u[a.gate_off + ch], nv = v == tid ? norm0 : static_cast<const float*>(a.norm)[v];
+    y[a.y_off + ch] = vs[v] * inv * nv * (g * sigmoid_f(g)) * a.out_scale;
   }
 }
 

@@ -37,16 +37,25 @@ __device__ __forceinline__ PolyCoef poly_coef(const tlhip_polynorm& p, PolySums 
 }
 
 // Elements [i0, i1) of one row by a block of NT threads; the three means are taken over the whole row
-// by every block that works on it.
+// by every block that works on it. Eight loads of a thread are asked for at once, and with the first ones the elements that it writes:
+// one by one a row of 8192 was six round trips.
 template <int NT>
 __device__ __forceinline__ void polynorm_block(const tlhip_polynorm& p, const float* __restrict__ z, float* __restrict__ y,
                                                int i0, int i1, float* red) {
   const int tid = threadIdx.x, ff = (int)p.ff, n4 = ff >> 2;
   PolySums s;
-  for (int i = tid; i < n4; i += NT) s.add(reinterpret_cast<const float4*>(z)[i]);
+  const float own0 = z[min(i0 + tid, ff - 1)], own1 = z[min(i0 + tid + NT, ff - 1)];
+  for (int i = tid; i < n4; i += 8 * NT) {
+    float4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = reinterpret_cast<const float4*>(z)[min(i + k * NT, n4 - 1)];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (i + k * NT < n4) s.add(v[k]);
+  }
   for (int i = 4 * n4 + tid; i < ff; i += NT) s.add(z[i]);
   const PolyCoef f = poly_coef<NT>(p, s, red);
-  for (int i = i0 + tid; i < i1; i += NT) y[i] = f(z[i]);
+  for (int i = i0 + tid; i < i1; i += NT) y[i] = f(i == i0 + tid ? own0 : i == i0 + tid + NT ? own1 : z[i]);
 }
 
 // A whole row whose values stay in registers: ff a multiple of 4 up to 4 * NT * L, z and y 16-byte aligned.
