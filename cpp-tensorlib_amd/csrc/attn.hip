@@ -123,11 +123,10 @@ __device__ __forceinline__ float4 kv_store4(uint16_t* p, float4 v, bool store) {
 // [0, pos0 + p_g]; later keys of a tile are masked per row. Longest rows first.
 template <int D, int G, typename KT, bool PRE, bool QKV = false>
 __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kernel(
-    const float* __restrict__ q, const KT* __restrict__ K, const KT* __restrict__ V,
+    const float* __restrict__ q, const KT* __restrict__ K, const KT* __restrict__ V, int64_t kv_stride, int n_kv_heads, int S,
+    int n_head_groups, int chunk, int shape, int group,     // (up to here in registers with the block; shape = TK | wavefronts << 8)
     float* __restrict__ out, float* __restrict__ part_m, float* __restrict__ part_l,
-    float* __restrict__ part_acc, int group, int ctx, int64_t kv_stride, int chunk, int TK,
-    float scale, int S, int T, int pos0, const uint32_t* __restrict__ dpos, QkvFuse fz, int kv_rows,
-    int n_kv_heads, int n_head_groups) {
+    float* __restrict__ part_acc, int ctx, float scale, int T, int pos0, const uint32_t* __restrict__ dpos, QkvFuse fz) {
   constexpr int EPL = D / 16;        // floats of a key row per lane (4 or 8)
   constexpr int NV = EPL / 4;        // float4 loads per lane per key
   // Lane c of a row holds elements [4c, 4c+4) of each of the NV consecutive 64-element
@@ -146,7 +145,9 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
   __shared__ float st_m[NWMAX][G], st_l[NWMAX][G];  // per-wave softmax state for the block merge
   __shared__ float st_acc[NWMAX][G][D];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = shape >> 8, threads = nw * 64;
+  int TK = shape & 255;
+  const int last_row = (int)min(kv_stride / D - 1, (int64_t)0x7fffffff);
   const int slot = lane >> 4, c = lane & 15;     // DPP row = key slot, c = position in the row
   // Decode launches a 1-D grid and deals (kv head, split, head group) from the block number so
   // that the head groups of one (kv head, split) - which read the same K/V rows - run on the
@@ -157,11 +158,12 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
   int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
   if constexpr (!PRE) {
     const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    bz = seq % n_head_groups;
-    const int pair = (seq / n_head_groups) * 8 + xcd;
+    const int turn = n_head_groups == 1 ? seq : seq / n_head_groups;
+    bz = seq - turn * n_head_groups;
+    const int pair = turn * 8 + xcd;
     if (pair >= n_kv_heads * S) return;          // (uniform for the block; no barrier was passed)
-    bx = pair % n_kv_heads;
-    by = pair / n_kv_heads;
+    by = small_div(pair, n_kv_heads);            // (at most 65535 kv heads, or one or two blocks per CU)
+    bx = pair - by * n_kv_heads;
   }
   const int split = by;
   TLHIP_MARK(0);
@@ -183,7 +185,7 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
   } else {
     kvh = bx;
     g0 = bz * G;
-    ng = min(G, group - g0);
+    ng = G == 1 ? 1 : min(G, group - g0);
     row0 = (size_t)kvh * group + g0;
     k_begin = k_end = 0;                         // set below, once the position is known
   }
@@ -231,7 +233,7 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
     const int kb0 = chunk ? split * chunk + wave * TK : (split * nw + wave) * TK;
 #pragma unroll
     for (int u = 0; u < UNR; u++) {
-      const int key = min(kb0 + u * 4 + slot, kv_rows - 1);
+      const int key = min(kb0 + u * 4 + slot, last_row);
 #pragma unroll
       for (int v = 0; v < NV; v++) {
         kpre[u][v] = KvLoad<KT>::ld(K + hoff + (size_t)key * D + dim0(c, v));
@@ -259,7 +261,7 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
       *reinterpret_cast<float4*>(&tabs[(tq - QT) * 4]) = t_own;
     }
     // blocks of one or two wavefronts (short contexts) have fewer threads than there are float4s
-    for (int t2 = tq + (int)blockDim.x; t2 < QT + (QKV ? D / 4 : 0); t2 += (int)blockDim.x) {
+    for (int t2 = tq + threads; t2 < QT + (QKV ? D / 4 : 0); t2 += threads) {
       if (t2 < QT) {
         const int gq = t2 / (D / 4), dq = (t2 - gq * (D / 4)) * 4;
         const size_t r = (row0 + (size_t)min(gq, ng - 1)) * D;
@@ -528,7 +530,7 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
   TLHIP_MARK(5);
 
   // ---- block merge (fixed wave order) and store ---------------------------------------------
-  for (int e = threadIdx.x; e < ng * D; e += blockDim.x) {
+  for (int e = threadIdx.x; e < ng * D; e += threads) {
     const int g = e / D, d = e - g * D;
     float M = st_m[0][g];
     for (int w = 1; w < nw; w++) M = fmaxf(M, st_m[w][g]);
@@ -549,6 +551,62 @@ __global__ __launch_bounds__((!PRE && G <= 4) ? 512 : 256) void attn_decode_kern
     }
   }
   TLHIP_MARK(6);
+}
+
+// Merge of up to 128 split partials of a head: grid (heads, 64-column parts), 256 threads, 16 column quads x 16 split groups (split s
+// in group s % 16, u = s / 16 <= U - 1). The kernel is a chain of latencies and little else: every load is requested at the top, every
+// wavefront weighs all splits by itself, a lane to a split, and the one barrier is that of the groups' sums, added up in order. With
+// 1024 threads and the weights formed by the block it was five barriers: 28 heads of 128 in 64 splits 3.96 us, 3.2 so (in a step's trace).
+template <int D, int U>
+__global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ part_m, const float* __restrict__ part_l,
+                                                         const float* __restrict__ part_acc, float* __restrict__ out, int S) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // (an odd number of maxima and sums lies ahead of the values)
+  __shared__ f32x4 red[16][16];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, cq = tid & 15, g = tid >> 4;
+  const float *pm = part_m + (size_t)h * S, *pl = part_l + (size_t)h * S;
+  const float* pa = part_acc + (size_t)h * S * D + blockIdx.y * 64 + 4 * cq;
+  constexpr int NL = U > 4 ? 2 : 1;    // splits of a lane
+  float m[NL], l[NL];
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    m[i] = pm[min(lane + 64 * i, S - 1)];
+    l[i] = pl[min(lane + 64 * i, S - 1)];
+  }
+  f32x4 v[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) v[u] = *reinterpret_cast<const f32x4u*>(pa + (size_t)min(g + 16 * u, S - 1) * D);
+  float M = -INFINITY, w[NL], L = 0.f;
+#pragma unroll
+  for (int i = 0; i < NL; i++) M = fmaxf(M, m[i]);   // (a split read twice changes no maximum)
+  M = wave_max(M);
+#pragma unroll
+  for (int i = 0; i < NL; i++) {
+    const bool live = lane + 64 * i < S;
+    w[i] = live ? __expf(m[i] - M) : 0.f;
+    L = add_rn(L, live ? mul_rn(l[i], w[i]) : 0.f);
+  }
+  L = wave_sum(L);
+  f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int sp = g + 16 * u;
+    const float f = __shfl(w[u / 4], sp & 63, kWave);
+#pragma unroll
+    for (int e = 0; e < 4; e++) a[e] = sp < S ? fmaf(f, v[u][e], a[e]) : a[e];
+  }
+  red[g][cq] = a;
+  __syncthreads();
+  if (tid < 64) {
+    const float* r = reinterpret_cast<const float*>(red) + tid;
+    float x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = r[64 * k];
+    float A = x[0];
+#pragma unroll
+    for (int k = 1; k < 16; k++) A += x[k];
+    out[(size_t)h * D + blockIdx.y * 64 + tid] = A / L;
+  }
 }
 
 // grid = Hq, block = 1024: merge the S split partials of one head. The threads are D
@@ -982,6 +1040,17 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
 
 }  // namespace gqa
 
+// The splits' partials of Hq heads -> out. More than 128 splits: the kernel that takes any number.
+template <int D>
+static void launch_merge(const float* pm, const float* pl, const float* pacc, float* out, int Hq, int S) {
+  hipStream_t st = tlhip::ctx().stream;
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)Hq, D / 64), dim3(256), 0, st, pm, pl, pacc, out, S); };
+  if (S <= 16) go(attn_merge_kernel<D, 1>);
+  else if (S <= 64) go(attn_merge_kernel<D, 4>);
+  else if (S <= 128) go(attn_merge_kernel<D, 8>);
+  else hipLaunchKernelGGL(attn_combine_kernel, dim3(Hq), dim3(1024), (size_t)(S + 1024) * sizeof(float), st, pm, pl, pacc, out, S, D);
+}
+
 struct AttnPlan { int G, gz, nw, TK, S, chunk; };
 
 // Split-KV plan. Work is cut into wave tiles of TK keys; the chip wants 4 to 8
@@ -1114,8 +1183,7 @@ static int launch_gqa(const float* q, const float* K, const float* V, float* out
 #undef TLHIP_GQA
   if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(LDS)");
   if (S > 1 && out)
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(Hq), dim3(1024), (size_t)(S + 1024) * sizeof(float),
-                       c.stream, pm, pl, pacc, out, S, D);
+    launch_merge<D>(pm, pl, pacc, out, Hq, S);
   TLHIP_CHECK_LAUNCH(TLHIP_C_ATTN_DECODE);
 }
 
@@ -1160,12 +1228,12 @@ static int launch_attn(const float* q, const KT* K, const KT* V, float* out, int
 #define TLHIP_ATTN(GG)                                                                            \
   if (fuse)                                                                                       \
     hipLaunchKernelGGL((attn_decode_kernel<D, GG, KT, false, true>), grid, block, 0, c.stream, q, \
-                       K, V, out, pm, pl, pacc, group, ctx, kv_stride, p.chunk, p.TK, scale, S,   \
-                       1, 0, dpos, fz, (int)kv_max, Hkv, p.gz);                                   \
+                       K, V, kv_stride, Hkv, S, p.gz, p.chunk, p.TK | (int)(block.x / 64) << 8, group, out, pm, pl, pacc, ctx, scale, \
+                       1, 0, dpos, fz);                                                           \
   else                                                                                            \
     hipLaunchKernelGGL((attn_decode_kernel<D, GG, KT, false>), grid, block, 0, c.stream, q, K, V, \
-                       out, pm, pl, pacc, group, ctx, kv_stride, p.chunk, p.TK, scale, p.S, 1, 0, \
-                       dpos, fz, (int)kv_max, Hkv, p.gz)
+                       kv_stride, Hkv, p.S, p.gz, p.chunk, p.TK | (int)(block.x / 64) << 8, group, out, pm, pl, pacc, ctx, scale, 1, 0, \
+                       dpos, fz)
   switch (p.G) {
     case 1: TLHIP_ATTN(1); break;
     case 2: TLHIP_ATTN(2); break;
@@ -1174,8 +1242,7 @@ static int launch_attn(const float* q, const KT* K, const KT* V, float* out, int
   }
 #undef TLHIP_ATTN
   if (S > 1)
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(Hq), dim3(1024), (size_t)(S + 1024) * sizeof(float),
-                       c.stream, pm, pl, pacc, out, S, D);
+    launch_merge<D>(pm, pl, pacc, out, Hq, S);
   TLHIP_CHECK_LAUNCH(TLHIP_C_ATTN_DECODE);
 }
 
@@ -1213,9 +1280,9 @@ static int launch_prefill(const float* q, const KT* K, const KT* V, float* out, 
   if (token_major) return fail(TLHIP_EUNSUPPORTED, "tlhip_attn_prefill_tok: the VALU kernel writes head-major only");
   constexpr int G = 8;   // query positions per block
   const dim3 grid(Hq, 1, (T + 4 * G - 1) / (4 * G)), block(256);   // 4 wavefronts x G query rows
-  hipLaunchKernelGGL((attn_decode_kernel<D, G, KT, true>), grid, block, 0, c.stream, q, K, V, out,
-                     (float*)nullptr, (float*)nullptr, (float*)nullptr, Hq / Hkv, pos0 + T,
-                     kv_max * D, 0, 64, scale, 1, T, pos0, (const uint32_t*)nullptr, QkvFuse{}, (int)kv_max, 0, 1);
+  hipLaunchKernelGGL((attn_decode_kernel<D, G, KT, true>), grid, block, 0, c.stream, q, K, V, kv_max * D, 0, 1, 1, 0, 64 | 4 << 8,
+                     Hq / Hkv, out, (float*)nullptr, (float*)nullptr, (float*)nullptr, pos0 + T, scale, T, pos0, (const uint32_t*)nullptr,
+                     QkvFuse{});
   TLHIP_CHECK_LAUNCH(TLHIP_C_ATTN_PREFILL);
 }
 

@@ -120,8 +120,11 @@ struct MixSplits {
 //   delta    Producer::delta; kAttnMerge: splits | heads << 8 | head size << 24
 //   len      16-byte units of a row | chunks / KW << 13 | chunks % KW << 22
 //   tiles    ntiles / blocks | ntiles % blocks << 19: a block's row tiles, one more for the first ones
+// TWO: every wavefront has exactly two items, both asked for ahead of the staging pass. Taken for int4 behind a norm or an attention merge
+// (1152 x 896 and 896 x 896 in a recorded 0.5B step: 499 -> 486 us for either, 475 for both). Not where there are more (9728 x 8192
+// normed 13.9 -> 14.3 us), nor for bf16 (9728 x 896 gated behind a post-norm, a small Girirax turn 6890 -> 7160; behind a norm no change).
 //   block    KW | wavefronts << 5 | blocks << 10 | (ceil(256 / KW) - 1) << 24
-template <typename Fmt, int R, int PRO, int LPR, int EPI = kStore>
+template <typename Fmt, int R, int PRO, int LPR, int EPI = kStore, bool TWO = false>
 __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
     const float* x, const uint4* __restrict__ W, const float* __restrict__ scales, const float* delta, const float* norm_w,
     int N, uint32_t len, uint32_t tiles, uint32_t block, float* __restrict__ y, const ProducerArgs pro) {
@@ -240,11 +243,12 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
   };
   RowFrag<Fmt, R, EPI> frag[NS];
   load_item(frag[0]);
+  if constexpr (TWO) load_item(frag[1]);
   TLHIP_MARK(1);
 
   if constexpr (PRO == kAttnMerge) {
     // The splits' weights e^(m_s - M) and each head's sum, once per block into LDS: sixteen adjacent
-    // lanes hold the (up to) sixteen splits of a head. Sums in the order of attn_combine_kernel's
+    // lanes hold the (up to) sixteen splits of a head. Sums in the order of attn_merge_kernel's
     // wavefront sum over its first sixteen lanes: partners 8, 4, 2 and 1 lanes away in turn.
     const int S = am_S, hs = am_heads * S;
     const auto weigh = [&](int e, float m, float l) {
@@ -520,7 +524,10 @@ __global__ __launch_bounds__(R >= 8 ? 512 : 1024) void gemv_rows_kernel(
       c++;
     }
   };
-  if (n_items >= NS) {
+  if constexpr (TWO) {
+    compute_item(frag[0]);
+    compute_item(frag[1]);
+  } else if (n_items >= NS) {
 #pragma unroll
     for (int k = 1; k < NS; k++) load_item(frag[k]);
     int it = 0;
@@ -803,16 +810,16 @@ static RowCfg pick_rows_cfg(int64_t N, int upr, int E, int pro, int cus, int lds
   return c;
 }
 
-template <typename Fmt, int PRO, int LPR, int EPI>
+template <typename Fmt, int PRO, int LPR, int EPI, bool TWO = false>
 static auto pick_rows_fn(int R) -> void (*)(const float*, const uint4*, const float*, const float*, const float*, int, uint32_t,
                                             uint32_t, uint32_t, float*, const ProducerArgs) {
   switch (R) {
     case 1:
-      if constexpr (EPI == kStore) return gemv_rows_kernel<Fmt, 1, PRO, LPR, EPI>;   // (a pair needs two rows)
+      if constexpr (EPI == kStore) return gemv_rows_kernel<Fmt, 1, PRO, LPR, EPI, TWO>;   // (a pair needs two rows)
       else return nullptr;
-    case 2: return gemv_rows_kernel<Fmt, 2, PRO, LPR, EPI>;
-    case 4: return gemv_rows_kernel<Fmt, 4, PRO, LPR, EPI>;
-    case 8: return gemv_rows_kernel<Fmt, 8, PRO, LPR, EPI>;
+    case 2: return gemv_rows_kernel<Fmt, 2, PRO, LPR, EPI, TWO>;
+    case 4: return gemv_rows_kernel<Fmt, 4, PRO, LPR, EPI, TWO>;
+    case 8: return gemv_rows_kernel<Fmt, 8, PRO, LPR, EPI, TWO>;
     default: return nullptr;
   }
 }
@@ -860,6 +867,10 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
     auto fn = cfg.lpr == 16 ? pick_rows_fn<Fmt, PRO, 16, EPI>(cfg.R) : pick_rows_fn<Fmt, PRO, 64, EPI>(cfg.R);
     if constexpr (PRO == kPostnorm)
       if (!held) fn = cfg.lpr == 16 ? pick_rows_fn<Fmt, kPostnormLong, 16, EPI>(cfg.R) : pick_rows_fn<Fmt, kPostnormLong, 64, EPI>(cfg.R);
+    const int chunks = (upr + cfg.lpr - 1) / cfg.lpr;
+    if constexpr (Fmt::kScaled && (PRO == kRmsnorm || PRO == kAttnMerge))
+      if (ntiles % cfg.blocks == 0 && chunks % cfg.KW == 0 && ntiles / cfg.blocks * (chunks / cfg.KW) == 2)
+        fn = cfg.lpr == 16 ? pick_rows_fn<Fmt, PRO, 16, EPI, true>(cfg.R) : pick_rows_fn<Fmt, PRO, 64, EPI, true>(cfg.R);
     if (!fn) return fail(TLHIP_EINVAL, "rows per wavefront must be 1, 2, 4 or 8");
     if (cfg.lds > 48 * 1024) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
@@ -868,7 +879,6 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
     }
     const uint4* Wn = static_cast<const uint4*>(W) + (size_t)n0 * upr;
     const float* sn = scales ? scales + (size_t)n0 * upr : nullptr;
-    const int chunks = (upr + cfg.lpr - 1) / cfg.lpr;
     if (upr > 0x1fff || chunks / cfg.KW > 0x1ff || cfg.KW > 16 || cfg.nw > 16 || cfg.blocks > 0x2000 || ntiles / cfg.blocks > 0x7ffff)
       return fail(TLHIP_EUNSUPPORTED, "gemv: launch shape out of range");   // (rows that LDS holds end far below)
     const uint32_t len = (uint32_t)upr | (uint32_t)(chunks / cfg.KW) << 13 | (uint32_t)(chunks % cfg.KW) << 22;

@@ -75,6 +75,21 @@ def test_attn_several_tiles_a_split(lib, orc, D, Hq, Hkv, ctx):
     assert np.array_equal(_run(lib, q, K, V, ctx, scale), got)
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,ctx", [(64, 7, 1, 1024), (64, 7, 1, 1025), (128, 3, 1, 4096), (64, 7, 1, 4097), (64, 7, 1, 8192), (64, 3, 1, 100),
+                                          (128, 1, 1, 9000), (64, 5, 5, 3000)])
+def test_attn_split_counts(lib, orc, D, Hq, Hkv, ctx):
+    """As many splits as one, four and eight of each of the merge's sixteen groups take (16, 64, 128), one more, few and many, an odd
+    number of maxima and sums ahead of the values."""
+    print("case attn splits", D, Hq, Hkv, ctx, flush=True)
+    q = orc.normal(Hq * D, 41).reshape(Hq, D) * 4.0      # (a few keys with most of the weight: splits of very different maxima)
+    K = orc.normal(Hkv * ctx * D, 42).reshape(Hkv, ctx, D)
+    V = orc.normal(Hkv * ctx * D, 43).reshape(Hkv, ctx, D)
+    scale = 1.0 / np.sqrt(float(D))
+    want = orc.attn_decode(q, K, V, scale, ctx=ctx)
+    got = _run(lib, q, K, V, ctx, scale)
+    assert allclose(got, want, RTOL, ATOL), maxrel(got, want)
+
+
 def test_attn_closed_forms(lib, orc):
     H, D, ctx = 4, 128, 300
     q = orc.normal(H * D, 1).reshape(H, D)
