@@ -22,7 +22,11 @@
 // contiguous kilobytes, copied by 48 global_load_lds_dwordx4 (1 KB each, whole cache lines, no
 // registers), six per wavefront. A block is eight wavefronts (4 x 2) on a 256 x 256 tile, 64 x 128
 // per wavefront (or 128 x 256 and 32 x 128: gemm_f16w_impl chooses), one block per CU, a ring of three slabs
-// in LDS (144 KB), one barrier per slab; a copy has two slab times to land. Products of f16 are exact in fp32, the MFMA sums in fp32, and
+// in LDS (144 KB), one barrier per slab; a copy has two slab times to land. What bounds it where it fills the chip is power: over
+// activations of zeros, the same instructions, 512 x 3584 x 18944 in four parts takes 116 us where it took 157 over random ones, and five
+// stages of 128 rows or copies spread evenly over a slab changed nothing. So the products are 16 x 16 x 32: 32 x 32 x 16 reads
+// and writes twice the accumulators per product. Measured for it at 512 rows, images included: 3584 x 18944 in parts 158.7 -> 137
+// us, 18944 gated x 3584 262 -> 231, 4608 x 3584 in parts 45.9 -> 43.4; 1024 x 3584 x 3584 76.6 -> 67.6. Products of f16 are exact in fp32, the MFMA sums in fp32, and
 // the result leaves as acc * 2^-(ea[m] + ew[n]), an exact scaling: the error is fp32 summation
 // error plus one fp32-rounding-sized term per product, as in the reference's fp32 FMA loop
 // (tensorlib_cuda.cu:509-519).
@@ -387,44 +391,40 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
     }
   };
 
-  f32x16 acc[TM][4];
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int RT = 2 * TM;                         // 16-row tiles of a wavefront
+  f32x4 acc[RT][8];
 #pragma unroll
-  for (int i = 0; i < TM; i++)
+  for (int i = 0; i < RT; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    for (int j = 0; j < 8; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // this lane's first fragment of A (hi plane, tile row 0) and of W (tile column 0) within a
-  // stage, per 16-k step; the other fragments are constant offsets from these
-  int aoff[2], boff[2];
+  // stage; the other fragments are constant offsets from these
+  const int aoff = image_off(wm * 32 * TM + (lane & 15), lane >> 4), boff = 2 * kAPlane + image_off(wn * 128 + (lane & 15), lane >> 4);
+  frag16 af[RT][2], bf[2][4];
+  auto fetch_w = [&](const char* stage, auto H) {
+    constexpr int h = decltype(H)::value;
 #pragma unroll
-  for (int ks = 0; ks < 2; ks++) {
-    const int kc = ks * 2 + (lane >> 5);
-    aoff[ks] = image_off(wm * 32 * TM + (lane & 31), kc);
-    boff[ks] = 2 * kAPlane + image_off(wn * 128 + (lane & 31), kc);
-  }
-  // fragment sets: F[0] for the first 16 k of a slab, F[1] for the second
-  frag16 af[2][TM][2], bf[2][4];
-  auto fetch = [&](const char* stage, auto KS) {
-    constexpr int ks = decltype(KS)::value;
-#pragma unroll
-    for (int j = 0; j < 4; j++) bf[ks][j] = *reinterpret_cast<const frag16*>(stage + boff[ks] + j * 32 * kRowBytes);
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int p = 0; p < 2; p++)
-        af[ks][i][p] = *reinterpret_cast<const frag16*>(stage + aoff[ks] + p * kAPlane + i * 32 * kRowBytes);
+    for (int j = 0; j < 4; j++) bf[h][j] = *reinterpret_cast<const frag16*>(stage + boff + (h * 4 + j) * 16 * kRowBytes);
   };
-  // four products: fragment set KS, (tile row, plane) pair Q against the four tile columns. The
-  // weight fragment is the MFMA's first operand: the tile comes out transposed, D[n][m], so that a
-  // lane ends up with four consecutive COLUMNS of one row of C - a 16-byte store, not four 4-byte ones.
-  auto mul4 = [&](auto KS, auto Q) {
-    constexpr int ks = decltype(KS)::value, q = decltype(Q)::value;
+  auto fetch_a = [&](const char* stage, auto I) {
+    constexpr int i = decltype(I)::value;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-      acc[q >> 1][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, bf[ks][j]),
-                                                              __builtin_bit_cast(f16x8, af[ks][q >> 1][q & 1]), acc[q >> 1][j], 0, 0, 0);
+    for (int p = 0; p < 2; p++) af[i][p] = *reinterpret_cast<const frag16*>(stage + aoff + p * kAPlane + i * 16 * kRowBytes);
+  };
+  // tile row I against the four tile columns of half H, the second terms first: sums in that order end up a little nearer (512 x 3584
+  // over 3584 in four parts 2.76e-7 of the result, 2.81e-7 the other way round). The weight fragment is the MFMA's first operand:
+  // the tile comes out transposed, D[n][m], so that a lane ends up with four consecutive COLUMNS of one row of C - a 16-byte
+  // store, not four 4-byte ones.
+  auto mul8 = [&](auto H, auto I) {
+    constexpr int h = decltype(H)::value, i = decltype(I)::value;
+#pragma unroll
+    for (int p = 1; p >= 0; p--)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        acc[i][h * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bf[h][j]), __builtin_bit_cast(f16x8, af[i][p]),
+                                                                   acc[i][h * 4 + j], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
   // The block's barrier without the fence __syncthreads() puts before it: that fence would wait for
@@ -436,84 +436,73 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
   };
 
   // Three slabs in flight. Invariant at the top of iteration k: slab k has landed in stage k % 3
-  // for every wavefront and its first fragment set is on its way to registers; slabs k + 1 and
+  // for every wavefront and its fragments of A and of W's first half are on their way to registers; slabs k + 1 and
   // k + 2 are being copied.
   issue(0, 0);
   issue(1, 1);
   issue(2, 2);
-#ifdef TLHIP_TRACE
-  unsigned long long ph[2] = {0, 0}, tc = __builtin_readcyclecounter();
   TLHIP_MARK(0);
-#define TLHIP_PHASE(i) do { const unsigned long long n_ = __builtin_readcyclecounter(); ph[i] += n_ - tc; tc = n_; } while (0)
-#else
-#define TLHIP_PHASE(i)
-#endif
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kCopies) : "memory");   // my copies of slab 0
   barrier();
-  fetch(ring, Idx<0>{});
+  fetch_w(ring, Idx<0>{});
+  fetch_a(ring, Idx<0>{});
+  fetch_a(ring, Idx<1>{});
+  if constexpr (TM == 2) {
+    fetch_a(ring, Idx<2>{});
+    fetch_a(ring, Idx<3>{});
+  }
   TLHIP_MARK(1);
-  // A fragment set is requested a few MFMAs before the set that uses it starts, and nothing
-  // younger is outstanding when it is waited for. The copies of slab k + 3 go out one or two at a
-  // time between groups of MFMAs: issued together, the 48 of a block queue up in front of the
-  // CU's one vector memory path and hold back the MFMAs that follow them in each wavefront.
+  // Every fragment has registers once: W's second half is requested while the products of its first half run, the next slab's
+  // first half while those of the second run, and a tile row of A as soon as its last product of the slab has been issued. The
+  // copies of slab k + 3 go out one or two at a time between groups of MFMAs: issued together, the 48 of a block queue up in
+  // front of the CU's one vector memory path and hold back the MFMAs that follow them in each wavefront.
   int st = 0;
   for (int k = 0; k < ns; k++) {
     const char* stage = ring + st * kStage;
     const int nx = st == 2 ? 0 : st + 1;
-    mul4(Idx<0>{}, Idx<0>{});
-    fetch(stage, Idx<1>{});
+    const char* next = ring + nx * kStage;
+    const bool more = k + 1 < ns;
+    fetch_w(stage, Idx<1>{});
     __builtin_amdgcn_sched_barrier(0);
-    mul4(Idx<0>{}, Idx<1>{});
+    mul8(Idx<0>{}, Idx<0>{});
+    mul8(Idx<0>{}, Idx<1>{});
     if constexpr (TM == 2) {
-      mul4(Idx<0>{}, Idx<2>{});
-      mul4(Idx<0>{}, Idx<3>{});
+      mul8(Idx<0>{}, Idx<2>{});
+      mul8(Idx<0>{}, Idx<3>{});
     }
-    TLHIP_PHASE(0);
     // my reads of slab k are complete and my copies of slab k + 1 have landed (those of slab
     // k + 2 may still be in flight); past the barrier that holds for every wavefront
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kCopies) : "memory");
     barrier();
-    TLHIP_PHASE(1);
     // slab k + 3 into the stage slab k has just left
-    mul4(Idx<1>{}, Idx<0>{});
+    if (more) fetch_w(next, Idx<0>{});
+    __builtin_amdgcn_sched_barrier(0);
+    mul8(Idx<1>{}, Idx<0>{});
     copy(k + 3, st, Idx<0>{});
-    if (TM == 1) copy(k + 3, st, Idx<1>{});
-    if (k + 1 < ns) fetch(ring + nx * kStage, Idx<0>{});
+    copy(k + 3, st, Idx<1>{});
+    if (more) fetch_a(next, Idx<0>{});
     __builtin_amdgcn_sched_barrier(0);
-    mul4(Idx<1>{}, Idx<1>{});
-    if constexpr (TM == 1) {
-      copy(k + 3, st, Idx<2>{});
-      copy(k + 3, st, Idx<3>{});
-    } else {
-      copy(k + 3, st, Idx<1>{});
-      copy(k + 3, st, Idx<2>{});
-      __builtin_amdgcn_sched_barrier(0);
-      mul4(Idx<1>{}, Idx<2>{});
-      copy(k + 3, st, Idx<3>{});
+    mul8(Idx<1>{}, Idx<1>{});
+    copy(k + 3, st, Idx<2>{});
+    copy(k + 3, st, Idx<3>{});
+    if (more) fetch_a(next, Idx<1>{});
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (TM == 2) {
+      mul8(Idx<1>{}, Idx<2>{});
       copy(k + 3, st, Idx<4>{});
+      if (more) fetch_a(next, Idx<2>{});
       __builtin_amdgcn_sched_barrier(0);
-      mul4(Idx<1>{}, Idx<3>{});
+      mul8(Idx<1>{}, Idx<3>{});
       copy(k + 3, st, Idx<5>{});
+      if (more) fetch_a(next, Idx<3>{});
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
     st = nx;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies past the end
-#ifdef TLHIP_TRACE
-  {
-    const unsigned b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    if (lane == 0 && b < kTraceBlocks) {
-      unsigned long long* g = &g_trace[(b * kTraceWaves + wave) * kTraceSlots];
-      g[2] = ph[0]; g[3] = ph[1]; g[7] = ns;
-    }
-  }
   TLHIP_MARK(5);
-#endif
-#undef TLHIP_PHASE
-
-  // acc[v] of lane l (transposed tile): column of C 8*(v/4) + 4*(l/32) + v%4 of the tile, row of C
-  // l%32. Four consecutive v are four consecutive columns: one 16-byte store where the row stride
-  // allows it. The exponents come back out, -(ea[row] + ew[W row of the column]); ldexpf is exact.
+  // acc[e] of lane l (transposed tile): column of C 4 (l / 16) + e of the 16 x 16 tile, row of C l % 16: four consecutive columns, one
+  // 16-byte store where the row stride allows it. The exponents come back out, -(ea[row] + ew[W row of the column]); ldexpf is exact.
   const int ltn = tn - tn0;                          // column tile within this launch
   const int nlim = N + (GU ? tn0 * 128 : tn0 * kTile);   // first unit of N past this launch, absolute
   const bool wide = (ldc & 3) == 0;
@@ -535,7 +524,6 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
       e4[e] = r >= 0 ? (int)ew[r] : 0;
     }
   };
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
   // Where small elements were counted - in a row of A (a_image_kernel) or in a row of W
   // (w_range_kernel) - their absolute errors add up to at most n 2^-10 in the units of acc, i.e.
   // n 2^-10 2^-(ea + ew) in the result's. After the tile has been stored, a result for which that
@@ -558,8 +546,8 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
     }
     wsome = __any(wsome);
 #pragma unroll 1
-    for (int i = 0; i < TM; i++) {
-      const int gm = tm * BM + wm * 32 * TM + i * 32 + (lane & 31);
+    for (int i = 0; i < RT; i++) {
+      const int gm = tm * BM + wm * 32 * TM + i * 16 + (lane & 15);
       const int raw = gm < M ? ea[gm] : 0;
       const uint32_t nsm = (uint32_t)raw >> 8;
       if (!wsome && !__any(nsm != 0u)) continue;      // the ordinary case: nothing to weigh
@@ -584,11 +572,11 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
         return x;
       };
 #pragma unroll 1
-      for (int idx = 0; idx < (gated_out ? 32 : 64); idx++) {
-        const int j = idx >> 4, v = idx & 15;
-        const int c = wn * 128 + j * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+      for (int idx = 0; idx < (gated_out ? 16 : 32); idx++) {
+        const int j = idx >> 2, v = idx & 3;
+        const int c = wn * 128 + j * 16 + 4 * (lane >> 4) + v;
         if (gated_out) {
-          const int f = ltn * 128 + wn * 64 + j * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+          const int f = ltn * 128 + wn * 64 + j * 16 + 4 * (lane >> 4) + v;
           const int rg = weight_row(GU, tn, c, nlim, ff), ru = weight_row(GU, tn, c + 64, nlim, ff);
           if (f >= N || rg < 0 || ru < 0 || !(needs(rg) || needs(ru))) continue;
           const int af = f + tn0 * 128;
@@ -604,80 +592,76 @@ __global__ __launch_bounds__(512, 1) void gemm_f16t_kernel(const char* __restric
   };
   if (GU && gridDim.y == 1) {
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int gm = tm * BM + wm * 32 * TM + i * 32 + (lane & 31);
+    for (int i = 0; i < RT; i++) {
+      const int gm = tm * BM + wm * 32 * TM + i * 16 + (lane & 15);
       if (gm >= M) continue;
       const int em = (int)(int8_t)(ea[gm] & 0xff);
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < 4; j++) {
+        const int c = wn * 128 + j * 16 + 4 * (lane >> 4);      // gate column of the tile; its up value is 64 further
+        const int f = ltn * 128 + wn * 64 + j * 16 + 4 * (lane >> 4);
+        if (f >= N) continue;
+        int eg[4], eu[4];
+        wexp4(c, eg);
+        wexp4(c + 64, eu);
+        float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (ACT == kGelu) {
+          const float* b = bias + f + tn0 * 128;
+          if (by4 && f + 3 < N) {
+            const f32x4 g4 = *reinterpret_cast<const f32x4*>(b), u4 = *reinterpret_cast<const f32x4*>(b + ff);
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const int c = wn * 128 + j * 32 + 8 * g + 4 * (lane >> 5);      // gate column of the tile; its up value is 64 further
-          const int f = ltn * 128 + wn * 64 + j * 32 + 8 * g + 4 * (lane >> 5);
-          if (f >= N) continue;
-          int eg[4], eu[4];
-          wexp4(c, eg);
-          wexp4(c + 64, eu);
-          float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (ACT == kGelu) {
-            const float* b = bias + f + tn0 * 128;
-            if (by4 && f + 3 < N) {
-              const f32x4 g4 = *reinterpret_cast<const f32x4*>(b), u4 = *reinterpret_cast<const f32x4*>(b + ff);
-#pragma unroll
-              for (int e = 0; e < 4; e++) { bg[e] = g4[e]; bu[e] = u4[e]; }
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; e++) {
-                const int k = min(e, N - 1 - f);
-                bg[e] = b[k];
-                bu[e] = b[ff + k];
-              }
-            }
-          }
-          f32x4 o;
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            o[e] = gate(ldexpf(acc[i][j][4 * g + e], -(em + eg[e])), ldexpf(acc[i][j + 2][4 * g + e], -(em + eu[e])), bg[e], bu[e]);
-          float* dst = C + (size_t)gm * ldc + f;
-          if (wide && f + 3 < N) {
-            *reinterpret_cast<f32x4*>(dst) = o;
+            for (int e = 0; e < 4; e++) { bg[e] = g4[e]; bu[e] = u4[e]; }
           } else {
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-              if (f + e < N) dst[e] = o[e];
+            for (int e = 0; e < 4; e++) {
+              const int k = min(e, N - 1 - f);
+              bg[e] = b[k];
+              bu[e] = b[ff + k];
+            }
           }
         }
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          o[e] = gate(ldexpf(acc[i][j][e], -(em + eg[e])), ldexpf(acc[i][j + 4][e], -(em + eu[e])), bg[e], bu[e]);
+        float* dst = C + (size_t)gm * ldc + f;
+        if (wide && f + 3 < N) {
+          *reinterpret_cast<f32x4*>(dst) = o;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (f + e < N) dst[e] = o[e];
+        }
+      }
     }
     again(true);
     TLHIP_MARK(6);
     return;
   }
 #pragma unroll
-  for (int i = 0; i < TM; i++) {
-    const int gm = tm * BM + wm * 32 * TM + i * 32 + (lane & 31);
+  for (int i = 0; i < RT; i++) {
+    const int gm = tm * BM + wm * 32 * TM + i * 16 + (lane & 15);
     if (gm >= M) continue;
     const int em = (int)(int8_t)(ea[gm] & 0xff);
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < 8; j++) {
+      const int c = wn * 128 + j * 16 + 4 * (lane >> 4);
+      const int gn = ltn * kTile + c;
+      if (!GU && gn >= N) continue;   // gated parts are whole tiles wide
+      int e4[4];
+      wexp4(c, e4);
+      f32x4 o;
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int c = wn * 128 + j * 32 + 8 * g + 4 * (lane >> 5);
-        const int gn = ltn * kTile + c;
-        if (!GU && gn >= N) continue;   // gated parts are whole tiles wide
-        int e4[4];
-        wexp4(c, e4);
-        f32x4 o;
+      for (int e = 0; e < 4; e++) o[e] = ldexpf(acc[i][j][e], -(em + e4[e]));
+      float* dst = C + (size_t)gm * ldc + gn;
+      if (wide && (GU || gn + 3 < N)) {
+        *reinterpret_cast<f32x4*>(dst) = o;
+      } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = ldexpf(acc[i][j][4 * g + e], -(em + e4[e]));
-        float* dst = C + (size_t)gm * ldc + gn;
-        if (wide && (GU || gn + 3 < N)) {
-          *reinterpret_cast<f32x4*>(dst) = o;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            if (GU || gn + e < N) dst[e] = o[e];
-        }
+        for (int e = 0; e < 4; e++)
+          if (GU || gn + e < N) dst[e] = o[e];
       }
+    }
   }
   again(false);
   TLHIP_MARK(6);
