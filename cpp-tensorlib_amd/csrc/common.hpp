@@ -35,8 +35,9 @@ struct Context {
   // exists, an outgrown scratch buffer is retired (kept allocated), never freed.
   int graphs_recorded = 0;
   std::vector<void*> retired_scratch;
-  int* argmax_dev = nullptr;      // one int32 result slot
+  int* argmax_dev = nullptr;      // a few words nobody reads (the warm-up reads' sums)
   int* argmax_host = nullptr;     // pinned landing slot for the 4-byte result
+  int* argmax_slot = nullptr;     // the same as the device addresses it
   uint64_t census[TLHIP_C_COUNT] = {};
   uint64_t alloc_calls = 0;       // hipMalloc / hipFree / hipHostMalloc / hipHostFree calls the library has made
   // int4 GEMV launch-shape override (tlhip_tune_gemv_q4)

@@ -216,7 +216,7 @@ int tlq_prefill_hidden(void* hv, float* out, int64_t T) {
 // Greedy step; logits_out (may be NULL) receives the [vocab] logits.
 int64_t tlq_step(void* hv, int64_t token, int64_t pos, float* logits_out) {
   auto* h = static_cast<handle*>(hv);
-  const int64_t id = qwen::step_greedy(h->M, token, pos);
+  const int64_t id = qwen::step_greedy(h->M, token, pos, logits_out != nullptr);
   if (id >= 0 && logits_out)
     std::memcpy(logits_out, qwen::logits(h->M), (size_t)h->M.d.vocab * sizeof(float));
   return id;
@@ -267,7 +267,7 @@ int tlq_decoder_feed(void* hv, int64_t id) {
 }
 int64_t tlq_decoder_step(void* hv, int64_t id, float* logits_out) {
   auto* h = static_cast<handle*>(hv);
-  const int64_t tok = h->dec.step(h->M, id);
+  const int64_t tok = h->dec.step(h->M, id, logits_out != nullptr);
   if (tok >= 0 && logits_out)
     std::memcpy(logits_out, qwen::logits(h->M), (size_t)h->M.d.vocab * sizeof(float));
   return tok;

@@ -189,6 +189,7 @@ int tlhip_init(int device) {
   if ((e = hipMalloc((void**)&c.argmax_dev, 256)) != hipSuccess) return hip_fail(e, "hipMalloc");
   if ((e = hipHostMalloc((void**)&c.argmax_host, 256, hipHostMallocDefault)) != hipSuccess)
     return hip_fail(e, "hipHostMalloc");
+  if ((e = hipHostGetDevicePointer((void**)&c.argmax_slot, c.argmax_host, 0)) != hipSuccess) return hip_fail(e, "hipHostGetDevicePointer");
   if (int rc = attn_static_setup(device)) return rc;
   c.device = device;
   c.cus = prop.multiProcessorCount;

@@ -31,10 +31,11 @@ namespace tl {
 namespace loops {
 
 // embed -> layers -> device argmax. Returns the greedy token, or -1 when any
-// launch was declined.
+// launch was declined. want_logits: logits() is called next, their copy is queued ahead of the wait for the token.
 template <class M>
-int64_t step_greedy(M& m, int64_t token, int64_t pos) {
+int64_t step_greedy(M& m, int64_t token, int64_t pos, bool want_logits = false) {
   if (!stage_embed(m, token) || !step_layers(m, pos)) return -1;
+  if (want_logits) hip::queue_to_host(logits_device(m));
   int64_t idx = -1;
   if (!hip::argmax(logits_device(m), vocab_size(m), &idx)) return -1;
   return idx;
@@ -195,8 +196,9 @@ struct captured_decoder {
     return ok;
   }
   // One decode step: feed + greedy token (-1 when the cache is full or a launch failed).
-  int64_t step(M& m, int64_t id) {
+  int64_t step(M& m, int64_t id, bool want_logits = false) {
     if (!feed(m, id)) return -1;
+    if (want_logits) hip::queue_to_host(logits_device(m));
     int64_t idx = -1;
     return hip::argmax(logits_device(m), vocab_size(m), &idx) ? idx : -1;
   }

@@ -721,6 +721,13 @@ inline void release(void* buf, int64_t, float*) {
   else c.f.free_(e.base);   // device-only extents are not kept for reuse
 }
 
+// sync_to_host will follow: what it would have to copy is queued now, behind the launches so far, where a kernel can do it.
+inline void queue_to_host(void* native) {
+  auto& c = context::get();
+  extent* e = c.ready ? c.buffers.containing(native) : nullptr;
+  if (e && e->staging && e->live == extent::side::device && c.queue_pull(*e)) c.pending = true;
+}
+
 // The host is about to read (for_write: and then modify) the buffer through its host half.
 inline void sync_to_host(void* native, bool for_write) {
   auto& c = context::get();

@@ -91,6 +91,22 @@ def test_argmax(lib, orc, n):
         assert lib.argmax(dv, n) == 123 == orc.argmax(v)
 
 
+@pytest.mark.parametrize("n", [255, 257, 2047, 2049, 3 * 2048 + 5, 151936, 1024 * 2048 + 777])
+def test_argmax_winner_anywhere(lib, orc, n):
+    """Eight numbers a thread at once, the last of them past the end: first, last and numbers in between win, also among -inf."""
+    v = np.full(n, -np.inf, np.float32)
+    dv = lib.to_device(v)
+    for at in sorted({0, n // 2, n - 1, max(n - 257, 0), 7 * (n // 8)}):
+        v[:] = -np.inf
+        v[at] = -1e30
+        dv.upload(v)
+        assert lib.argmax(dv, n) == at
+    v = orc.normal(n, 5)
+    dv.upload(v)
+    assert lib.argmax(dv, n) == int(np.argmax(v))
+    dv.free()
+
+
 def test_kv_append_fill(lib, orc):
     Hkv, D, kv_max = 4, 128, 50
     Kc = np.zeros((Hkv, kv_max, D), np.float32); Vc = Kc.copy()
