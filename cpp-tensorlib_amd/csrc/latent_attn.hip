@@ -398,8 +398,9 @@ __global__ __launch_bounds__(512) void latent_attend_kernel(const uint16_t* __re
   const int DS = steps & 0xffff, LT = steps >> 16, H = hs & 0xffff, S = hs >> 16;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kt = wave & 1, dq = wave >> 1;
-  const int rt = (int)blockIdx.z * 65535 + (int)blockIdx.y, split = blockIdx.x;
-  if (rt * 32 >= rows) return;
+  const int tile = (int)blockIdx.z * 65535 + (int)blockIdx.y, split = blockIdx.x;
+  if (tile * 32 >= rows) return;
+  const int rt = T == 1 ? tile : rows / 32 - 1 - tile;   // the last queries see the most keys: first
   const int row = rt * 32 + c;                       // this lane's query row
   const u32x4* kc = reinterpret_cast<const u32x4*>(keys) + lane;
   const u32x4* vc = reinterpret_cast<const u32x4*>(values) + lane;
@@ -544,8 +545,9 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const uint16_t
   const int S = hs >> 16;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, c = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rt = (int)blockIdx.z * 65535 + (int)blockIdx.y, split = blockIdx.x;
-  if (rt * 32 >= rows) return;
+  const int tile = (int)blockIdx.z * 65535 + (int)blockIdx.y, split = blockIdx.x;
+  if (tile * 32 >= rows) return;
+  const int rt = T == 1 ? tile : rows / 32 - 1 - tile;   // the last queries see the most keys: first
   const int p0 = d_pos ? (int)*d_pos : pos0;
   const int row = rt * 32 + c;                       // this lane's query row
   const int limit = row < T * d.H ? p0 + row / d.H : -1;
@@ -566,7 +568,7 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const uint16_t
   float m = -INFINITY, l = 0.f;
   __syncthreads();
   int par = 0;
-  for (int tile = split; tile < ntiles; tile += S, par ^= 1) {
+  for (int kt = split; kt < ntiles; kt += S, par ^= 1) {
     // values of this tile, requested before the scores are formed
     u32x4 vr[NL][NC][2];
 #pragma unroll
@@ -576,7 +578,7 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const uint16_t
 #pragma unroll
         for (int k = 0; k < 2; k++) {
           const int lt = min(wave + 4 * i, d.LT - 1);
-          vr[i][n][k] = vc[((((size_t)tile * NC + n) * d.LT + lt) * 2 + k) * 64];
+          vr[i][n][k] = vc[((((size_t)kt * NC + n) * d.LT + lt) * 2 + k) * 64];
         }
     f32x16 s;
 #pragma unroll
@@ -584,7 +586,7 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const uint16_t
     for (int st = wave; st < d.DS; st += 4) {
       u32x4 kr[NC], qr[NQ];
 #pragma unroll
-      for (int n = 0; n < NC; n++) kr[n] = kc[(((size_t)tile * NC + n) * d.DS + st) * 64];
+      for (int n = 0; n < NC; n++) kr[n] = kc[(((size_t)kt * NC + n) * d.DS + st) * 64];
 #pragma unroll
       for (int n = 0; n < NQ; n++) qr[n] = qs[(n * d.DS + st) * 64 + lane];
 #pragma unroll
@@ -603,7 +605,7 @@ __global__ __launch_bounds__(256) void latent_attend_exact_kernel(const uint16_t
 #pragma unroll
       for (int w = 1; w < 4; w++) t += red[(par * 16 + 4 * w + i) * 64 + lane];
 #pragma unroll
-      for (int b = 0; b < 4; b++) s[4 * i + b] = tile * 32 + 8 * i + 4 * g + b <= limit ? t[b] : -INFINITY;
+      for (int b = 0; b < 4; b++) s[4 * i + b] = kt * 32 + 8 * i + 4 * g + b <= limit ? t[b] : -INFINITY;
     }
     float mt = s[0];
 #pragma unroll
