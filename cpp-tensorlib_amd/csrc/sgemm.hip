@@ -248,12 +248,12 @@ __global__ __launch_bounds__(64 * kSrWaves, 2) void sgemm_rows_kernel(const floa
   extern __shared__ __attribute__((aligned(16))) float sums[];
   float (*red)[BM][kSrLD] = reinterpret_cast<float (*)[BM][kSrLD]>(sums);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, quarter = lane >> 4;
-  // one contiguous run of tiles per XCD, row blocks fastest: they read the same columns of B
-  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
-  const int lid = xcd * q8 + min(xcd, r8) + within;
+  // row blocks fastest: they read the same columns of B (with parts in an XCD's run 90 x 896 x 4864 16.4 -> 15.7 us, 33 rows 11.9 -> 11.2)
+  const BlockPlace place = block_place(gridDim.x, gridDim.y);
+  const int lid = place.tile;
   const int m0 = lid % row_blocks * BM, n0 = lid / row_blocks * kSrBN;
-  const int kbeg = blockIdx.y * kchunk, kend = min(K, kbeg + kchunk);
-  C += (size_t)blockIdx.y * M * N;                 // K-split parts are dense
+  const int kbeg = place.part * kchunk, kend = min(K, kbeg + kchunk);
+  C += (size_t)place.part * M * N;                 // K-split parts are dense
   // whole steps, the first `whole` of this block's range; what is left of K is one ragged step
   const int steps = (kend - kbeg) / kSrStep, mine = wave < steps ? (steps - wave + kSrWaves - 1) / kSrWaves : 0;
   const bool edge = n0 + kSrBN > N;                // (the block's last columns are read one by one, clamped)

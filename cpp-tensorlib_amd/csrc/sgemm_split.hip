@@ -74,20 +74,21 @@ __device__ __forceinline__ void cut(const float (&x)[8], Terms& t, Range& range,
 template <int TM, int TB>
 __global__ __launch_bounds__(64 * kWaves, 2) void sgemm_split_kernel(const float* __restrict__ A, uint32_t lda, const float* __restrict__ B,
                                                                      uint32_t ldb, float* __restrict__ C, int M, int N, int K, float scale,
-                                                                     float offset, int epi, int kchunk, int row_blocks) {
+                                                                     float offset, int epi, int kchunk, int split) {
   constexpr int BM = 32 * TM;
   extern __shared__ __attribute__((aligned(16))) float sums[];
   __shared__ float seen_most[2][kWaves];
   __shared__ uint32_t seen_least[2][kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
-  // one contiguous run of tiles per XCD, row blocks fastest: they read the same columns of B
-  const int nb = gridDim.x, xcd = blockIdx.x & 7, within = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7;
-  const int lid = xcd * q8 + min(xcd, r8) + within;
+  // row blocks fastest: they read the same columns of B (with parts in an XCD's run 333 x 896 x 4864 29.1 -> 28.0 us)
+  const int row_blocks = split & 0xffff;           // (split: row blocks | parts << 16)
+  const BlockPlace place = block_place(gridDim.x, split >> 16);
+  const int lid = place.tile;
   // (the last columns' tile is moved back to end with the matrix: it stores only the columns from `own` on, for those before them the
   // tile ahead of it may have taken the other way through the range check below)
   const int m0 = lid % row_blocks * BM, own = lid / row_blocks * kBN, n0 = min(own, N - kBN);
-  const int kbeg = blockIdx.y * kchunk, kend = min(K, kbeg + kchunk);
-  C += (size_t)blockIdx.y * M * N;                 // K-split parts are dense
+  const int kbeg = place.part * kchunk, kend = min(K, kbeg + kchunk);
+  C += (size_t)place.part * M * N;                 // K-split parts are dense
   const int steps = (kend - kbeg) / kStep, mine = wave < steps ? (steps - wave + kWaves - 1) / kWaves : 0;
   // column tile j of this lane
   const auto column = [&](int j) { return n0 + (TB ? 32 * j + l32 : 64 * (j >> 1) + 2 * l32 + (j & 1)); };
@@ -364,7 +365,7 @@ int launch_sgemm_split(const float* pa, int64_t lda, const float* pb, int64_t ld
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (set != hipSuccess) return hip_fail(set, "hipFuncSetAttribute");
     sgemm_split_kernel<TM_, TB_><<<dim3((unsigned)tiles, (unsigned)S), dim3(64 * kWaves), lds, ctx().stream>>>(
-        pa, (uint32_t)lda, pb, (uint32_t)ldb, dst, M, N, K, scale, offset, kepi, kchunk, rb);
+        pa, (uint32_t)lda, pb, (uint32_t)ldb, dst, M, N, K, scale, offset, kepi, kchunk, rb | S << 16);   // (rows: up to 1024)
     return 0;
   };
   using std::integral_constant;

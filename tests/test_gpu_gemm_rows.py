@@ -60,6 +60,13 @@ def test_plain_and_parts(lib, orc, fmt, M, N, K):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "q4"])
+@pytest.mark.parametrize("M,N,K", [(50, 890, 4864), (90, 17, 8192), (200, 890, 4864), (500, 300, 2048), (130, 3590, 1024), (300, 1000, 8192)])
+def test_parts_and_tiles_in_runs(lib, orc, fmt, M, N, K):
+    """Tiles that are no multiple of 8, fewer than 8 and several row blocks, times K-split parts: every part of every tile once."""
+    test_plain_and_parts(lib, orc, fmt, M, N, K)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "q4"])
 @pytest.mark.parametrize("M,ff,K", [(1, 8, 128), (5, 4864, 896), (16, 100, 128), (33, 31, 256), (77, 4864, 896), (81, 200, 384), (128, 17, 128), (300, 200, 896), (16, 40, 4864), (40, 72, 4864),
                                     (150, 4864, 896), (200, 25, 1024)])
 def test_gated(lib, orc, fmt, M, ff, K):
