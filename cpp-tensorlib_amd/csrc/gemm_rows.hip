@@ -58,6 +58,13 @@ __host__ __device__ constexpr int lds_bytes_bf16(int TM, int TN) {
   const int ring = ring_bf16(TM, TN, weight_steps(TM, TN)), sums = sums_bf16(TM, TN);
   return ring > sums ? ring : sums;
 }
+// Blocks that fit a CU: by their registers, as the compiler reports them (two wavefronts a SIMD each), and by the LDS above, of which
+// a CU has 160 KB. The plan prices rounds of blocks by it.
+constexpr int blocks_a_cu(int TM, int TN) {
+  constexpr int by_registers[kMaxTM][4] = {{4, 4, 4, 2}, {4, 3, 2, 2}, {3, 2, 2, 1}, {3, 3, 1, 1}, {2, 2, 1, 1}};
+  const int by_lds = 160 * 1024 / lds_bytes_bf16(TM, TN), by_reg = by_registers[TM - 1][TN - 1];
+  return by_lds < by_reg ? by_lds : by_reg;
+}
 
 // 8 floats -> their three bf16 terms (by truncation: x = hi + mid + lo exactly for normal x)
 __device__ __forceinline__ void split3(const f32x4& x0, const f32x4& x1, frag16 p[3]) {
@@ -685,18 +692,22 @@ static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t m
 // CUs are idle; blocks that share a CU cost half again each, more where their steps are many. Fitted up to 128 rows to 25000
 // runs in the chains allowed (2 to 128 rows, 256 to 16000 columns, K 256 to 18944: error 8 %, the shape it chooses 1.1 % slower than the
 // fastest one on average), above to 13980 others (12800 runs of 129 to 1024 rows take 1.1 times as much, error 9 %, the shape 1.1 %).
+// Since weights are copied into LDS a CU takes other numbers of blocks than those runs had. With them the shape is 1.2 % slower than the
+// fastest of up to twelve over 900 products to 128 rows and 1.7 % over 400 above (1.4 and 2.1 % by the earlier numbers; all constants fitted
+// anew 1.5 and 1.4 %, but longer chains), constants as they were but for the price of sums above 128 rows (0.144; 129 x 3085 gated x 1056
+// takes 12.8 us by 194 blocks and 12.7 by 387). Of 11000 drawn products of 2 to 1024 rows 3 % are run another way for them; 150 of those
+// take 0.71 to 1.19 of their time, 0.942 on average (86 x 5216 gated x 416 8.2 -> 6.8 us, 131 x 21064 gated x 352 34.8 -> 28.2, 43 x 39656 x 6080
+// 133 -> 150, 87 x 34840 x 2560, which was in tiles, 72 -> 86).
 // Measured, us, tiles -> this kernel: 896 x 896 at 37 / 77 / 512 rows 10.3 / 20.9 / 21.7 -> 3.8 / 4.4 / 7.7; 4864 x 896 gated at 37 / 77 / 256
 // 15.0 / 25.2 / 28.3 -> 8.3 / 10.7 / 24.4; 896 x 4864 at 37 / 77 / 150 10.9 / 21.4 / 22.5 -> 6.5 / 8.7 / 10.6; 1152 x 896 at 77 / 300 20.9 / 21.4 -> 5.1 / 7.3;
 // 18944 x 3584 gated at 37 / 64 104 / 105 -> 73 / 89.
 static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
-  // blocks of [row tiles][column tiles] that fit a CU (registers, LDS)
-  static constexpr int kFit[5][4] = {{4, 3, 2, 2}, {4, 2, 2, 1}, {3, 2, 1, 1}, {2, 2, 1, 1}, {2, 1, 1, 1}};
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   RowsPlan best;
   const int64_t rows_w = (gu ? 2 : 1) * N, cus = cu_count(), units = K / rows::kStep, t16 = cdiv(M, 16);
   struct Cost { double start, share, share_n, steps, fill, whole, rows, cols, idle, sums, dispatch, parts, weights, all; };
   static constexpr Cost kFew = {2.33, 0.40, 0.35, 20, 0.77, 0, 0.229, 0.184, 0.827, 0.165, 0.317, 0, 0.051, 1};
-  static constexpr Cost kMany = {2.08, 0.424, 0.593, 10, 0.86, 0.086, 0.194, 0.182, 0.877, 0.144, 0, 0.179, 0.103, 1.1};
+  static constexpr Cost kMany = {2.08, 0.424, 0.593, 10, 0.86, 0.086, 0.194, 0.182, 0.877, 0.14, 0, 0.179, 0.103, 1.106};
   const Cost& k = M > 128 ? kMany : kFew;
   // What adds the parts up beside reading them: a launch, or where a narrow product is left as parts their consumer. (Both
   // forms of a narrow product take one plan: two products of this kernel with room for as many parts are the same bits.)
@@ -710,7 +721,7 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
   for (int64_t row_blocks = few; row_blocks <= std::min(few + 1, t16); row_blocks++)
     for (int TN = 4; TN >= (gu ? 2 : 1); TN--) {
       const int TM = (int)cdiv(t16, row_blocks);
-      const int64_t tiles = cdiv(rows_w, 16 * TN), fit = kFit[TM - 1][TN - 1], at_once = fit * cus;
+      const int64_t tiles = cdiv(rows_w, 16 * TN), fit = rows::blocks_a_cu(TM, TN), at_once = fit * cus;
       if (row_blocks > few && t16 <= 4 && tiles * few > cus / 2) continue;   // (weights read twice for CUs that are busy anyway)
       const int64_t unsplit = tiles * row_blocks;
       // (K is split no further than keeps every CU busy)

@@ -107,6 +107,17 @@ def test_the_faster_kernel_is_chosen(plans, M, N, K, gated, parts, tiles, rows):
     assert plans.plan_gemm_bf16(M, N, K, gated, parts)[0] == (rows < tiles)
 
 
+# M, N, K, gated, room for parts; row and column tiles of a block, us measured with them and with the tiles that an estimate took which
+# had other numbers of blocks on a CU than the kernel's LDS allows
+TILES = [(86, 5216, 416, True, 0, 2, 4, 6.75, 8.21), (24, 13272, 320, True, 0, 2, 4, 6.58, 8.00), (178, 2976, 256, False, 0, 3, 3, 4.28, 5.10),
+         (142, 18080, 352, True, 0, 3, 3, 22.9, 27.9), (186, 8988, 352, False, 0, 3, 3, 9.30, 11.4), (18, 38236, 384, True, 0, 2, 4, 16.2, 20.4)]
+
+
+@pytest.mark.parametrize("M,N,K,gated,parts,TM,TN,us,other", TILES)
+def test_blocks_on_a_cu_are_those_its_lds_takes(plans, M, N, K, gated, parts, TM, TN, us, other):
+    assert us < other and plans.plan_gemm_bf16(M, N, K, gated, parts)[:3] == (1, TM, TN)
+
+
 @pytest.mark.parametrize("M,N,K", [(129, 999, 8192), (200, 1151, 4864), (150, 3585, 3584), (1000, 301, 12288)])
 def test_a_k_that_cannot_be_split_has_no_longer_chains_above_128_rows(plans, M, N, K):
     """The tiles cannot split it either: theirs would be all of K (129 x 999 x 8192 369 us, 26 here)."""
