@@ -175,6 +175,40 @@ def test_attn_decode_device_position(lib, orc, D, Hq, Hkv, kv_max):
         b.free()
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,kv_max", [(128, 28, 4, 4352), (128, 28, 4, 1500), (128, 24, 8, 6153), (64, 56, 2, 8192), (64, 14, 2, 8192), (64, 14, 2, 700),
+                                             (128, 28, 4, 500)])
+def test_merge_error_of_many_splits(lib, D, Hq, Hkv, kv_max):
+    """Splits are added up in pairs of pairs and then over 1024 / D groups: over the partials that a launch leaves, the merge's rounding
+    error is no larger than that order's. A query of zeros makes every weight 1 and every sum a count, so nothing else rounds."""
+    print("case merge error", D, Hq, Hkv, kv_max, flush=True)
+    rng = np.random.default_rng(11)
+    q = np.zeros((Hq, D), np.float32)
+    K, V = (rng.standard_normal((Hkv, kv_max, D)).astype(np.float32) for _ in range(2))
+    dq, dk, dv, do = lib.to_device(q), lib.to_device(K), lib.to_device(V), lib.empty((Hq, D))
+    nb = lib.attn_partials_bytes(Hq, Hkv, kv_max, D) // 4 * 4
+    part, dpos = lib.to_device(np.full(nb // 4, np.nan, np.float32)), lib.to_device(np.array([kv_max - 1], np.uint32))
+    lib.attn_decode_dpos(dq, dk, dv, do, Hq, Hkv, dpos, kv_max, D, 1.0, part)
+    got, p = do.numpy(), part.numpy()
+    S = int(np.argmax(p != 0)) // Hq                    # (the maxima, all zero, lie ahead of the sums)
+    assert 1 < S <= 8 * (1024 // D)
+    l, acc = p[Hq * S:2 * Hq * S].reshape(Hq, S), p[2 * Hq * S:Hq * S * (2 + D)].reshape(Hq, S, D)
+    assert np.all(l.sum(1) == kv_max)
+    a = np.zeros((Hq, 8 * (1024 // D), D), np.float32)
+    a[:, :S] = acc
+    a = a.reshape(Hq, 8, 1024 // D, D)
+    b = [a[:, i] + a[:, i + 4] for i in range(4)]
+    b = (b[0] + b[1]) + (b[2] + b[3])
+    t = b[:, 0]
+    for k in range(1, 1024 // D):
+        t = t + b[:, k]
+    want = acc.astype(np.float64).sum(1) / kv_max
+    err = lambda x: np.sqrt(np.mean((x.astype(np.float64) - want) ** 2))
+    print(S, "splits: error", err(got), "pairs", err(t / np.float32(kv_max)), flush=True)
+    assert err(got) <= 1.01 * err(t / np.float32(kv_max))
+    for x in (dq, dk, dv, do, part, dpos):
+        x.free()
+
+
 def test_attn_full_size_properties(lib, orc):
     """BASELINE config 3 at its largest context (ctx 32768, 0.94 GB of f32 K/V) through
     properties that need no oracle run: constant keys make the output the plain mean of V
