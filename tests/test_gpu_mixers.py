@@ -157,6 +157,25 @@ def test_window_chunks_deep_in_a_context(lib, capi, H, G):
     close(outs[1], outs[0], 2e-4)
 
 
+@pytest.mark.parametrize("window,rows", [(5, 32), (33, 96), (90, 96), (700, 1056), (2100, 2144)])
+def test_window_ring_far_into_a_sequence(lib, capi, window, rows):
+    """Ring rows at positions up to the largest that a step takes: tokens whose whole window was fed there come out as at the start of a
+    sequence (no temperature, so that only distances count); rings of a power of two and of other lengths."""
+    H, G, dim, n = 2, 1, 32, 4
+    T = window + n
+    for base in (999999937, 3 * 2 ** 28 + 11, 2 ** 30 - T + 1):
+        print("case ring far", window, rows, base, flush=True)
+        w = Window(lib, capi, H, G, dim, window, chunk=rows - window + 1, coef=0.0)
+        assert w.at.ring_rows == rows
+        u = w.rows(T, window, amp=2.0)
+        want = w.want(u)[window - 1:]
+        got = np.stack([w.step(u[t], base + t) for t in range(T)])[window - 1:]
+        close(got, want)
+        d_pos = lib.to_device(np.array([base + T - 1], np.uint32))
+        assert np.array_equal(w.step(u[T - 1], 0, d_pos), got[-1])
+        d_pos.free()
+
+
 def test_window_long_context_and_splits(lib, capi):
     """A window of several splits: decode at far positions equals the chunk kernel and the plain
     form; the device position gives the host position's bits."""

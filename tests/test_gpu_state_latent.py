@@ -217,6 +217,24 @@ def test_latent_attention_chunks_and_steps(lib, capi, H, D, R, V, L, planes, tol
     close(np.concatenate([a.run(v[:2], r[:2], 0), a.run(v[2:3], r[2:3], 2), a.run(v[3:], r[3:], 3)]), a.want(v, r), 2 * tol)
 
 
+@pytest.mark.parametrize("planes,tol", PLANES)
+@pytest.mark.parametrize("H,D,R,V,L", [(2, 128, 8, 16, 64), (2, 130, 4, 24, 200), (3, 300, 6, 16, 72), (1, 1024, 2, 8, 40)])
+def test_wide_latent_queries_token_by_token(lib, capi, H, D, R, V, L, planes, tol):
+    """Query dims past the 128 whose weights are asked for ahead, and past the 256 that the block's threads hold; the device position
+    gives the host position's bits."""
+    print("case latent wide", H, D, R, V, L, planes, flush=True)
+    T = 40
+    a = Latent(lib, capi, H, D, R, V, L, 64, planes, seed=D)
+    u, q = a.rows(T, D + 1)
+    want = a.want(u, q)
+    steps = np.concatenate([a.run(u[t:t + 1], q[t:t + 1], t) for t in range(T)])
+    close(steps, want, tol)
+    d_pos = lib.to_device(np.array([T - 1], np.uint32))
+    assert np.array_equal(a.run(u[T - 1:], q[T - 1:], T - 1, d_pos)[0], steps[T - 1])
+    d_pos.free()
+    close(a.run(u, q, 0), want, tol)
+
+
 @pytest.mark.parametrize("planes", [3, 1])
 @pytest.mark.parametrize("H", [1, 3, 40])
 def test_single_keys_show(lib, capi, H, planes):
