@@ -132,10 +132,11 @@ __global__ __launch_bounds__(512) void ssm_step_kernel(const float* __restrict__
 // The same by slices: a block takes 16 of a head's columns (grid: slices, heads), a thread one float4 column of ROWS state rows and of
 // every 128th after those. The step is a chain of round trips, which this is there to shorten: four times the blocks, the sum
 // over the rows across lanes instead of 32 LDS reads in turn (28 heads of 128 x 64: 6.6 us whole, 5.1 in slices). Each slice convolves
-// its group's B and C again. Nothing waits for another load before it is asked for: what the requests need are the 14
-// dwords of arguments that arrive with the block, the state is read in both slots and the convolution's ring (four taps) whole, and
-// the position, which may have to be loaded itself, only picks among what came (TAPS4 false: other taps wait for it).
-// (28 heads of 128 x 64, a small Girirax turn of six such layers: 7263 -> 7174 us.)
+// its group's B and C again. What the first requests need are the 14 dwords of arguments that arrive with the block: the convolution's
+// ring (four taps) is read whole, and the position, which may have to be loaded itself, only picks among what came (TAPS4 false: other taps
+// wait for it). The state is asked for next, in the position's slot. (Both slots ahead of the position were more traffic than they
+// saved: 28, 64 and 112 heads of 128 x 64 in a turn's trace 3.63, 5.76 and 7.0 us, so 3.42, 5.1 and 5.49; the kernel for whole heads or
+// slices before this one 5.05, 5.35 and 6.38.)
 // dims = state rows | taps << 10 | heads << 17, vper = head size | heads per group << 16; inv: ceil(2^32 / heads per group), 0 for one.
 struct SsmRest {
   const float *conv_b, *dt_bias, *decay, *skip;
@@ -159,12 +160,7 @@ __global__ __launch_bounds__(512) void ssm_step_sliced_kernel(const float* __res
   const size_t slot = (size_t)H * N * V;
   const uint32_t at = (uint32_t)h * (uint32_t)(N * V) + col0 + 4 * v4;       // (a head's rows: below 2^32 floats by the sizes taken)
   const auto channel = [&](int i) { return i < 16 ? h * V + col0 + i : i - 16 < N ? inner + g * N + i - 16 : inner + (G + g) * N + i - 16 - N; };
-  f32x4 st[2][ROWS];
-#pragma unroll
-  for (int i = 0; i < ROWS; i++)
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-      st[k][i] = *reinterpret_cast<const f32x4*>(state + k * slot + at + (size_t)min(row0 + 128 * i, N - 1) * V);
+  const int p = d_pos ? (int)*d_pos : a.pos;
   const int c0 = channel(min(tid, chans - 1));
   float now = u[x_off + c0], x[4], f[4];
   if constexpr (TAPS4) {
@@ -175,9 +171,12 @@ __global__ __launch_bounds__(512) void ssm_step_sliced_kernel(const float* __res
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  const float* src = state + (size_t)(p & 1) * slot + at;
+  f32x4 st[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; i++) st[i] = *reinterpret_cast<const f32x4*>(src + (size_t)min(row0 + 128 * i, N - 1) * V);
   const float bias0 = a.conv_b[c0], z = u[a.z_off + h * V + col0 + (tid & 15)];
   const float dt = softplus_f(u[a.dt_off + h] + a.dt_bias[h]), w = exp2f(a.decay[h] * dt), skip = a.skip[h];
-  const int p = d_pos ? (int)*d_pos : a.pos;
   // sum over the taps of channel c for the token at position p; `now` is the token's own input
   const auto conv4 = [&](const float r[4], const float f[4], float now, float bias) {
     float q[4] = {r[0], r[1], r[2], r[3]};           // the ring from slot (p + 1) % 4 on: positions p - 3, p - 2, p - 1
@@ -234,9 +233,9 @@ __global__ __launch_bounds__(512) void ssm_step_sliced_kernel(const float* __res
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < ROWS; i++)
-    if (row0 + 128 * i < N) row(row0 + 128 * i, p > 0 ? ((p & 1) ? st[1][i] : st[0][i]) : zero);
+    if (row0 + 128 * i < N) row(row0 + 128 * i, p > 0 ? st[i] : zero);
   for (int n = row0 + 128 * ROWS; n < N; n += 128)
-    row(n, p > 0 ? *reinterpret_cast<const f32x4*>(state + (size_t)(p & 1) * slot + at + (size_t)n * V) : zero);
+    row(n, p > 0 ? *reinterpret_cast<const f32x4*>(src + (size_t)n * V) : zero);
 #pragma unroll
   for (int e = 0; e < 4; e++) {        // over the lanes of one column: 32, 16, 8 and 4 apart
     LanePair t = swap32(o[e], o[e]);
