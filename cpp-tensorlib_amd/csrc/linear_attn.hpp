@@ -37,8 +37,9 @@ __device__ __forceinline__ float decay_logit(const tlhip_linear_attn& a, const f
 __host__ __device__ inline int64_t linear_state_ld(int64_t vdim) { return (vdim + 3) & ~(int64_t)3; }
 
 // Decode step of head h, one block of 512 threads. The state is read from the slot of `pos` and
-// written to the other one; a thread owns one float4 column of every ng-th row. Of its first rows both slots are asked for: the
-// position may be on the device, and what depends on it would be asked for a round trip later.
+// written to the other one; a thread owns one float4 column of every ng-th row. (Both slots of a thread's first rows, asked for ahead of a
+// position that may be on the device, were more traffic than they saved: the mixers of 7, 16 and 28 heads of 64 x 128 in a turn's trace 5.06,
+// 5.14 and 5.12 us, so 4.65, 5.05 and 4.98.)
 __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, const float* __restrict__ u,
                                                   float* __restrict__ y, int pos, int h, float* smem) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -52,14 +53,12 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
   float* red = vs + ld + ((4 - (3 * dim + ld) % 4) & 3);   // [ng][ld], 16-byte aligned
   float* sums = red + 2048;       // [8]
   const size_t slot = (size_t)a.heads * dim * ld;
-  const float* both = static_cast<const float*>(a.state) + (size_t)h * dim * ld;
+  const float* src = static_cast<const float*>(a.state) + (size_t)(pos & 1) * slot + (size_t)h * dim * ld;
+  float* dst = static_cast<float*>(a.state) + (size_t)((pos + 1) & 1) * slot + (size_t)h * dim * ld;
   constexpr int PRE = 4;          // rows of this thread requested up front
-  float4 st[2][PRE];
+  float4 st[PRE];
 #pragma unroll
-  for (int i = 0; i < PRE; i++)
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-      st[k][i] = *reinterpret_cast<const float4*>(both + k * slot + (size_t)min(dg + i * ng, dim - 1) * ld + 4 * v4);
+  for (int i = 0; i < PRE; i++) st[i] = *reinterpret_cast<const float4*>(src + (size_t)min(dg + i * ng, dim - 1) * ld + 4 * v4);
   const int64_t ch0 = (int64_t)h * vdim + min(tid, vdim - 1);
   const float gate0 = u[a.gate_off + ch0], norm0 = static_cast<const float*>(a.norm)[min(tid, vdim - 1)];   // of what this thread writes first
   for (int d = tid; d < dim; d += 512) {
@@ -71,8 +70,6 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
   }
   for (int v = tid; v < ld; v += 512) vs[v] = v < vdim ? u[a.v_off + (int64_t)h * vdim + v] : 0.f;
   __syncthreads();
-  const float* src = both + (size_t)(pos & 1) * slot;
-  float* dst = static_cast<float*>(a.state) + (size_t)((pos + 1) & 1) * slot + (size_t)h * dim * ld;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   if (live) {
     const float v0 = vs[4 * v4], v1 = vs[4 * v4 + 1], v2 = vs[4 * v4 + 2], v3 = vs[4 * v4 + 3];
@@ -84,7 +81,7 @@ __device__ __forceinline__ void linear_step_block(const tlhip_linear_attn& a, co
     };
 #pragma unroll
     for (int i = 0; i < PRE; i++)
-      if (dg + i * ng < dim) row(dg + i * ng, pos > 0 ? ((pos & 1) ? st[1][i] : st[0][i]) : make_float4(0.f, 0.f, 0.f, 0.f));
+      if (dg + i * ng < dim) row(dg + i * ng, pos > 0 ? st[i] : make_float4(0.f, 0.f, 0.f, 0.f));
     for (int d = dg + PRE * ng; d < dim; d += ng)
       row(d, pos > 0 ? *reinterpret_cast<const float4*>(src + (size_t)d * ld + 4 * v4) : make_float4(0.f, 0.f, 0.f, 0.f));
     *reinterpret_cast<float4*>(red + dg * ld + 4 * v4) = o;
