@@ -627,12 +627,9 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
   }
 }
 
-// grid = Hq, block = 1024: merge the S split partials of one head. The threads are D
-// columns x (1024/D) split groups. The kernel is a chain of memory latencies and little
-// else, so with up to 8 splits per group (S <= 64 at D = 128) every load - the partial
-// maxima and sums and the thread's own accumulator values - is requested at the top and
-// waited for once; the split weights exp(m_s - M) are formed once per split in LDS, each
-// thread sums its splits in a fixed order and the groups are summed in a fixed order.
+// Merge of any number of split partials of a head (more than the 128 that the kernel above takes: a long context of few kv heads):
+// grid = heads, block = 1024, D columns x 1024 / D split groups. The splits' weights are formed once in LDS, each thread sums its
+// splits in a fixed order, and the groups are summed in a fixed order.
 __global__ __launch_bounds__(1024) void attn_combine_kernel(const float* __restrict__ part_m,
                                                             const float* __restrict__ part_l,
                                                             const float* __restrict__ part_acc,
@@ -640,25 +637,13 @@ __global__ __launch_bounds__(1024) void attn_combine_kernel(const float* __restr
   extern __shared__ float sm[];   // f[S] | red[1024]
   float* f = sm;
   float* red = sm + S;
-  constexpr int kUp = 8;          // accumulator loads a thread issues up front
   const int h = blockIdx.x, tid = threadIdx.x;
   const float* pm = part_m + (size_t)h * S;
   const float* pl = part_l + (size_t)h * S;
   const int groups = 1024 / D, d = tid % D, sg = tid / D;
   const float* pa = part_acc + (size_t)h * S * D + d;
-  const bool upfront = S <= kUp * groups;        // (then S <= 1024 as well)
-  float pv[kUp], my_m = -INFINITY, my_l = 0.f;
-  if (upfront) {
-#pragma unroll
-    for (int u = 0; u < kUp; u++) {
-      const int s = sg + u * groups;
-      pv[u] = s < S ? pa[(size_t)s * D] : 0.f;
-    }
-    if (tid < S) { my_m = pm[tid]; my_l = pl[tid]; }
-  }
-  float mx = my_m;
-  if (!upfront)
-    for (int s = tid; s < S; s += 1024) mx = fmaxf(mx, pm[s]);
+  float mx = -INFINITY;
+  for (int s = tid; s < S; s += 1024) mx = fmaxf(mx, pm[s]);
   mx = wave_max(mx);
   if ((tid & 63) == 0) red[tid >> 6] = mx;
   __syncthreads();
@@ -667,18 +652,10 @@ __global__ __launch_bounds__(1024) void attn_combine_kernel(const float* __restr
   for (int w = 1; w < 16; w++) M = fmaxf(M, red[w]);
   __syncthreads();
   float lsum = 0.f;
-  if (upfront) {
-    if (tid < S) {
-      const float w = __expf(my_m - M);
-      f[tid] = w;
-      lsum = my_l * w;
-    }
-  } else {
-    for (int s = tid; s < S; s += 1024) {
-      const float w = __expf(pm[s] - M);
-      f[s] = w;
-      lsum = fmaf(pl[s], w, lsum);
-    }
+  for (int s = tid; s < S; s += 1024) {
+    const float w = __expf(pm[s] - M);
+    f[s] = w;
+    lsum = fmaf(pl[s], w, lsum);
   }
   lsum = wave_sum(lsum);
   if ((tid & 63) == 0) red[tid >> 6] = lsum;
@@ -688,27 +665,16 @@ __global__ __launch_bounds__(1024) void attn_combine_kernel(const float* __restr
   for (int w = 1; w < 16; w++) L += red[w];
   __syncthreads();
   float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-  if (upfront) {
-#pragma unroll
-    for (int u = 0; u < kUp; u += 4) {
-      const int s = sg + u * groups;
-      a0 = fmaf(s < S ? f[s] : 0.f, pv[u], a0);
-      a1 = fmaf(s + groups < S ? f[s + groups] : 0.f, pv[u + 1], a1);
-      a2 = fmaf(s + 2 * groups < S ? f[s + 2 * groups] : 0.f, pv[u + 2], a2);
-      a3 = fmaf(s + 3 * groups < S ? f[s + 3 * groups] : 0.f, pv[u + 3], a3);
-    }
-  } else {
-    int s = sg;
-    for (; s + 3 * groups < S; s += 4 * groups) {
-      const float v0 = pa[(size_t)s * D], v1 = pa[(size_t)(s + groups) * D],
-                  v2 = pa[(size_t)(s + 2 * groups) * D], v3 = pa[(size_t)(s + 3 * groups) * D];
-      a0 = fmaf(f[s], v0, a0);
-      a1 = fmaf(f[s + groups], v1, a1);
-      a2 = fmaf(f[s + 2 * groups], v2, a2);
-      a3 = fmaf(f[s + 3 * groups], v3, a3);
-    }
-    for (; s < S; s += groups) a0 = fmaf(f[s], pa[(size_t)s * D], a0);
+  int s = sg;
+  for (; s + 3 * groups < S; s += 4 * groups) {
+    const float v0 = pa[(size_t)s * D], v1 = pa[(size_t)(s + groups) * D],
+                v2 = pa[(size_t)(s + 2 * groups) * D], v3 = pa[(size_t)(s + 3 * groups) * D];
+    a0 = fmaf(f[s], v0, a0);
+    a1 = fmaf(f[s + groups], v1, a1);
+    a2 = fmaf(f[s + 2 * groups], v2, a2);
+    a3 = fmaf(f[s + 3 * groups], v3, a3);
   }
+  for (; s < S; s += groups) a0 = fmaf(f[s], pa[(size_t)s * D], a0);
   red[tid] = (a0 + a1) + (a2 + a3);
   __syncthreads();
   if (sg == 0) {
@@ -750,7 +716,7 @@ __global__ __launch_bounds__(1024) void attn_combine_kernel(const float* __restr
 // copies the next tile into a second LDS stage while it works on the current one. The deal does
 // not depend on the live context, so a grid planned for the cache capacity (position on the
 // device) and one planned for the live context give the same bits: splits without keys write
-// neutral partials, which add exact zeros in the combine.
+// neutral partials, which add exact zeros in the merge.
 // QKV: as in the kernel above, the raw [q | k | v] projection comes in; the block's query rows get
 // their bias and rotation on the way into LDS, and the block whose tile holds the step's position
 // forms the new key/value row (same arithmetic as the stand-alone epilogue, so cache rows are
@@ -1044,7 +1010,7 @@ __global__ __launch_bounds__(64 * (GRP + 1)) void attn_gqa_kernel(
     if (lane < CH) {
       const size_t head = (size_t)kvh * GRP + h;
       if (S == 1 && out) {
-        // (divisions, as in the combine kernel: a grid with one split and one with more give the same bits)
+        // (divisions, as in the merge kernel: a grid with one split and one with more give the same bits)
         *reinterpret_cast<float4*>(out + head * D + lane * 4) = make_float4(acc.x / l, acc.y / l, acc.z / l, acc.w / l);
       } else {
         const size_t ps = head * S + split;
@@ -1134,8 +1100,8 @@ template <typename KT> static bool gqa_applies(int group) { return false; }
 template <> bool gqa_applies<float>(int group) { return group >= 3 && group <= 8; }
 
 // Splits: one tile each while there are CUs for them (a block per CU and kv head), never more
-// than the combine kernel sums in one pass (8 per column group; beyond that its summation order
-// would depend on the count). stages: 2 when a split holds more than one tile.
+// than eight for each of the merge's 1024 / D groups: 64 at head size 128, 128 at 64, whose sums have one order for every number
+// of splits (the kernel for more has an order that depends on it). stages: 2 when a split holds more than one tile.
 struct GqaPlan { int S, stages; };
 static GqaPlan plan_gqa(int Hkv, int ctx, int cus, int D) {
   const int tiles = (ctx + gqa::kKeys - 1) / gqa::kKeys;

@@ -164,10 +164,9 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// a / n and a % n for 0 <= a < 2^20, n > 0, by a reciprocal that is off by an ulp (a / n + 1 / 2n is never that close to a whole
+// a / n for 0 <= a < 2^20, n > 0, by a reciprocal that is off by an ulp (a / n + 1 / 2n is never that close to a whole
 // number): six instructions where the compiler's division is a chain of thirty, at the head of kernels that wait for its result.
 __device__ __forceinline__ int small_div(int a, int n) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)n)); }
-__device__ __forceinline__ int small_mod(int a, int n) { return a - small_div(a, n) * n; }
 
 // Where a block of a product works: tile `tile` of nb, K-split part `part`. The hardware deals blocks round-robin to the 8 XCDs,
 // x fastest; each XCD, which has an L2 of its own, gets one contiguous run of tiles, or with parts > 1 of the pairs (part, tile), fewer

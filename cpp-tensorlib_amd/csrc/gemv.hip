@@ -885,6 +885,7 @@ static int launch_rows(const float* x, const void* W, const float* scales, float
     const uint32_t tiles = (uint32_t)(ntiles / cfg.blocks) | (uint32_t)(ntiles % cfg.blocks) << 19;
     const uint32_t block = (uint32_t)cfg.KW | (uint32_t)cfg.nw << 5 | (uint32_t)cfg.blocks << 10 |
                            (uint32_t)((256 + cfg.KW - 1) / cfg.KW - 1) << 24;
+    static_assert(!Fmt::kScaled || PRO != kPostnorm, "the third argument is an int4 weight's scales or the post-norm's bias");
     const float* third = PRO == kPostnorm ? pro.bias : sn;
     const float* fourth = pro.delta;
     if (PRO == kAttnMerge) fourth = reinterpret_cast<const float*>((uint64_t)pro.S | (uint64_t)pro.heads << 8 | (uint64_t)pro.D << 24);
@@ -990,7 +991,7 @@ static int check_attn_merge(const void* parts, int64_t n_parts, int64_t heads, i
   if (!parts || !aligned16(parts)) return fail(TLHIP_EINVAL, "%s: partials pointer null or not 16-byte aligned", who);
   if (heads <= 0 || heads > 4096 || (D != 64 && D != 128) || heads * D != K)
     return fail(TLHIP_EINVAL, "%s: K must be heads x head_dim, head_dim 64 or 128", who);
-  // as many splits as the merge kernel sums one after the other: one per column group of its 1024 threads
+  // as many splits as the merge kernel has groups, which it sums one after the other
   const int64_t most = D == 64 ? kMergeMax : kMergeMax / 2;
   if (n_parts < 1 || n_parts > most) return fail(TLHIP_EUNSUPPORTED, "%s: 1 to %d split partials", who, (int)most);
   if (((2 * heads * n_parts) % 4) != 0) return fail(TLHIP_EUNSUPPORTED, "%s: heads x splits must be even", who);
