@@ -58,13 +58,18 @@ __host__ __device__ constexpr int lds_bytes_bf16(int TM, int TN) {
   const int ring = ring_bf16(TM, TN, weight_steps(TM, TN)), sums = sums_bf16(TM, TN);
   return ring > sums ? ring : sums;
 }
-// Blocks that fit a CU: by their registers, as the compiler reports them (two wavefronts a SIMD each), and by the LDS above, of which
-// a CU has 160 KB. The plan prices rounds of blocks by it.
-constexpr int blocks_a_cu(int TM, int TN) {
-  constexpr int by_registers[kMaxTM][4] = {{4, 4, 4, 2}, {4, 3, 2, 2}, {3, 2, 2, 1}, {3, 3, 1, 1}, {2, 2, 1, 1}};
-  const int by_lds = 160 * 1024 / lds_bytes_bf16(TM, TN), by_reg = by_registers[TM - 1][TN - 1];
-  return by_lds < by_reg ? by_lds : by_reg;
-}
+// Blocks of [row tiles - 1][column tiles - 1] that fit a CU: by their registers, as the compiler reports them (two wavefronts a SIMD each), and
+// by the LDS above, of which a CU has 160 KB. The plan prices rounds of blocks by it.
+struct BlocksOfACu {
+  int n[kMaxTM][4] = {{4, 4, 4, 2}, {4, 3, 2, 2}, {3, 2, 2, 1}, {3, 3, 1, 1}, {2, 2, 1, 1}};
+  constexpr BlocksOfACu() {
+    for (int TM = 1; TM <= kMaxTM; TM++)
+      for (int TN = 1; TN <= 4; TN++) {
+        const int by_lds = 160 * 1024 / lds_bytes_bf16(TM, TN);
+        if (by_lds < n[TM - 1][TN - 1]) n[TM - 1][TN - 1] = by_lds;
+      }
+  }
+};
 
 // 8 floats -> their three bf16 terms (by truncation: x = hi + mid + lo exactly for normal x)
 __device__ __forceinline__ void split3(const f32x4& x0, const f32x4& x1, frag16 p[3]) {
@@ -702,6 +707,7 @@ static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t m
 // 15.0 / 25.2 / 28.3 -> 8.3 / 10.7 / 24.4; 896 x 4864 at 37 / 77 / 150 10.9 / 21.4 / 22.5 -> 6.5 / 8.7 / 10.6; 1152 x 896 at 77 / 300 20.9 / 21.4 -> 5.1 / 7.3;
 // 18944 x 3584 gated at 37 / 64 104 / 105 -> 73 / 89.
 static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t max_S) {
+  static constexpr rows::BlocksOfACu kFit;
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   RowsPlan best;
   const int64_t rows_w = (gu ? 2 : 1) * N, cus = cu_count(), units = K / rows::kStep, t16 = cdiv(M, 16);
@@ -721,7 +727,7 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
   for (int64_t row_blocks = few; row_blocks <= std::min(few + 1, t16); row_blocks++)
     for (int TN = 4; TN >= (gu ? 2 : 1); TN--) {
       const int TM = (int)cdiv(t16, row_blocks);
-      const int64_t tiles = cdiv(rows_w, 16 * TN), fit = rows::blocks_a_cu(TM, TN), at_once = fit * cus;
+      const int64_t tiles = cdiv(rows_w, 16 * TN), fit = kFit.n[TM - 1][TN - 1], at_once = fit * cus;
       if (row_blocks > few && t16 <= 4 && tiles * few > cus / 2) continue;   // (weights read twice for CUs that are busy anyway)
       const int64_t unsplit = tiles * row_blocks;
       // (K is split no further than keeps every CU busy)
