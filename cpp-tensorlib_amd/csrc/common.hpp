@@ -169,12 +169,13 @@ __device__ __forceinline__ float wave_max(float v) {
 __device__ __forceinline__ int small_div(int a, int n) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)n)); }
 
 // Where a block of a product works: tile `tile` of nb, K-split part `part`. The hardware deals blocks round-robin to the 8 XCDs,
-// x fastest; each XCD, which has an L2 of its own, gets one contiguous run of tiles, or with parts > 1 of the pairs (part, tile), fewer
-// than 2^20, so that it reads a few parts of the activations whole instead of some of all: the tiles of a part that lie
-// apart in x by a multiple of 8 would otherwise meet on an XCD only where nb is one too.
+// x fastest; each XCD, which has an L2 of its own, gets one contiguous run of tiles, or with parts > 1 (at most 16) of the pairs (part,
+// tile), so that it reads a few parts of the activations whole instead of some of all: the tiles of a part that lie
+// apart in x by a multiple of 8 would otherwise meet on an XCD only where nb is one too. From 65536 tiles on the pairs would pass what
+// small_div is exact for: the part is the grid's y there.
 struct BlockPlace { int tile, part; };
 __device__ __forceinline__ BlockPlace block_place(int nb, int parts) {
-  const bool pairs = parts > 1;
+  const bool pairs = parts > 1 && nb < (1 << 16);
   const int all = pairs ? nb * parts : nb, at = blockIdx.x + (pairs ? blockIdx.y * nb : 0), xcd = at & 7, within = at >> 3;
   const int i = xcd * (all >> 3) + min(xcd, all & 7) + within, part = pairs ? small_div(i, nb) : blockIdx.y;
   return BlockPlace{pairs ? i - part * nb : i, part};
