@@ -26,7 +26,9 @@
 // activations of zeros, the same instructions, 512 x 3584 x 18944 in four parts takes 116 us where it took 157 over random ones, and five
 // stages of 128 rows or copies spread evenly over a slab changed nothing. So the products are 16 x 16 x 32: 32 x 32 x 16 reads
 // and writes twice the accumulators per product. Measured for it at 512 rows, images included: 3584 x 18944 in parts 158.7 -> 137
-// us, 18944 gated x 3584 262 -> 231, 4608 x 3584 in parts 45.9 -> 43.4; 1024 x 3584 x 3584 76.6 -> 67.6. Products of f16 are exact in fp32, the MFMA sums in fp32, and
+// us, 18944 gated x 3584 262 -> 231, 4608 x 3584 in parts 45.9 -> 43.4; 1024 x 3584 x 3584 76.6 -> 67.6. Errors of whole models by them
+// (eight seeds): 7B prompt of 512 over four layers 1.89e-6 -> 1.86e-6 of the logits, a document of 1001 tokens 1.40e-6 -> 1.37e-6.
+// Products of f16 are exact in fp32, the MFMA sums in fp32, and
 // the result leaves as acc * 2^-(ea[m] + ew[n]), an exact scaling: the error is fp32 summation
 // error plus one fp32-rounding-sized term per product, as in the reference's fp32 FMA loop
 // (tensorlib_cuda.cu:509-519).

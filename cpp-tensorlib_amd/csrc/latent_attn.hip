@@ -387,6 +387,8 @@ __global__ __launch_bounds__(256) void latent_query_mfma_kernel(const float* __r
 // Grid: splits, query tiles (65535 to a z). The arguments up to `rows` arrive with the block (steps = DS | LT << 16, hs = heads |
 // S << 16), and with them alone keys, queries and values of the first pair are asked for: which keys there are is known only when the
 // position, which may be on the device, has come. Until then tiles are bound by the cache; a value tile past the last is taken as zeros.
+// (Splits that hold no key read for nothing: 28 heads of 576 numbers in 64 splits of 4096 positions 7.3 us at position 30 and 8.5 at 2000, 7.8 and
+// 8.8 with everything asked for behind the position; 14 heads of 288 and 16 of 576 at position 30 5.8 and 8.5 us either way.)
 template <int KS, int NL>
 __global__ __launch_bounds__(512) void latent_attend_kernel(const uint16_t* __restrict__ qimg, const void* __restrict__ keys,
                                                             const void* __restrict__ values, const uint32_t* __restrict__ d_pos,
