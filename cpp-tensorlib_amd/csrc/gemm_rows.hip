@@ -698,11 +698,11 @@ static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t m
 // runs in the chains allowed (2 to 128 rows, 256 to 16000 columns, K 256 to 18944: error 8 %, the shape it chooses 1.1 % slower than the
 // fastest one on average), above to 13980 others (12800 runs of 129 to 1024 rows take 1.1 times as much, error 9 %, the shape 1.1 %).
 // Since weights are copied into LDS a CU takes other numbers of blocks than those runs had. With them the shape is 1.2 % slower than the
-// fastest of up to twelve over 900 products to 128 rows and 1.7 % over 400 above (1.4 and 2.1 % by the earlier numbers; all constants fitted
-// anew 1.5 and 1.4 %, but longer chains), constants as they were but for the price of sums above 128 rows (0.144; 129 x 3085 gated x 1056
-// takes 12.8 us by 194 blocks and 12.7 by 387). Of 11000 drawn products of 2 to 1024 rows 3 % are run another way for them; 150 of those
-// take 0.71 to 1.19 of their time, 0.942 on average (86 x 5216 gated x 416 8.2 -> 6.8 us, 131 x 21064 gated x 352 34.8 -> 28.2, 43 x 39656 x 6080
-// 133 -> 150, 87 x 34840 x 2560, which was in tiles, 72 -> 86).
+// fastest of up to twelve over 3000 products to 128 rows and 1.7 % over 400 above (1.4 and 2.1 % by the earlier numbers; all constants fitted
+// anew 1.5 and 1.4 %, or with the sharing alone 0.95 to 128 rows, but longer chains), constants as they were but for the price of sums
+// above 128 rows (0.144 before; 129 x 3085 gated x 1056 takes 12.8 us by 194 blocks and 12.7 by 387). Of drawn products of 2 to 1024 rows
+// 3 % are run another way for them: 150 of those take 0.79 to 1.14 of their time, 0.941 on average, 27 of the models' sizes 0.74 to 1.03,
+// 0.912 (89 x 4608 x 3584 22.8 -> 16.7 us, 89 x 10304 x 2048 24.2 -> 21.0, 131 x 21064 gated x 352 34.8 -> 28.2; 592 x 13304 gated x 352 70 -> 80).
 // Measured, us, tiles -> this kernel: 896 x 896 at 37 / 77 / 512 rows 10.3 / 20.9 / 21.7 -> 3.8 / 4.4 / 7.7; 4864 x 896 gated at 37 / 77 / 256
 // 15.0 / 25.2 / 28.3 -> 8.3 / 10.7 / 24.4; 896 x 4864 at 37 / 77 / 150 10.9 / 21.4 / 22.5 -> 6.5 / 8.7 / 10.6; 1152 x 896 at 77 / 300 20.9 / 21.4 -> 5.1 / 7.3;
 // 18944 x 3584 gated at 37 / 64 104 / 105 -> 73 / 89.
@@ -713,7 +713,7 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
   const int64_t rows_w = (gu ? 2 : 1) * N, cus = cu_count(), units = K / rows::kStep, t16 = cdiv(M, 16);
   struct Cost { double start, share, share_n, steps, fill, whole, rows, cols, idle, sums, dispatch, parts, weights, all; };
   static constexpr Cost kFew = {2.33, 0.40, 0.35, 20, 0.77, 0, 0.229, 0.184, 0.827, 0.165, 0.317, 0, 0.051, 1};
-  static constexpr Cost kMany = {2.08, 0.424, 0.593, 10, 0.86, 0.086, 0.194, 0.182, 0.877, 0.14, 0, 0.179, 0.103, 1.106};
+  static constexpr Cost kMany = {2.08, 0.424, 0.593, 10, 0.86, 0.086, 0.194, 0.182, 0.877, 0.141, 0, 0.179, 0.103, 1.1};
   const Cost& k = M > 128 ? kMany : kFew;
   // What adds the parts up beside reading them: a launch, or where a narrow product is left as parts their consumer. (Both
   // forms of a narrow product take one plan: two products of this kernel with room for as many parts are the same bits.)
@@ -740,7 +740,10 @@ static RowsPlan plan_rows_bf16(int64_t M, int64_t N, int64_t K, bool gu, int64_t
         // gated x 1600, 50 steps, 1.75e-7 of error in 13 parts and 1.51e-7 in 7)
         if (M <= 128 && S > least_S && ((int)units + rows::kWaves * steps - 1) / (rows::kWaves * steps) != S) continue;
         const double n = (double)steps;
-        const auto share = [&](int64_t on_a_cu) { return 1 + (k.share + k.share_n * n / (n + k.steps)) * (double)(on_a_cu - 1); };
+        // (blocks of nine accumulator tiles leave each other less from the start: 41 x 18944 gated x 3584 by two of them on a CU 85 us, 78 by
+        // one of twelve)
+        const Cost& sh = TM * TN > 8 ? kMany : k;
+        const auto share = [&](int64_t on_a_cu) { return 1 + (sh.share + sh.share_n * n / (n + sh.steps)) * (double)(on_a_cu - 1); };
         double rounds = 1;
         if (blocks > cus) {
           const int64_t rest = blocks % at_once;
