@@ -701,7 +701,7 @@ static int64_t longest_chain(int64_t M, int64_t N, int64_t K, bool gu, int64_t m
 // fastest of up to twelve over 3000 products to 128 rows and 1.7 % over 400 above (1.4 and 2.1 % by the earlier numbers; all constants fitted
 // anew 1.5 and 1.4 %, or with the sharing alone 0.95 to 128 rows, but longer chains), constants as they were but for the price of sums
 // above 128 rows (0.144 before; 129 x 3085 gated x 1056 takes 12.8 us by 194 blocks and 12.7 by 387). Of drawn products of 2 to 1024 rows
-// 3 % are run another way for them: 150 of those take 0.79 to 1.14 of their time, 0.941 on average, 27 of the models' sizes 0.74 to 1.03,
+// 3 % are run another way for them: 150 of those take 0.79 to 1.14 of their time, 0.941 on average, 27 of the models' sizes 0.74 to 1.05,
 // 0.912 (89 x 4608 x 3584 22.8 -> 16.7 us, 89 x 10304 x 2048 24.2 -> 21.0, 131 x 21064 gated x 352 34.8 -> 28.2; 592 x 13304 gated x 352 70 -> 80).
 // Measured, us, tiles -> this kernel: 896 x 896 at 37 / 77 / 512 rows 10.3 / 20.9 / 21.7 -> 3.8 / 4.4 / 7.7; 4864 x 896 gated at 37 / 77 / 256
 // 15.0 / 25.2 / 28.3 -> 8.3 / 10.7 / 24.4; 896 x 4864 at 37 / 77 / 150 10.9 / 21.4 / 22.5 -> 6.5 / 8.7 / 10.6; 1152 x 896 at 77 / 300 20.9 / 21.4 -> 5.1 / 7.3;
