@@ -164,15 +164,17 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// a / n for 0 <= a < 2^20, n > 0, by a reciprocal that is off by an ulp (a / n + 1 / 2n is never that close to a whole
-// number): six instructions where the compiler's division is a chain of thirty, at the head of kernels that wait for its result.
+// a / n for 0 <= a < 2^21, n > 0, by a reciprocal that is off by an ulp (a / n + 1 / 2n is never that close to a whole number; every n, with
+// the ends of each quotient's range and reciprocals an ulp off either way, gives the quotient, and from 2^21 + 3582 on some do not): six
+// instructions where the compiler's division is a chain of thirty, at the head of kernels that wait for its result. The largest a
+// is a mixer step's block, 65535 heads in 32 splits.
 __device__ __forceinline__ int small_div(int a, int n) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)n)); }
 
 // Where a block of a product works: tile `tile` of nb, K-split part `part`. The hardware deals blocks round-robin to the 8 XCDs,
 // x fastest; each XCD, which has an L2 of its own, gets one contiguous run of tiles, or with parts > 1 (at most 16) of the pairs (part,
 // tile), so that it reads a few parts of the activations whole instead of some of all: the tiles of a part that lie
-// apart in x by a multiple of 8 would otherwise meet on an XCD only where nb is one too. From 65536 tiles on the pairs would pass what
-// small_div is exact for: the part is the grid's y there.
+// apart in x by a multiple of 8 would otherwise meet on an XCD only where nb is one too. The pairs stay below 2^20, within what
+// small_div is exact for: from 65536 tiles on the part is the grid's y.
 struct BlockPlace { int tile, part; };
 __device__ __forceinline__ BlockPlace block_place(int nb, int parts) {
   const bool pairs = parts > 1 && nb < (1 << 16);
